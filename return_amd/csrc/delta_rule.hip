@@ -18,9 +18,10 @@
 // with DPT rows in registers; the two sums over rows are finished by data-parallel moves. Columns of
 // one head are independent, so a head is spread over V / VB workgroups: the walk over the tokens is the
 // long pole, and it is as long for 16 columns as for 128. The output kernel norms a head's read-out
-// over all its columns, weighs and gates it: a wave per (row, head). Steps whose longest request has eight
-// rows or more take the recurrence kernel with feeder waves (below); single tokens and short portions the plain
-// one, which needs half the threads, few registers and little LDS, so that many workgroups share a CU.
+// over all its columns, weighs and gates it: a wave per (row, head). In bf16 requests of RC_MIN_ROWS rows and
+// more go by chunks on the matrix cores (recurrence_chunks.hip) if a head has at most 128 channels; other requests of eight
+// rows and more take the recurrence kernel with feeder waves (below); single tokens and short portions the plain one, which
+// needs half the threads, few registers and little LDS, so that many workgroups share a CU.
 //
 // A second rule runs on the same kernels (rule 1, "outer"): the gated outer-product memory of a linear attention,
 //     S <- diag(alpha_t) S + k_t v_t^T;   o_t = S^T q_t,    alpha_t[i] = sigmoid(a_t[h,i] + bias[h,i])^rate
@@ -38,6 +39,7 @@
 // head and token, g = exp(-exp(A_log[h]) softplus(a_t[h] + dt_bias[h])), formed once per row by the exact routines,
 // and the output gate silu(c).
 #include "common.h"
+#include "recurrence_chunks.h"
 
 #define DR_TC_MAX 32      // rows of a chunk; fewer where a head's rows would not fit the LDS
 #define DR_PAD 4
@@ -74,14 +76,14 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     const T* __restrict__ qkv, long long ld_qkv, const T* __restrict__ b, long long ld_b, const T* __restrict__ ag,
     long long ld_ag, const float* __restrict__ A_log, const float* __restrict__ dt_bias, float* __restrict__ S,
     const int* __restrict__ cu_q, const int* __restrict__ slot_ids, float* __restrict__ o_raw, int H, int G, int D, int V,
-    int RS, int VB, int TC, int rule, float rate) {
+    int RS, int VB, int TC, int rule, float rate, int below) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wave = tid >> 6, n_waves = NT >> 6;
     const int col_blocks = (V + VB - 1) / VB;
     const int h = blockIdx.x / col_blocks, j0 = (blockIdx.x - h * col_blocks) * VB;
     const int s = blockIdx.y, kvh = h / (H / G);
     const int base = cu_q[s], q_len = cu_q[s + 1] - base;
-    if (q_len <= 0) return;
+    if (q_len <= 0 || q_len >= below) return;       // (requests of `below` rows and more are another kernel's)
     const int PS = DPT + DR_PAD;                    // a lane group's rows in LDS, padded against bank conflicts
     const int DP = RS * PS;
     float* k_s = smem;                              // [TC][DP]
@@ -283,14 +285,14 @@ __global__ __launch_bounds__(DR_WALKERS + DR_FEEDERS) __attribute__((amdgpu_wave
     const T* __restrict__ qkv, long long ld_qkv, const T* __restrict__ b, long long ld_b, const T* __restrict__ ag,
     long long ld_ag, const float* __restrict__ A_log, const float* __restrict__ dt_bias, float* __restrict__ S,
     const int* __restrict__ cu_q, const int* __restrict__ slot_ids, float* __restrict__ o_raw, int H, int G, int D, int V,
-    int RS, int VB, int TC, int rule, float rate) {
+    int RS, int VB, int TC, int rule, float rate, int below) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     const int tid = threadIdx.x, lane = tid & 63;
     const int col_blocks = (V + VB - 1) / VB;
     const int h = blockIdx.x / col_blocks, j0 = (blockIdx.x - h * col_blocks) * VB;
     const int s = blockIdx.y, kvh = h / (H / G);
     const int base = cu_q[s], q_len = cu_q[s + 1] - base;
-    if (q_len <= 0) return;
+    if (q_len <= 0 || q_len >= below) return;       // (requests of `below` rows and more are another kernel's)
     const int PS = DPT + DR_PAD;                    // a lane group's rows in LDS, padded against bank conflicts
     const int DP = RS * PS;
     const int BUF = (TC * (3 * DP + VB) + TC + 3) & ~3;        // floats of one buffer: k, q, g [TC][DP], v [TC][VB], beta [TC]
@@ -544,11 +546,18 @@ extern "C" int ra_delta_rule_fits(int D, int V) {
     return delta_rule_chunk(DPT, RS, VB) > 0 ? 1 : 0;
 }
 
+// Floats of scratch `ws` that the recurrences below want for requests of q_lens rows (host memory; rule as in
+// delta_rule_run). 0: none, ws and q_lens may then be null.
+extern "C" long long ra_recurrence_scratch(const int* q_lens, int n_seqs, int H, int D, int V, int rule) {
+    return recurrence_chunks_workspace(q_lens, n_seqs, H, D, V, rule);
+}
+
 template <typename T>
 static int delta_rule_fed_launch(hipStream_t st, int DPT, dim3 grid, size_t lds, const void* qkv, long long ld_qkv,
                                  const void* b, long long ld_b, const void* ag, long long ld_ag, const float* A_log,
                                  const float* dt_bias, float* S, const int* cu_q, const int* slot_ids, float* o_raw, int H,
-                                 int G, int D, int V, int RS, int VB, int TC, int rule, float rate) {
+                                 int G, int D, int V, int RS, int VB, int TC, int rule, float rate,
+                                 int below) {
 #define DR_FED(DPT_)                                                                                                  \
     do {                                                                                                              \
         if (lds > 64 * 1024 &&                                                                                        \
@@ -557,7 +566,7 @@ static int delta_rule_fed_launch(hipStream_t st, int DPT, dim3 grid, size_t lds,
             return RA_ERR_LAUNCH;                                                                                     \
         hipLaunchKernelGGL((delta_rule_fed_kernel<T, DPT_>), grid, dim3(DR_WALKERS + DR_FEEDERS), lds, st, (const T*)qkv, \
                            ld_qkv, (const T*)b, ld_b, (const T*)ag, ld_ag, A_log, dt_bias, S, cu_q, slot_ids, o_raw, H, G, \
-                           D, V, RS, VB, TC, rule, rate);                                                                       \
+                           D, V, RS, VB, TC, rule, rate, below);                                                      \
     } while (0)
     switch (DPT) {
         case 4: DR_FED(4); break;
@@ -575,7 +584,7 @@ template <typename T>
 static int delta_rule_launch(hipStream_t st, int DPT, dim3 grid, dim3 block, size_t lds, const void* qkv, long long ld_qkv,
                              const void* b, long long ld_b, const void* ag, long long ld_ag, const float* A_log,
                              const float* dt_bias, float* S, const int* cu_q, const int* slot_ids, float* o_raw, int H, int G,
-                             int D, int V, int RS, int VB, int TC, int rule, float rate) {
+                             int D, int V, int RS, int VB, int TC, int rule, float rate, int below) {
 #define DR_GO(DPT_)                                                                                               \
     do {                                                                                                          \
         if (lds > 64 * 1024 &&                                                                                    \
@@ -583,7 +592,8 @@ static int delta_rule_launch(hipStream_t st, int DPT, dim3 grid, dim3 block, siz
                                 (int)lds) != hipSuccess)                                                          \
             return RA_ERR_LAUNCH;                                                                                 \
         hipLaunchKernelGGL((delta_rule_kernel<T, DPT_>), grid, block, lds, st, (const T*)qkv, ld_qkv, (const T*)b, ld_b, \
-                           (const T*)ag, ld_ag, A_log, dt_bias, S, cu_q, slot_ids, o_raw, H, G, D, V, RS, VB, TC, rule, rate); \
+                           (const T*)ag, ld_ag, A_log, dt_bias, S, cu_q, slot_ids, o_raw, H, G, D, V, RS, VB, TC, rule, rate, \
+                           below);                                                                                \
     } while (0)
     switch (DPT) {
         case 4: DR_GO(4); break;
@@ -604,8 +614,8 @@ static int delta_rule_launch(hipStream_t st, int DPT, dim3 grid, dim3 block, siz
 static int delta_rule_run(const void* qkv, long long ld_qkv, const void* b, long long ld_b, const void* ag,
                           long long ld_ag, const void* gate, long long ld_gate, const float* A_log, const float* dt_bias,
                           const float* norm_w, float eps, float* S, const int* cu_q, const int* slot_ids, float* o_raw,
-                          void* out, int n_seqs, int T_tokens, int max_q_len, int H, int G, int D, int V, int rule,
-                          float rate, int dtype, void* stream) {
+                          void* out, int n_seqs, int T_tokens, int max_q_len, const int* q_lens, float* ws,
+                          long long ws_floats, int H, int G, int D, int V, int rule, float rate, int dtype, void* stream) {
     if (n_seqs <= 0 || T_tokens <= 0) return RA_OK;
     int RS, DPT, VB;
     if (!delta_rule_plan(D, V, &RS, &DPT, &VB) || H < 1 || G < 1 || H % G || n_seqs > 65535) return RA_ERR_ARG;
@@ -615,6 +625,23 @@ static int delta_rule_run(const void* qkv, long long ld_qkv, const void* b, long
     if (dtype != RA_DTYPE_F32 && dtype != RA_DTYPE_BF16) return RA_ERR_ARG;
     int TC = delta_rule_chunk(DPT, RS, VB);
     if (TC <= 0 || max_q_len < 1) return RA_ERR_ARG;
+    hipStream_t st = (hipStream_t)stream;
+    int rc;
+    // Requests of RC_MIN_ROWS rows and more go by chunks on the matrix cores, as far as the heads fit those kernels (in bf16;
+    // the 32-bit mode, which checks are run in, keeps its one order of sums);
+    // the others of the step, if there are any, walk their rows here.
+    int below = 0x7fffffff;
+    bool walk = true;
+    if (dtype == RA_DTYPE_BF16 && recurrence_chunks_workspace(q_lens, n_seqs, H, D, V, rule) > 0) {
+        rc = recurrence_chunks_run(st, qkv, ld_qkv, b, ld_b, ag, ld_ag, A_log, dt_bias, S, cu_q, slot_ids, o_raw, q_lens, n_seqs,
+                                   H, G, D, V, rule, rate, ws, ws_floats, dtype);
+        if (rc != RA_OK) return rc;
+        below = RC_MIN_ROWS;
+        max_q_len = 0;
+        for (int i = 0; i < n_seqs; ++i)
+            if (q_lens[i] < RC_MIN_ROWS && q_lens[i] > max_q_len) max_q_len = q_lens[i];
+        walk = max_q_len > 0;
+    }
     // no chunk longer than the step's longest request: a step of single tokens takes an eighth of the LDS, and
     // eight times the workgroups share a CU while each waits for its state
     while (TC > 4 && (TC >> 1) >= max_q_len) TC >>= 1;
@@ -622,9 +649,7 @@ static int delta_rule_run(const void* qkv, long long ld_qkv, const void* b, long
     const int col_blocks = (V + VB - 1) / VB;
     if ((long long)H * col_blocks > 0x7fffffffLL) return RA_ERR_ARG;
     dim3 grid(H * col_blocks, n_seqs), block(((VB * RS + 63) / 64) * 64);
-    hipStream_t st = (hipStream_t)stream;
-    int rc;
-    // requests of eight rows and more: the kernel whose feeder waves prepare the next chunk while this one is walked
+    // requests of eight rows and more (that do not go by chunks): the kernel whose feeder waves prepare the next chunk while this one is walked
     // (while the workgroups are few: from about one and a half per CU on, the CUs' other workgroups fill the waits, and
     // the plain kernel's smaller footprint wins: measured, 32 heads of 128 x 128, four requests of 512 rows 1.48 against
     // 1.77 ms, one of 2,048 rows 2.75 against 1.76 ms)
@@ -636,22 +661,24 @@ static int delta_rule_run(const void* qkv, long long ld_qkv, const void* b, long
     }
     const bool few = (long long)grid.x * grid.y <= (long long)cus * 3 / 2;
     const int TCF = (max_q_len >= 8 && few) ? delta_rule_fed_chunk(DPT, RS, VB) : 0;
-    if (TCF > 0 && VB * RS <= DR_WALKERS) {
+    if (!walk) {
+        rc = RA_OK;
+    } else if (TCF > 0 && VB * RS <= DR_WALKERS) {
         int tcf = TCF;
         while (tcf > 8 && (tcf >> 1) >= max_q_len) tcf >>= 1;
         const size_t flds = delta_rule_fed_lds(DPT, RS, VB, tcf);
         if (dtype == RA_DTYPE_F32)
             rc = delta_rule_fed_launch<float>(st, DPT, grid, flds, qkv, ld_qkv, b, ld_b, ag, ld_ag, A_log, dt_bias, S, cu_q,
-                                              slot_ids, o_raw, H, G, D, V, RS, VB, tcf, rule, rate);
+                                              slot_ids, o_raw, H, G, D, V, RS, VB, tcf, rule, rate, below);
         else
             rc = delta_rule_fed_launch<bf16>(st, DPT, grid, flds, qkv, ld_qkv, b, ld_b, ag, ld_ag, A_log, dt_bias, S, cu_q,
-                                             slot_ids, o_raw, H, G, D, V, RS, VB, tcf, rule, rate);
+                                             slot_ids, o_raw, H, G, D, V, RS, VB, tcf, rule, rate, below);
     } else if (dtype == RA_DTYPE_F32)
         rc = delta_rule_launch<float>(st, DPT, grid, block, lds, qkv, ld_qkv, b, ld_b, ag, ld_ag, A_log, dt_bias, S, cu_q,
-                                      slot_ids, o_raw, H, G, D, V, RS, VB, TC, rule, rate);
+                                      slot_ids, o_raw, H, G, D, V, RS, VB, TC, rule, rate, below);
     else
         rc = delta_rule_launch<bf16>(st, DPT, grid, block, lds, qkv, ld_qkv, b, ld_b, ag, ld_ag, A_log, dt_bias, S, cu_q,
-                                     slot_ids, o_raw, H, G, D, V, RS, VB, TC, rule, rate);
+                                     slot_ids, o_raw, H, G, D, V, RS, VB, TC, rule, rate, below);
     if (rc != RA_OK) return rc;
     if (rule == 2) return RA_OK;                      // (the caller's own kernel takes the read-outs)
     const long long n_rows = (long long)T_tokens * H;
@@ -668,12 +695,13 @@ static int delta_rule_run(const void* qkv, long long ld_qkv, const void* b, long
 extern "C" int ra_delta_rule(const void* qkv, long long ld_qkv, const void* b, long long ld_b, const void* ag,
                              long long ld_ag, const float* A_log, const float* dt_bias, const float* norm_w, float eps,
                              float* S, const int* cu_q, const int* slot_ids, float* o_raw, void* out, int n_seqs,
-                             int T_tokens, int max_q_len, int H, int G, int D, int V, int dtype, void* stream) {
+                             int T_tokens, int max_q_len, const int* q_lens, float* ws, long long ws_floats, int H, int G,
+                             int D, int V, int dtype, void* stream) {
     if (ld_ag < (long long)H * D + (long long)H * V) return RA_ERR_ARG;
     const size_t el = dtype == RA_DTYPE_F32 ? 4 : 2;
     const void* gate = (const char*)ag + (size_t)H * D * el;
     return delta_rule_run(qkv, ld_qkv, b, ld_b, ag, ld_ag, gate, ld_ag, A_log, dt_bias, norm_w, eps, S, cu_q, slot_ids,
-                          o_raw, out, n_seqs, T_tokens, max_q_len, H, G, D, V, 0, 0.f, dtype, stream);
+                          o_raw, out, n_seqs, T_tokens, max_q_len, q_lens, ws, ws_floats, H, G, D, V, 0, 0.f, dtype, stream);
 }
 
 // The delta rule with one decay per head: a [T, H] the decay's projection before its bias, b [T, H] beta before the
@@ -682,10 +710,11 @@ extern "C" int ra_delta_rule_head(const void* qkv, long long ld_qkv, const void*
                                   long long ld_a, const void* gate, long long ld_gate, const float* A_log,
                                   const float* dt_bias, const float* norm_w, float eps, float* S, const int* cu_q,
                                   const int* slot_ids, float* o_raw, void* out, int n_seqs, int T_tokens, int max_q_len,
-                                  int H, int G, int D, int V, int dtype, void* stream) {
+                                  const int* q_lens, float* ws, long long ws_floats, int H, int G, int D, int V, int dtype,
+                                  void* stream) {
     if (A_log == nullptr || dt_bias == nullptr || norm_w == nullptr) return RA_ERR_ARG;
     return delta_rule_run(qkv, ld_qkv, b, ld_b, a, ld_a, gate, ld_gate, A_log, dt_bias, norm_w, eps, S, cu_q, slot_ids,
-                          o_raw, out, n_seqs, T_tokens, max_q_len, H, G, D, V, 3, 0.f, dtype, stream);
+                          o_raw, out, n_seqs, T_tokens, max_q_len, q_lens, ws, ws_floats, H, G, D, V, 3, 0.f, dtype, stream);
 }
 
 // The outer-product rule: qkv rows [q: H D | k: H D | v: H V]; a [T, H D] the decay's logits before their bias;
@@ -693,10 +722,11 @@ extern "C" int ra_delta_rule_head(const void* qkv, long long ld_qkv, const void*
 extern "C" int ra_outer_rule(const void* qkv, long long ld_qkv, const void* a, long long ld_a, const void* gate,
                              long long ld_gate, const float* bias, float rate, const float* norm_w, float eps, float* S,
                              const int* cu_q, const int* slot_ids, float* o_raw, void* out, int n_seqs, int T_tokens,
-                             int max_q_len, int H, int D, int V, int dtype, void* stream) {
+                             int max_q_len, const int* q_lens, float* ws, long long ws_floats, int H, int D, int V, int dtype,
+                             void* stream) {
     if (!(rate > 0.f) || bias == nullptr) return RA_ERR_ARG;
     return delta_rule_run(qkv, ld_qkv, nullptr, 0, a, ld_a, gate, ld_gate, nullptr, bias, norm_w, eps, S, cu_q, slot_ids,
-                          o_raw, out, n_seqs, T_tokens, max_q_len, H, H, D, V, 1, rate, dtype, stream);
+                          o_raw, out, n_seqs, T_tokens, max_q_len, q_lens, ws, ws_floats, H, H, D, V, 1, rate, dtype, stream);
 }
 
 // out[t, part] = y / sqrt(mean over the part of y^2 + eps) * norm_w with y = (o[t, c] + skip[head of c] v[t, c]) * silu(z[t, c]),
@@ -750,14 +780,15 @@ __global__ __launch_bounds__(256) void scalar_out_kernel(const float* __restrict
 extern "C" int ra_scalar_rule(const void* qkv, long long ld_qkv, const void* d, long long ld_d, const void* gate,
                               long long ld_gate, const float* A_log, const float* d_bias, const float* skip,
                               const float* norm_w, int n_parts, float eps, float* S, const int* cu_q, const int* slot_ids,
-                              float* o_raw, void* out, int n_seqs, int T_tokens, int max_q_len, int H, int G, int D, int V,
-                              int dtype, void* stream) {
+                              float* o_raw, void* out, int n_seqs, int T_tokens, int max_q_len, const int* q_lens, float* ws,
+                              long long ws_floats, int H, int G, int D, int V, int dtype, void* stream) {
     if (n_seqs <= 0 || T_tokens <= 0) return RA_OK;
     if (A_log == nullptr || d_bias == nullptr || skip == nullptr || norm_w == nullptr || n_parts < 1 ||
         ((long long)H * V) % n_parts)
         return RA_ERR_ARG;
     const int rc = delta_rule_run(qkv, ld_qkv, nullptr, 0, d, ld_d, gate, ld_gate, A_log, d_bias, norm_w, eps, S, cu_q,
-                                  slot_ids, o_raw, out, n_seqs, T_tokens, max_q_len, H, G, D, V, 2, 0.f, dtype, stream);
+                                  slot_ids, o_raw, out, n_seqs, T_tokens, max_q_len, q_lens, ws, ws_floats, H, G, D, V, 2, 0.f, dtype,
+                                  stream);
     if (rc != RA_OK) return rc;
     const int L = (int)((long long)H * V / n_parts);
     const long long n_units = (long long)T_tokens * n_parts;

@@ -68,12 +68,12 @@ def _declare(lib):
         "ra_gate_rows": [P, L, P, L, I, I, I, P],
         "ra_qkv_rows_prepare": [P, L, I, I, I, I, P, P, I, I, F, P, P, P, I, P, P, P, P, I, L, I, P],
         "ra_causal_conv_bias": [P, L, P, P, P, P, P, P, P, L, I, I, I, I, I, I, P],
-        "ra_scalar_rule": [P, L, P, L, P, L, P, P, P, P, I, F, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
+        "ra_scalar_rule": [P, L, P, L, P, L, P, P, P, P, I, F, P, P, P, P, P, I, I, I, P, P, L, I, I, I, I, I, P],
         "ra_attention_latent_plain_fits": [I, I],
         "ra_attention_latent_mfma_bf16": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, P, I, P, P],
         "ra_attention_latent_mfma_fits": [I, I, I],
         "ra_attention_latent_mfma_tile_tokens": [I],
-        "ra_outer_rule": [P, L, P, L, P, L, P, F, P, F, P, P, P, P, P, I, I, I, I, I, I, I, P],
+        "ra_outer_rule": [P, L, P, L, P, L, P, F, P, F, P, P, P, P, P, I, I, I, P, P, L, I, I, I, I, P],
         "ra_moe_route_law": [P, L, P, I, I, I, I, I, F, P, P, I, P],
         "ra_moe_product_act": [P, P, P, P, P, P, I, I, I, I, I, I, I, F, F, P, I, P],
         "ra_add_rmsnorm": [P, P, P, F, P, P, I, I, I, P],
@@ -110,8 +110,8 @@ def _declare(lib):
         "ra_gemm_sweep_norm_bf16": [P, P, P, I, I, I, I, I, I, P, I, I, F, P, P, P, P],
         "ra_attention_plain": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, I, P, F, I, I, P, F, L, P],
         "ra_causal_conv": [P, L, P, P, P, P, P, L, I, I, I, I, I, I, P],
-        "ra_delta_rule": [P, L, P, L, P, L, P, P, P, F, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
-        "ra_delta_rule_head": [P, L, P, L, P, L, P, L, P, P, P, F, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
+        "ra_delta_rule": [P, L, P, L, P, L, P, P, P, F, P, P, P, P, P, I, I, I, P, P, L, I, I, I, I, I, P],
+        "ra_delta_rule_head": [P, L, P, L, P, L, P, L, P, P, P, F, P, P, P, P, P, I, I, I, P, P, L, I, I, I, I, I, P],
         "ra_channel_recurrence": [P, P, P, P, P, L, P, P, P, P, P, F, P, L, I, I, I, I, I, I, I, P],
         "ra_channel_recurrence_chunk": [I],
         "ra_channel_recurrence_mfma": [I, I, I],
@@ -140,6 +140,8 @@ def _declare(lib):
         fn = getattr(lib, name)
         fn.argtypes = args
         fn.restype = _c_int
+    lib.ra_recurrence_scratch.argtypes = [P, I, I, I, I, I]
+    lib.ra_recurrence_scratch.restype = _c_ll
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -762,6 +764,16 @@ class HipOps:
             "causal_conv")
         return out
 
+    def _recurrence_scratch(self, step, H, D, V, rule, dtype):
+        """(rows that every request brings, as a host array; scratch; its floats) for the recurrences' kernels by chunks
+        of rows, as the library's entries take them; nothing for a step of single tokens or in 32-bit."""
+        if step.max_q_len <= 1 or dtype != torch.bfloat16:
+            return None, None, 0
+        cu = step.cu_q_host
+        rows = (_c_int * step.n_seqs)(*[cu[i + 1] - cu[i] for i in range(step.n_seqs)])
+        floats = self.lib.ra_recurrence_scratch(rows, step.n_seqs, H, D, V, rule)
+        return rows, torch.empty(floats, dtype=torch.float32, device=self.device) if floats > 0 else None, floats
+
     def delta_rule_fits(self, D, V):
         return bool(self.lib.ra_delta_rule_fits(int(D), int(V)))
 
@@ -791,10 +803,11 @@ class HipOps:
         if not self.delta_rule_fits(D, V):
             raise KernelError(f"delta_rule: heads of {D} x {V} are beyond the kernel")
         o_raw = torch.empty(T, H * V, dtype=torch.float32, device=self.device)
+        rows, scratch, floats = self._recurrence_scratch(step, H, D, V, 0, qkv.dtype)
         self._check(self.lib.ra_delta_rule(
             _ptr(qkv), ld_qkv, _ptr(beta), ld_b, _ptr(ag), ld_ag, _ptr(a_log), _ptr(dt_bias), _ptr(norm_w), float(eps),
             _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), _ptr(o_raw), _ptr(out), step.n_seqs, T,
-            max(1, int(step.max_q_len)), H, G, D, V,
+            max(1, int(step.max_q_len)), rows, _ptr(scratch), floats, H, G, D, V,
             _code(qkv.dtype), self._stream()), "delta_rule")
         return out
 
@@ -825,10 +838,12 @@ class HipOps:
         if not self.delta_rule_fits(D, V):
             raise KernelError(f"delta_rule_head: heads of {D} x {V} are beyond the kernel")
         o_raw = torch.empty(T, H * V, dtype=torch.float32, device=self.device)
+        rows, scratch, floats = self._recurrence_scratch(step, H, D, V, 3, qkv.dtype)
         self._check(self.lib.ra_delta_rule_head(
             _ptr(qkv), ld_qkv, _ptr(beta), ld_b, _ptr(a), ld_a, _ptr(gate), ld_g, _ptr(a_log), _ptr(dt_bias), _ptr(norm_w),
             float(eps), _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), _ptr(o_raw), _ptr(out), step.n_seqs, T,
-            max(1, int(step.max_q_len)), H, G, D, V, _code(qkv.dtype), self._stream()), "delta_rule_head")
+            max(1, int(step.max_q_len)), rows, _ptr(scratch), floats, H, G, D, V, _code(qkv.dtype),
+            self._stream()), "delta_rule_head")
         return out
 
     def channel_recurrence(self, u, w_gates, gate_bias, rate, y, y_bias, state, step, out, out_scale=1.0):
@@ -973,10 +988,12 @@ class HipOps:
         if not self.delta_rule_fits(D, V) or not float(tau) > 0:
             raise KernelError(f"outer_rule: heads of {D} x {V} (tau {tau}) are beyond the kernel")
         o_raw = torch.empty(T, H * V, dtype=torch.float32, device=self.device)
+        rows, scratch, floats = self._recurrence_scratch(step, H, D, V, 1, qkv.dtype)
         self._check(self.lib.ra_outer_rule(
             _ptr(qkv), ld_qkv, _ptr(a), ld_a, _ptr(gate), ld_g, _ptr(decay_bias), 1.0 / float(tau), _ptr(norm_w), float(eps),
             _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), _ptr(o_raw), _ptr(out), step.n_seqs, T,
-            max(1, int(step.max_q_len)), H, D, V, _code(qkv.dtype), self._stream()), "outer_rule")
+            max(1, int(step.max_q_len)), rows, _ptr(scratch), floats, H, D, V, _code(qkv.dtype),
+            self._stream()), "outer_rule")
         return out
 
     def scalar_rule(self, qkv, dt, a_log, dt_bias, skip, gate, norm_w, norm_groups, eps, state, step, out, H, G, D, V):
@@ -1007,10 +1024,12 @@ class HipOps:
         if not self.delta_rule_fits(D, V):
             raise KernelError(f"scalar_rule: heads of {D} x {V} are beyond the kernel")
         o_raw = torch.empty(T, H * V, dtype=torch.float32, device=self.device)
+        rows, scratch, floats = self._recurrence_scratch(step, H, D, V, 2, qkv.dtype)
         self._check(self.lib.ra_scalar_rule(
             _ptr(qkv), ld_qkv, _ptr(dt), ld_dt, _ptr(gate), ld_g, _ptr(a_log), _ptr(dt_bias), _ptr(skip), _ptr(norm_w),
             int(norm_groups), float(eps), _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), _ptr(o_raw), _ptr(out),
-            step.n_seqs, T, max(1, int(step.max_q_len)), H, G, D, V, _code(qkv.dtype), self._stream()), "scalar_rule")
+            step.n_seqs, T, max(1, int(step.max_q_len)), rows, _ptr(scratch), floats, H, G, D, V,
+            _code(qkv.dtype), self._stream()), "scalar_rule")
         return out
 
     def token_side(self, h, delta, token_ids, table, offset, gate, proj, weight, eps):
