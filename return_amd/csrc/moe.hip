@@ -10,39 +10,21 @@
 //             choice is made on s, a group's score is its largest s, the weights are the chosen s as they are. Law 3:
 //             as law 0, the weights are the chosen s as they are.
 //   plan      pairs p = t * top + k grouped by expert: order[] lists the pairs expert by expert, and tiles[]
-//             lists (expert, first place in order[], places) for runs of at most `rows` places of one expert.
+//             lists (expert, first place in order[], places) for runs of at most `rows` places of one expert (runs of
+//             MOE_TILE_ROWS: as many as that takes, but of even length, in groups of 16).
 //             One workgroup (a counting sort). A pair's result does not depend on its place in a tile.
 //   product   for every tile: y[p] = W_e x[row(p)] with row(p) = p / top (the token's row) or p itself;
 //             gated: W_e = [gate rows; up rows], y = silu(gate) * up; with in_scale [n_pairs] the pair's row of x is
 //             taken times in_scale[p] (the two sums are, which is the same). An FMA form for every size and both
 //             storage types, and two matrix-core forms for bfloat16 with K % 8 == 0: operands straight from
 //             memory for tiles of 16 or 64 rows (few rows an expert: the weights are read once, the time is
-//             the reading), tiles of 128 rows staged in LDS where an expert has many rows.
+//             the reading), tiles staged in LDS where an expert has many rows: of up to 256 rows (moe_tile.hip), or of
+//             128 where K is no multiple of 32.
 //   combine   out[t] = sum_k weights[t][k] * y[t * top + k], k in order, 32-bit sums; optionally one more term,
 //             extra[t] * sigmoid(logit[t]) (an expert that every token uses, behind a gate of one number a token).
-#include "common.h"
+#include "moe_tile.h"
 
 #define MOE_MAX_EXPERTS 1024
-
-// What a gated product makes of its two halves: kind 0, silu(g) * u; kind 1 ("clamped"), with g <- min(g, limit)
-// and u <- clamp(u, -limit, limit): g * sigmoid(slope * g) * (u + 1).
-struct MoeAct {
-    int kind;
-    float limit, slope;
-    const float* in_scale;      // a factor on a pair's input row (null: none)
-};
-// both halves of pair p from their 32-bit sums: scaled, rounded to what a product kernel would have stored, activated
-template <typename T>
-__device__ __forceinline__ float moe_gate(float g, float u, const MoeAct act, float in_scale) {
-    g = round_to<T>(g * in_scale);
-    u = round_to<T>(u * in_scale);
-    if (act.kind == 1) {
-        g = fminf(g, act.limit);
-        u = fminf(fmaxf(u, -act.limit), act.limit);
-        return g / (1.0f + expf(-act.slope * g)) * (u + 1.0f);
-    }
-    return g / (1.0f + expf(-g)) * u;
-}
 
 // ------------------------------------------------------------------ route: one wave per token
 __global__ __launch_bounds__(256) void moe_route_kernel(const float* __restrict__ z, long long ld_z, const float* __restrict__ bias,
@@ -144,6 +126,16 @@ extern "C" int ra_moe_route(const float* z, const float* bias, int T, int E, int
 }
 
 // ------------------------------------------------------------------ plan: one workgroup
+// Rows of an expert's tiles, and how many tiles its n rows make.
+__device__ __forceinline__ int moe_rows_of_tile(int n, int rows) {
+    if (rows < MOE_TILE_ROWS) return rows;
+    const int t = (n + rows - 1) / rows;
+    return t > 1 ? min(rows, ((n + t - 1) / t + 15) & ~15) : rows;
+}
+__device__ __forceinline__ int moe_tiles_of(int n, int rows) {
+    const int per = moe_rows_of_tile(n, rows);
+    return (n + per - 1) / per;
+}
 // meta[0] = number of tiles. order [n_pairs], tiles [max_tiles][3].
 __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ ids, int n_pairs, int E, int rows,
                                                         int* __restrict__ order, int* __restrict__ tiles,
@@ -162,7 +154,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
             first[e] = at;
             tile_first[e] = tl;
             at += count[e];
-            tl += (count[e] + rows - 1) / rows;
+            tl += moe_tiles_of(count[e], rows);
         }
         first[E] = at;
         tile_first[E] = tl;
@@ -179,11 +171,11 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
         order[first[e] + atomicAdd(&running[e], 1)] = p;
     }
     for (int e = tid; e < E; e += n_thr) {
-        const int n = count[e];
-        for (int i = 0, tl = tile_first[e]; i < n; i += rows, ++tl) {
+        const int n = count[e], per = moe_rows_of_tile(n, rows);
+        for (int i = 0, tl = tile_first[e]; i < n; i += per, ++tl) {
             tiles[3 * tl] = e;
             tiles[3 * tl + 1] = first[e] + i;
-            tiles[3 * tl + 2] = min(rows, n - i);
+            tiles[3 * tl + 2] = min(per, n - i);
         }
     }
 }
@@ -470,10 +462,14 @@ __global__ __launch_bounds__(256) void moe_product_tile_kernel(
     }
 }
 
-// rows of a tile that the product kernel behind these arguments takes (what ra_moe_plan is to be called with)
-extern "C" int ra_moe_tile_rows(int n_pairs, int E, int K, int dtype) {
-    if (dtype == RA_DTYPE_BF16 && K % 8 == 0) return n_pairs >= 64 * E ? 128 : (n_pairs >= 24 * E ? 64 : 16);
-    return MOE_FMA_ROWS;
+// rows of a tile that the product kernel behind these arguments takes (what ra_moe_plan is to be called with); n_rows: rows
+// of one expert's matrix. From eight pairs an expert on the tiles staged in LDS are the fastest (32 experts of 6,144 x 4,096,
+// gate-up and down together: 64 tokens 442 us against 492 with operands straight from memory, 120 tokens 448 against 649,
+// 500 tokens 515 against 1,215; 16 tokens 422 against 402).
+extern "C" int ra_moe_tile_rows(int n_pairs, int E, int n_rows, int K, int dtype) {
+    if (dtype != RA_DTYPE_BF16 || K % 8 != 0) return MOE_FMA_ROWS;
+    if (n_pairs >= 8 * E && moe_tile_fits(n_pairs, n_rows, K)) return MOE_TILE_ROWS;
+    return n_pairs >= 64 * E ? MT_BM : (n_pairs >= 24 * E ? 64 : 16);
 }
 
 // x [rows][K]; w [E][N or 2N][K]; y [n_pairs][N]; the row of pair p in x is p / top_div (top_div = top: the
@@ -488,6 +484,9 @@ extern "C" int ra_moe_product_act(const void* x, const void* w, void* y, const i
     if (N < 1 || K < 1 || top_div < 1 || act_kind < 0 || act_kind > 1 || (in_scale != nullptr && !gated)) return RA_ERR_ARG;
     const MoeAct act = {act_kind, limit, slope, in_scale};
     hipStream_t st = (hipStream_t)stream;
+    if (dtype == RA_DTYPE_BF16 && tile_rows == MOE_TILE_ROWS)
+        return moe_tile_launch(st, (const bf16*)x, (const bf16*)w, (bf16*)y, order, tiles, meta, max_tiles, N, K, top_div, gated != 0,
+                               act);
     if (dtype == RA_DTYPE_BF16 && K % 8 == 0 && tile_rows == MT_BM) {
         const int cn = gated ? 64 : 128;
         dim3 grid((N + cn - 1) / cn, max_tiles);

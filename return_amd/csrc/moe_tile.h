@@ -1,0 +1,31 @@
+// The experts' products for many rows an expert (moe_tile.hip) and what moe.hip shares with them.
+#pragma once
+#include "common.h"
+
+// What a gated product makes of its halves. Kind 0: silu(g) * u. Kind 1: with g <- min(g, limit)
+// and u <- clamp(u, -limit, limit): g * sigmoid(slope * g) * (u + 1).
+struct MoeAct {
+    int kind;
+    float limit, slope;
+    const float* in_scale;      // a factor on a pair's input row (null: none)
+};
+// both halves of pair p from their 32-bit sums: scaled, rounded to what a product kernel would have stored, activated
+template <typename T>
+__device__ __forceinline__ float moe_gate(float g, float u, const MoeAct act, float in_scale) {
+    g = round_to<T>(g * in_scale);
+    u = round_to<T>(u * in_scale);
+    if (act.kind == 1) {
+        g = fminf(g, act.limit);
+        u = fminf(fmaxf(u, -act.limit), act.limit);
+        return g / (1.0f + expf(-act.slope * g)) * (u + 1.0f);
+    }
+    return g / (1.0f + expf(-g)) * u;
+}
+
+#define MOE_TILE_ROWS 256
+// Whether the kernel takes an expert's matrix of n_rows rows and n_pairs rows of x, all of K elements.
+static inline bool moe_tile_fits(long long n_pairs, long long n_rows, int K) {
+    return K % 32 == 0 && n_pairs * K * 2 < 0x7fffff00ll && n_rows * K * 2 < 0x7fffff00ll;
+}
+int moe_tile_launch(hipStream_t st, const bf16* x, const bf16* w, bf16* y, const int* order, const int* tiles,
+                    const int* meta, int max_tiles, int N, int K, int top_div, bool gated, const MoeAct& act);

@@ -86,7 +86,7 @@ def _declare(lib):
         "ra_attention_diff_plain_fits": [I, I],
         "ra_moe_route": [P, P, I, I, I, I, I, F, P, P, P],
         "ra_moe_plan": [P, I, I, I, P, P, P, P],
-        "ra_moe_tile_rows": [I, I, I, I],
+        "ra_moe_tile_rows": [I, I, I, I, I],
         "ra_moe_product": [P, P, P, P, P, P, I, I, I, I, I, I, I, P],
         "ra_moe_combine": [P, P, P, I, I, I, I, P],
         "ra_moe_combine_extra": [P, P, P, I, I, I, P, P, I, L, I, P],
@@ -2085,7 +2085,7 @@ class HipOps:
             return order, tiles, meta, max_tiles, rows
 
         # the two products may take tiles of different heights (their K differ): a plan each where they do
-        rows_up, rows_down = (int(self.lib.ra_moe_tile_rows(n_pairs, E, K, code)) for K in (H, I))
+        rows_up, rows_down = (int(self.lib.ra_moe_tile_rows(n_pairs, E, N, K, code)) for N, K in ((I2, H), (H, I)))
         up = plan(rows_up)
         down = up if rows_down == rows_up else plan(rows_down)
         order, tiles, meta, max_tiles, rows = up
