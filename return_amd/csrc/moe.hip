@@ -16,10 +16,10 @@
 //   product   for every tile: y[p] = W_e x[row(p)] with row(p) = p / top (the token's row) or p itself;
 //             gated: W_e = [gate rows; up rows], y = silu(gate) * up; with in_scale [n_pairs] the pair's row of x is
 //             taken times in_scale[p] (the two sums are, which is the same). An FMA form for every size and both
-//             storage types, and two matrix-core forms for bfloat16 with K % 8 == 0: operands straight from
-//             memory for tiles of 16 or 64 rows (few rows an expert: the weights are read once, the time is
-//             the reading), tiles staged in LDS where an expert has many rows: of up to 256 rows (moe_tile.hip), or of
-//             128 where K is no multiple of 32.
+//             storage types, and matrix-core forms for bfloat16 with K % 8 == 0: tiles of 16 rows with W read in whole
+//             runs (moe_sweep.hip: few rows an expert, the time is the reading) and tiles of up to 256 rows staged in LDS
+//             (moe_tile.hip: many). Sizes that these do not take: operands straight from memory for tiles of 16 (K beyond
+//             4,096) or 64 rows, tiles of 128 rows in LDS (K no multiple of 32).
 //   combine   out[t] = sum_k weights[t][k] * y[t * top + k], k in order, 32-bit sums; optionally one more term,
 //             extra[t] * sigmoid(logit[t]) (an expert that every token uses, behind a gate of one number a token).
 #include "moe_tile.h"
@@ -463,12 +463,14 @@ __global__ __launch_bounds__(256) void moe_product_tile_kernel(
 }
 
 // rows of a tile that the product kernel behind these arguments takes (what ra_moe_plan is to be called with); n_rows: rows
-// of one expert's matrix. From eight pairs an expert on the tiles staged in LDS are the fastest (32 experts of 6,144 x 4,096,
-// gate-up and down together: 64 tokens 442 us against 492 with operands straight from memory, 120 tokens 448 against 649,
-// 500 tokens 515 against 1,215; 16 tokens 422 against 402).
+// of one expert's matrix. Up to twelve pairs an expert W is read in whole runs for tiles of 16 (moe_sweep.hip), beyond that,
+// where more and more experts would have two such tiles, by tiles staged in LDS (moe_tile.hip). 32 experts of 6,144 x 4,096,
+// four a token, gate-up and down together, sweep / LDS tiles: 16 tokens 369 / 422 us, 64 tokens 443 / 453, 80 tokens 464 / 458;
+// of 4,096 x 2,048: 64 tokens 155 / 194, 80 tokens 157 / 195. (Operands straight from memory: 402, 492 and 193 us at 16 and
+// 64 tokens, 649 at 120, 1,215 at 500, where the LDS tiles take 448 and 515.)
 extern "C" int ra_moe_tile_rows(int n_pairs, int E, int n_rows, int K, int dtype) {
     if (dtype != RA_DTYPE_BF16 || K % 8 != 0) return MOE_FMA_ROWS;
-    if (n_pairs >= 8 * E && moe_tile_fits(n_pairs, n_rows, K)) return MOE_TILE_ROWS;
+    if (n_pairs >= (moe_sweep_fits(K) ? 12 : 8) * E && moe_tile_fits(n_pairs, n_rows, K)) return MOE_TILE_ROWS;
     return n_pairs >= 64 * E ? MT_BM : (n_pairs >= 24 * E ? 64 : 16);
 }
 
@@ -499,6 +501,8 @@ extern "C" int ra_moe_product_act(const void* x, const void* w, void* y, const i
                                (bf16*)y, order, tiles, meta, N, K, top_div, act);
         return ra_launch_status();
     }
+    if (dtype == RA_DTYPE_BF16 && tile_rows == 16 && moe_sweep_fits(K))
+        return moe_sweep_launch(st, (const bf16*)x, (const bf16*)w, (bf16*)y, order, tiles, meta, N, K, top_div, gated != 0, act);
     if (dtype == RA_DTYPE_BF16 && K % 8 == 0 && (tile_rows == 16 || tile_rows == 64)) {
         const bf16 *xb = (const bf16*)x, *wb = (const bf16*)w;
         bf16* yb = (bf16*)y;

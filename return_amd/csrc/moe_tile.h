@@ -1,4 +1,4 @@
-// The experts' products for many rows an expert (moe_tile.hip) and what moe.hip shares with them.
+// The experts' products for many rows an expert (moe_tile.hip) and for few (moe_sweep.hip), and what moe.hip shares with them.
 #pragma once
 #include "common.h"
 
@@ -29,3 +29,8 @@ static inline bool moe_tile_fits(long long n_pairs, long long n_rows, int K) {
 }
 int moe_tile_launch(hipStream_t st, const bf16* x, const bf16* w, bf16* y, const int* order, const int* tiles,
                     const int* meta, int max_tiles, int N, int K, int top_div, bool gated, const MoeAct& act);
+
+// Few rows an expert: tiles of up to 16 rows.
+bool moe_sweep_fits(int K);
+int moe_sweep_launch(hipStream_t st, const bf16* x, const bf16* w, bf16* y, const int* order, const int* tiles,
+                     const int* meta, int N, int K, int top_div, bool gated, const MoeAct& act);

@@ -1,0 +1,66 @@
+"""The experts' products on the matrix cores (bf16) against a 64-bit product of the same bfloat16 operands: tiles of up to 256
+rows in LDS (twelve pairs an expert and more) at every count of groups of 16 rows, few k-steps, experts without rows, widths
+that are no multiple of a tile; tiles of 16 rows with W read in whole runs (fewer pairs) at one to eight waves, columns shared
+out unevenly, more tiles than workgroups; both activations, factors on what an expert reads."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.fixture(scope="module")
+def ops():
+    from return_amd.kernels.hip_ops import HipOps
+    return HipOps(DEV)
+
+
+def check(ops, rows, E, H, I, ids, kind):
+    """One expert a token, so that the counts are exact. A result is two bf16 roundings (2^-9 each of the halves and of the
+    activation) away from the 64-bit one, grown by the product with them: 2^-6 of the largest."""
+    g = torch.Generator().manual_seed(len(ids) + H)
+    x = torch.randn(len(ids), H, generator=g).bfloat16()
+    w_up = (torch.randn(E, 2 * I, H, generator=g) * H ** -0.5).bfloat16()
+    w_down = (torch.randn(E, H, I, generator=g) * I ** -0.5).bfloat16()
+    factor = 0.5 + torch.rand(len(ids), 1, generator=g)
+    kw = {"clamped": dict(activation="clamped", limit=1.0), "input": dict(weigh="input"), "silu": {}}[kind]
+    assert ops.lib.ra_moe_tile_rows(len(ids), E, 2 * I, H, 1) == rows        # (the kernel that this is about)
+    got = ops.moe_experts(x.to(DEV), ids.int()[:, None].to(DEV), factor.to(DEV), w_up.to(DEV), w_down.to(DEV), **kw)
+    want = torch.zeros(len(ids), H, dtype=torch.float64)
+    for e in ids.unique().tolist():
+        t = (ids == e).nonzero()[:, 0]
+        h = (x[t].double() * (factor[t].double() if kind == "input" else 1.0)) @ w_up[e].double().T
+        a, b = h[:, :I], h[:, I:]
+        if kind == "clamped":
+            a, b = a.clamp(max=1.0), b.clamp(-1.0, 1.0) + 1.0
+            mid = a * torch.sigmoid(1.702 * a) * b
+        else:
+            mid = a * torch.sigmoid(a) * b
+        want[t] = (mid @ w_down[e].double().T) * (1.0 if kind == "input" else factor[t].double())
+    err = (got.cpu().double() - want).abs().max() / want.abs().max()
+    assert err < 2.0 ** -6, float(err)
+
+
+def shuffled(counts):
+    ids = torch.cat([torch.full((n,), e) for e, n in enumerate(counts)])
+    return ids[torch.randperm(len(ids), generator=torch.Generator().manual_seed(len(ids)))]
+
+
+KINDS = ["silu", "clamped", "input"]
+
+
+@pytest.mark.parametrize("E,H,I,counts", [
+    (4, 32, 32, [8, 9, 31, 33]), (3, 64, 96, [16, 20, 0]), (2, 224, 40, [64, 65]), (5, 256, 160, [128, 129, 144, 145, 0]),
+    (3, 96, 300, [160, 192, 193]), (4, 160, 128, [224, 225, 256, 257]), (2, 1024, 224, [272, 700]), (1, 128, 64, [12]),
+    (6, 192, 2, [0, 0, 48, 0, 0, 500])])
+@pytest.mark.parametrize("kind", KINDS)
+def test_products_of_many_rows(ops, E, H, I, counts, kind):
+    check(ops, 256, E, H, I, shuffled(counts), kind)
+
+
+@pytest.mark.parametrize("E,H,I,counts", [
+    (4, 8, 8, [1, 0, 2, 0]), (3, 520, 24, [5, 16, 7]), (2, 1032, 40, [1, 20]), (8, 2048, 136, [1, 0, 0, 3, 17, 0, 33, 9]),
+    (3, 4096, 56, [15, 1, 0]), (2, 2568, 1000, [1, 1]), (1, 3080, 16, [11]), (700, 64, 24, [1] * 650 + [0] * 50), (5, 512, 7, [0, 4, 0, 1, 0])])
+@pytest.mark.parametrize("kind", KINDS)
+def test_products_of_few_rows(ops, E, H, I, counts, kind):
+    check(ops, 16, E, H, I, shuffled(counts), kind)
