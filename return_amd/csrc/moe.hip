@@ -137,46 +137,74 @@ __device__ __forceinline__ int moe_tiles_of(int n, int rows) {
     return (n + per - 1) / per;
 }
 // meta[0] = number of tiles. order [n_pairs], tiles [max_tiles][3].
+// What bounds it is the chain of dependent steps of one workgroup: ids from memory, counts, sums over the experts, places.
+// So a thread asks for eight ids at once; with up to MOE_PLAN_EXPERTS experts every wave counts for itself (the lanes of
+// sixteen waves would queue at the same few LDS words); and the sums over the experts are a scan over the threads, not a
+// loop of one of them (32 experts: 32 pairs 5.4 -> 4.0 us, 12,432 pairs 18.8 -> 9.9; 1,024
+// experts, 1,200 pairs 108 -> 4.4).
+#define MOE_PLAN_EXPERTS 128
 __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ ids, int n_pairs, int E, int rows,
                                                         int* __restrict__ order, int* __restrict__ tiles,
                                                         int* __restrict__ meta) {
-    __shared__ int count[MOE_MAX_EXPERTS];
-    __shared__ int first[MOE_MAX_EXPERTS + 1];
-    __shared__ int tile_first[MOE_MAX_EXPERTS + 1];
-    const int tid = threadIdx.x, n_thr = blockDim.x;
-    for (int e = tid; e < E; e += n_thr) count[e] = 0;
+    __shared__ int place[MOE_MAX_EXPERTS > 16 * MOE_PLAN_EXPERTS ? MOE_MAX_EXPERTS : 16 * MOE_PLAN_EXPERTS];
+    __shared__ unsigned long long wave_total[16];
+    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int copies = E <= MOE_PLAN_EXPERTS ? 16 : 1;
+    int* mine = place + (copies == 16 ? wave : 0) * E;
+    for (int i = tid; i < copies * E; i += 1024) place[i] = 0;
     __syncthreads();
-    for (int p = tid; p < n_pairs; p += n_thr) atomicAdd(&count[ids[p]], 1);
-    __syncthreads();
-    if (tid == 0) {
-        int at = 0, tl = 0;
-        for (int e = 0; e < E; ++e) {
-            first[e] = at;
-            tile_first[e] = tl;
-            at += count[e];
-            tl += moe_tiles_of(count[e], rows);
-        }
-        first[E] = at;
-        tile_first[E] = tl;
-        meta[0] = tl;
+    for (int p0 = tid; p0 < n_pairs; p0 += 8 * 1024) {
+        int id[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) id[j] = p0 + j * 1024 < n_pairs ? ids[p0 + j * 1024] : -1;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (id[j] >= 0) atomicAdd(&mine[id[j]], 1);
     }
     __syncthreads();
-    // a pair's place among its expert's pairs is whatever the atomic gives: a row's result does not depend
-    // on its place in a tile
-    __shared__ int running[MOE_MAX_EXPERTS];
-    for (int e = tid; e < E; e += n_thr) running[e] = 0;
-    __syncthreads();
-    for (int p = tid; p < n_pairs; p += n_thr) {
-        const int e = ids[p];
-        order[first[e] + atomicAdd(&running[e], 1)] = p;
+    // thread e: its expert's pairs and tiles, and how many of both the experts before it have
+    int n = 0;
+    if (tid < E)
+        for (int c = 0; c < copies; ++c) n += place[c * E + tid];
+    const int own_tiles = tid < E && n > 0 ? moe_tiles_of(n, rows) : 0;
+    unsigned long long sum = ((unsigned long long)n << 32) | (unsigned)own_tiles;
+    const unsigned long long own = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const unsigned long long t = __shfl_up(sum, o, 64);
+        if (lane >= o) sum += t;
     }
-    for (int e = tid; e < E; e += n_thr) {
-        const int n = count[e], per = moe_rows_of_tile(n, rows);
-        for (int i = 0, tl = tile_first[e]; i < n; i += per, ++tl) {
-            tiles[3 * tl] = e;
-            tiles[3 * tl + 1] = first[e] + i;
+    if (lane == 63) wave_total[wave] = sum;
+    __syncthreads();
+    for (int v = 0; v < wave; ++v) sum += wave_total[v];
+    if (tid == 1023) meta[0] = (int)(sum & 0xffffffffull);
+    sum -= own;
+    const int first = (int)(sum >> 32);
+    if (tid < E) {
+        int tl = (int)(sum & 0xffffffffull);
+        const int per = moe_rows_of_tile(n, rows);
+        for (int i = 0; i < n; i += per, ++tl) {
+            tiles[3 * tl] = tid;
+            tiles[3 * tl + 1] = first + i;
             tiles[3 * tl + 2] = min(per, n - i);
         }
+        // a pair's place among its expert's pairs is whatever the atomic gives: a row's result does not depend on its
+        // place in a tile
+        int at = first;
+        for (int c = 0; c < copies; ++c) {
+            const int k = place[c * E + tid];
+            place[c * E + tid] = at;
+            at += k;
+        }
+    }
+    __syncthreads();
+    for (int p0 = tid; p0 < n_pairs; p0 += 8 * 1024) {
+        int id[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) id[j] = p0 + j * 1024 < n_pairs ? ids[p0 + j * 1024] : -1;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (id[j] >= 0) order[atomicAdd(&mine[id[j]], 1)] = p0 + j * 1024;
     }
 }
 
@@ -550,6 +578,58 @@ __global__ void moe_combine_kernel(const T* __restrict__ y, const float* __restr
     out[i] = from_f<T>(acc);
 }
 
+// The same for bfloat16 rows of whole 16-byte pieces, eight columns a thread: every row's piece of a token is asked for at
+// once. Bound by reading the pairs' rows (2,048 tokens of four rows of 4,096: 43 us with a column a thread, 17 now).
+template <typename L>
+__global__ __launch_bounds__(256) void moe_combine_bf16x8_kernel(
+    const uint4* __restrict__ y, const float* __restrict__ weights, uint4* __restrict__ out, int top, int n8, long long total8,
+    const uint4* __restrict__ extra, const L* __restrict__ logit, long long ld_logit) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= total8) return;
+    const long long t = i / n8;
+    const int c = (int)(i - t * n8);
+    float acc[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) acc[e] = 0.f;
+    auto add = [&](float w, uint4 v) {
+        const uint32_t p[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            acc[2 * e] = fmaf(w, __uint_as_float(p[e] << 16), acc[2 * e]);
+            acc[2 * e + 1] = fmaf(w, __uint_as_float(p[e] & 0xffff0000u), acc[2 * e + 1]);
+        }
+    };
+    const uint4* row = y + t * top * n8 + c;
+    uint4 ex = make_uint4(0, 0, 0, 0);
+    float lg = 0.f;
+    if (extra != nullptr) {
+        ex = extra[i];
+        lg = to_f(logit[t * ld_logit]);
+    }
+    for (int k0 = 0; k0 < top; k0 += 4) {
+        uint4 v[4];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (k0 + k < top) v[k] = row[(long long)(k0 + k) * n8];
+#pragma unroll
+        for (int k = 0; k < 4; ++k)
+            if (k0 + k < top) add(weights != nullptr ? weights[t * top + k0 + k] : 1.0f, v[k]);
+    }
+    if (extra != nullptr) {
+        const float w = 1.0f / (1.0f + expf(-lg));
+        const uint32_t p[4] = {ex.x, ex.y, ex.z, ex.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            acc[2 * e] = fmaf(__uint_as_float(p[e] << 16), w, acc[2 * e]);
+            acc[2 * e + 1] = fmaf(__uint_as_float(p[e] & 0xffff0000u), w, acc[2 * e + 1]);
+        }
+    }
+    uint32_t r[4];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) r[e] = (uint32_t)f2bf_bits(acc[2 * e]) | ((uint32_t)f2bf_bits(acc[2 * e + 1]) << 16);
+    out[i] = make_uint4(r[0], r[1], r[2], r[3]);
+}
+
 // weights null: factors of one. extra [T, N] and logit (one number a token, rows ld_logit elements apart, of type
 // logit_dtype: the rows' own or 32-bit) may be null: no further term
 extern "C" int ra_moe_combine_extra(const void* y, const float* weights, void* out, int T, int top, int N,
@@ -560,6 +640,16 @@ extern "C" int ra_moe_combine_extra(const void* y, const float* weights, void* o
     if ((extra == nullptr) != (logit == nullptr) || (extra != nullptr && ld_logit < 1) ||
         (logit_dtype != dtype && logit_dtype != RA_DTYPE_F32))
         return RA_ERR_ARG;
+    if (dtype == RA_DTYPE_BF16 && N % 8 == 0 && (((size_t)y | (size_t)out | (size_t)extra) & 15) == 0) {
+        const dim3 grid8((unsigned)((total / 8 + 255) / 256));
+#define MOE_COMBINE8(L_)                                                                                                     \
+    hipLaunchKernelGGL((moe_combine_bf16x8_kernel<L_>), grid8, dim3(256), 0, (hipStream_t)stream, (const uint4*)y, weights,  \
+                       (uint4*)out, top, N / 8, total / 8, (const uint4*)extra, (const L_*)logit, ld_logit)
+        if (logit_dtype == RA_DTYPE_BF16) MOE_COMBINE8(bf16);
+        else MOE_COMBINE8(float);
+#undef MOE_COMBINE8
+        return ra_launch_status();
+    }
     dim3 block(256), grid((unsigned)((total + 255) / 256));
 #define MOE_COMBINE(T_, L_)                                                                                              \
     hipLaunchKernelGGL((moe_combine_kernel<T_, L_>), grid, block, 0, (hipStream_t)stream, (const T_*)y, weights, (T_*)out, \
