@@ -1,5 +1,5 @@
 // Token choice from fp32 logits: greedy, temperature, top-k, top-p; and the chosen token's
-// log-probability under the raw logits. One block per row.
+// log-probability under the raw logits. One block per row; several for few rows of a large vocabulary (sample_parts).
 //
 // What the reference samples with (rollout/model.py:15-61): temperature <= 0 is argmax;
 // otherwise logits / temperature; keep the top_k largest; over the kept values in descending
@@ -18,8 +18,10 @@
 // largest) are first collected into a list in LDS, in vocabulary order; if they fit, and if the
 // thresholds lie among them (k is at most their number; their mass is more than top_p of the whole),
 // the thresholds are searched and the token is drawn from the list alone, which takes microseconds.
-// Otherwise (a flat row, a large k, top_p near 1) the searches go over the whole row, pass by pass.
+// Otherwise (a flat row, a large k, top_p near 1) the searches go over the whole row, in two passes as a rule.
 // Which way a row goes depends on that row alone.
+// One block a row is bound by its chain of barriers and short sums (a peaked row of 16,384: 20 us, 6 of them for the
+// maximum) and, flat, by one CU's arithmetic (32,000: 41 us; before the searches of two passes 54, and peaked 32).
 #include "common.h"
 
 #define SAMPLE_THREADS 1024
@@ -27,6 +29,8 @@
 #define CAND_PER_WAVE 512                                        // list entries of one wave's run of the row
 #define CAND_OWN (CAND_WAVES * CAND_PER_WAVE / SAMPLE_THREADS)   // entries a thread looks after in a search: 8
 #define CAND_SPAN 16.0f
+#define WEIGHS_NOTHING 28.5f      // (max - x) / T from which to_fixed(exp(-that)) is 0: 2^-41 is exp(-28.42)
+#define TOP_K_SPAN 32.0f          // logits: top-k beyond the list is searched closely so far from the largest
 #define SAMPLE_BLOCKS 64                                         // blocks of 256 tokens in a wave's run whose masses are kept
 
 __device__ __forceinline__ uint32_t order_key(float f) {
@@ -102,7 +106,7 @@ __device__ __forceinline__ fixed_t block_sum_fixed(fixed_t v, fixed_t* wsum) {
 // pass visits).
 #define FIXED_UNKNOWN (~0ull)
 template <typename Visit>
-__device__ uint32_t search_threshold(Visit visit, int tid, uint32_t lo, uint32_t hi, fixed_t limit, fixed_t* fx,
+__device__ __noinline__ uint32_t search_threshold(Visit visit, int tid, uint32_t lo, uint32_t hi, fixed_t limit, fixed_t* fx,
                                      fixed_t* wsum, int* sh_b, fixed_t* sh_above, fixed_t* above = nullptr,
                                      fixed_t* at = nullptr) {
     fixed_t at_t = FIXED_UNKNOWN;
@@ -155,6 +159,95 @@ __device__ uint32_t search_threshold(Visit visit, int tid, uint32_t lo, uint32_t
     return lo;
 }
 
+// The same threshold among few tokens (OWN a thread), in one pass where the logits spread: run_of(key), 0 for the
+// largest logits up to SEARCH_BUCKETS - 1, is a run of equal width in the logit, token(e, key) tells a token's key and
+// gives its measure (0: no token), limit_of(sum) the limit for their sum. What falls into the boundary's run, a handful, every wave puts in order
+// for itself. (By halving the keys' range, as above, 300 tokens took three passes, 14 us of a row's 31; the row takes 20 this way.)
+// Gives whether there is a boundary among them; `key` is left alone if its run holds more than 64 tokens (many that tie):
+// then found == FEW_CROWDED, and the caller searches as above. limit: what limit_of gave.
+#define SEARCH_FEW 64
+enum { FEW_NONE = 0, FEW_FOUND = 1, FEW_CROWDED = 2 };
+struct FewLds { fixed_t mass[SEARCH_FEW], above; uint32_t key[SEARCH_FEW]; int run, n; };
+// The masses of the runs are in fx: finds the run in which their sum, from run 0 on, passes the limit (few->run; -1:
+// none), and the sum before it. Barriers before and after.
+template <typename Limit>
+__device__ __forceinline__ int crossing_run(Limit limit_of, int tid, const fixed_t* fx, fixed_t* wsum, FewLds* few,
+                                            fixed_t& limit) {
+    const int wave = tid >> 6, lane = tid & 63;
+    __syncthreads();
+    const fixed_t f0 = fx[2 * tid], f1 = fx[2 * tid + 1];
+    fixed_t upto = f0 + f1;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const fixed_t t = __shfl_up(upto, o, 64);
+        if (lane >= o) upto += t;
+    }
+    if (lane == 63) wsum[wave] = upto;
+    __syncthreads();
+    fixed_t sum = 0ull, before = 0ull;
+#pragma unroll
+    for (int w = 0; w < CAND_WAVES; ++w) {
+        const fixed_t t = wsum[w];
+        sum += t;
+        before += w < wave ? t : 0ull;
+    }
+    limit = limit_of(sum);
+    const fixed_t b1 = before + upto - f1, b0 = b1 - f0;              // measure before runs 2 tid + 1 and 2 tid
+    if (b0 <= limit && b1 > limit) { few->run = 2 * tid; few->above = b0; }
+    if (b1 <= limit && b1 + f1 > limit) { few->run = 2 * tid + 1; few->above = b1; }
+    __syncthreads();
+    return few->run;
+}
+__device__ __forceinline__ void clear_runs(int tid, fixed_t* fx, FewLds* few) {
+    fx[2 * tid] = 0ull;
+    fx[2 * tid + 1] = 0ull;
+    if (tid == 0) { few->run = -1; few->n = 0; }
+    __syncthreads();
+}
+template <int OWN, typename Run, typename Token, typename Limit>
+__device__ __forceinline__ int search_few(Run run_of, Token token, Limit limit_of, int tid,
+                                          fixed_t* fx, fixed_t* wsum, FewLds* few, uint32_t& key, fixed_t& limit,
+                                          fixed_t& above, fixed_t& at) {
+    const int lane = tid & 63;
+    clear_runs(tid, fx, few);
+#pragma unroll 4
+    for (int e = 0; e < OWN; ++e) {
+        uint32_t k;
+        const fixed_t m = token(e, k);
+        if (m) atomicAdd(&fx[run_of(k)], m);
+    }
+    const int run = crossing_run(limit_of, tid, fx, wsum, few, limit);
+    if (run < 0) return FEW_NONE;
+#pragma unroll 4
+    for (int e = 0; e < OWN; ++e) {
+        uint32_t k;
+        const fixed_t m = token(e, k);
+        if (m && run_of(k) == run) {
+            const int i = atomicAdd(&few->n, 1);
+            if (i < SEARCH_FEW) { few->key[i] = k; few->mass[i] = m; }
+        }
+    }
+    __syncthreads();
+    const int n = few->n;
+    if (n > SEARCH_FEW) return FEW_CROWDED;
+    const uint32_t mine = lane < n ? few->key[lane] : 0u;
+    fixed_t over = few->above, same = 0ull;
+    for (int j = 0; j < n; ++j) {
+        const uint32_t k = few->key[j];
+        const fixed_t m = few->mass[j];
+        over += k > mine ? m : 0ull;
+        same += k == mine ? m : 0ull;
+    }
+    uint32_t t = lane < n && over <= limit ? mine : 0xffffffffu;     // the smallest with at most the limit above it
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) t = min(t, (uint32_t)__shfl_xor((int)t, o, 64));
+    const int who = __ffsll((long long)__ballot(lane < n && mine == t)) - 1;
+    key = t;
+    above = __shfl(over, who, 64);
+    at = __shfl(same, who, 64);
+    return FEW_FOUND;
+}
+
 // Of the tokens that tie at a boundary, the first `stay` in vocabulary order stay: returns the index of the
 // last of them (`upto` if all of them stay). count_ties(f) calls f(index) for every tying token of this thread
 // with index <= upto. One pass counts them; only if they are more than may stay, the index is searched.
@@ -174,7 +267,7 @@ __device__ __noinline__ int tie_cut(Ties ties, int tid, int V, unsigned long lon
     if (stay == 0ull) return -1;
     // the stay-th tie from the front: the smallest t with at most stay - 1 ties at keys V - 1 - index above it
     const uint32_t t = search_threshold(
-        [&](uint32_t lo, uint32_t hi, auto add) {
+        [=](uint32_t lo, uint32_t hi, auto add) {
             ties([&](int i) {
                 const uint32_t key = (uint32_t)(V - 1 - i);
                 if (key > lo && key <= hi) add(key, 1ull << 40);
@@ -188,18 +281,23 @@ __device__ __noinline__ int tie_cut(Ties ties, int tid, int V, unsigned long lon
 // Gives the wave in whose run the running sum passes u times the total (the last run with kept mass if it
 // never does), the sum before that run and the target. Every thread computes the same.
 __device__ __forceinline__ void pick_wave(const float* wmass, float u, int& owner, float& before, float& target) {
-    float total = 0.f;
-    for (int w = 0; w < CAND_WAVES; ++w) total += wmass[w];
+    float m[CAND_WAVES], total = 0.f;
+#pragma unroll
+    for (int w = 0; w < CAND_WAVES; ++w) m[w] = wmass[w];            // (all on their way at once)
+#pragma unroll
+    for (int w = 0; w < CAND_WAVES; ++w) total += m[w];
     target = u * total;
     float run = 0.f;
     owner = -1;
     before = 0.f;
+    bool passed = false;
+#pragma unroll
     for (int w = 0; w < CAND_WAVES; ++w) {
-        if (wmass[w] > 0.f) {
+        if (!passed && m[w] > 0.f) {
             owner = w;
             before = run;
-            if (run + wmass[w] > target) break;
-            run += wmass[w];
+            passed = run + m[w] > target;
+            run += m[w];
         }
     }
 }
@@ -214,33 +312,55 @@ __device__ __forceinline__ float wave_running_sum(float v, int lane) {
     return v;
 }
 
-__global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
-    const float* __restrict__ logits, int V, const float* __restrict__ temperature,
-    const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ u,
-    int* __restrict__ out, int* __restrict__ path) {
-    extern __shared__ __attribute__((aligned(16))) float dyn[];           // the list (64 KB), then the search's runs (16 KB)
-    __shared__ float scratch[16];
-    __shared__ float wmass[CAND_WAVES];
-    __shared__ fixed_t wsum[CAND_WAVES];
-    __shared__ fixed_t sh_above;
-    __shared__ int sh_b;
-    fixed_t* fx = reinterpret_cast<fixed_t*>(dyn + 2 * CAND_WAVES * CAND_PER_WAVE);
-    const int row = blockIdx.x, tid = threadIdx.x;
-    const float* x = logits + (size_t)row * V;
+// ---- Large vocabularies, few rows: one block a row leaves the chip idle (a flat row of 151,936 takes it 111 us, all
+// of it one CU's arithmetic over five passes; 45 this way), so kernels over CAND_WAVES * parts blocks a row find what the
+// last one, sample_kernel, needs:
+//   sample_top      largest logit, first index that holds it, smallest, sum of exp, of every part of the row
+//   sample_span     marks (a bit a token) of those within CAND_SPAN of the largest, their number and mass; for top-p
+//                   alone the masses of HIST runs of equal width in the logit, which hold every token that weighs anything
+//   sample_gather   flat rows under top-p alone: the tokens of the run in which the boundary lies
+//   sample_settle   the boundary itself, searched among those (one block a row)
+//   sample_masses   the kept mass of every 256 tokens
+// Whole numbers are added, so that thresholds are the ones that the passes over the row find, bit for bit, and the
+// masses of 256 tokens are summed as the draw sums them. Rows that need none of a kernel leave it at once; what none
+// of them settles (top-k beyond the list, a run with more than GATHER tokens, a largest logit that is no number) goes
+// the way it goes without them.
+#define HIST 512
+#define GATHER 8192
+#define PART_THREADS 256
+#define MAX_PARTS 64
 
-    // ---- one pass: running maximum, first index that holds it, sum of exp(x - maximum)
-    float mx = -INFINITY, se = 0.f;
-    int arg = 0x7fffffff;
-    for_each_logit(x, V, tid, [&](int i, float v) {
-        if (v > mx) {
-            se = se * __expf(mx - v) + 1.0f;          // mx = -inf: se is 0 and stays finite
-            mx = v;
-            arg = i;
-        } else {
-            se += __expf(v - mx);
-        }
-    });
-    // merge (mx, se, arg) over the wave, then over the waves in wave order
+struct RowPart { float mx, se, mn; int arg, count; float rest; fixed_t mass; };
+struct RowState { uint32_t keep_key; int tie_limit, status, gathered; };
+enum { ROW_OPEN = 0, ROW_SETTLED = 1 };
+struct RowTop { float mx, se, mn; int arg; };
+
+struct SampleWs {
+    char* base;
+    size_t row_bytes, marks_at, masses_at;
+    static constexpr size_t HIST_AT = MAX_PARTS * sizeof(RowPart), STATE_AT = HIST_AT + HIST * sizeof(fixed_t),
+                            LIST_AT = STATE_AT + sizeof(RowState);
+    __device__ char* at(int row) const { return base + (size_t)row * row_bytes; }
+    __device__ RowPart* parts(int row) const { return reinterpret_cast<RowPart*>(at(row)); }
+    __device__ fixed_t* hist(int row) const { return reinterpret_cast<fixed_t*>(at(row) + HIST_AT); }
+    __device__ RowState& state(int row) const { return *reinterpret_cast<RowState*>(at(row) + STATE_AT); }
+    __device__ uint2* list(int row) const { return reinterpret_cast<uint2*>(at(row) + LIST_AT); }      // key, token
+    __device__ fixed_t* marks(int row) const { return reinterpret_cast<fixed_t*>(at(row) + marks_at); } // four words per 256
+    __device__ float* masses(int row) const { return reinterpret_cast<float*>(at(row) + masses_at); }
+};
+
+static SampleWs sample_ws(char* base, int V) {
+    const size_t blocks = (size_t)(V + 255) / 256;
+    SampleWs w{base, 0, SampleWs::LIST_AT + GATHER * sizeof(uint2), 0};
+    w.masses_at = w.marks_at + blocks * 4 * sizeof(fixed_t);
+    w.row_bytes = (w.masses_at + blocks * sizeof(float) + 255) / 256 * 256;
+    return w;
+}
+
+__device__ __forceinline__ bool finite(float f) { return fabsf(f) < INFINITY; }
+
+// merges (mx, se, arg) over the lanes of a wave: every lane gets the same
+__device__ __forceinline__ void merge_top(float& mx, float& se, int& arg) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         const float m2 = __shfl_xor(mx, o, 64), s2 = __shfl_xor(se, o, 64);
@@ -252,22 +372,464 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         se = s1 + s3;                                 // the same two numbers in both lanes of a pair
         mx = m;
     }
-    __shared__ float wm[16], ws[16];
-    __shared__ int wa[16];
-    if ((tid & 63) == 0) { wm[tid >> 6] = mx; ws[tid >> 6] = se; wa[tid >> 6] = arg; }
+}
+
+// The whole row's from its parts' (n <= 64); every wave does it for itself.
+__device__ __forceinline__ RowTop row_top(const RowPart* parts, int n) {
+    const int lane = threadIdx.x & 63;
+    RowTop t{-INFINITY, 0.f, INFINITY, 0x7fffffff};
+    if (lane < n) t = RowTop{parts[lane].mx, parts[lane].se, parts[lane].mn, parts[lane].arg};
+    merge_top(t.mx, t.se, t.arg);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) t.mn = fminf(t.mn, __shfl_xor(t.mn, o, 64));
+    return t;
+}
+
+// One part's tokens: run (part / parts) of the row, which is what one wave of sample_kernel has, cut into `parts`
+// pieces of whole 256s. f(token of the lane's first, its four logits, -inf beyond the end; number of the 256).
+struct PartRange { int beg, end; };
+__device__ __forceinline__ PartRange part_range(int V, int part, int parts) {
+    const int seg = ((V + CAND_WAVES - 1) / CAND_WAVES + 255) / 256 * 256;
+    const int piece = (seg / 256 + parts - 1) / parts * 256;
+    const int run = part / parts, k = part - run * parts;
+    const int end = min(V, run * seg + min(seg, (k + 1) * piece));
+    return {min(end, run * seg + k * piece), end};
+}
+template <typename F>
+__device__ __forceinline__ void for_each_256(const float* __restrict__ x, int V, PartRange r, F f) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const bool vec = (V & 3) == 0 && (reinterpret_cast<uintptr_t>(x) & 15) == 0;
+    constexpr int STEP = 256 * (PART_THREADS / 64), AHEAD = 4;
+    for (int b0 = r.beg + 256 * wave; b0 < r.end; b0 += AHEAD * STEP) {
+        float a[AHEAD][4];
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j) {
+            const int i = b0 + j * STEP + 4 * lane;
+            if (vec) {
+                float4 t = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+                if (i < r.end) t = *reinterpret_cast<const float4*>(x + i);
+                a[j][0] = t.x; a[j][1] = t.y; a[j][2] = t.z; a[j][3] = t.w;
+            } else {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) a[j][c] = i + c < r.end ? x[i + c] : -INFINITY;
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < AHEAD; ++j)
+            if (b0 + j * STEP < r.end) f(b0 + j * STEP + 4 * lane, a[j], (b0 + j * STEP) / 256);
+    }
+}
+
+__global__ __launch_bounds__(PART_THREADS) void sample_top_kernel(const float* __restrict__ logits, int V, SampleWs ws,
+                                                                  int parts) {
+    const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x;
+    for (int i = part * PART_THREADS + tid; i < HIST; i += gridDim.x * PART_THREADS) ws.hist(row)[i] = 0ull;
+    if (part == 0 && tid == 0) ws.state(row).gathered = 0;
+    const PartRange r = part_range(V, part, parts);
+    float mx = -INFINITY, se = 0.f, mn = INFINITY;
+    int arg = 0x7fffffff;
+    for_each_256(logits + (size_t)row * V, V, r, [&](int i, const float (&a)[4], int) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            if (i + c >= r.end) continue;
+            const float v = a[c];
+            mn = fminf(mn, v);
+            if (v > mx) {
+                se = se * __expf(mx - v) + 1.0f;      // mx = -inf: se is 0 and stays finite
+                mx = v;
+                arg = i + c;
+            } else {
+                se += __expf(v - mx);
+            }
+        }
+    });
+    merge_top(mx, se, arg);
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) mn = fminf(mn, __shfl_xor(mn, o, 64));
+    __shared__ RowTop w[PART_THREADS / 64];
+    if ((tid & 63) == 0) w[tid >> 6] = RowTop{mx, se, mn, arg};
     __syncthreads();
-    float gmax = wm[0];
-    int argmax = wa[0];
-    for (int w = 1; w < SAMPLE_THREADS / 64; ++w) {
-        if (wm[w] > gmax) { gmax = wm[w]; argmax = wa[w]; }
-        else if (wm[w] == gmax) argmax = min(argmax, wa[w]);
+    if (tid != 0) return;
+    for (int k = 1; k < PART_THREADS / 64; ++k) {
+        const float m = fmaxf(mx, w[k].mx);
+        const float s1 = (mx == -INFINITY) ? 0.f : se * __expf(mx - m);
+        const float s2 = (w[k].mx == -INFINITY) ? 0.f : w[k].se * __expf(w[k].mx - m);
+        if (w[k].mx > mx) arg = w[k].arg;
+        else if (w[k].mx == mx) arg = min(arg, w[k].arg);
+        mx = m;
+        se = s1 + s2;
+        mn = fminf(mn, w[k].mn);
+    }
+    RowPart& p = ws.parts(row)[part];
+    p.mx = mx; p.se = se; p.mn = mn; p.arg = arg;
+}
+
+// The run of equal width in the logit that a token belongs to: 0 holds the largest. -1: it weighs nothing.
+struct Runs {
+    float mx, inv_t, scale;
+    __device__ Runs(const RowTop& t, float temp) : mx(t.mx), inv_t(1.0f / temp) {
+        scale = fminf((float)HIST / fminf(WEIGHS_NOTHING * temp, t.mx - t.mn), 1e30f);      // (one value only: 1e30, all in run 0)
+    }
+    __device__ int operator()(float v) const {
+        return (mx - v) * inv_t < WEIGHS_NOTHING ? (int)fminf((mx - v) * scale, (float)(HIST - 1)) : -1;
+    }
+};
+
+__global__ __launch_bounds__(PART_THREADS) void sample_span_kernel(
+    const float* __restrict__ logits, int V, const float* __restrict__ temperature, const int* __restrict__ top_k,
+    const float* __restrict__ top_p, SampleWs ws, int parts) {
+    const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x, lane = tid & 63;
+    const float temp = temperature[row];
+    const int k = top_k[row];
+    const bool want_k = k > 0 && k < V, want_p = top_p[row] < 1.0f;
+    if (!(temp > 0.f) || !(want_k || want_p)) return;
+    const RowTop top = row_top(ws.parts(row), gridDim.x);
+    if (!finite(top.mx)) return;
+    const bool masses = want_p && !want_k;
+    const Runs run_of(top, temp);
+    const float gmax = top.mx, inv_t = 1.0f / temp, cut = gmax - CAND_SPAN * temp;
+    __shared__ fixed_t h[HIST];
+    for (int i = tid; i < HIST; i += PART_THREADS) h[i] = 0ull;
+    __syncthreads();
+    int count = 0;
+    float rest = 0.f;
+    fixed_t mass = 0ull;
+    const PartRange r = part_range(V, part, parts);
+    for_each_256(logits + (size_t)row * V, V, r, [&](int i, const float (&a)[4], int b) {
+        fixed_t mark = 0ull;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const bool in = a[c] >= cut;
+            const unsigned long long m = __ballot(in);
+            count += __popcll(m);
+            if (lane == c) mark = m;
+            if (masses && i + c < r.end) {
+                const float weight = __expf((a[c] - gmax) * inv_t);
+                const int at = run_of(a[c]);
+                if (at >= 0) {
+                    const fixed_t f = to_fixed(weight);
+                    atomicAdd(&h[at], f);
+                    mass += in ? f : 0ull;
+                }
+                rest += in ? 0.f : weight;
+            }
+        }
+        if (lane < 4) ws.marks(row)[4 * (size_t)b + lane] = mark;
+    });
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        rest += __shfl_xor(rest, o, 64);
+        mass += __shfl_xor(mass, o, 64);
+    }
+    __shared__ int wc[PART_THREADS / 64];
+    __shared__ float wr[PART_THREADS / 64];
+    __shared__ fixed_t wm[PART_THREADS / 64];
+    if (lane == 0) { wc[tid >> 6] = count; wr[tid >> 6] = rest; wm[tid >> 6] = mass; }
+    __syncthreads();
+    if (masses)
+        for (int i = tid; i < HIST; i += PART_THREADS)
+            if (h[i]) atomicAdd(&ws.hist(row)[i], h[i]);
+    if (tid != 0) return;
+    for (int w = 1; w < PART_THREADS / 64; ++w) { count += wc[w]; rest += wr[w]; mass += wm[w]; }
+    RowPart& p = ws.parts(row)[part];
+    p.count = count; p.rest = rest; p.mass = mass;
+}
+
+// Whether a row under top-p alone is one for the searches over the whole row: too many candidates for the list in
+// one run, or less than top_p of the mass among them. Every wave finds it for itself.
+__device__ __forceinline__ bool row_is_flat(const RowPart* all, int parts, float gmax, float temp, float top_p) {
+    const int lane = threadIdx.x & 63;
+    if (order_key(gmax - CAND_SPAN * temp) == 0u) return true;
+    int count = 0;
+    if (lane < CAND_WAVES)
+        for (int j = 0; j < parts; ++j) count += all[lane * parts + j].count;
+    if (__ballot(count > CAND_PER_WAVE)) return true;
+    fixed_t mass = lane < CAND_WAVES * parts ? all[lane].mass : 0ull;
+    float rest = lane < CAND_WAVES * parts ? all[lane].rest : 0.f;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        mass += __shfl_xor(mass, o, 64);
+        rest += __shfl_xor(rest, o, 64);
+    }
+    const fixed_t z = mass + (fixed_t)((double)rest * (double)FIXED_ONE_F);
+    return mass <= (fixed_t)((double)top_p * (double)z);
+}
+
+// The run in which the top-p boundary lies, the mass of the runs before it, and what may lie above the boundary.
+struct Boundary { int run; fixed_t above, limit; };
+__device__ __forceinline__ Boundary boundary_run(const fixed_t* hist, float top_p) {
+    const int lane = threadIdx.x & 63;
+    constexpr int EACH = HIST / 64;
+    fixed_t h[EACH], mine = 0ull;
+#pragma unroll
+    for (int e = 0; e < EACH; ++e) { h[e] = hist[lane * EACH + e]; mine += h[e]; }
+    fixed_t upto = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const fixed_t t = __shfl_up(upto, o, 64);
+        if (lane >= o) upto += t;
+    }
+    const fixed_t z = __shfl(upto, 63, 64);
+    const fixed_t limit = (fixed_t)((double)top_p * (double)z);
+    const unsigned long long past = __ballot(upto > limit);
+    const int who = past ? __ffsll((long long)past) - 1 : 63;
+    fixed_t above = upto - mine;
+    int run = lane * EACH;
+#pragma unroll
+    for (int e = 0; e < EACH - 1; ++e)
+        if (run == lane * EACH + e && above + h[e] <= limit) { above += h[e]; ++run; }
+    return {__shfl(run, who, 64), __shfl(above, who, 64), limit};
+}
+
+__global__ __launch_bounds__(PART_THREADS) void sample_gather_kernel(
+    const float* __restrict__ logits, int V, const float* __restrict__ temperature, const int* __restrict__ top_k,
+    const float* __restrict__ top_p, SampleWs ws, int parts) {
+    const int row = blockIdx.y, part = blockIdx.x, lane = threadIdx.x & 63;
+    const float temp = temperature[row], p = top_p[row];
+    const int k = top_k[row];
+    if (!(temp > 0.f) || !(p < 1.0f) || (k > 0 && k < V)) return;
+    const RowTop top = row_top(ws.parts(row), gridDim.x);
+    if (!finite(top.mx) || !row_is_flat(ws.parts(row), parts, top.mx, temp, p)) return;
+    const Boundary b = boundary_run(ws.hist(row), p);
+    const Runs run_of(top, temp);
+    const PartRange r = part_range(V, part, parts);
+    for_each_256(logits + (size_t)row * V, V, r, [&](int i, const float (&a)[4], int) {
+        int before = 0, all = 0;
+        bool in[4];
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            in[c] = i + c < r.end && run_of(a[c]) == b.run;
+            const unsigned long long m = __ballot(in[c]);
+            before += __popcll(m & ((1ull << lane) - 1ull));
+            all += __popcll(m);
+        }
+        if (all == 0) return;
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&ws.state(row).gathered, all);
+        at = __shfl(at, 0, 64) + before;
+#pragma unroll
+        for (int c = 0; c < 4; ++c)
+            if (in[c]) {
+                if (at < GATHER) ws.list(row)[at] = make_uint2(order_key(a[c]), (uint32_t)(i + c));
+                ++at;
+            }
+    });
+}
+
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_settle_kernel(
+    int V, const float* __restrict__ temperature, const int* __restrict__ top_k, const float* __restrict__ top_p,
+    SampleWs ws, int parts) {
+    __shared__ fixed_t fx[SEARCH_BUCKETS], wsum[CAND_WAVES], sh_above;
+    __shared__ int sh_b;
+    __shared__ FewLds few;
+    const int row = blockIdx.x, tid = threadIdx.x;
+    const float temp = temperature[row], p = top_p[row];
+    const int k = top_k[row];
+    RowState& st = ws.state(row);
+    const bool want_k = k > 0 && k < V, want_p = p < 1.0f;
+    const RowTop top = row_top(ws.parts(row), CAND_WAVES * parts);
+    if (!(temp > 0.f) || want_k || !finite(top.mx)) {
+        if (tid == 0) st.status = ROW_OPEN;
+        return;
+    }
+    if (!want_p) {                                     // all of it is kept
+        if (tid == 0) { st.keep_key = 0u; st.tie_limit = 0x7fffffff; st.status = ROW_SETTLED; }
+        return;
+    }
+    const int n = st.gathered;
+    if (n > GATHER || n == 0 || !row_is_flat(ws.parts(row), parts, top.mx, temp, p)) {
+        if (tid == 0) st.status = ROW_OPEN;
+        return;
+    }
+    const Boundary b = boundary_run(ws.hist(row), p);
+    const float inv_t = 1.0f / temp;
+    constexpr int OWN = GATHER / SAMPLE_THREADS;
+    const uint2* list = ws.list(row);
+    auto entry = [list, tid, n](int e, uint32_t& key, int& i) {
+        const int at = tid + e * SAMPLE_THREADS;
+        const uint2 t = at < n ? list[at] : make_uint2(0u, 0u);
+        key = t.x;
+        i = (int)t.y;
+        return at < n;
+    };
+    auto weighed = [=](int e, uint32_t& key) {
+        int i;
+        return entry(e, key, i) ? to_fixed(__expf((key_value(key) - top.mx) * inv_t)) : 0ull;
+    };
+    const Runs runs(top, temp);
+    fixed_t above = 0ull, at = FIXED_UNKNOWN, limit_in;
+    uint32_t keep = 0u;
+    if (search_few<OWN>(
+            [=](uint32_t key) {                        // the run's width, cut once more
+                const float d = ((top.mx - key_value(key)) * runs.scale - (float)b.run) * (float)SEARCH_BUCKETS;
+                return (int)fminf(fmaxf(d, 0.f), (float)(SEARCH_BUCKETS - 1));
+            },
+            weighed, [=](fixed_t) { return b.limit - b.above; }, tid, fx, wsum, &few, keep, limit_in, above, at) != FEW_FOUND) {
+        __syncthreads();
+        keep = search_threshold(
+            [=](uint32_t lo, uint32_t hi, auto add) {
+                for (int e = 0; e < OWN; ++e) {
+                    uint32_t key;
+                    const fixed_t m = weighed(e, key);
+                    if (m && key > lo && key <= hi) add(key, m);
+                }
+            },
+            tid, 0u, order_key(top.mx), b.limit - b.above, fx, wsum, &sh_b, &sh_above, &above, &at);
+    }
+    // of the tokens that tie with the boundary value, as in sample_kernel
+    const fixed_t each = to_fixed(__expf((key_value(keep) - top.mx) * inv_t));
+    const unsigned long long stay = each ? (b.limit - b.above - above) / each + 1ull : ~0ull;
+    const int limit = tie_cut(
+        [entry, keep](auto f) {
+            for (int e = 0; e < OWN; ++e) {
+                uint32_t key;
+                int i;
+                if (entry(e, key, i) && key == keep) f(i);
+            }
+        },
+        tid, V, stay, 0x7fffffff, at != FIXED_UNKNOWN && each ? at / each : FIXED_UNKNOWN, fx, wsum, &sh_b, &sh_above);
+    if (tid == 0) { st.keep_key = keep; st.tie_limit = limit; st.status = ROW_SETTLED; }
+}
+
+__global__ __launch_bounds__(PART_THREADS) void sample_masses_kernel(const float* __restrict__ logits, int V,
+                                                                     const float* __restrict__ temperature, SampleWs ws,
+                                                                     int parts) {
+    const int row = blockIdx.y, lane = threadIdx.x & 63;
+    const RowState st = ws.state(row);
+    if (st.status != ROW_SETTLED) return;
+    const float gmax = row_top(ws.parts(row), gridDim.x).mx, inv_t = 1.0f / temperature[row];
+    const PartRange r = part_range(V, blockIdx.x, parts);
+    for_each_256(logits + (size_t)row * V, V, r, [&](int i, const float (&a)[4], int b) {
+        float m = 0.f;
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const uint32_t key = order_key(a[c]);
+            const bool kept = i + c < r.end && (key > st.keep_key || (key == st.keep_key && i + c <= st.tie_limit));
+            m += kept ? __expf((a[c] - gmax) * inv_t) : 0.f;
+        }
+        m = wave_sum(m);
+        if (lane == 0) ws.masses(row)[b] = m;
+    });
+}
+
+// A wave's part of the list from the marks of its run of the row (n 256s, at most SAMPLE_BLOCKS = 64: one a lane), in
+// vocabulary order: entry e is the e-th mark. Gives the number of marks; nothing is written if they are too many.
+__device__ __forceinline__ int list_of_marks(const fixed_t* __restrict__ marks, int n, const float* __restrict__ x,
+                                             int beg, int lane, float* cv, int* ci) {
+    int mine = 0;
+    if (lane < n)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) mine += __popcll(marks[4 * lane + c]);
+    int upto = mine;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int t = __shfl_up(upto, o, 64);
+        if (lane >= o) upto += t;
+    }
+    const int all = __shfl(upto, 63, 64);
+    if (all > CAND_PER_WAVE) return all;
+    for (int e0 = 0; e0 < all; e0 += 64) {
+        const int e = e0 + lane;
+        int b = 0;                                     // the first 256 with more than e marks up to its end
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+            if (__shfl(upto, b + o - 1, 64) <= e) b += o;
+        const int left = e - __shfl(upto - mine, b, 64);       // (all lanes take part in the shuffles)
+        if (e < all) {
+            fixed_t m[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) m[c] = marks[4 * b + c];
+            int l = 0, below = 0;                      // the lane of the 256 that holds it: marks of the lanes before it <= left
+#pragma unroll
+            for (int o = 32; o > 0; o >>= 1) {
+                const unsigned long long mask = (1ull << (l + o)) - 1ull;
+                int c2 = 0;
+#pragma unroll
+                for (int c = 0; c < 4; ++c) c2 += __popcll(m[c] & mask);
+                if (c2 <= left) { l += o; below = c2; }
+            }
+            int want = left - below, c = 0;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int bit = (int)((m[q] >> l) & 1ull);
+                if (bit && want == 0) c = q;
+                want -= bit;
+            }
+            const int token = beg + 256 * b + 4 * l + c;
+            cv[e] = x[token];
+            ci[e] = token;
+        }
+    }
+    return all;
+}
+
+// PREPARED: the row's sums, candidates and block masses were found by the kernels above (ws); else this block finds
+// them itself.
+template <bool PREPARED>
+__global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
+    const float* __restrict__ logits, int V, const float* __restrict__ temperature,
+    const int* __restrict__ top_k, const float* __restrict__ top_p, const float* __restrict__ u,
+    int* __restrict__ out, int* __restrict__ path, SampleWs ws_all, int parts) {
+    extern __shared__ __attribute__((aligned(16))) float dyn[];           // the list (64 KB), then the search's runs (16 KB)
+    __shared__ float scratch[16];
+    __shared__ float wmass[CAND_WAVES];
+    __shared__ fixed_t wsum[CAND_WAVES];
+    __shared__ fixed_t sh_above;
+    __shared__ int sh_b;
+    __shared__ FewLds few;
+    fixed_t* fx = reinterpret_cast<fixed_t*>(dyn + 2 * CAND_WAVES * CAND_PER_WAVE);
+    const int row = blockIdx.x, tid = threadIdx.x;
+    const float* x = logits + (size_t)row * V;
+
+    float gmax, total_e = 0.f;
+    int argmax;
+    [[maybe_unused]] const int n_parts = CAND_WAVES * parts;
+    if constexpr (PREPARED) {
+        const RowTop t = row_top(ws_all.parts(row), n_parts);
+        gmax = t.mx;
+        argmax = t.arg;
+        total_e = t.se;
+    } else {
+        // ---- one pass: running maximum, first index that holds it, sum of exp(x - maximum)
+        float mx = -INFINITY, se = 0.f;
+        int arg = 0x7fffffff;
+        for_each_logit(x, V, tid, [&](int i, float v) {
+            if (v > mx) {
+                se = se * __expf(mx - v) + 1.0f;          // mx = -inf: se is 0 and stays finite
+                mx = v;
+                arg = i;
+            } else {
+                se += __expf(v - mx);
+            }
+        });
+        // merge (mx, se, arg) over the wave, then over the waves in wave order
+    #pragma unroll
+        for (int o = 32; o > 0; o >>= 1) {
+            const float m2 = __shfl_xor(mx, o, 64), s2 = __shfl_xor(se, o, 64);
+            const int a2 = __shfl_xor(arg, o, 64);
+            const float m = fmaxf(mx, m2);
+            const float s1 = (mx == -INFINITY) ? 0.f : se * __expf(mx - m);
+            const float s3 = (m2 == -INFINITY) ? 0.f : s2 * __expf(m2 - m);
+            arg = (m2 > mx) ? a2 : ((m2 == mx) ? min(arg, a2) : arg);
+            se = s1 + s3;                                 // the same two numbers in both lanes of a pair
+            mx = m;
+        }
+        __shared__ float wm[16], ws[16];
+        __shared__ int wa[16];
+        if ((tid & 63) == 0) { wm[tid >> 6] = mx; ws[tid >> 6] = se; wa[tid >> 6] = arg; }
+        __syncthreads();
+        gmax = wm[0];
+        argmax = wa[0];
+        for (int w = 1; w < SAMPLE_THREADS / 64; ++w) {
+            if (wm[w] > gmax) { gmax = wm[w]; argmax = wa[w]; }
+            else if (wm[w] == gmax) argmax = min(argmax, wa[w]);
+        }
+        for (int w = 0; w < SAMPLE_THREADS / 64; ++w)
+            total_e += (wm[w] == -INFINITY) ? 0.f : ws[w] * __expf(wm[w] - gmax);
     }
     // a row with no value above -inf (all -inf, or NaN after an overflow upstream) never set an index:
     // token 0 then, so that nothing below reads beyond the row
     if ((unsigned)argmax >= (unsigned)V) argmax = 0;
-    float total_e = 0.f;
-    for (int w = 0; w < SAMPLE_THREADS / 64; ++w)
-        total_e += (wm[w] == -INFINITY) ? 0.f : ws[w] * __expf(wm[w] - gmax);
     const float lse = gmax + logf(total_e);
 
     const float temp = temperature[row];
@@ -310,7 +872,16 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     int tie_limit = 0x7fffffff;
     auto kept = [&](uint32_t key, int i) { return key > keep_key || (key == keep_key && i <= tie_limit); };
 
-    if (want_k || want_p) {
+    bool settled = false;                              // thresholds and block masses are there already
+    if constexpr (PREPARED) {
+        const RowState st = ws_all.state(row);
+        if (st.status == ROW_SETTLED) {
+            settled = true;
+            keep_key = st.keep_key;
+            tie_limit = st.tie_limit;
+        }
+    }
+    if (!settled && (want_k || want_p)) {
         // ---- the list: wave w goes through its run of the row, 64 tokens a load, and appends the tokens
         // within CAND_SPAN of the largest to its part of the list, in their order
         float* cv = dyn;                                                   // [CAND_WAVES][CAND_PER_WAVE] logits
@@ -325,40 +896,48 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         {
             int have = 0;
             float rest = 0.f;
-            const unsigned long long below = (1ull << lane) - 1ull;        // the lanes before this one
-            for (int i0 = beg + 4 * lane; i0 - 4 * lane < end; i0 += 4 * 256) {      // four loads on their way
-                if (have > CAND_PER_WAVE) break;          // (a flat row: this run alone is too much for the list)
-                float v[4][4];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) load4(i0 + 256 * j, v[j]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    int before = 0, all = 0;
-                    bool in[4];
-#pragma unroll
-                    for (int c = 0; c < 4; ++c) {
-                        in[c] = v[j][c] >= cut;
-                        const unsigned long long m = __ballot(in[c]);
-                        before += __popcll(m & below);
-                        all += __popcll(m);
-                    }
-                    if (all != 0) {
-                        int at = have + before;
-#pragma unroll
+            [[maybe_unused]] bool marked = false;
+            if constexpr (PREPARED) marked = finite(gmax);
+            if (marked) {
+                have = list_of_marks(ws_all.marks(row) + 4 * (beg / 256), (end - beg + 255) / 256, x, beg, lane,
+                                     cv + wave * CAND_PER_WAVE, ci + wave * CAND_PER_WAVE);
+                if (sum_rest && tid < n_parts) rest = ws_all.parts(row)[tid].rest;
+            } else {
+                const unsigned long long below = (1ull << lane) - 1ull;        // the lanes before this one
+                for (int i0 = beg + 4 * lane; i0 - 4 * lane < end; i0 += 4 * 256) {      // four loads on their way
+                    if (have > CAND_PER_WAVE) break;          // (a flat row: this run alone is too much for the list)
+                    float v[4][4];
+    #pragma unroll
+                    for (int j = 0; j < 4; ++j) load4(i0 + 256 * j, v[j]);
+    #pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        int before = 0, all = 0;
+                        bool in[4];
+    #pragma unroll
                         for (int c = 0; c < 4; ++c) {
-                            if (in[c]) {
-                                if (at < CAND_PER_WAVE) {
-                                    cv[wave * CAND_PER_WAVE + at] = v[j][c];
-                                    ci[wave * CAND_PER_WAVE + at] = i0 + 256 * j + c;
-                                }
-                                ++at;
-                            }
+                            in[c] = v[j][c] >= cut;
+                            const unsigned long long m = __ballot(in[c]);
+                            before += __popcll(m & below);
+                            all += __popcll(m);
                         }
-                        have += all;
-                    }
-                    if (sum_rest) {
-#pragma unroll
-                        for (int c = 0; c < 4; ++c) rest += in[c] ? 0.f : __expf((v[j][c] - gmax) * inv_t);
+                        if (all != 0) {
+                            int at = have + before;
+    #pragma unroll
+                            for (int c = 0; c < 4; ++c) {
+                                if (in[c]) {
+                                    if (at < CAND_PER_WAVE) {
+                                        cv[wave * CAND_PER_WAVE + at] = v[j][c];
+                                        ci[wave * CAND_PER_WAVE + at] = i0 + 256 * j + c;
+                                    }
+                                    ++at;
+                                }
+                            }
+                            have += all;
+                        }
+                        if (sum_rest) {
+    #pragma unroll
+                            for (int c = 0; c < 4; ++c) rest += in[c] ? 0.f : __expf((v[j][c] - gmax) * inv_t);
+                        }
                     }
                 }
             }
@@ -374,61 +953,91 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
 
             // a thread's entries for the searches: place (tid % CAND_PER_WAVE) of every other wave's part
             if (listed) {
-                uint32_t key[CAND_OWN];
-                float weight[CAND_OWN];                    // exp((x - max) / T), made a whole number where it is added
-                int idx[CAND_OWN];                         // the entry's token; -1: no entry
                 const int half = tid / CAND_PER_WAVE, off = tid - half * CAND_PER_WAVE;
-#pragma unroll
-                for (int e = 0; e < CAND_OWN; ++e) {
+                const int* held = cnt;
+                auto entry = [cv, ci, held, half, off](int e, float& v, int& i) {
                     const int w = half + (SAMPLE_THREADS / CAND_PER_WAVE) * e;
-                    const bool there = off < cnt[w];
-                    const float v = there ? cv[w * CAND_PER_WAVE + off] : 0.f;
-                    key[e] = there ? order_key(v) : 0u;
-                    weight[e] = there ? __expf((v - gmax) * inv_t) : 0.f;
-                    idx[e] = there ? ci[w * CAND_PER_WAVE + off] : -1;
-                }
+                    v = cv[w * CAND_PER_WAVE + off];
+                    i = ci[w * CAND_PER_WAVE + off];
+                    return off < held[w];
+                };
                 // the entries that tie at key t, up to token `upto`
-                auto ties_at = [&](uint32_t t, int upto) {
-                    return [&key, &idx, t, upto](auto f) {
-#pragma unroll
-                        for (int e = 0; e < CAND_OWN; ++e)
-                            if (idx[e] >= 0 && key[e] == t && idx[e] <= upto) f(idx[e]);
+                auto ties_at = [entry](uint32_t t, int upto) {
+                    return [entry, t, upto](auto f) {
+#pragma unroll 4
+                        for (int e = 0; e < CAND_OWN; ++e) {
+                            float v;
+                            int i;
+                            if (entry(e, v, i) && order_key(v) == t && i <= upto) f(i);
+                        }
                     };
+                };
+                const float scale = fminf((float)SEARCH_BUCKETS / (CAND_SPAN * temp), 1e30f);
+                auto run_of = [=](uint32_t key) {
+                    return (int)fminf(fmaxf((gmax - key_value(key)) * scale, 0.f), (float)(SEARCH_BUCKETS - 1));
                 };
                 // top-k: the k-th largest is on the list; below cut_key - 1 nothing of it lies
                 if (want_k) {
-                    fixed_t above = 0ull, at = FIXED_UNKNOWN;
-                    keep_key = search_threshold(
-                        [&](uint32_t lo, uint32_t hi, auto add) {
-#pragma unroll
-                            for (int e = 0; e < CAND_OWN; ++e)
-                                if (key[e] > lo && key[e] <= hi) add(key[e], 1ull << 40);
-                        },
-                        tid, cut_key - 1u, top_key, (fixed_t)(k - 1) << 40, fx, wsum, &sh_b, &sh_above, &above, &at);
+                    auto one = [=](int e, uint32_t& key) {
+                        float v;
+                        int i;
+                        const bool there = entry(e, v, i);
+                        key = order_key(v);
+                        return there ? 1ull << 40 : 0ull;
+                    };
+                    fixed_t above = 0ull, at = FIXED_UNKNOWN, limit;
+                    if (search_few<CAND_OWN>(run_of, one, [=](fixed_t) { return (fixed_t)(k - 1) << 40; }, tid, fx, wsum, &few,
+                                             keep_key, limit, above, at) != FEW_FOUND) {
+                        __syncthreads();
+                        keep_key = search_threshold(
+                            [=](uint32_t lo, uint32_t hi, auto add) {
+                                for (int e = 0; e < CAND_OWN; ++e) {
+                                    uint32_t key;
+                                    const fixed_t m = one(e, key);
+                                    if (m && key > lo && key <= hi) add(key, m);
+                                }
+                            },
+                            tid, cut_key - 1u, top_key, (fixed_t)(k - 1) << 40, fx, wsum, &sh_b, &sh_above, &above, &at);
+                    }
                     // of the tokens that tie with the k-th value, as many stay as make k with those above them
                     tie_limit = tie_cut(ties_at(keep_key, 0x7fffffff), tid, V, (unsigned long long)k - (above >> 40),
                                         0x7fffffff, at == FIXED_UNKNOWN ? at : at >> 40, fx, wsum, &sh_b, &sh_above);
+                    __syncthreads();
                 }
                 if (want_p) {
-                    fixed_t zc = 0ull;
-#pragma unroll
-                    for (int e = 0; e < CAND_OWN; ++e) zc += idx[e] >= 0 && kept(key[e], idx[e]) ? to_fixed(weight[e]) : 0ull;
-                    zc = block_sum_fixed(zc, wsum);
-                    const fixed_t z = zc + (fixed_t)((double)z_rest * (double)FIXED_ONE_F);
-                    const fixed_t limit = (fixed_t)((double)p * (double)z);
+                    const uint32_t k_key = keep_key;         // what top-k left: the search goes over that
+                    const int k_limit = tie_limit;
+                    auto weighed = [=](int e, uint32_t& key) {
+                        float v;
+                        int i;
+                        const bool there = entry(e, v, i);
+                        key = order_key(v);
+                        return there && (key > k_key || (key == k_key && i <= k_limit)) ? to_fixed(__expf((v - gmax) * inv_t))
+                                                                                        : 0ull;
+                    };
+                    fixed_t above = 0ull, at = FIXED_UNKNOWN, limit, zc = 0ull;
+                    const int found = search_few<CAND_OWN>(
+                        run_of, weighed,
+                        [&](fixed_t sum) {
+                            zc = sum;
+                            const fixed_t z = sum + (fixed_t)((double)z_rest * (double)FIXED_ONE_F);
+                            return (fixed_t)((double)p * (double)z);
+                        },
+                        tid, fx, wsum, &few, keep_key, limit, above, at);
                     // the boundary is on the list if the list's mass is more than p of the whole (always, after top-k)
                     if (want_k || zc > limit) {
-                        const uint32_t k_key = keep_key;     // what top-k left: the search goes over that
-                        const int k_limit = tie_limit;
-                        fixed_t above = 0ull, at = FIXED_UNKNOWN;
-                        keep_key = search_threshold(
-                            [&](uint32_t lo, uint32_t hi, auto add) {
-#pragma unroll
-                                for (int e = 0; e < CAND_OWN; ++e)
-                                    if (idx[e] >= 0 && key[e] > lo && key[e] <= hi &&
-                                        (key[e] > k_key || idx[e] <= k_limit)) add(key[e], to_fixed(weight[e]));
-                            },
-                            tid, want_k ? k_key : cut_key - 1u, top_key, limit, fx, wsum, &sh_b, &sh_above, &above, &at);
+                        if (found != FEW_FOUND) {
+                            __syncthreads();
+                            keep_key = search_threshold(
+                                [=](uint32_t lo, uint32_t hi, auto add) {
+                                    for (int e = 0; e < CAND_OWN; ++e) {
+                                        uint32_t key;
+                                        const fixed_t m = weighed(e, key);
+                                        if (m && key > lo && key <= hi) add(key, m);
+                                    }
+                                },
+                                tid, want_k ? k_key : cut_key - 1u, top_key, limit, fx, wsum, &sh_b, &sh_above, &above, &at);
+                        }
                         // of the tokens that tie with the boundary value, the i-th in vocabulary order stays while
                         // what lies before it, the mass above them and i of their own, is at most top_p of the whole
                         const fixed_t each = to_fixed(__expf((key_value(keep_key) - gmax) * inv_t));
@@ -446,12 +1055,16 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                 // ---- the draw over the list, which is in vocabulary order: wave w has its own part,
                 // a lane CAND_PER_WAVE / 64 consecutive entries of it
                 constexpr int RUN = CAND_PER_WAVE / 64;
-                const int o0 = min(cnt[wave], RUN * lane), o1 = min(cnt[wave], o0 + RUN);
-                float mine = 0.f;
-                for (int o = o0; o < o1; ++o) {
-                    const float v = cv[wave * CAND_PER_WAVE + o];
-                    if (kept(order_key(v), ci[wave * CAND_PER_WAVE + o])) mine += __expf((v - gmax) * inv_t);
-                }
+                float* cw = cv + wave * CAND_PER_WAVE;      // every entry's kept mass first, in the logit's place
+                for (int o = lane; o < CAND_PER_WAVE; o += 64)
+                    cw[o] = o < cnt[wave] && kept(order_key(cw[o]), ci[wave * CAND_PER_WAVE + o])
+                                ? __expf((cw[o] - gmax) * inv_t) : 0.f;
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                float own[RUN], mine = 0.f;
+#pragma unroll
+                for (int o = 0; o < RUN; ++o) own[o] = cw[RUN * lane + o];
+#pragma unroll
+                for (int o = 0; o < RUN; ++o) mine += own[o];
                 const float upto = wave_running_sum(mine, lane);
                 __syncthreads();
                 if (lane == 63) wmass[wave] = upto;
@@ -474,15 +1087,16 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                 const int who = passed ? __ffsll((long long)passed) - 1 : 63 - __builtin_clzll(any);
                 if (lane == who) {
                     float run = before + (upto - mine);
-                    int tok = argmax;
-                    for (int o = o0; o < o1; ++o) {
-                        const float v = cv[wave * CAND_PER_WAVE + o];
-                        if (kept(order_key(v), ci[wave * CAND_PER_WAVE + o])) {
-                            tok = ci[wave * CAND_PER_WAVE + o];      // the last kept entry if the target is never passed
-                            run += __expf((v - gmax) * inv_t);
-                            if (run > target) break;
+                    int at = -1;                           // the last kept entry if the target is never passed
+                    bool over = false;
+#pragma unroll
+                    for (int o = 0; o < RUN; ++o)
+                        if (!over && own[o] > 0.f) {
+                            at = o;
+                            run += own[o];
+                            over = run > target;
                         }
-                    }
+                    const int tok = at < 0 ? argmax : ci[wave * CAND_PER_WAVE + RUN * lane + at];
                     out[2 * row] = tok;
                     out[2 * row + 1] = __float_as_int(x[tok] - lse);
                     if (path) path[row] = 1;
@@ -502,41 +1116,90 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
             };
         };
 
-        // ---- over the whole row. top-k: the key of the k-th largest value is the smallest key with at most
-        // k - 1 tokens above it
-        if (want_k) {
-            fixed_t above = 0ull, at = FIXED_UNKNOWN;
-            keep_key = search_threshold(
-                [&](uint32_t lo, uint32_t hi, auto add) {
-                    for_each_logit(x, V, tid, [&](int, float v) {
-                        const uint32_t key = order_key(v);
-                        if (key > lo && key <= hi) add(key, 1ull << 40);
-                    });
+        // ---- over the whole row, in two passes: masses of runs of equal width in the logit (beyond `span` from the
+        // largest all in the last one), then the tokens of the run in which the boundary lies, into the list's place. mass(i, v):
+        // a token's measure. False (too many tokens in it): the keys' range is halved, pass by pass, instead.
+        auto search_row = [&](float span, auto mass, auto limit_of, fixed_t& limit, fixed_t& above, fixed_t& at) {
+            const float scale = fminf((float)SEARCH_BUCKETS / span, 1e30f);
+            auto place = [=](float v) { return (gmax - v) * scale; };
+            auto cut_to_runs = [](float d) { return (int)fminf(fmaxf(d, 0.f), (float)(SEARCH_BUCKETS - 1)); };
+            clear_runs(tid, fx, &few);
+            for_each_logit(x, V, tid, [&](int i, float v) {
+                const fixed_t m = mass(i, v);
+                if (m) atomicAdd(&fx[cut_to_runs(place(v))], m);
+            });
+            const int run = crossing_run(limit_of, tid, fx, wsum, &few, limit);
+            if (run < 0) return false;
+            const fixed_t before = few.above;
+            for_each_logit(x, V, tid, [&](int i, float v) {
+                if (cut_to_runs(place(v)) == run && mass(i, v)) {
+                    const int at = atomicAdd(&few.n, 1);
+                    if (at < CAND_WAVES * CAND_PER_WAVE) {
+                        cv[at] = v;
+                        ci[at] = i;
+                    }
+                }
+            });
+            __syncthreads();
+            const int n = few.n;
+            __syncthreads();
+            if (n > CAND_WAVES * CAND_PER_WAVE) return false;
+            fixed_t limit_in;
+            const bool found = search_few<CAND_OWN>(
+                [=](uint32_t key) { return cut_to_runs((place(key_value(key)) - (float)run) * (float)SEARCH_BUCKETS); },
+                [=](int e, uint32_t& key) {
+                    const int o = tid + e * SAMPLE_THREADS;
+                    if (o >= n) return (fixed_t)0ull;
+                    key = order_key(cv[o]);
+                    return mass(ci[o], cv[o]);
                 },
-                tid, 0u, top_key, (fixed_t)(k - 1) << 40, fx, wsum, &sh_b, &sh_above, &above, &at);
+                [=](fixed_t) { return limit - before; }, tid, fx, wsum, &few, keep_key, limit_in, above, at) == FEW_FOUND;
+            above += before;
+            return found;
+        };
+        // top-k: the key of the k-th largest value is the smallest key with at most k - 1 tokens above it
+        if (want_k) {
+            fixed_t above = 0ull, at = FIXED_UNKNOWN, limit;
+            if (!search_row(TOP_K_SPAN, [=](int, float v) { return v <= gmax ? 1ull << 40 : 0ull; },
+                            [=](fixed_t) { return (fixed_t)(k - 1) << 40; }, limit, above, at)) {
+                __syncthreads();
+                at = FIXED_UNKNOWN;
+                keep_key = search_threshold(
+                    [=](uint32_t lo, uint32_t hi, auto add) {
+                        for_each_logit(x, V, tid, [&](int, float v) {
+                            const uint32_t key = order_key(v);
+                            if (key > lo && key <= hi) add(key, 1ull << 40);
+                        });
+                    },
+                    tid, 0u, top_key, (fixed_t)(k - 1) << 40, fx, wsum, &sh_b, &sh_above, &above, &at);
+            }
             tie_limit = tie_cut(ties_at(keep_key, 0x7fffffff), tid, V, (unsigned long long)k - (above >> 40),
                                 0x7fffffff, at == FIXED_UNKNOWN ? at : at >> 40, fx, wsum, &sh_b, &sh_above);
+            __syncthreads();
         }
         // top-p: the smallest key with at most p of the kept mass above it
         if (want_p) {
-            fixed_t z = 0ull;
-            for_each_logit(x, V, tid, [&](int i, float v) {
-                if (kept(order_key(v), i)) z += to_fixed(__expf((v - gmax) * inv_t));
-            });
-            z = block_sum_fixed(z, wsum);
-            const fixed_t limit = (fixed_t)((double)p * (double)z);
             const uint32_t k_key = keep_key;             // what top-k left: the search goes over that
             const int k_limit = tie_limit;
-            fixed_t above = 0ull, at = FIXED_UNKNOWN;
-            keep_key = search_threshold(
-                [&](uint32_t lo, uint32_t hi, auto add) {
-                    for_each_logit(x, V, tid, [&](int i, float v) {
-                        const uint32_t key = order_key(v);
-                        if (key > lo && key <= hi && (key > k_key || i <= k_limit))
-                            add(key, to_fixed(__expf((v - gmax) * inv_t)));
-                    });
-                },
-                tid, k_key, top_key, limit, fx, wsum, &sh_b, &sh_above, &above, &at);
+            auto mass = [=](int i, float v) {
+                const uint32_t key = order_key(v);
+                return v <= gmax && (key > k_key || (key == k_key && i <= k_limit)) ? to_fixed(__expf((v - gmax) * inv_t)) : 0ull;
+            };
+            fixed_t above = 0ull, at = FIXED_UNKNOWN, limit;
+            if (!search_row(WEIGHS_NOTHING * temp, mass, [=](fixed_t sum) { return (fixed_t)((double)p * (double)sum); }, limit,
+                            above, at)) {
+                __syncthreads();
+                at = FIXED_UNKNOWN;
+                keep_key = search_threshold(
+                    [=](uint32_t lo, uint32_t hi, auto add) {
+                        for_each_logit(x, V, tid, [&](int i, float v) {
+                            const uint32_t key = order_key(v);
+                            if (key > lo && key <= hi && (key > k_key || i <= k_limit))
+                                add(key, to_fixed(__expf((v - gmax) * inv_t)));
+                        });
+                    },
+                    tid, k_key, top_key, limit, fx, wsum, &sh_b, &sh_above, &above, &at);
+            }
             const fixed_t each = to_fixed(__expf((key_value(keep_key) - gmax) * inv_t));
             const unsigned long long stay = each ? (limit - above) / each + 1ull : ~0ull;
             const int upto = keep_key == k_key ? k_limit : 0x7fffffff;
@@ -557,7 +1220,11 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         const int n_it = (end - beg + 255) / 256;            // this wave's blocks
         const bool by_block = seg / 256 <= SAMPLE_BLOCKS;    // (a vocabulary beyond 262,144: the whole run is gone through again)
         float mine = 0.f;
-        for (int it0 = 0; it0 < n_it; it0 += 4) {            // four loads on their way
+        if (settled) {                                       // (at most SAMPLE_BLOCKS blocks: ra_sample_traced sees to it)
+            const float m = lane < n_it ? ws_all.masses(row)[beg / 256 + lane] : 0.f;
+            if (lane < n_it) bmass[wave][lane] = m;
+            for (int it = 0; it < n_it; ++it) mine += __shfl(m, it, 64);
+        } else for (int it0 = 0; it0 < n_it; it0 += 4) {     // four loads on their way
             float a[4][4];
 #pragma unroll
             for (int j = 0; j < 4; ++j) load4(beg + 256 * (it0 + j) + 4 * lane, a[j]);
@@ -641,28 +1308,64 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
     }
 }
 
+// How many pieces a wave's run of the row is cut into for the kernels over several blocks a row; 0: one block a row.
+// The line, one block a row / several blocks, microseconds a call, logits near normal at T 0.7, greedy | top-p 0.9 with
+// 300 large logits | top-p 0.9, flat:
+//   vocabulary  65,536   1 row  10.3 / 13.1 | 29 / 32 |  60 / 37      32 rows 11.0 / 16.3 | 30 / 37 |  62 / 47
+//              128,256   1      16.4 / 13.8 | 41 / 33 |  99 / 42      32      16.9 / 18.0 | 41 / 41 | 101 / 62
+//              151,936   1      18.0 / 14.0 | 45 / 34 | 111 / 45      32      18.7 / 18.9 | 45 / 44 | 116 / 67
+//              151,936  64      20.5 / 23.6 | 52 / 54 | 123 / 84
+// so that from about 100,000 tokens and up to 32 rows no kind of row loses; beyond SAMPLE_BLOCKS 256s a run the masses
+// have no room.
+static int sample_parts(int M, int V) {
+    if (V < 98304 || V > CAND_WAVES * 256 * SAMPLE_BLOCKS || M > 32) return 0;
+    return M <= 8 ? 4 : (M <= 24 ? 2 : 1);
+}
+
+extern "C" long long ra_sample_scratch(int M, int V) {
+    return M > 0 && sample_parts(M, V) ? (long long)M * (long long)sample_ws(nullptr, V).row_bytes : 0;
+}
+
 // path (may be nullptr): per row 0 = no threshold was needed, 1 = thresholds and draw from the list of the
-// largest logits, 2 = by passes over the whole row.
+// largest logits, 2 = by passes over the whole row. ws: ra_sample_scratch bytes, 16-byte aligned (nullptr: one block
+// a row).
 extern "C" int ra_sample_traced(const float* logits, int M, int V, const float* temperature,
                                 const int* top_k, const float* top_p, const float* u, int* out, int* path,
-                                void* stream) {
+                                char* ws, long long ws_bytes, void* stream) {
     if (M <= 0) return RA_OK;
     if (V <= 0) return RA_ERR_ARG;
     const size_t lds = (size_t)2 * CAND_WAVES * CAND_PER_WAVE * sizeof(float) + SEARCH_BUCKETS * sizeof(fixed_t);   // 80 KB
     static bool allowed = false;
     if (!allowed) {
-        if (hipFuncSetAttribute(reinterpret_cast<const void*>(sample_kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+        if (hipFuncSetAttribute(reinterpret_cast<const void*>(sample_kernel<false>), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)lds) != hipSuccess ||
+            hipFuncSetAttribute(reinterpret_cast<const void*>(sample_kernel<true>), hipFuncAttributeMaxDynamicSharedMemorySize,
                                 (int)lds) != hipSuccess)
             return RA_ERR_ARG;
         allowed = true;
     }
-    hipLaunchKernelGGL(sample_kernel, dim3(M), dim3(SAMPLE_THREADS), lds, (hipStream_t)stream, logits,
-                       V, temperature, top_k, top_p, u, out, path);
+    hipStream_t s = (hipStream_t)stream;
+    const SampleWs w = sample_ws(ws, V);
+    const int parts = ws ? sample_parts(M, V) : 0;
+    if (parts == 0) {
+        hipLaunchKernelGGL(sample_kernel<false>, dim3(M), dim3(SAMPLE_THREADS), lds, s, logits, V, temperature, top_k, top_p,
+                           u, out, path, w, 0);
+        return ra_launch_status();
+    }
+    if (ws_bytes < (long long)M * (long long)w.row_bytes || (reinterpret_cast<uintptr_t>(ws) & 15) != 0) return RA_ERR_ARG;
+    const dim3 grid(CAND_WAVES * parts, M), block(PART_THREADS);
+    hipLaunchKernelGGL(sample_top_kernel, grid, block, 0, s, logits, V, w, parts);
+    hipLaunchKernelGGL(sample_span_kernel, grid, block, 0, s, logits, V, temperature, top_k, top_p, w, parts);
+    hipLaunchKernelGGL(sample_gather_kernel, grid, block, 0, s, logits, V, temperature, top_k, top_p, w, parts);
+    hipLaunchKernelGGL(sample_settle_kernel, dim3(M), dim3(SAMPLE_THREADS), 0, s, V, temperature, top_k, top_p, w, parts);
+    hipLaunchKernelGGL(sample_masses_kernel, grid, block, 0, s, logits, V, temperature, w, parts);
+    hipLaunchKernelGGL(sample_kernel<true>, dim3(M), dim3(SAMPLE_THREADS), lds, s, logits, V, temperature, top_k, top_p,
+                       u, out, path, w, parts);
     return ra_launch_status();
 }
 
 extern "C" int ra_sample(const float* logits, int M, int V, const float* temperature,
                          const int* top_k, const float* top_p, const float* u, int* out,
                          void* stream) {
-    return ra_sample_traced(logits, M, V, temperature, top_k, top_p, u, out, nullptr, stream);
+    return ra_sample_traced(logits, M, V, temperature, top_k, top_p, u, out, nullptr, nullptr, 0, stream);
 }

@@ -133,7 +133,7 @@ def _declare(lib):
         "ra_attention_prefill_bf16": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, F, I, P, F, I, I, P, F, L, I, P],
         "ra_attention_prefill_tile_rows": [I],
         "ra_sample": [P, I, I, P, P, P, P, P, P],
-        "ra_sample_traced": [P, I, I, P, P, P, P, P, P, P],
+        "ra_sample_traced": [P, I, I, P, P, P, P, P, P, P, L, P],
         "ra_stream_read": [P, L, P, I, P],
     }
     for name, args in sigs.items():
@@ -142,6 +142,8 @@ def _declare(lib):
         fn.restype = _c_int
     lib.ra_recurrence_scratch.argtypes = [P, I, I, I, I, I]
     lib.ra_recurrence_scratch.restype = _c_ll
+    lib.ra_sample_scratch.argtypes = [I, I]
+    lib.ra_sample_scratch.restype = _c_ll
 
 
 def _ptr(t: Optional[torch.Tensor]):
@@ -2140,6 +2142,8 @@ class HipOps:
             self._want(path, "path", torch.int32, 1)
             if path.shape[0] != M:
                 raise KernelError(f"sample: path has {path.shape[0]} entries for {M} rows")
+        need = self.lib.ra_sample_scratch(M, V)
+        ws = torch.empty(need, dtype=torch.uint8, device=self.device) if need else None
         self._check(self.lib.ra_sample_traced(_ptr(logits), M, V, _ptr(temperature), _ptr(top_k), _ptr(top_p),
-                                              _ptr(u), _ptr(out), _ptr(path), self._stream()), "sample")
+                                              _ptr(u), _ptr(out), _ptr(path), _ptr(ws), need, self._stream()), "sample")
         return out

@@ -1,0 +1,99 @@
+"""The sampler's searches at the edges of their ranges: several workgroups a row against one, and the searches of few
+passes against the distribution in 64 bits."""
+import pytest
+import torch
+
+from return_amd.kernels.hip_ops import _ptr
+from tests.test_kernels_gpu import DEV, ops  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+
+KINDS = ["flat", "peaked", "very flat", "ties", "one value", "masked", "two far apart", "crowded", "all -inf", "inf"]
+
+
+def _rows(V, seed):
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randn(len(KINDS), V, generator=g)
+    x[1, torch.randint(0, V, (300,), generator=g)] = 14 + 8 * torch.rand(300, generator=g)
+    x[2] *= 0.02
+    x[3] = torch.randint(-2, 3, (V,), generator=g).float()
+    x[4] = 1.5
+    x[5, torch.rand(V, generator=g) < 0.9] = float("-inf")
+    x[6] = -1e4
+    x[6, V // 3], x[6, V - 1] = 3.0, 2.9
+    x[7, 777:777 + 600] = 9 + torch.rand(600, generator=g)
+    x[8] = float("-inf")
+    x[9, 5] = float("inf")
+    return x
+
+
+def _options(M, seed):
+    g = torch.Generator().manual_seed(seed)
+    pick = lambda values, dt: torch.tensor(values, dtype=dt)[torch.randint(0, len(values), (M,), generator=g)].to(DEV)
+    return (pick([0.0, 0.3, 0.7, 1.0, 1.0, 4.0], torch.float32), pick([0, 0, 0, 1, 50, 3000], torch.int32),
+            pick([0.0, 0.01, 0.5, 0.9, 0.999, 1.0], torch.float32), torch.rand(M, generator=g).to(DEV))
+
+
+@pytest.mark.parametrize("M", [1, 8, 9, 25, 32])
+@pytest.mark.parametrize("V", [98304, 98305, 131075, 151936, 262144])
+def test_several_workgroups_a_row_draw_what_one_draws(ops, V, M):
+    """Whole numbers are added, and masses in the same order: the same tokens, from the same search. The
+    log-probabilities' sum of exp is formed in another order (2^-24 a step of some dozens)."""
+    assert ops.lib.ra_sample_scratch(M, V) > 0
+    base = _rows(V, V).to(DEV)
+    for seed in range(3 if M > 1 else 24):
+        kinds = torch.randperm(len(KINDS), generator=torch.Generator().manual_seed(seed))
+        x = base[kinds.repeat(4)[:M]].contiguous()
+        t, k, p, u = _options(M, seed)
+        path = [torch.full((M,), -1, dtype=torch.int32, device=DEV) for _ in range(2)]
+        one = torch.empty(M, 2, dtype=torch.int32, device=DEV)
+        got = ops.sample(x, t, k, p, u, path=path[0])
+        ops._check(ops.lib.ra_sample_traced(_ptr(x), M, V, _ptr(t), _ptr(k), _ptr(p), _ptr(u), _ptr(one), _ptr(path[1]),
+                                            None, 0, ops._stream()), "sample")
+        assert got[:, 0].tolist() == one[:, 0].tolist(), (seed, [KINDS[i] for i in kinds.repeat(4)[:M]])
+        assert path[0].tolist() == path[1].tolist()
+        torch.testing.assert_close(got[:, 1].contiguous().view(torch.float32), one[:, 1].contiguous().view(torch.float32),
+                                   atol=2e-5, rtol=1e-6, equal_nan=True)
+
+
+@pytest.mark.parametrize("V", [63, 4096, 8193, 20001, 98303, 98304])
+def test_kept_tokens_are_those_of_the_distribution(ops, V):
+    """Every kind of row under every option: the token is where the running sum of the plain distribution (64 bits),
+    in vocabulary order, passes the uniform number. 2^-24 of a weight and a running sum in float32 over runs
+    of 256: 1e-4, the bound that the other tests of the sampler have."""
+    from tests.plain import qwen3_plain as plain
+    x = _rows(V, V) if V > 4096 else torch.randn(len(KINDS), V, generator=torch.Generator().manual_seed(V)) * torch.arange(1, 11)[:, None]
+    x = x[:8]                                      # (without a finite largest logit there is no distribution)
+    for seed in range(4):
+        t, k, p, u = _options(8, 100 + seed)
+        out = ops.sample(x.to(DEV), t, k, p, u).cpu()
+        for r in range(8):
+            tok = int(out[r, 0])
+            if float(t[r]) == 0.0:
+                assert tok == int(x[r].argmax())
+                continue
+            d = plain.sample_distribution(x[r], float(t[r]), int(k[r]), float(p[r])).double()
+            assert d[tok] > 0, (KINDS[r], seed, tok, float(t[r]), int(k[r]), float(p[r]))
+            c = d.cumsum(0)
+            before = float(c[tok - 1]) if tok else 0.0
+            assert before - 1e-4 <= float(u[r]) <= float(c[tok]) + 1e-4, (KINDS[r], seed, tok)
+
+
+def test_captured_and_replayed(ops):
+    """Several workgroups a row in a graph: every replay gives what a call gives, other logits and calls between."""
+    V, M = 131072, 8
+    x = torch.empty(M, V, device=DEV)
+    t, k, p, u = _options(M, 5)
+    t[:] = 0.8
+    base = _rows(V, 3).to(DEV)
+    x.copy_(base[:M])
+    ops.sample(x, t, k, p, u)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = ops.sample(x, t, k, p, u)
+    for it in range(4):
+        x.copy_(base[:M].roll(it, 0) * (1.0 + 0.1 * it))
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, ops.sample(x, t, k, p, u)), f"replay {it}"
