@@ -176,7 +176,7 @@ class HipOps:
         self.decode_merge_waves = 0          # waves of such a workgroup; 0: by the number of pairs and the context
         self.prefill_key_split = 0           # groups of waves that share a q tile's keys (1 or 2); 0: by the number of tiles
         self.prefill_small_tiles = True      # q tiles of 64 rows instead of 128 while those would not fill the chip
-        self.overlap_attention = True        # mixed steps: the decode and the prefill attention side by side on two streams
+        self.overlap_attention = None        # mixed steps: the decode and the prefill attention side by side on two streams; None: by size
         self._side_stream = None
         self.skinny_max_grid = 0             # 0: one workgroup per 16 weight rows
         self.gated_skinny_rows = 8           # up to this many rows gate-up and SiLU-mul are one kernel
@@ -1509,6 +1509,19 @@ class HipOps:
             return (rows,) if rows == 64 else (rows, 64)
         return None
 
+    def _side_by_side(self, step, window):
+        """Whether a mixed step's two attention kernels go to two streams: from 512 Ki keys of decoded tokens on. A fork and
+        a join cost the host 30 us a layer and the device gaps as long, and the other kernel's workgroups disturb the
+        prefill kernel's order over the XCDs. Measured, a layer's attention between two products, microseconds, side
+        by side / one after the other: heads 32 over 8 of 128, portions of 2,048 rows after 2,048: 8 requests of 1,024
+        417 / 328, 64 of 4,096 519 / 502, 16 of 32,768 696 / 730, 128 of 16,384 1,748 / 1,798; portions of 512 after 16,384:
+        8 of 1,024 355 / 347, 64 of 4,096 594 / 594, 128 of 8,192 1,034 / 1,125; heads 8 over 2 of 64, 128 of 8,192 341 / 406. A
+        whole mixed step of the 4B shape (24 requests of about 450 tokens, a portion of 512) 11.0 / 8.7 ms."""
+        if self.overlap_attention is not None:
+            return self.overlap_attention
+        keys = min(step.max_decode_seq_len, window) if window > 0 else step.max_decode_seq_len
+        return step.n_decode * keys >= 1 << 19
+
     def attention(self, q, out, k_pool, v_pool, step, group, scale, window=0, head_scale=None, softcap=0.0,
                   keep_first=0, sink=False, sink_logit=None, out_scale=1.0, fine_weights=False):
         """Attention of the step's queries over the paged cache. Optional: head_scale (fp32, one factor per query
@@ -1605,9 +1618,9 @@ class HipOps:
         if fast_decode and fast_prefill and step.n_prefill_tokens > 0:
             # A step of prompt portions beside decoded tokens: the two kernels work on different rows of q and
             # out, one is bound by memory and the other by the matrix cores and the latency inside its waves,
-            # so they run side by side on two streams (never while a graph is being captured: such steps are
-            # not captured anyway, and a fork and join inside a graph costs more than it gives).
-            if self.overlap_attention and not torch.cuda.is_current_stream_capturing():
+            # so where the decoding is long they run side by side on two streams (never while a graph is being
+            # captured: such steps are not captured anyway, and a fork and join inside a graph costs more than it gives).
+            if self._side_by_side(step, window) and not torch.cuda.is_current_stream_capturing():
                 main = torch.cuda.current_stream(self.device)
                 if self._side_stream is None:
                     self._side_stream = torch.cuda.Stream(self.device)      # (default priority, like every stream here)
