@@ -2,8 +2,8 @@
 // rollout/monkey_patch/qwen3.py:21). This file holds the plain tiled kernel: products and
 // sums in true 32-bit FMA, K walked in order, so a row's result does not depend on M.
 // It is the matrix product of the float32 path and the fallback of the bfloat16 path. For up to
-// 16 rows of x in float32 (decoding) there is a second kernel that streams W once with 16-byte
-// loads; it sums a row's products in another order than the tiled kernel, 32-bit all the same.
+// 16 rows of x in float32 (decoding) there are two kernels that stream W once with 16-byte
+// loads, x in LDS or from the cache; they sum a row's products in another order than the tiled kernel, 32-bit all the same.
 #include "common.h"
 
 #define BM 64
@@ -125,6 +125,74 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__
         }
 }
 
+// The same without LDS: a lane takes its floats of x from the cache beside those of W, so that no barrier holds the waves
+// together, and asks for the next 256 columns before it multiplies the last ones. A lane's sums are formed in the same order,
+// so the results are the same bits. Bound by the reading of W; microseconds with LDS / without, and rate of W: 4,096 x 12,288
+// at 1 row 46 / 32 (6.2 TB/s), 4 rows 61 / 35, 8 rows 84 / 46; 6,144 x 4,096 at 1 row 27 / 23, 4 rows 33 / 26, 8 rows 41 / 33;
+// 24,576 x 4,096 at 1 row 80 / 72, 4 rows 90 / 76. (512 columns ahead: the same to 8 % slower.)
+template <int MR>
+__global__ __launch_bounds__(256) void gemv_f32_direct_kernel(const float* __restrict__ x, const float* __restrict__ W,
+                                                              float* __restrict__ y, int M, int N, int K) {
+    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int n0 = (blockIdx.x * 4 + wave) * 4;
+    if (n0 >= N) return;
+    const float *wr[4], *xr[MR];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) wr[r] = W + (size_t)min(n0 + r, N - 1) * K + 4 * lane;      // clamped: loads stay inside
+#pragma unroll
+    for (int m = 0; m < MR; ++m) xr[m] = x + (size_t)min(m, M - 1) * K + 4 * lane;
+    float acc[4][MR];
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int m = 0; m < MR; ++m) acc[r][m] = 0.f;
+    struct Cols { gv_f4 w[4], x[MR]; };
+    auto load = [&](Cols& c, int k) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) c.w[r] = __builtin_nontemporal_load(reinterpret_cast<const gv_f4*>(wr[r] + k));
+#pragma unroll
+        for (int m = 0; m < MR; ++m) c.x[m] = *reinterpret_cast<const gv_f4*>(xr[m] + k);
+    };
+    auto multiply = [&](const Cols& l) {
+#pragma unroll
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+#pragma unroll
+                for (int c = 0; c < 4; ++c) acc[r][m] = fmaf(l.w[r][c], l.x[m][c], acc[r][m]);
+    };
+    const int nb = K / 256;
+    Cols a, b;
+    if (nb > 0) {
+        load(a, 0);
+        int j = 0;
+        for (; j + 2 < nb; j += 2) {
+            load(b, (j + 1) * 256);
+            multiply(a);
+            load(a, (j + 2) * 256);
+            multiply(b);
+        }
+        if (j + 1 < nb) {
+            load(b, (j + 1) * 256);
+            multiply(a);
+            multiply(b);
+        } else {
+            multiply(a);
+        }
+    }
+    if (nb * 256 + 4 * lane < K) {
+        load(a, nb * 256);
+        multiply(a);
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r)
+#pragma unroll
+        for (int m = 0; m < MR; ++m) {
+            const float s = wave_sum(acc[r][m]);
+            if (lane == 0 && m < M && n0 + r < N) y[(size_t)m * N + n0 + r] = s;
+        }
+}
+
 // in_dtype / out_dtype: RA_DTYPE_F32 or RA_DTYPE_BF16 (x and W share in_dtype)
 extern "C" int ra_gemm_nt(const void* A, const void* W, void* C, int M, int N, int K, int in_dtype,
                           int out_dtype, void* stream) {
@@ -136,11 +204,20 @@ extern "C" int ra_gemm_nt(const void* A, const void* W, void* C, int M, int N, i
         const dim3 g16((N + 15) / 16);
         const float *xa = (const float*)A, *wa = (const float*)W;
         float* ya = (float*)C;
-        if (M <= 1) hipLaunchKernelGGL(gemv_f32_kernel<1>, g16, block, 0, s, xa, wa, ya, M, N, K);
-        else if (M <= 2) hipLaunchKernelGGL(gemv_f32_kernel<2>, g16, block, 0, s, xa, wa, ya, M, N, K);
-        else if (M <= 4) hipLaunchKernelGGL(gemv_f32_kernel<4>, g16, block, 0, s, xa, wa, ya, M, N, K);
-        else if (M <= 8) hipLaunchKernelGGL(gemv_f32_kernel<8>, g16, block, 0, s, xa, wa, ya, M, N, K);
-        else hipLaunchKernelGGL(gemv_f32_kernel<16>, g16, block, 0, s, xa, wa, ya, M, N, K);
+        // x from the cache up to 8 rows; from 5 rows on x is as much to load as W or more, which shows where W is long
+        // (151,936 x 4,096 at 5 rows 465 with LDS, 483 without) and beyond 8 rows wherever there are more workgroups than
+        // CUs (9 rows: 4,096 x 4,096 49 / 32, 6,144 x 4,096 53 / 58, 24,576 x 4,096 151 / 171)
+        if (M <= 4 || (M <= 8 && N < 65536) || N <= 4096) {
+            if (M <= 1) hipLaunchKernelGGL(gemv_f32_direct_kernel<1>, g16, block, 0, s, xa, wa, ya, M, N, K);
+            else if (M <= 2) hipLaunchKernelGGL(gemv_f32_direct_kernel<2>, g16, block, 0, s, xa, wa, ya, M, N, K);
+            else if (M <= 4) hipLaunchKernelGGL(gemv_f32_direct_kernel<4>, g16, block, 0, s, xa, wa, ya, M, N, K);
+            else if (M <= 8) hipLaunchKernelGGL(gemv_f32_direct_kernel<8>, g16, block, 0, s, xa, wa, ya, M, N, K);
+            else hipLaunchKernelGGL(gemv_f32_direct_kernel<16>, g16, block, 0, s, xa, wa, ya, M, N, K);
+        } else if (M <= 8) {
+            hipLaunchKernelGGL(gemv_f32_kernel<8>, g16, block, 0, s, xa, wa, ya, M, N, K);
+        } else {
+            hipLaunchKernelGGL(gemv_f32_kernel<16>, g16, block, 0, s, xa, wa, ya, M, N, K);
+        }
         return ra_launch_status();
     }
     if (in_dtype == RA_DTYPE_F32 && out_dtype == RA_DTYPE_F32)
