@@ -803,7 +803,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
             }
         });
         // merge (mx, se, arg) over the wave, then over the waves in wave order
-    #pragma unroll
+#pragma unroll
         for (int o = 32; o > 0; o >>= 1) {
             const float m2 = __shfl_xor(mx, o, 64), s2 = __shfl_xor(se, o, 64);
             const int a2 = __shfl_xor(arg, o, 64);
@@ -907,13 +907,13 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                 for (int i0 = beg + 4 * lane; i0 - 4 * lane < end; i0 += 4 * 256) {      // four loads on their way
                     if (have > CAND_PER_WAVE) break;          // (a flat row: this run alone is too much for the list)
                     float v[4][4];
-    #pragma unroll
+#pragma unroll
                     for (int j = 0; j < 4; ++j) load4(i0 + 256 * j, v[j]);
-    #pragma unroll
+#pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         int before = 0, all = 0;
                         bool in[4];
-    #pragma unroll
+#pragma unroll
                         for (int c = 0; c < 4; ++c) {
                             in[c] = v[j][c] >= cut;
                             const unsigned long long m = __ballot(in[c]);
@@ -922,7 +922,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                         }
                         if (all != 0) {
                             int at = have + before;
-    #pragma unroll
+#pragma unroll
                             for (int c = 0; c < 4; ++c) {
                                 if (in[c]) {
                                     if (at < CAND_PER_WAVE) {
@@ -935,7 +935,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                             have += all;
                         }
                         if (sum_rest) {
-    #pragma unroll
+#pragma unroll
                             for (int c = 0; c < 4; ++c) rest += in[c] ? 0.f : __expf((v[j][c] - gmax) * inv_t);
                         }
                     }
