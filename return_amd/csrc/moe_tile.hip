@@ -14,8 +14,8 @@
 //
 // Why: with tiles of 128 x 128 staged through registers (what this replaces for K % 32 == 0) every k-step moved 16 KB
 // for 64 MFMAs of a workgroup; here it is 24 to 32 KB for 160 to 256. Measured, gate-up of 32 experts
-// of 6,144 x 4,096, four a token: 8,192 pairs 656 us (0.63 PFLOP/s) where the smaller tiles took 1,150, 12,432 pairs 754 (0.83)
-// against 1,409, 32,000 pairs 1,830 (0.88) against 3,192. At 2,000 pairs and fewer the time is the reading of W: 300 to 345 us for
+// of 6,144 x 4,096, four a token: 8,192 pairs 638 us (0.65 PFLOP/s) where the smaller tiles took 1,150, 12,432 pairs 731 (0.86)
+// against 1,409, 32,000 pairs 1,802 (0.89) against 3,192. At 2,000 pairs and fewer the time is the reading of W: 300 to 345 us for
 // 1.6 GB (5.4 TB/s at 480 pairs), where operands straight from memory took 415 to 790. What is lost at 8,192 pairs is the last
 // rounds of tiles: half of the experts have a few rows more than 256 and so two tiles of 140.
 #include "moe_tile.h"
@@ -29,10 +29,12 @@ typedef float mt_float4_t __attribute__((ext_vector_type(4)));
 #define MB_STAGE (2 * MB_HALF)
 #define MB_LDS (4 * MB_STAGE)                    // 128 KB
 
-template <int N>
-__device__ __forceinline__ void mb_wait_copies() {
-    // s_waitcnt vmcnt(N) alone: expcnt and lgkmcnt at their maxima
-    __builtin_amdgcn_s_waitcnt(0x0F70 | N);
+// Waits until at most COPIES of the wave's copies and READS of its LDS reads are on their way (the last ones: both finish in
+// their order). A barrier waits for neither.
+template <int COPIES, int READS>
+__device__ __forceinline__ void mb_wait() {
+    static_assert(COPIES < 16 && READS < 16, "fields of s_waitcnt");
+    __builtin_amdgcn_s_waitcnt(0x0070 | COPIES | (READS << 8));        // (expcnt at its maximum)
 }
 
 // A tile of 32 NB rows at most. xoff: where this lane's rows of x begin (bytes), one for each of its copies.
@@ -73,7 +75,8 @@ __device__ __forceinline__ void mb_tile(unsigned char* lds, const __amdgpu_buffe
     copy_stage(0, 0);
     if (nk > 1) copy_stage(1, 1);
     if (nk > 2) copy_stage(2, 2);
-    if (nk > 2) mb_wait_copies<PER>(); else mb_wait_copies<0>();
+    if (nk > 2) mb_wait<PER, 15>(); else mb_wait<0, 15>();
+    mb_wait<15, 0>();                                          // (no reads are; the compiled branches of two sizes meet here)
     __builtin_amdgcn_s_barrier();
     mt_bf16x8_t fwA[4], fxA[NB], fwB[4], fxB[NB];
 #pragma unroll
@@ -81,18 +84,18 @@ __device__ __forceinline__ void mb_tile(unsigned char* lds, const __amdgpu_buffe
 #pragma unroll
     for (int b = 0; b < NB; ++b) fxA[b] = read_x(0, b);
 
-    // (as in gemm_tile.hip: step it's operands are in registers, stage it + 1 is in LDS and is read meanwhile, stages
-    // it + 2 and it + 3 are on their way; every other step asks for two stages)
+    // Step it's operands are in registers, stage it + 1 is in LDS and is read meanwhile, stages it + 2 and it + 3 are on their
+    // way. A step refills the stage of step it - 1, which was read in step it - 2: every wave has to have finished those reads
+    // when it passes the barrier behind step it - 1, so at a step's end a wave waits until only that step's own reads are on
+    // their way. (Two stages asked for in every other step, the halves of the same 128-byte lines, would refill a stage behind
+    // the very barrier before which it was read: the wait for the reads cost that form 2 to 6 % at 2,000 to 12,000 pairs.)
     auto step = [&](int it, auto stage_c, auto steady_c, mt_bf16x8_t (&fw_c)[4], mt_bf16x8_t (&fx_c)[NB], mt_bf16x8_t (&fw_n)[4],
                     mt_bf16x8_t (&fx_n)[NB]) {
         constexpr int stage = decltype(stage_c)::value;
         constexpr bool steady = decltype(steady_c)::value;
         constexpr int nxt = (stage + 1) & 3;
         const bool more = steady || it + 1 < nk;
-        if constexpr ((stage & 1) == 0) {
-            if (steady || it + 3 < nk) copy_stage((stage + 3) & 3, it + 3);
-            if (steady || it + 4 < nk) copy_stage(stage, it + 4);
-        }
+        if (steady || it + 3 < nk) copy_stage((stage + 3) & 3, it + 3);
         if (more) {
 #pragma unroll
             for (int a = 0; a < 4; ++a) fw_n[a] = read_w(nxt, a);
@@ -111,17 +114,11 @@ __device__ __forceinline__ void mb_tile(unsigned char* lds, const __amdgpu_buffe
             for (int b = 0; b + 2 < NB; ++b) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                if constexpr ((stage & 1) == 0) {
-                    if (b < 2) __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
-                    else __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-                }
+                if (b < PER) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
             }
         }
-        if constexpr (steady) {
-            if constexpr ((stage & 1) == 0) mb_wait_copies<2 * PER>(); else mb_wait_copies<PER>();
-        } else {
-            mb_wait_copies<0>();
-        }
+        if constexpr (steady) mb_wait<PER, 4 + NB>();
+        else mb_wait<0, 0>();
         __builtin_amdgcn_s_barrier();
     };
     using std::integral_constant;
