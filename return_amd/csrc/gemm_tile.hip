@@ -8,8 +8,7 @@
 // of W as 8 x 4 MFMA 16x16x32 tiles (128 accumulator registers). Tiles of both operands go straight
 // from memory into LDS (buffer_load ... lds: the 64 lanes' 16 bytes land at consecutive addresses),
 // four stages of 32 KB; which 16-byte piece of a row a lane fetches is chosen so that a row's pieces
-// lie rotated by (row / 4) % 4 and the operand reads meet no bank conflict without padding. Every
-// other k-step asks for two stages (the two halves of the same 128-byte lines). The operands of
+// lie rotated by (row / 4) % 4 and the operand reads meet no bank conflict without padding. The operands of
 // k-step i+1 are read from LDS between the MFMAs of k-step i, an operand of x as soon as two of this
 // step's are used up, so that operands take 72 registers and nothing spills; the loop holds no vector
 // instruction but MFMAs, LDS reads and the copies. Workgroups go to the XCDs round-robin by their
@@ -31,10 +30,12 @@ typedef float float4_t __attribute__((ext_vector_type(4)));
 #define GT_STAGE (2 * GT_HALF)                   // 32 KB
 #define GT_LDS (GT_STAGES * GT_STAGE)            // 128 KB
 
-template <int N>
-__device__ __forceinline__ void gt_wait_copies() {
-    // s_waitcnt vmcnt(N) alone: expcnt and lgkmcnt at their maxima
-    __builtin_amdgcn_s_waitcnt(0x0F70 | N);
+// Waits until at most COPIES of the wave's copies and READS of its LDS reads are on their way (the last ones: both finish in
+// their order). A barrier waits for neither.
+template <int COPIES, int READS>
+__device__ __forceinline__ void gt_wait() {
+    static_assert(COPIES < 16 && READS < 16, "fields of s_waitcnt");
+    __builtin_amdgcn_s_waitcnt(0x0070 | COPIES | (READS << 8));        // (expcnt at its maximum)
 }
 
 template <typename TO>
@@ -112,7 +113,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
     copy_stage(0, 0);
     if (nk > 1) copy_stage(1, 1);
     if (nk > 2) copy_stage(2, 2);
-    if (nk > 2) gt_wait_copies<4>(); else gt_wait_copies<0>();      // stages 0 and 1 have landed
+    if (nk > 2) gt_wait<4, 15>(); else gt_wait<0, 15>();      // stages 0 and 1 have landed
     __builtin_amdgcn_s_barrier();
     bf16x8_t fwA[4], fxA[8], fwB[4], fxB[8];
 #pragma unroll
@@ -122,18 +123,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
 
     // step it: its operands are in registers (fw_c, fx_c); stage it+1 is in LDS and is read into
     // (fw_n, fx_n) between the MFMAs, an operand of x as soon as two of this step's are used up;
-    // stages it+2 and it+3 are on their way
+    // stages it+2 and it+3 are on their way; what is refilled is the stage of step it-1
     auto step = [&](int it, auto stage_c, auto steady_c, bf16x8_t (&fw_c)[4], bf16x8_t (&fx_c)[8],
                     bf16x8_t (&fw_n)[4], bf16x8_t (&fx_n)[8]) {
         constexpr int stage = decltype(stage_c)::value;       // it & 3
         constexpr bool steady = decltype(steady_c)::value;
         constexpr int nxt = (stage + 1) & 3;
         const bool more = steady || it + 1 < nk;
-        // every other step asks for two stages, the halves of the same 128-byte lines of x and W
-        if constexpr ((stage & 1) == 0) {
-            if (steady || it + 3 < nk) copy_stage((stage + 3) & 3, it + 3);
-            if (steady || it + 4 < nk) copy_stage(stage, it + 4);
-        }
+        if (steady || it + 3 < nk) copy_stage((stage + 3) & 3, it + 3);
         if (more) {
 #pragma unroll
             for (int a = 0; a < 4; ++a) fw_n[a] = read_w(nxt, a);
@@ -153,19 +150,14 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void g
             for (int b = 0; b < 6; ++b) {
                 __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
                 __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-                if constexpr ((stage & 1) == 0) {
-                    if (b < 2) __builtin_amdgcn_sched_group_barrier(0x020, 2, 0);
-                    else __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-                }
+                if (b < 4) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
             }
             __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
         }
-        // stage it+2 must have landed (for everyone) before the next step reads it
-        if constexpr (steady) {
-            if constexpr ((stage & 1) == 0) gt_wait_copies<8>(); else gt_wait_copies<4>();
-        } else {
-            gt_wait_copies<0>();
-        }
+        // stage it+2 must have landed (for everyone) before the next step reads it, and the reads of step it-1 must have
+        // finished (for everyone) before the next step refills what they read, stage it
+        if constexpr (steady) gt_wait<4, 12>();
+        else gt_wait<0, 0>();
         __builtin_amdgcn_s_barrier();
     };
     using std::integral_constant;

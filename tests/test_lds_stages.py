@@ -104,7 +104,7 @@ def test_the_walk_finds_what_it_is_for():
 
 
 @pytest.mark.skipif(not (shutil.which("hipcc") or os.path.exists("/opt/rocm/bin/hipcc")), reason="no hipcc")
-@pytest.mark.parametrize("source", ["moe_tile.hip"])
+@pytest.mark.parametrize("source", ["moe_tile.hip", "gemm_tile.hip"])
 def test_no_stage_is_refilled_before_it_is_read(source, tmp_path):
     kernels = {n: b for n, b in _kernels(_compiled(source, tmp_path)).items() if any(" lds" in i for _, c in b for i in c)}
     assert kernels
