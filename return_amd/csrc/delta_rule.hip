@@ -18,7 +18,7 @@
 // with DPT rows in registers; the two sums over rows are finished by data-parallel moves. Columns of
 // one head are independent, so a head is spread over V / VB workgroups: the walk over the tokens is the
 // long pole, and it is as long for 16 columns as for 128. The output kernel norms a head's read-out
-// over all its columns, weighs and gates it: a wave per (row, head). In bf16 requests of RC_MIN_ROWS rows and
+// over all its columns, weighs and gates it: a wave per (row, head). In bf16 requests of rc_min_rows rows and
 // more go by chunks on the matrix cores (recurrence_chunks.hip) if a head has at most 128 channels; other requests of eight
 // rows and more take the recurrence kernel with feeder waves (below); single tokens and short portions the plain one, which
 // needs half the threads, few registers and little LDS, so that many workgroups share a CU.
@@ -627,7 +627,7 @@ static int delta_rule_run(const void* qkv, long long ld_qkv, const void* b, long
     if (TC <= 0 || max_q_len < 1) return RA_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
     int rc;
-    // Requests of RC_MIN_ROWS rows and more go by chunks on the matrix cores, as far as the heads fit those kernels (in bf16;
+    // Requests of rc_min_rows rows and more go by chunks on the matrix cores, as far as the heads fit those kernels (in bf16;
     // the 32-bit mode, which checks are run in, keeps its one order of sums);
     // the others of the step, if there are any, walk their rows here.
     int below = 0x7fffffff;
@@ -636,10 +636,10 @@ static int delta_rule_run(const void* qkv, long long ld_qkv, const void* b, long
         rc = recurrence_chunks_run(st, qkv, ld_qkv, b, ld_b, ag, ld_ag, A_log, dt_bias, S, cu_q, slot_ids, o_raw, q_lens, n_seqs,
                                    H, G, D, V, rule, rate, ws, ws_floats, dtype);
         if (rc != RA_OK) return rc;
-        below = RC_MIN_ROWS;
+        below = rc_min_rows(rule);
         max_q_len = 0;
         for (int i = 0; i < n_seqs; ++i)
-            if (q_lens[i] < RC_MIN_ROWS && q_lens[i] > max_q_len) max_q_len = q_lens[i];
+            if (q_lens[i] < below && q_lens[i] > max_q_len) max_q_len = q_lens[i];
         walk = max_q_len > 0;
     }
     // no chunk longer than the step's longest request: a step of single tokens takes an eighth of the LDS, and

@@ -13,7 +13,7 @@
 // no state: unit vectors and decays, products of decays along the rows, A and L by products of 16 x 16 tiles, T by
 // substitution in its two diagonal tiles and one product between them, U and W by products with T. The second (carry), a
 // workgroup per (request, head, 16 or 32 columns of S), goes through the chunks with its part of S in registers. All
-// products are 32-bit matrix instructions (16x16x4), every sum is 32-bit; nothing is rounded on the way.
+// products are 32-bit matrix instructions (16x16x4), every sum is 32-bit.
 //
 // The quotients P_i / P_j never overflow: products of decays are formed from one row to the next, between the two halves
 // of a chunk as (P_i from the later half's start) times (product from j to the earlier half's end), both at most one,
@@ -26,14 +26,22 @@
 // (n + 16 g), the rows 4 g .. 4 g + 3 of column n: the state's result tiles are the next product's B operands as they
 // are, without a trip through LDS. The scratch of a step is cut into runs of chunks of about RC_SCRATCH floats.
 //
+// Digits. The walk rounds a state twice a row; here the roundings are fewer but fall on products that many rows share, so they
+// are kept few: a decay near one is held as what it lacks to one, products of decays are formed as pairs of numbers, an
+// operand is an input times one factor that was formed as a pair (rounded once), numbers of a row are formed in 64 bits, and
+// every sum of products is several sums (a chain of 4 to 16 roundings). Errors against 64 bits, the walk's taken as 1, over the
+// designs' decays, 24 / 64 / 250 / 2,048 rows: read-outs of rule 0 0.93 / 0.85 / 0.67 / 0.55, rule 1 0.82 / 0.63 / 0.33 / 0.12,
+// rule 2 0.99 / 0.89 / 0.53 / 0.16, rule 3 1.00 / 0.91 / 0.74 / 0.46, states 0.79 and less; where a state forgets in a row or two,
+// read-outs 1.02 and states up to 1.15 (of 6e-8). With products of decays as single numbers and one sum each it was 1.06 to 1.37
+// and 1.0.
+//
 // Bounds and what it measured (bf16, one layer, recurrence without the output kernel): one request of 2,048 rows, 32 heads
-// of 128 x 128, rule 0: 195 us (prepare 72, carry 123) where the walk took 1,417; rule 3 180 (1,155), rule 1 134 (1,211);
-// four requests of 700 rows 260 (2,344), eight of 250 rows 181 (1,670); 64 heads of 128 x 64, rule 2, eight of 250 rows 148
-// (1,107). The products are 11 GFLOP at 32 heads of 128 x 128, about 100 us at the 32-bit matrix rate; of the carry's 1.9 us
+// of 128 x 128, rule 0: 215 us (prepare 90, carry 125) where the walk took 1,408; rule 3 197 (1,155), rule 1 147 (1,211);
+// four requests of 700 rows 287 (2,344), eight of 250 rows 199 (1,670); 64 heads of 128 x 64, rule 2, eight of 250 rows 171
+// (1,116). The products are 11 GFLOP at 32 heads of 128 x 128, about 100 us at the 32-bit matrix rate; of the carry's 1.9 us
 // a chunk 0.85 are its 56 products a wave, the rest the way of W S through LDS, which the state waits for. Asking for
 // operands two chunks ahead instead of one changes nothing; 16 columns a workgroup in place of 32 when the chip is full
-// anyway take 181 us in place of 149 (four of 700 rows). In front of the sums of four for A and L the errors against 64
-// bits were a third larger; with them they are those of the walk within a fifth (2e-7 of a state's size on random rows).
+// anyway took 181 us in place of 149 (four of 700 rows). The digits cost 4 to 12 % of the time.
 #include "common.h"
 #include "recurrence_chunks.h"
 
@@ -45,24 +53,69 @@
 typedef float rc_f4 __attribute__((ext_vector_type(4)));
 
 __device__ __forceinline__ rc_f4 rc_mfma(float a, float b, rc_f4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ rc_f4 rc_mul4(rc_f4 a, rc_f4 b, rc_f4 c) {
+// A product of two tiles as four sums, which rc_sum4 adds up: a chain of roundings is as long as four rows, not sixteen.
+struct RcSums { rc_f4 s[4]; };
+__device__ __forceinline__ RcSums rc_zero() {
+    const rc_f4 z = {0.f, 0.f, 0.f, 0.f};
+    return RcSums{{z, z, z, z}};
+}
+__device__ __forceinline__ RcSums rc_mul4(rc_f4 a, rc_f4 b, RcSums c) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) c = rc_mfma(a[r], b[r], c);
+    for (int r = 0; r < 4; ++r) c.s[r] = rc_mfma(a[r], b[r], c.s[r]);
     return c;
 }
+__device__ __forceinline__ rc_f4 rc_sum4(const RcSums& c) { return (c.s[0] + c.s[1]) + (c.s[2] + c.s[3]); }
 
 // Floats per (chunk, head): W and q P [2][DT], k P_C / P [DT][2], U [VT][2], A [3] tiles of 256, P_C [16 DT]
 __host__ __device__ static inline long long rc_stride(int DT, int VT, bool delta) {
     return (long long)((delta ? 6 : 4) * DT + 2 * VT + 3) * 256 + 16 * DT;
 }
 
-__device__ __forceinline__ float rc_sigmoid(float x) { return 1.f / (1.f + expf(-x)); }
-__device__ __forceinline__ float rc_softplus_exact(float x) { return x > 30.f ? x : log1pf(expf(x)); }
-// (as in delta_rule.hip: the decay of a key channel by the hardware's exponential and logarithm)
-__device__ __forceinline__ float rc_decay(float neg_a, float x) {
-    const float sp = x > 20.f ? x : __logf(1.f + __expf(x));
-    return __expf(neg_a * sp);
+// Numbers of a row (one or two a row and head) are formed in 64 bits: an error in them is in all of the row's elements alike.
+__device__ __forceinline__ double rc_softplus(double x) { return x > 40.0 ? x : log1p(exp(x)); }
+
+// e^x for x <= 20 to about one unit in the last place: the hardware's power of two, of a product with log2 e in two parts.
+__device__ __forceinline__ float rc_exp(float x) {
+    x = x < -150.f ? -150.f : x;
+    const float y = x * 1.44269502f, rest = fmaf(x, 1.92596303e-8f, fmaf(x, 1.44269502f, -y));
+    const float e = __builtin_amdgcn_exp2f(y);
+    return fmaf(e * 0.693147182f, rest, e);
 }
+// log(1 + t) for t >= 0: what 1 + t rounds away goes in behind; near zero by the series
+__device__ __forceinline__ float rc_log1p(float t) {
+    const float u = 1.f + t;
+    const float far = fmaf(__builtin_amdgcn_logf(u), 0.693147182f, (t - (u - 1.f)) * __builtin_amdgcn_rcpf(u));
+    const float near = t * fmaf(t, fmaf(t, fmaf(t, fmaf(t, 0.2f, -0.25f), 0.333333343f), -0.5f), 1.f);
+    return t < 0.015625f ? near : far;
+}
+// A decay e^g, g <= 0, in one word: near one as e^g - 1 with the sign set, which has the digits that e^g in 32 bits has
+// not, else e^g itself.
+#define RC_NEAR_ONE (-0.25f)
+__device__ __forceinline__ float rc_decay(float g) {
+    float e = fmaf(g, 1.f / 7.f, 1.f);
+#pragma unroll
+    for (int n = 6; n >= 2; --n) e = fmaf(g * e, 1.f / n, 1.f);
+    return g > RC_NEAR_ONE ? -fabsf(g * e) : rc_exp(g);
+}
+__device__ __forceinline__ float rc_decay(double g) { return g > RC_NEAR_ONE ? -fabsf((float)expm1(g)) : (float)exp(g); }
+// A number as the sum of two.
+struct RcPair { float hi, lo; };
+__device__ __forceinline__ RcPair rc_decay_pair(float word) {
+    if (!(__float_as_uint(word) & 0x80000000u)) return {word, 0.f};
+    const float hi = 1.f + word;
+    return {hi, word - (hi - 1.f)};
+}
+__device__ __forceinline__ RcPair rc_times(RcPair p, RcPair a) {
+    const float h = p.hi * a.hi, e = fmaf(p.lo, a.hi, fmaf(p.hi, a.lo, fmaf(p.hi, a.hi, -h))), hi = h + e;
+    return {hi, e - (hi - h)};
+}
+__device__ __forceinline__ RcPair rc_one_over(RcPair p) {
+    const float hi = __builtin_amdgcn_rcpf(p.hi);
+    return {hi, hi * fmaf(-p.lo, hi, fmaf(-p.hi, hi, 1.f))};
+}
+__device__ __forceinline__ RcPair rc_pair(double x) { return {(float)x, (float)(x - (double)(float)x)}; }
+// x times a pair, rounded once
+__device__ __forceinline__ float rc_scaled(float x, RcPair p) { return fmaf(x, p.hi, x * p.lo); }
 #define RC_DPP(v, ctrl) ((v) + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, (v)), ctrl, 0xF, 0xF, true)))
 // sums over 8 and 16 neighbouring lanes, in every one of them
 __device__ __forceinline__ float rc_sum8(float v) {
@@ -76,10 +129,10 @@ __device__ __forceinline__ float rc_sum16(float v) {
 }
 
 // Chunks of request s that the run of `run` chunks from chunk `first` on holds.
-__device__ __forceinline__ int rc_chunks(const int* cu_q, int s, int n_seqs, int first, int run) {
+__device__ __forceinline__ int rc_chunks(const int* cu_q, int s, int n_seqs, int first, int run, int min_rows) {
     if (s >= n_seqs) return 0;
     const int len = cu_q[s + 1] - cu_q[s];
-    if (len < RC_MIN_ROWS) return 0;
+    if (len < min_rows) return 0;
     return max(0, min(run, (len + RC_C - 1) / RC_C - first));
 }
 
@@ -93,9 +146,9 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
     constexpr int DP = 16 * DT, LD = DP + 4, EP = DP / 8;
     constexpr int VW = 128, LV = VW + 4;                     // columns of v that are staged at a time
     extern __shared__ __attribute__((aligned(16))) float sm[];
-    float* qs = sm;                                          // [32][LD]  q, then q P
-    float* ks = qs + RC_C * LD;                              // [32][LD]  k, then k P
-    float* as = ks + RC_C * LD;                              // [32][LD]  decays, then k / P
+    float* qs = sm;                                          // [32][LD]  q as it comes, then unit q times P
+    float* ks = qs + RC_C * LD;                              // [32][LD]  k as it comes, then unit k times P
+    float* as = ks + RC_C * LD;                              // [32][LD]  decays (rc_decay's words), then k / P
     float* kt = as + RC_C * LD;                              // [16][LD]  first half: k times the decays behind it in the half
     // [32][LV] values: with heads of 128 in the place of k / P, once A and L are formed (two workgroups share a CU's LDS)
     float* vs = DT == 8 ? as : kt + 16 * LD;
@@ -106,7 +159,9 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
     float* SL = SA + 512;
     float* pt = SL + 512;                                    // [2][DP]   product of a half's decays
     float* beta_s = pt + 2 * DP;                             // [32]
-    int* slow = (int*)(beta_s + RC_C);                       // [2]
+    RcPair* nq_s = (RcPair*)(beta_s + RC_C);                 // [32] factors that make q and k of a row unit vectors, q times its scale
+    RcPair* nk_s = nq_s + RC_C;                              // [32]
+    int* slow = (int*)(nk_s + RC_C);                         // [2]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int h = blockIdx.x, kvh = h / (H / G);
     const bool delta = rule == 0 || rule == 3;
@@ -117,7 +172,7 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
         int before = 0;
         const int want = blockIdx.y;
         for (int s0 = 0; s0 < n_seqs; s0 += 64) {
-            const int n = rc_chunks(cu_q, s0 + lane, n_seqs, first, run);
+            const int n = rc_chunks(cu_q, s0 + lane, n_seqs, first, run, rc_min_rows(rule));
             int incl = n;
 #pragma unroll
             for (int o = 1; o < 64; o <<= 1) {
@@ -146,9 +201,10 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
     float* oA = oU + 2 * VT * 256;
     float* oP = oA + 3 * 256;
 
-    const float neg_a = rule == 1 ? -rate : -expf(A_log[h]);
+    const double neg_a = rule == 1 ? -(double)rate : -exp((double)A_log[h]);
+    const float neg_a32 = (float)neg_a;
     const float a_sign = rule == 1 ? -1.f : 1.f;
-    const float q_scale = rule == 2 ? 1.f : 1.0f / sqrtf((float)D);
+    const double q_scale = rule == 2 ? 1.0 : rsqrt((double)D);
 
     // ---- rows: 8 threads each, EP neighbouring elements a thread
     const int row = tid >> 3, e0 = (tid & 7) * EP;
@@ -179,31 +235,42 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
     const T* vrow = qrow + (size_t)2 * G * D + (size_t)h * V;
     const int v0 = (tid & 7) * (VW / 8);
     take(fv, vrow + v0, v0, V, VW / 8);
-    float step = 0.f;
-    if (rule >= 2 && live) step = to_f(arow[h]) + dt_bias[h];
+    double sp = 0.0;                                         // rules 2 and 3: the row's step
+    if (rule >= 2 && live) sp = rc_softplus((double)to_f(arow[h]) + dt_bias[h]);
     float bet = 0.f;
-    if (live) bet = rule == 1 ? 1.f : rule == 2 ? rc_softplus_exact(step) : rc_sigmoid(to_f(b[(size_t)(base + c0 + row) * ld_b + h]));
+    if (live)
+        bet = rule == 1 ? 1.f : rule == 2 ? (float)sp : (float)(1.0 / (1.0 + exp(-(double)to_f(b[(size_t)(base + c0 + row) * ld_b + h]))));
     if ((tid & 7) == 0) beta_s[row] = bet;
     if (tid < 2) slow[tid] = 0;
-    float nk = 1.f, nq = q_scale;
+    double nk = 1.0, nq = q_scale;
     if (delta) {
-        float sk = 0.f, sq = 0.f;
+        double sk = 0.0, sq = 0.0;
 #pragma unroll
         for (int e = 0; e < EP; ++e) {
-            sk = fmaf(fk[e], fk[e], sk);
-            sq = fmaf(fq[e], fq[e], sq);
+            sk = fma((double)fk[e], (double)fk[e], sk);
+            sq = fma((double)fq[e], (double)fq[e], sq);
         }
-        nk = 1.0f / sqrtf(rc_sum8(sk) + 1e-6f);
-        nq = q_scale / sqrtf(rc_sum8(sq) + 1e-6f);
+        nk = rsqrt((double)rc_sum8((float)sk) + 1e-6);
+        nq = q_scale * rsqrt((double)rc_sum8((float)sq) + 1e-6);
     }
-    const float row_decay = rule >= 2 && live ? expf(neg_a * rc_softplus_exact(step)) : 1.f;
+    if ((tid & 7) == 0) {
+        nq_s[row] = rc_pair(nq);
+        nk_s[row] = rc_pair(nk);
+    }
+    const float one = -0.f;                                  // (rc_decay's word for it)
+    const float row_decay = rule >= 2 && live ? rc_decay(neg_a * sp) : one;
 #pragma unroll
     for (int e = 0; e < EP; ++e) {
         const bool in = live && e0 + e < D;
-        if (rule < 2) fa[e] = in ? rc_decay(neg_a, a_sign * (fa[e] + dt_bias[h * D + e0 + e])) : 1.f;
-        else fa[e] = in ? row_decay : 1.f;
-        qs[row * LD + e0 + e] = fq[e] * nq;
-        ks[row * LD + e0 + e] = fk[e] * nk;
+        if (rule < 2) {
+            const float x = in ? a_sign * (fa[e] + dt_bias[h * D + e0 + e]) : 0.f;
+            const float word = rc_decay(neg_a32 * (x > 20.f ? x : rc_log1p(rc_exp(x > 20.f ? 20.f : x))));
+            fa[e] = in ? word : one;
+        } else {
+            fa[e] = in ? row_decay : one;
+        }
+        qs[row * LD + e0 + e] = fq[e];
+        ks[row * LD + e0 + e] = fk[e];
         as[row * LD + e0 + e] = fa[e];
     }
     __syncthreads();
@@ -212,18 +279,20 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
     const int hf = tid / DP, d = tid - hf * DP;
     const bool chan = hf < 2;
     float ak[16], aq[16], aa[16];
+    RcPair pp[16];
     if (chan) {
-        float p = 1.f;
+        RcPair p = {1.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int at = (hf * 16 + i) * LD + d;
             aq[i] = qs[at];
             ak[i] = ks[at];
             aa[i] = as[at];
-            p *= aa[i];
+            p = rc_times(p, rc_decay_pair(aa[i]));
+            pp[i] = p;
         }
-        pt[hf * DP + d] = p;
-        if (!(p >= RC_TINY)) slow[hf] = 1;
+        pt[hf * DP + d] = p.hi;
+        if (!(p.hi >= RC_TINY)) slow[hf] = 1;
     }
     __syncthreads();
     // (a half whose decays go below RC_TINY: pairs one by one, 16 lanes to a column j, their channels' products carried
@@ -237,17 +306,18 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
 #pragma unroll
             for (int e = 0; e < DT; ++e) {
                 p[e] = 1.f;
-                kj[e] = ks[(x * 16 + j) * LD + sl + 16 * e];
+                kj[e] = rc_scaled(ks[(x * 16 + j) * LD + sl + 16 * e], nk_s[x * 16 + j]);
             }
             for (int i = 0; i < 16; ++i) {
+                const RcPair fq_i = nq_s[x * 16 + i], fk_i = nk_s[x * 16 + i];
                 float da = 0.f, dl = 0.f;
 #pragma unroll
                 for (int e = 0; e < DT; ++e) {
                     const int at = (x * 16 + i) * LD + sl + 16 * e;
-                    if (i > j) p[e] *= as[at];
+                    if (i > j) p[e] *= rc_decay_pair(as[at]).hi;
                     const float kp = kj[e] * p[e];
-                    da = fmaf(qs[at], kp, da);
-                    dl = fmaf(ks[at], kp, dl);
+                    da = fmaf(rc_scaled(qs[at], fq_i), kp, da);
+                    dl = fmaf(rc_scaled(ks[at], fk_i), kp, dl);
                 }
                 da = rc_sum16(da);
                 dl = rc_sum16(dl);
@@ -262,11 +332,12 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
     if (chan) {
         // k times the decays behind it in the half; times the second half's product it is k P_C / P
         const float other = hf == 0 ? pt[DP + d] : 1.f;
-        float p = 1.f, kend[16];
+        RcPair p = {1.f, 0.f};
+        float kend[16];
 #pragma unroll
         for (int i = 15; i >= 0; --i) {
-            kend[i] = ak[i] * p;
-            p *= aa[i];
+            kend[i] = rc_scaled(ak[i], rc_times(p, nk_s[hf * 16 + i]));
+            p = rc_times(p, rc_decay_pair(aa[i]));
         }
         if (hf == 0) {
 #pragma unroll
@@ -277,14 +348,13 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
             const rc_f4 x = {kend[4 * g] * other, kend[4 * g + 1] * other, kend[4 * g + 2] * other, kend[4 * g + 3] * other};
             *reinterpret_cast<rc_f4*>(oK + (((d >> 4) * 2 + hf) * 64 + g * 16 + (d & 15)) * 4) = x;
         }
-        p = 1.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int at = (hf * 16 + i) * LD + d;
-            p *= aa[i];
-            qs[at] = aq[i] * p;
-            ks[at] = ak[i] * p;
-            as[at] = ak[i] / p;
+            const RcPair fk_i = nk_s[hf * 16 + i];
+            qs[at] = rc_scaled(aq[i], rc_times(pp[i], nq_s[hf * 16 + i]));
+            ks[at] = rc_scaled(ak[i], rc_times(pp[i], fk_i));
+            as[at] = rc_scaled(ak[i], rc_times(rc_one_over(pp[i]), fk_i));
         }
     }
     __syncthreads();
@@ -296,24 +366,18 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
         const float* col = wave < 2 ? as + (bj * 16 + m16) * LD : kt + m16 * LD;
         const float* rq = qs + (bi * 16 + m16) * LD;
         const float* rk = ks + (bi * 16 + m16) * LD;
-        // (four sums each, so that no product waits for the one before, and short chains of roundings)
-        rc_f4 pa[4], pl[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) pa[i] = pl[i] = rc_f4{0.f, 0.f, 0.f, 0.f};
+        // (sixteen sums each: short chains of roundings)
+        RcSums pa[4] = {rc_zero(), rc_zero(), rc_zero(), rc_zero()}, pl[4] = {rc_zero(), rc_zero(), rc_zero(), rc_zero()};
 #pragma unroll
         for (int t = 0; t < DT; ++t) {
             const rc_f4 x = *reinterpret_cast<const rc_f4*>(col + 16 * t + g4);
             const rc_f4 y = *reinterpret_cast<const rc_f4*>(rq + 16 * t + g4);
-#pragma unroll
-            for (int r = 0; r < 4; ++r) pa[r] = rc_mfma(x[r], y[r], pa[r]);
-            if (delta) {
-                const rc_f4 z = *reinterpret_cast<const rc_f4*>(rk + 16 * t + g4);
-#pragma unroll
-                for (int r = 0; r < 4; ++r) pl[r] = rc_mfma(x[r], z[r], pl[r]);
-            }
+            pa[t & 3] = rc_mul4(x, y, pa[t & 3]);
+            if (delta) pl[t & 3] = rc_mul4(x, *reinterpret_cast<const rc_f4*>(rk + 16 * t + g4), pl[t & 3]);
         }
         MFMA_SETTLE();
-        rc_f4 ta = (pa[0] + pa[1]) + (pa[2] + pa[3]), tl = (pl[0] + pl[1]) + (pl[2] + pl[3]);
+        rc_f4 ta = (rc_sum4(pa[0]) + rc_sum4(pa[1])) + (rc_sum4(pa[2]) + rc_sum4(pa[3]));
+        rc_f4 tl = (rc_sum4(pl[0]) + rc_sum4(pl[1])) + (rc_sum4(pl[2]) + rc_sum4(pl[3]));
         // (lane m16 + 16 g: row i = m16, columns j = 4 g .. 4 g + 3)
         if (wave < 2) {
             if (wave ? slow1 : slow0) {
@@ -386,12 +450,11 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
                 x0[r] = ks[(g4 + r) * LD + 16 * t + m16] * beta_s[g4 + r];
                 x1[r] = ks[(16 + g4 + r) * LD + 16 * t + m16] * p0 * beta_s[16 + g4 + r];
             }
-            const rc_f4 zero = {0.f, 0.f, 0.f, 0.f};
-            const rc_f4 w0 = rc_mul4(x0, t00, zero);
-            const rc_f4 w1 = rc_mul4(x1, t11, rc_mul4(x0, t10, zero));
+            const RcSums w0 = rc_mul4(x0, t00, rc_zero());
+            const RcSums w1 = rc_mul4(x1, t11, rc_mul4(x0, t10, rc_zero()));
             MFMA_SETTLE();
-            *reinterpret_cast<rc_f4*>(oW + (t * 64 + lane) * 4) = w0;
-            *reinterpret_cast<rc_f4*>(oW + ((DT + t) * 64 + lane) * 4) = w1;
+            *reinterpret_cast<rc_f4*>(oW + (t * 64 + lane) * 4) = rc_sum4(w0);
+            *reinterpret_cast<rc_f4*>(oW + ((DT + t) * 64 + lane) * 4) = rc_sum4(w1);
         }
         // ---- U = T beta v, 128 columns of v at a time
         for (int vb = 0; vb < V; vb += VW) {
@@ -410,13 +473,12 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
                     x0[r] = vs[(g4 + r) * LV + 16 * n + m16];
                     x1[r] = vs[(16 + g4 + r) * LV + 16 * n + m16];
                 }
-                const rc_f4 zero = {0.f, 0.f, 0.f, 0.f};
-                const rc_f4 u0 = rc_mul4(t00, x0, zero);
-                const rc_f4 u1 = rc_mul4(t11, x1, rc_mul4(t10, x0, zero));
+                const RcSums u0 = rc_mul4(t00, x0, rc_zero());
+                const RcSums u1 = rc_mul4(t11, x1, rc_mul4(t10, x0, rc_zero()));
                 MFMA_SETTLE();
                 float* to = oU + (long long)(vb / 16 + n) * 512 + lane * 4;
-                *reinterpret_cast<rc_f4*>(to) = u0;
-                *reinterpret_cast<rc_f4*>(to + 256) = u1;
+                *reinterpret_cast<rc_f4*>(to) = rc_sum4(u0);
+                *reinterpret_cast<rc_f4*>(to + 256) = rc_sum4(u1);
             }
         }
         return;
@@ -448,7 +510,7 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
 
 static size_t rc_prepare_lds(int DT) {
     const int LD = 16 * DT + 4;
-    return sizeof(float) * ((size_t)(3 * RC_C + 16) * LD + (DT == 8 ? 0 : RC_C * 132) + 2 * RC_C * 36 + 16 * 20 + 1024 + 32 * DT + RC_C + 4);
+    return sizeof(float) * ((size_t)(3 * RC_C + 16) * LD + (DT == 8 ? 0 : RC_C * 132) + 2 * RC_C * 36 + 16 * 20 + 1024 + 32 * DT + 5 * RC_C + 4);
 }
 
 // ---------------------------------------------------------------------------------------------------- carry
@@ -461,9 +523,9 @@ struct RcChunk {
 // A wave holds 16 DPW rows of the workgroup's columns of S and takes part in every product with the state over its own
 // rows; the four waves' shares of W S and q P S meet in LDS (two buffers, one barrier a chunk).
 template <int DT, int NV, bool DELTA>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) void recur_carry_kernel(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DELTA ? 1 : 2, 2))) void recur_carry_kernel(
     const float* __restrict__ ws, float* __restrict__ S, const int* __restrict__ cu_q, const int* __restrict__ slot_ids,
-    float* __restrict__ o_raw, int n_seqs, int H, int D, int V, int first, int run, int splits) {
+    float* __restrict__ o_raw, int n_seqs, int H, int D, int V, int first, int run, int splits, int min_rows) {
     constexpr int DPW = DT / 4, PARTS = DELTA ? 4 : 2;
     __shared__ __attribute__((aligned(16))) float part[2][4][PARTS][NV][256];
     // the splits of one head lie eight workgroups apart, on one XCD, whose L2 then holds what they share
@@ -471,10 +533,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     const int s = unit / H, h = unit - s * H;
     if (s >= n_seqs) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m16 = lane & 15, g4 = (lane >> 4) * 4;
-    const int n_chunks = rc_chunks(cu_q, s, n_seqs, first, run);
+    const int n_chunks = rc_chunks(cu_q, s, n_seqs, first, run, min_rows);
     if (n_chunks <= 0) return;
     int before = 0;
-    for (int r = lane; r < s; r += 64) before += rc_chunks(cu_q, r, n_seqs, first, run);
+    for (int r = lane; r < s; r += 64) before += rc_chunks(cu_q, r, n_seqs, first, run, min_rows);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
     const int base = cu_q[s], q_len = cu_q[s + 1] - base;
@@ -537,41 +599,35 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
     };
 
     auto go = [&](const Chunk& x, int ci, int buf) {
-        rc_f4 sw[NV][2], sq[NV][2];
+        // (two sums each, as of S below: half the chain of roundings. W S first: the next chunk's state waits for it, q P S
+        // only for the read-out. The reads of these results sit in the same basic block, where the compiler keeps the
+        // distance by itself.)
+        auto with_state = [&](const rc_f4 (&m)[2][DPW], int what, int nv) {
+            rc_f4 s[2][2];
 #pragma unroll
-        for (int nv = 0; nv < NV; ++nv)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                sw[nv][i] = sq[nv][i] = rc_f4{0.f, 0.f, 0.f, 0.f};
-            }
-        // (W S first: the next chunk's state waits for it, q P S only for the read-out. The reads of these results sit in
-        // the same basic block, where the compiler keeps the distance by itself.)
-        if constexpr (DELTA) {
+            for (int i = 0; i < 2; ++i) s[0][i] = s[1][i] = rc_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int t = 0; t < DPW; ++t)
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
 #pragma unroll
-                    for (int nv = 0; nv < NV; ++nv)
+                    for (int i = 0; i < 2; ++i) s[r & 1][i] = rc_mfma(m[i][t][r], st[nv][t][r], s[r & 1][i]);
 #pragma unroll
-                        for (int i = 0; i < 2; ++i) sw[nv][i] = rc_mfma(x.w[i][t][r], st[nv][t][r], sw[nv][i]);
+            for (int i = 0; i < 2; ++i) *reinterpret_cast<rc_f4*>(&part[buf][wave][what + i][nv][lane * 4]) = s[0][i] + s[1][i];
+        };
+        if constexpr (DELTA) {
+#pragma unroll
+            for (int nv = 0; nv < NV; ++nv) with_state(x.w, 2, nv);
         }
 #pragma unroll
-        for (int t = 0; t < DPW; ++t)
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-#pragma unroll
-                for (int nv = 0; nv < NV; ++nv)
-#pragma unroll
-                    for (int i = 0; i < 2; ++i) sq[nv][i] = rc_mfma(x.q[i][t][r], st[nv][t][r], sq[nv][i]);
-#pragma unroll
-        for (int nv = 0; nv < NV; ++nv)
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                *reinterpret_cast<rc_f4*>(&part[buf][wave][i][nv][lane * 4]) = sq[nv][i];
-                if constexpr (DELTA) *reinterpret_cast<rc_f4*>(&part[buf][wave][2 + i][nv][lane * 4]) = sw[nv][i];
-            }
+        for (int nv = 0; nv < NV; ++nv) with_state(x.q, 0, nv);
         __syncthreads();
+        auto sum_waves = [&](int what, int nv) {
+            rc_f4 w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[i] = *reinterpret_cast<const rc_f4*>(&part[buf][i][what][nv][lane * 4]);
+            return (w[0] + w[1]) + (w[2] + w[3]);
+        };
         rc_f4 u[NV][2];
 #pragma unroll
         for (int nv = 0; nv < NV; ++nv)
@@ -579,40 +635,57 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
             for (int i = 0; i < 2; ++i) {
                 u[nv][i] = x.u[nv][i];
                 if constexpr (DELTA) {
-                    rc_f4 sum = *reinterpret_cast<const rc_f4*>(&part[buf][0][2 + i][nv][lane * 4]);
-#pragma unroll
-                    for (int w = 1; w < 4; ++w) sum += *reinterpret_cast<const rc_f4*>(&part[buf][w][2 + i][nv][lane * 4]);
-                    u[nv][i] -= sum;
+                    u[nv][i] -= sum_waves(2 + i, nv);
                 }
             }
+        auto move_on = [&]() {
 #pragma unroll
-        for (int nv = 0; nv < NV; ++nv)
+            for (int nv = 0; nv < NV; ++nv) {
+                rc_f4 ku[2][DPW];
 #pragma unroll
-            for (int t = 0; t < DPW; ++t) st[nv][t] *= x.p[t];
+                for (int t = 0; t < DPW; ++t) ku[0][t] = ku[1][t] = rc_f4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+                for (int i = 0; i < 2; ++i)
 #pragma unroll
-            for (int r = 0; r < 4; ++r)
+                    for (int r = 0; r < 4; ++r)
 #pragma unroll
-                for (int nv = 0; nv < NV; ++nv)
+                        for (int t = 0; t < DPW; ++t) ku[r & 1][t] = rc_mfma(x.k[t][i][r], u[nv][i][r], ku[r & 1][t]);
 #pragma unroll
-                    for (int t = 0; t < DPW; ++t) st[nv][t] = rc_mfma(x.k[t][i][r], u[nv][i][r], st[nv][t]);
+                for (int t = 0; t < DPW; ++t) {
+                    const rc_f4 add = ku[0][t] + ku[1][t];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) st[nv][t][r] = fmaf(st[nv][t][r], x.p[t][r], add[r]);
+                }
+            }
+        };
+        // (the delta rules' next chunk waits for S; without a correction nothing does, and the read-out first takes fewer registers)
+        if constexpr (DELTA) move_on();
         if (on < NV) {
-            rc_f4 o = *reinterpret_cast<const rc_f4*>(&part[buf][0][oi][on][lane * 4]);
-#pragma unroll
-            for (int w = 1; w < 4; ++w) o += *reinterpret_cast<const rc_f4*>(&part[buf][w][oi][on][lane * 4]);
+            rc_f4 o = sum_waves(oi, on);
             const rc_f4 u0 = on ? u[NV - 1][0] : u[0][0], u1 = on ? u[NV - 1][1] : u[0][1];
-            o = rc_mul4(x.a[0], u0, o);
-            if (oi) o = rc_mul4(x.a[1], u1, o);
+            constexpr int SUMS = DELTA || NV == 1 || DT < 8 ? 4 : 2;      // (what the registers of two workgroups a CU hold)
+            rc_f4 au[SUMS];
+#pragma unroll
+            for (int r = 0; r < SUMS; ++r) au[r] = rc_f4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < 4; ++r) au[r % SUMS] = rc_mfma(x.a[0][r], u0[r], au[r % SUMS]);
+            if (oi) {
+#pragma unroll
+                for (int r = 0; r < 4; ++r) au[r % SUMS] = rc_mfma(x.a[1][r], u1[r], au[r % SUMS]);
+            }
             MFMA_SETTLE();
+            if constexpr (SUMS == 4) o += (au[0] + au[1]) + (au[2] + au[3]);
+            else o += au[0] + au[1];
             const int v = (split * NV + on) * 16 + m16, c0 = (first + ci) * RC_C + oi * 16 + g4;
             if (v < V) {
 #pragma unroll
                 for (int r = 0; r < 4; ++r)
                     if (c0 + r < q_len) o_raw[(size_t)(base + c0 + r) * H * V + (size_t)h * V + v] = o[r];
             }
-        } else {
-            MFMA_SETTLE();
+        }
+        if constexpr (!DELTA) {
+            __builtin_amdgcn_sched_barrier(0);
+            move_on();
         }
     };
 
@@ -657,10 +730,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(1, 2))) voi
 static int rc_tiles(int D) { return D <= 64 ? 4 : 8; }
 
 // Chunks of every request that a run takes at once, so that the scratch of a group of requests stays near RC_SCRATCH.
-static int rc_run(const int* q_lens, int n, int H, long long stride, int* longest, long long* most) {
+static int rc_run(const int* q_lens, int n, int H, long long stride, int min_rows, int* longest, long long* most) {
     int count = 0, top = 0;
     for (int i = 0; i < n; ++i)
-        if (q_lens[i] >= RC_MIN_ROWS) {
+        if (q_lens[i] >= min_rows) {
             ++count;
             top = top > (q_lens[i] + RC_C - 1) / RC_C ? top : (q_lens[i] + RC_C - 1) / RC_C;
         }
@@ -671,7 +744,7 @@ static int rc_run(const int* q_lens, int n, int H, long long stride, int* longes
     if (run < 1) run = 1;
     if (run > top) run = top;
     for (int i = 0; i < n; ++i)
-        if (q_lens[i] >= RC_MIN_ROWS) {
+        if (q_lens[i] >= min_rows) {
             const long long c = (q_lens[i] + RC_C - 1) / RC_C;
             *most += c < run ? c : run;
         }
@@ -685,7 +758,7 @@ long long recurrence_chunks_workspace(const int* q_lens, int n_seqs, int H, int 
     for (int r0 = 0; r0 < n_seqs; r0 += RC_GROUP) {
         int longest;
         long long most;
-        rc_run(q_lens + r0, n_seqs - r0 < RC_GROUP ? n_seqs - r0 : RC_GROUP, H, stride, &longest, &most);
+        rc_run(q_lens + r0, n_seqs - r0 < RC_GROUP ? n_seqs - r0 : RC_GROUP, H, stride, rc_min_rows(rule), &longest, &most);
         if (most * H * stride > need) need = most * H * stride;
     }
     return need;
@@ -710,12 +783,12 @@ static int rc_launch(hipStream_t st, const T* qkv, long long ld_qkv, const T* b,
         const int n = n_seqs - r0 < RC_GROUP ? n_seqs - r0 : RC_GROUP;
         int longest;
         long long most;
-        const int run = rc_run(q_lens + r0, n, H, stride, &longest, &most);
+        const int run = rc_run(q_lens + r0, n, H, stride, rc_min_rows(rule), &longest, &most);
         for (int first = 0; first < longest; first += run) {
             long long chunks = 0;
             for (int i = 0; i < n; ++i) {
                 const int len = q_lens[r0 + i];
-                const long long c = len < RC_MIN_ROWS ? 0 : (len + RC_C - 1) / RC_C - first;
+                const long long c = len < rc_min_rows(rule) ? 0 : (len + RC_C - 1) / RC_C - first;
                 chunks += c < 0 ? 0 : c < run ? c : run;
             }
             if (chunks > 65535) return RA_ERR_ARG;
@@ -728,7 +801,7 @@ static int rc_launch(hipStream_t st, const T* qkv, long long ld_qkv, const T* b,
             const dim3 grid((unsigned)(units * splits));
 #define RC_CARRY(NV_, DE_)                                                                                                    \
     hipLaunchKernelGGL((recur_carry_kernel<DT, NV_, DE_>), grid, dim3(256), 0, st, ws, S, cu_q + r0, slot_ids + r0, o_raw, n, \
-                       H, D, V, first, run, splits)
+                       H, D, V, first, run, splits, rc_min_rows(rule))
             if (wide && delta) RC_CARRY(2, true);
             else if (wide) RC_CARRY(2, false);
             else if (delta) RC_CARRY(1, true);

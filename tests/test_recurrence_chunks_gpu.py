@@ -1,10 +1,13 @@
-"""The recurrences by chunks of rows on the matrix cores (bf16, requests of 16 rows and more) against the stand-ins that
+"""The recurrences by chunks of rows on the matrix cores (bf16, requests of 16 or 24 rows and more) against the stand-ins that
 walk the rows, at the edges of chunks and halves, of tiles of channels and columns, of runs of chunks and groups of requests,
 with decays from one to zero, and with rows that begin at unaligned addresses."""
+import ctypes
+
 import pytest
 import torch
 
-from tests.test_kofipel_gpu import DEV, ops, ref, rnd, state_step  # noqa: F401
+from return_amd.kernels.hip_ops import _ptr
+from tests.test_kofipel_gpu import DEV, i32, ops, ref, rnd, state_step  # noqa: F401
 
 pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
@@ -48,7 +51,7 @@ RULES = ["channel", "head", "outer", "scalar"]
 @pytest.mark.parametrize("H,G,D,V,q_lens,offset", [
     (2, 1, 128, 128, [16, 17, 15, 1, 31], 0), (3, 3, 64, 16, [32, 33, 2, 64], 0), (2, 2, 80, 40, [65, 96, 97], 0),
     (4, 2, 24, 8, [127], 8), (2, 1, 128, 130, [47, 16], 0), (2, 2, 33, 17, [48, 20], 1), (1, 1, 1, 1, [18], 3),
-    (2, 1, 66, 34, [40], 2), (8, 2, 128, 64, [9, 40] * 35, 0)])
+    (2, 1, 66, 34, [40], 2), (8, 2, 128, 64, [9, 40] * 35, 0), (2, 1, 128, 128, [24, 23, 31, 32], 0), (2, 2, 48, 24, [25, 26], 0)])
 def test_against_the_walk(ops, ref, rule, H, G, D, V, q_lens, offset):
     both(ops, ref, rule, q_lens, H, H if rule == "outer" else G, D, V, offset=offset)
 
@@ -82,3 +85,87 @@ def test_runs_of_chunks(ops, ref, rule):
     assert ops.lib.ra_recurrence_scratch((__import__("ctypes").c_int * 1)(T), 1, H, D, V, 3) < 30 * H * 17600
     torch.testing.assert_close(got[0][0], got[1][0], atol=0, rtol=0)        # the cut falls on a chunk's border
     torch.testing.assert_close(got[0][1], got[1][1], atol=0, rtol=0)
+
+
+# ------------------------------------------------------------------ read-outs and states as they come, before the norm
+NUMBER = {"channel": 0, "outer": 1, "scalar": 2, "head": 3}
+
+
+def drawn(rule, q_lens, H, G, D, V, seed):
+    """A layer's inputs as the designs have them: rows behind a SiLU, decays by the package's own laws (near one)."""
+    T, law = sum(q_lens), torch.Generator(device=DEV).manual_seed(seed)
+    uniform = lambda n, lo, hi: lo + (hi - lo) * torch.rand(n, generator=law, device=DEV)
+    per = H * D if rule in ("channel", "outer") else H
+    qkv = rnd(T, 2 * G * D + H * V, seed=seed)
+    return dict(qkv=(qkv if rule == "outer" else torch.nn.functional.silu(qkv)).to(BF), b=rnd(T, H, dtype=BF, seed=seed + 1, scale=0.5),
+                a=rnd(T, per + (H * V if rule == "channel" else 0), dtype=BF, seed=seed + 2, scale=0.5), a_log=uniform(H, 0.02, 1).log(),
+                bias=uniform(per, 2, 5) if rule == "outer" else uniform(per, -4, -1), rate=1 / 16)
+
+
+def recur(ops, rule, x, state, q_lens, H, G, D, V, chunks):
+    """Read-outs [T, H V] of the step, by chunks of rows or row by row; the state moves on."""
+    T, n, number = sum(q_lens), len(q_lens), NUMBER[rule]
+    step = state_step(q_lens, list(range(n)))
+    o, out = torch.empty(T, H * V, device=DEV), torch.empty(T, H * V, dtype=BF, device=DEV)
+    rows = (ctypes.c_int * n)(*q_lens) if chunks else None
+    floats = ops.lib.ra_recurrence_scratch(rows, n, H, D, V, number) if chunks else 0
+    assert not chunks or floats > 0
+    ws = torch.empty(floats, device=DEV) if chunks else None
+    ones, gate = torch.ones(H * V, device=DEV), torch.zeros(T, H * V, dtype=BF, device=DEV)
+    end = (_ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), _ptr(o), _ptr(out), n, T, max(q_lens), rows, _ptr(ws), floats, H)
+    qkv, a, lib, last = (_ptr(x["qkv"]), x["qkv"].stride(0)), (_ptr(x["a"]), x["a"].stride(0)), ops.lib, (D, V, 1, ops._stream())
+    b, g, law = (_ptr(x["b"]), H), (_ptr(gate), H * V), (_ptr(x["a_log"]), _ptr(x["bias"]))
+    if rule == "channel":
+        code = lib.ra_delta_rule(*qkv, *b, *a, *law, _ptr(ones), 1e-5, *end, G, *last)
+    elif rule == "head":
+        code = lib.ra_delta_rule_head(*qkv, *b, *a, *g, *law, _ptr(ones), 1e-5, *end, G, *last)
+    elif rule == "outer":
+        code = lib.ra_outer_rule(*qkv, *a, *g, law[1], x["rate"], _ptr(ones), 1e-5, *end, *last)
+    else:
+        code = lib.ra_scalar_rule(*qkv, *a, *g, *law, _ptr(ones), _ptr(ones), 1, 1e-5, *end, G, *last)
+    ops._check(code, rule)
+    return o
+
+
+def recur64(rule, x, state, q_lens, H, G, D, V):
+    """The same in 64 bits, row by row."""
+    f = {k: v.double() if torch.is_tensor(v) else v for k, v in x.items()}
+    T, per = sum(q_lens), D if rule in ("channel", "outer") else 1
+    q, k, v = (t.view(T, -1, w) for t, w in zip(f["qkv"].split([G * D, G * D, H * V], 1), (D, D, V)))
+    if rule in ("channel", "head"):
+        q, k = (t * torch.rsqrt((t * t).sum(-1, keepdim=True) + 1e-6) for t in (q, k))
+    q, k = (t.repeat_interleave(H // G, 1) for t in (q * (1.0 if rule == "scalar" else D ** -0.5), k))
+    a = (f["a"][:, :H * per] + f["bias"]).view(T, H, per)
+    step = torch.logaddexp(a, torch.zeros_like(a))
+    decay = torch.sigmoid(a) ** f["rate"] if rule == "outer" else torch.exp(-f["a_log"].exp()[:, None] * step)
+    k = k * step if rule == "scalar" else k
+    beta, S, out, at = torch.sigmoid(f["b"]), state.double(), torch.empty(T, H, V, dtype=torch.float64, device=DEV), 0
+    for s, n in enumerate(q_lens):
+        for t in range(at, at + n):
+            M = S[s] * decay[t][:, None]
+            u = v[t]
+            if rule in ("channel", "head"):
+                u = beta[t][:, None] * (u - (M @ k[t][:, :, None])[..., 0])
+            S[s] = M + u[:, :, None] * k[t][:, None]
+            out[t] = (S[s] @ q[t][:, :, None])[..., 0]
+        at += n
+    return out.view(T, H * V), S
+
+
+@pytest.mark.parametrize("rule,H,G,D,V", [("channel", 16, 4, 128, 128), ("head", 16, 4, 128, 128), ("outer", 16, 16, 128, 128),
+                                          ("scalar", 32, 8, 128, 64)])
+@pytest.mark.parametrize("q_lens", [[24] * 4, [33] * 3, [48] * 3, [250] * 2, [700]], ids=str)
+def test_no_further_from_64_bits_than_the_walk(ops, rule, H, G, D, V, q_lens):
+    """Over the designs' decays the chunks' read-outs and states are at most as far from the 64-bit recurrence as those of the
+    kernels that go row by row (three draws together, 2 % for their scatter)."""
+    far = {True: [0.0, 0.0], False: [0.0, 0.0]}
+    for seed in (1, 101, 201):
+        x = drawn(rule, q_lens, H, G, D, V, seed)
+        start = torch.zeros(len(q_lens), H, V, D, device=DEV)
+        want = recur64(rule, x, start, q_lens, H, G, D, V)
+        for chunks in (True, False):
+            state = start.clone()
+            got = recur(ops, rule, x, state, q_lens, H, G, D, V, chunks), state
+            for i in (0, 1):
+                far[chunks][i] += float((got[i].double() - want[i]).norm() / want[i].norm()) / 3
+    assert far[True][0] <= 1.02 * far[False][0] and far[True][1] <= 1.02 * far[False][1], far
