@@ -128,7 +128,8 @@ __device__ __forceinline__ float rc_sum16(float v) {
     return RC_DPP(v, 0x140);
 }
 
-// Chunks of request s that the run of `run` chunks from chunk `first` on holds.
+// Chunks of request s that the run of `run` chunks from chunk `first` on holds. (min_rows comes from the rule in the kernel:
+// not knowing that a request has at least 16 rows costs the carry 112 registers.)
 __device__ __forceinline__ int rc_chunks(const int* cu_q, int s, int n_seqs, int first, int run, int min_rows) {
     if (s >= n_seqs) return 0;
     const int len = cu_q[s + 1] - cu_q[s];
@@ -525,7 +526,7 @@ struct RcChunk {
 template <int DT, int NV, bool DELTA>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DELTA ? 1 : 2, 2))) void recur_carry_kernel(
     const float* __restrict__ ws, float* __restrict__ S, const int* __restrict__ cu_q, const int* __restrict__ slot_ids,
-    float* __restrict__ o_raw, int n_seqs, int H, int D, int V, int first, int run, int splits, int min_rows) {
+    float* __restrict__ o_raw, int n_seqs, int H, int D, int V, int first, int run, int splits, int rule) {
     constexpr int DPW = DT / 4, PARTS = DELTA ? 4 : 2;
     __shared__ __attribute__((aligned(16))) float part[2][4][PARTS][NV][256];
     // the splits of one head lie eight workgroups apart, on one XCD, whose L2 then holds what they share
@@ -533,10 +534,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DELTA ? 1 :
     const int s = unit / H, h = unit - s * H;
     if (s >= n_seqs) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, m16 = lane & 15, g4 = (lane >> 4) * 4;
-    const int n_chunks = rc_chunks(cu_q, s, n_seqs, first, run, min_rows);
+    const int n_chunks = rc_chunks(cu_q, s, n_seqs, first, run, rc_min_rows(rule));
     if (n_chunks <= 0) return;
     int before = 0;
-    for (int r = lane; r < s; r += 64) before += rc_chunks(cu_q, r, n_seqs, first, run, min_rows);
+    for (int r = lane; r < s; r += 64) before += rc_chunks(cu_q, r, n_seqs, first, run, rc_min_rows(rule));
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) before += __shfl_xor(before, o, 64);
     const int base = cu_q[s], q_len = cu_q[s + 1] - base;
@@ -801,7 +802,7 @@ static int rc_launch(hipStream_t st, const T* qkv, long long ld_qkv, const T* b,
             const dim3 grid((unsigned)(units * splits));
 #define RC_CARRY(NV_, DE_)                                                                                                    \
     hipLaunchKernelGGL((recur_carry_kernel<DT, NV_, DE_>), grid, dim3(256), 0, st, ws, S, cu_q + r0, slot_ids + r0, o_raw, n, \
-                       H, D, V, first, run, splits, rc_min_rows(rule))
+                       H, D, V, first, run, splits, rule)
             if (wide && delta) RC_CARRY(2, true);
             else if (wide) RC_CARRY(2, false);
             else if (delta) RC_CARRY(1, true);
