@@ -17,8 +17,8 @@
 //
 // The quotients P_i / P_j never overflow: products of decays are formed from one row to the next, between the two halves
 // of a chunk as (P_i from the later half's start) times (product from j to the earlier half's end), both at most one,
-// and inside a half as (q_i P_i) (k_j / P_j) only where the half's whole product is at least RC_TINY in every channel;
-// else the half's pairs are formed one by one with the products between them (recur_pairs).
+// and inside a half as (q_i P_i) (k_j / P_j) only where the half's whole product is at least RC_TINY in every channel
+// and no key is beyond RC_LARGE; else the half's pairs are formed one by one with the products between them (recur_pairs).
 //
 // What the carry reads lies in scratch in the order of the matrix instructions' operands: an A operand of the 16x16x4
 // product holds, lane (m + 16 g), the four columns 4 g .. 4 g + 3 of row m as one 16-byte load that serves four
@@ -36,17 +36,23 @@
 // and 1.0.
 //
 // Bounds and what it measured (bf16, one layer, recurrence without the output kernel): one request of 2,048 rows, 32 heads
-// of 128 x 128, rule 0: 215 us (prepare 90, carry 125) where the walk took 1,408; rule 3 197 (1,155), rule 1 147 (1,211);
-// four requests of 700 rows 287 (2,344), eight of 250 rows 199 (1,670); 64 heads of 128 x 64, rule 2, eight of 250 rows 171
+// of 128 x 128, rule 0: 224 us (prepare 97, carry 127) where the walk took 1,408; rule 3 202 (1,155), rule 1 148 (1,211);
+// four requests of 700 rows 295 (2,344), eight of 250 rows 208 (1,670); 64 heads of 128 x 64, rule 2, eight of 250 rows 172
 // (1,116). The products are 11 GFLOP at 32 heads of 128 x 128, about 100 us at the 32-bit matrix rate; of the carry's 1.9 us
 // a chunk 0.85 are its 56 products a wave, the rest the way of W S through LDS, which the state waits for. Asking for
 // operands two chunks ahead instead of one changes nothing; 16 columns a workgroup in place of 32 when the chip is full
-// anyway took 181 us in place of 149 (four of 700 rows). The digits cost 4 to 12 % of the time.
+// anyway took 181 us in place of 149 (four of 700 rows). The digits cost 4 to 12 % of the time, the look for
+// odd numbers 2 %.
+//
+// A row that is no number (infinite, NaN) reaches the rows behind it and no row before it, as in the walk; the carry goes through
+// a request and head that has one without asking for operands ahead.
 #include "common.h"
 #include "recurrence_chunks.h"
+#include <type_traits>
 
 #define RC_C 32                       // rows of a chunk: two tiles of 16
 #define RC_TINY 1e-20f
+#define RC_LARGE 1e15f
 #define RC_SCRATCH (48ll << 20)       // floats of scratch after which a step's chunks are cut into runs (192 MiB)
 #define RC_GROUP 64                   // requests of one launch at most
 
@@ -65,10 +71,55 @@ __device__ __forceinline__ RcSums rc_mul4(rc_f4 a, rc_f4 b, RcSums c) {
     return c;
 }
 __device__ __forceinline__ rc_f4 rc_sum4(const RcSums& c) { return (c.s[0] + c.s[1]) + (c.s[2] + c.s[3]); }
+// A and T have zeros behind the diagonal, and a product takes them times what stands in later rows: times an infinity or NaN
+// that gives NaN in rows before it, which do not know of it. So where a lane of the wave holds such a number (rc_odd; or one so
+// large that a sum of it may become one), the product with a diagonal tile is formed another way, and the carry goes through
+// such a request and head with code of its own.
+__device__ __forceinline__ bool rc_odd(rc_f4 x) {
+    return __ballot(!(fabsf(x[0]) + fabsf(x[1]) + (fabsf(x[2]) + fabsf(x[3])) < 1e30f)) != 0ull;
+}
+// c and the product of two tiles over the rows j <= i alone, one by one (ROWS: i is the result's row, else its column)
+template <bool ROWS>
+__device__ __forceinline__ rc_f4 rc_lower(rc_f4 a, rc_f4 b, rc_f4 c) {
+    const int lane = threadIdx.x & 63, m16 = lane & 15, g4 = (lane >> 4) * 4;
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {
+        const int from = 16 * (j >> 2);
+        const float y = __shfl(b[j & 3], from + m16, 64);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const float x = __shfl(a[j & 3], from + g4 + r, 64);
+            if (j <= (ROWS ? g4 + r : m16)) c[r] = fmaf(x, y, c[r]);
+        }
+    }
+    return c;
+}
+// The same on the matrix instructions, for a tile u whose columns are the result's: takes what is no number out of u and gives
+// what the result lacks then, NaN for the rows from there on, zero for those before.
+__device__ __forceinline__ rc_f4 rc_spoilt(rc_f4& u) {
+    const int lane = threadIdx.x & 63;
+    rc_f4 e;
+    float run = 0.f;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const bool odd = !(fabsf(u[r]) < INFINITY);
+        run += odd ? NAN : 0.f;
+        e[r] = run;
+        u[r] = odd ? 0.f : u[r];
+    }
+    float before = 0.f;
+#pragma unroll
+    for (int g = 1; g < 4; ++g) {
+        const float x = __shfl_up(run, 16 * g, 64);
+        before += lane >= 16 * g ? x : 0.f;
+    }
+    return e + before;
+}
 
-// Floats per (chunk, head): W and q P [2][DT], k P_C / P [DT][2], U [VT][2], A [3] tiles of 256, P_C [16 DT]
+// Floats per (chunk, head): W and q P [2][DT], k P_C / P [DT][2], U [VT][2], A [3] tiles of 256, P_C [16 DT], a word that says
+// whether an odd number (rc_odd) is among them, and three to keep the next one's tiles at 16 bytes
 __host__ __device__ static inline long long rc_stride(int DT, int VT, bool delta) {
-    return (long long)((delta ? 6 : 4) * DT + 2 * VT + 3) * 256 + 16 * DT;
+    return (long long)((delta ? 6 : 4) * DT + 2 * VT + 3) * 256 + 16 * DT + 4;
 }
 
 // Numbers of a row (one or two a row and head) are formed in 64 bits: an error in them is in all of the row's elements alike.
@@ -201,6 +252,8 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
     float* oU = oK + 2 * DT * 256;
     float* oA = oU + 2 * VT * 256;
     float* oP = oA + 3 * 256;
+    int* odd = (int*)(oP + DP);
+    if (tid == 0) *odd = 0;                                  // (waves that find one set it behind barriers)
 
     const double neg_a = rule == 1 ? -(double)rate : -exp((double)A_log[h]);
     const float neg_a32 = (float)neg_a;
@@ -283,20 +336,22 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
     RcPair pp[16];
     if (chan) {
         RcPair p = {1.f, 0.f};
+        float top = 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
             const int at = (hf * 16 + i) * LD + d;
             aq[i] = qs[at];
             ak[i] = ks[at];
             aa[i] = as[at];
+            top = fmaxf(top, fabsf(ak[i]));
             p = rc_times(p, rc_decay_pair(aa[i]));
             pp[i] = p;
         }
         pt[hf * DP + d] = p.hi;
-        if (!(p.hi >= RC_TINY)) slow[hf] = 1;
+        if (!(p.hi >= RC_TINY) || !(top <= RC_LARGE)) slow[hf] = 1;
     }
     __syncthreads();
-    // (a half whose decays go below RC_TINY: pairs one by one, 16 lanes to a column j, their channels' products carried
+    // (a half whose decays go below RC_TINY or whose keys go beyond RC_LARGE: pairs one by one, 16 lanes to a column j, their channels' products carried
     // from row to row)
     const int slow0 = slow[0], slow1 = slow[1];
     if (slow0 | slow1) {
@@ -434,7 +489,8 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
         __syncthreads();
         v = 0.f;
 #pragma unroll
-        for (int j = 0; j < 16; ++j) v = fmaf(-Ts[(16 + ti) * 36 + 16 + j], Ms[j * 20 + tc], v);
+        for (int j = 0; j < 16; ++j)
+            if (j <= ti) v = fmaf(-Ts[(16 + ti) * 36 + 16 + j], Ms[j * 20 + tc], v);
         Ts[(16 + ti) * 36 + tc] = v;
         __syncthreads();
         // ---- W^T = (beta k P)^T T^T: rows d, columns i
@@ -451,11 +507,16 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
                 x0[r] = ks[(g4 + r) * LD + 16 * t + m16] * beta_s[g4 + r];
                 x1[r] = ks[(16 + g4 + r) * LD + 16 * t + m16] * p0 * beta_s[16 + g4 + r];
             }
-            const RcSums w0 = rc_mul4(x0, t00, rc_zero());
-            const RcSums w1 = rc_mul4(x1, t11, rc_mul4(x0, t10, rc_zero()));
+            const RcSums s0 = rc_mul4(x0, t00, rc_zero()), s10 = rc_mul4(x0, t10, rc_zero()), s1 = rc_mul4(x1, t11, s10);
             MFMA_SETTLE();
-            *reinterpret_cast<rc_f4*>(oW + (t * 64 + lane) * 4) = rc_sum4(w0);
-            *reinterpret_cast<rc_f4*>(oW + ((DT + t) * 64 + lane) * 4) = rc_sum4(w1);
+            rc_f4 w0 = rc_sum4(s0), w1 = rc_sum4(s1);
+            if (rc_odd(w0) || rc_odd(w1)) {
+                if (lane == 0) *odd = 1;
+                w0 = rc_lower<false>(x0, t00, rc_f4{0.f, 0.f, 0.f, 0.f});
+                w1 = rc_lower<false>(x1, t11, rc_sum4(s10));
+            }
+            *reinterpret_cast<rc_f4*>(oW + (t * 64 + lane) * 4) = w0;
+            *reinterpret_cast<rc_f4*>(oW + ((DT + t) * 64 + lane) * 4) = w1;
         }
         // ---- U = T beta v, 128 columns of v at a time
         for (int vb = 0; vb < V; vb += VW) {
@@ -474,12 +535,17 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
                     x0[r] = vs[(g4 + r) * LV + 16 * n + m16];
                     x1[r] = vs[(16 + g4 + r) * LV + 16 * n + m16];
                 }
-                const RcSums u0 = rc_mul4(t00, x0, rc_zero());
-                const RcSums u1 = rc_mul4(t11, x1, rc_mul4(t10, x0, rc_zero()));
+                const RcSums s0 = rc_mul4(t00, x0, rc_zero()), s10 = rc_mul4(t10, x0, rc_zero()), s1 = rc_mul4(t11, x1, s10);
                 MFMA_SETTLE();
+                rc_f4 u0 = rc_sum4(s0), u1 = rc_sum4(s1);
+                if (rc_odd(u0) || rc_odd(u1)) {
+                    if (lane == 0) *odd = 1;
+                    u0 = rc_lower<true>(t00, x0, rc_f4{0.f, 0.f, 0.f, 0.f});
+                    u1 = rc_lower<true>(t11, x1, rc_sum4(s10));
+                }
                 float* to = oU + (long long)(vb / 16 + n) * 512 + lane * 4;
-                *reinterpret_cast<rc_f4*>(to) = rc_sum4(u0);
-                *reinterpret_cast<rc_f4*>(to + 256) = rc_sum4(u1);
+                *reinterpret_cast<rc_f4*>(to) = u0;
+                *reinterpret_cast<rc_f4*>(to + 256) = u1;
             }
         }
         return;
@@ -502,6 +568,7 @@ __global__ __launch_bounds__(256, 2) void recur_prepare_kernel(
                 x0[r] = vs[(g4 + r) * LV + 16 * n + m16];
                 x1[r] = vs[(16 + g4 + r) * LV + 16 * n + m16];
             }
+            if ((rc_odd(x0) || rc_odd(x1)) && lane == 0) *odd = 1;
             float* to = oU + (long long)(vb / 16 + n) * 512 + lane * 4;
             *reinterpret_cast<rc_f4*>(to) = x0;
             *reinterpret_cast<rc_f4*>(to + 256) = x1;
@@ -599,7 +666,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DELTA ? 1 :
         x.a[1] = *reinterpret_cast<const rc_f4*>(a + (2 * 64 + lane) * 4);
     };
 
-    auto go = [&](const Chunk& x, int ci, int buf) {
+    auto go = [&](const Chunk& x, int ci, int buf, auto odd_c) {
         // (two sums each, as of S below: half the chain of roundings. W S first: the next chunk's state waits for it, q P S
         // only for the read-out. The reads of these results sit in the same basic block, where the compiler keeps the
         // distance by itself.)
@@ -663,7 +730,11 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DELTA ? 1 :
         if constexpr (DELTA) move_on();
         if (on < NV) {
             rc_f4 o = sum_waves(oi, on);
-            const rc_f4 u0 = on ? u[NV - 1][0] : u[0][0], u1 = on ? u[NV - 1][1] : u[0][1];
+            rc_f4 u0 = on ? u[NV - 1][0] : u[0][0], u1 = on ? u[NV - 1][1] : u[0][1];
+            if constexpr (decltype(odd_c)::value) {          // (what meets A's diagonal tile)
+                if (oi) o += rc_spoilt(u1);
+                else o += rc_spoilt(u0);
+            }
             constexpr int SUMS = DELTA || NV == 1 || DT < 8 ? 4 : 2;      // (what the registers of two workgroups a CU hold)
             rc_f4 au[SUMS];
 #pragma unroll
@@ -692,23 +763,36 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DELTA ? 1 :
 
     // (a chunk's operands are asked for while the one before it is worked on; the last chunk has code of its own, because
     // behind a branch around the loads the compiler waits for those of the next chunk too)
-    Chunk x, y;
-    load(x, at);
-    for (int c = 0;; c += 2) {
-        if (c + 1 >= n_chunks) {
-            go(x, c, 0);
-            break;
+    constexpr std::integral_constant<bool, false> plain{};
+    constexpr std::integral_constant<bool, true> odd{};
+    int any_odd = 0;
+    for (int c = lane; c < n_chunks; c += 64)
+        any_odd |= reinterpret_cast<const int*>(at + (long long)c * stride)[rc_stride(DT, VT, DELTA) - 4];
+    if (__ballot(any_odd != 0)) {                            // (the same in every wave)
+        Chunk z;
+        for (int c = 0; c < n_chunks; ++c) {
+            load(z, at + (long long)c * stride);
+            go(z, c, c & 1, odd);
         }
-        load(y, at + (long long)(c + 1) * stride);
-        __builtin_amdgcn_sched_barrier(0);
-        go(x, c, 0);
-        if (c + 2 >= n_chunks) {
-            go(y, c + 1, 1);
-            break;
+    } else {
+        Chunk x, y;
+        load(x, at);
+        for (int c = 0;; c += 2) {
+            if (c + 1 >= n_chunks) {
+                go(x, c, 0, plain);
+                break;
+            }
+            load(y, at + (long long)(c + 1) * stride);
+            __builtin_amdgcn_sched_barrier(0);
+            go(x, c, 0, plain);
+            if (c + 2 >= n_chunks) {
+                go(y, c + 1, 1, plain);
+                break;
+            }
+            load(x, at + (long long)(c + 2) * stride);
+            __builtin_amdgcn_sched_barrier(0);
+            go(y, c + 1, 1, plain);
         }
-        load(x, at + (long long)(c + 2) * stride);
-        __builtin_amdgcn_sched_barrier(0);
-        go(y, c + 1, 1);
     }
 #pragma unroll
     for (int nv = 0; nv < NV; ++nv)

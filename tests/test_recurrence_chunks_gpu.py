@@ -169,3 +169,40 @@ def test_no_further_from_64_bits_than_the_walk(ops, rule, H, G, D, V, q_lens):
             for i in (0, 1):
                 far[chunks][i] += float((got[i].double() - want[i]).norm() / want[i].norm()) / 3
     assert far[True][0] <= 1.02 * far[False][0] and far[True][1] <= 1.02 * far[False][1], far
+
+
+def strange(x, what, rule, row, value, H, G, D, V):
+    """The inputs with one number of one row replaced."""
+    x = dict(x)
+    name, column = {"q": ("qkv", 7), "k": ("qkv", G * D + 7), "v": ("qkv", 2 * G * D + 3), "decay": ("a", 7 if rule in ("channel", "outer") else 1),
+                    "beta": ("b", 1)}[what]
+    x[name] = x[name].clone()
+    x[name][row, column] = value
+    return x
+
+
+@pytest.mark.parametrize("rule", RULES)
+@pytest.mark.parametrize("what", ["q", "k", "v", "decay", "beta"])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), 1e30], ids=str)
+def test_rows_before_one_that_is_no_number(ops, rule, what, value):
+    """An infinity, NaN or very large number in one row: what the walk gives as a number is one by chunks too, rows before it
+    and the other request among it (there the same: 32-bit sums of at most 90 rows of a unit's size in another order); what the
+    walk does not, neither do the chunks."""
+    H = G = 2
+    q_lens = [90, 40]
+    for D, V in ((64, 32), (128, 40)):
+        base = drawn(rule, q_lens, H, G, D, V, 5)
+        for row in (0, 3, 15, 16, 30, 31, 33, 50, 89):
+            x = strange(base, what, rule, row, value, H, G, D, V)
+            start = rnd(2, H, V, D, seed=8, scale=0.3)
+            both = []
+            for chunks in (True, False):
+                state = start.clone()
+                both.append((recur(ops, rule, x, state, q_lens, H, G, D, V, chunks), state))
+            for got, want in zip(*both):
+                assert torch.equal(want.isfinite(), got.isfinite()), row
+            (o, state), (o_walk, state_walk) = both
+            clear = torch.tensor([i < row or i >= q_lens[0] for i in range(sum(q_lens))], device=DEV)
+            assert bool(o[clear].isfinite().all()), row
+            torch.testing.assert_close(o[clear], o_walk[clear], atol=1e-4, rtol=1e-4)
+            torch.testing.assert_close(state[1], state_walk[1], atol=1e-4, rtol=1e-4)
