@@ -53,7 +53,7 @@
 #define RC_C 32                       // rows of a chunk: two tiles of 16
 #define RC_TINY 1e-20f
 #define RC_LARGE 1e15f
-#define RC_SCRATCH (48ll << 20)       // floats of scratch after which a step's chunks are cut into runs (192 MiB)
+#define RC_SCRATCH (48ll << 20)       // floats of scratch beyond which a step is cut into groups of requests and runs of chunks (192 MiB)
 #define RC_GROUP 64                   // requests of one launch at most
 
 typedef float rc_f4 __attribute__((ext_vector_type(4)));
@@ -814,7 +814,13 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(DELTA ? 1 :
 // ---------------------------------------------------------------------------------------------------- host
 static int rc_tiles(int D) { return D <= 64 ? 4 : 8; }
 
-// Chunks of every request that a run takes at once, so that the scratch of a group of requests stays near RC_SCRATCH.
+// Requests that one launch takes at most: as many as have room for a chunk each in RC_SCRATCH (one that has not goes alone).
+static int rc_group(int H, long long stride) {
+    const long long fit = RC_SCRATCH / (stride * H);
+    return fit < 1 ? 1 : fit > RC_GROUP ? RC_GROUP : (int)fit;
+}
+
+// Chunks of every request that a run takes at once, so that the scratch of a group of requests is at most RC_SCRATCH.
 static int rc_run(const int* q_lens, int n, int H, long long stride, int min_rows, int* longest, long long* most) {
     int count = 0, top = 0;
     for (int i = 0; i < n; ++i)
@@ -839,11 +845,12 @@ static int rc_run(const int* q_lens, int n, int H, long long stride, int min_row
 long long recurrence_chunks_workspace(const int* q_lens, int n_seqs, int H, int D, int V, int rule) {
     if (q_lens == nullptr || n_seqs < 1 || H < 1 || D < 1 || D > 128 || V < 1 || V > 4096) return 0;
     const long long stride = rc_stride(rc_tiles(D), (V + 15) / 16, rule == 0 || rule == 3);
+    const int group = rc_group(H, stride);
     long long need = 0;
-    for (int r0 = 0; r0 < n_seqs; r0 += RC_GROUP) {
+    for (int r0 = 0; r0 < n_seqs; r0 += group) {
         int longest;
         long long most;
-        rc_run(q_lens + r0, n_seqs - r0 < RC_GROUP ? n_seqs - r0 : RC_GROUP, H, stride, rc_min_rows(rule), &longest, &most);
+        rc_run(q_lens + r0, n_seqs - r0 < group ? n_seqs - r0 : group, H, stride, rc_min_rows(rule), &longest, &most);
         if (most * H * stride > need) need = most * H * stride;
     }
     return need;
@@ -864,8 +871,9 @@ static int rc_launch(hipStream_t st, const T* qkv, long long ld_qkv, const T* b,
     const size_t per = 16 / sizeof(T);
     const bool vec = D % per == 0 && V % per == 0 && ld_qkv % per == 0 && ((size_t)qkv & 15) == 0 &&
                      (rule >= 2 || (ld_ag % per == 0 && ((size_t)ag & 15) == 0));
-    for (int r0 = 0; r0 < n_seqs; r0 += RC_GROUP) {
-        const int n = n_seqs - r0 < RC_GROUP ? n_seqs - r0 : RC_GROUP;
+    const int group = rc_group(H, stride);
+    for (int r0 = 0; r0 < n_seqs; r0 += group) {
+        const int n = n_seqs - r0 < group ? n_seqs - r0 : group;
         int longest;
         long long most;
         const int run = rc_run(q_lens + r0, n, H, stride, rc_min_rows(rule), &longest, &most);

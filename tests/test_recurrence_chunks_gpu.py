@@ -51,7 +51,8 @@ RULES = ["channel", "head", "outer", "scalar"]
 @pytest.mark.parametrize("H,G,D,V,q_lens,offset", [
     (2, 1, 128, 128, [16, 17, 15, 1, 31], 0), (3, 3, 64, 16, [32, 33, 2, 64], 0), (2, 2, 80, 40, [65, 96, 97], 0),
     (4, 2, 24, 8, [127], 8), (2, 1, 128, 130, [47, 16], 0), (2, 2, 33, 17, [48, 20], 1), (1, 1, 1, 1, [18], 3),
-    (2, 1, 66, 34, [40], 2), (8, 2, 128, 64, [9, 40] * 35, 0), (2, 1, 128, 128, [24, 23, 31, 32], 0), (2, 2, 48, 24, [25, 26], 0)])
+    (2, 1, 66, 34, [40], 2), (8, 2, 128, 64, [9, 40] * 35, 0), (2, 1, 128, 128, [24, 23, 31, 32], 0), (2, 2, 48, 24, [25, 26], 0),
+    (96, 1, 128, 128, [25] * 33, 0)])
 def test_against_the_walk(ops, ref, rule, H, G, D, V, q_lens, offset):
     both(ops, ref, rule, q_lens, H, H if rule == "outer" else G, D, V, offset=offset)
 
