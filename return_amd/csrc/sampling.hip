@@ -359,6 +359,22 @@ static SampleWs sample_ws(char* base, int V) {
 
 __device__ __forceinline__ bool finite(float f) { return fabsf(f) < INFINITY; }
 
+// One pass's maximum, first index that holds it and sum of exp(x - maximum). What is subtracted is never -inf, so that a
+// token of logit -inf weighs nothing, in front of the first other one too (-inf less -inf would be NaN).
+struct RunningTop {
+    float mx = -INFINITY, ref = -3.402823466e38f, se = 0.f;
+    int arg = 0x7fffffff;
+    __device__ __forceinline__ void add(int i, float v) {
+        if (v > mx) {
+            se = se * __expf(mx - v) + 1.0f;              // mx = -inf: se is 0 and stays finite
+            mx = ref = v;
+            arg = i;
+        } else {
+            se += __expf(v - ref);
+        }
+    }
+};
+
 // merges (mx, se, arg) over the lanes of a wave: every lane gets the same
 __device__ __forceinline__ void merge_top(float& mx, float& se, int& arg) {
 #pragma unroll
@@ -426,23 +442,18 @@ __global__ __launch_bounds__(PART_THREADS) void sample_top_kernel(const float* _
     for (int i = part * PART_THREADS + tid; i < HIST; i += gridDim.x * PART_THREADS) ws.hist(row)[i] = 0ull;
     if (part == 0 && tid == 0) ws.state(row).gathered = 0;
     const PartRange r = part_range(V, part, parts);
-    float mx = -INFINITY, se = 0.f, mn = INFINITY;
-    int arg = 0x7fffffff;
+    RunningTop top;
+    float mn = INFINITY;
     for_each_256(logits + (size_t)row * V, V, r, [&](int i, const float (&a)[4], int) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
             if (i + c >= r.end) continue;
-            const float v = a[c];
-            mn = fminf(mn, v);
-            if (v > mx) {
-                se = se * __expf(mx - v) + 1.0f;      // mx = -inf: se is 0 and stays finite
-                mx = v;
-                arg = i + c;
-            } else {
-                se += __expf(v - mx);
-            }
+            mn = fminf(mn, a[c]);
+            top.add(i + c, a[c]);
         }
     });
+    float mx = top.mx, se = top.se;
+    int arg = top.arg;
     merge_top(mx, se, arg);
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) mn = fminf(mn, __shfl_xor(mn, o, 64));
@@ -791,29 +802,11 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         total_e = t.se;
     } else {
         // ---- one pass: running maximum, first index that holds it, sum of exp(x - maximum)
-        float mx = -INFINITY, se = 0.f;
-        int arg = 0x7fffffff;
-        for_each_logit(x, V, tid, [&](int i, float v) {
-            if (v > mx) {
-                se = se * __expf(mx - v) + 1.0f;          // mx = -inf: se is 0 and stays finite
-                mx = v;
-                arg = i;
-            } else {
-                se += __expf(v - mx);
-            }
-        });
-        // merge (mx, se, arg) over the wave, then over the waves in wave order
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float m2 = __shfl_xor(mx, o, 64), s2 = __shfl_xor(se, o, 64);
-            const int a2 = __shfl_xor(arg, o, 64);
-            const float m = fmaxf(mx, m2);
-            const float s1 = (mx == -INFINITY) ? 0.f : se * __expf(mx - m);
-            const float s3 = (m2 == -INFINITY) ? 0.f : s2 * __expf(m2 - m);
-            arg = (m2 > mx) ? a2 : ((m2 == mx) ? min(arg, a2) : arg);
-            se = s1 + s3;                                 // the same two numbers in both lanes of a pair
-            mx = m;
-        }
+        RunningTop top;
+        for_each_logit(x, V, tid, [&](int i, float v) { top.add(i, v); });
+        float mx = top.mx, se = top.se;
+        int arg = top.arg;
+        merge_top(mx, se, arg);                           // over the wave; then over the waves in wave order
         __shared__ float wm[16], ws[16];
         __shared__ int wa[16];
         if ((tid & 63) == 0) { wm[tid >> 6] = mx; ws[tid >> 6] = se; wa[tid >> 6] = arg; }

@@ -97,3 +97,45 @@ def test_captured_and_replayed(ops):
         graph.replay()
         torch.cuda.synchronize()
         assert torch.equal(out, ops.sample(x, t, k, p, u)), f"replay {it}"
+
+
+@pytest.mark.parametrize("V,M", [(63, 7), (4096, 7), (20001, 7), (98304, 7), (151936, 7), (151936, 40)])
+def test_log_probabilities_of_masked_rows(ops, V, M):
+    """Tokens of logit -inf weigh nothing, wherever they stand: the log-probability is log_softmax's. A sum of V numbers in
+    32 bits, chains of V / 1024 and a tree: (V / 1024 + 16) 2^-24, and a rounding of the logit and of the logarithm."""
+    g = torch.Generator().manual_seed(V)
+    x = 4 * torch.randn(M, V, generator=g)
+    low = float("-inf")
+    for r in range(M):
+        kind = r % 7
+        if kind == 0:
+            x[r, torch.rand(V, generator=g) < 0.9] = low
+        elif kind == 1:
+            x[r, :V // 2] = low
+        elif kind == 2:
+            x[r, V // 2:] = low
+        elif kind == 3:
+            x[r, :V - 1] = low
+        elif kind == 4:
+            x[r, 1:] = low
+        elif kind == 5:
+            x[r, : V // 2] = torch.finfo(torch.float32).min
+        # (kind 6: nothing masked)
+    rows = x.to(DEV)
+    want = torch.log_softmax(x.double(), -1)
+    u = torch.rand(M, generator=g).to(DEV)
+    for temperature, top_k, top_p in ((0.0, 0, 1.0), (0.8, 0, 1.0), (0.8, 0, 0.9), (0.8, 40, 0.9), (1.0, 3000, 1.0)):
+        t = torch.full((M,), temperature, device=DEV)
+        k = torch.full((M,), top_k, dtype=torch.int32, device=DEV)
+        p = torch.full((M,), top_p, device=DEV)
+        path = torch.zeros(M, dtype=torch.int32, device=DEV)
+        one = torch.empty(M, 2, dtype=torch.int32, device=DEV)
+        got = ops.sample(rows, t, k, p, u)
+        ops._check(ops.lib.ra_sample_traced(_ptr(rows), M, V, _ptr(t), _ptr(k), _ptr(p), _ptr(u), _ptr(one), _ptr(path), None, 0,
+                                            ops._stream()), "sample")
+        for out in (got, one):
+            tokens, logs = out[:, 0].cpu(), out[:, 1].contiguous().view(torch.float32).cpu().double()
+            chosen = want[torch.arange(M), tokens]
+            assert bool(chosen.isfinite().all()), tokens
+            bound = (V / 1024 + 16) * 2.0 ** -24 + 2.0 ** -23 * (chosen.abs() + x.double().clamp(min=-100).abs().max())
+            assert bool(((logs - chosen).abs() <= bound).all()), (logs, chosen)
