@@ -19,8 +19,10 @@
 // thresholds lie among them (k is at most their number; their mass is more than top_p of the whole),
 // the thresholds are searched and the token is drawn from the list alone, which takes microseconds.
 // Otherwise (a flat row, a large k, top_p near 1) the searches go over the whole row, in two passes as a rule.
-// Which way a row goes depends on that row alone.
-// One block a row is bound by its chain of barriers and short sums (a peaked row of 16,384: 20 us, 6 of them for the
+// Which way a row goes and which token it draws depends on that row alone, and not on the rows beside it: what decides either
+// is a sum of whole numbers, or a sum in an order of its own. (The log-probability's sum of exponentials is formed in the order
+// of the kernels that serve so many rows: its last bits depend on their number.)
+// One block a row is bound by its chain of barriers and short sums (a peaked row of 16,384: 21 us, 6 of them for the
 // maximum) and, flat, by one CU's arithmetic (32,000: 41 us; before the searches of two passes 54, and peaked 32).
 #include "common.h"
 
@@ -79,6 +81,11 @@ __device__ __forceinline__ fixed_t to_fixed(float w) {          // 0 <= w <= 1
     const float hi = floorf(t);
     return ((fixed_t)(uint32_t)hi << 32) + (fixed_t)(uint32_t)((t - hi) * 4294967296.0f);
 }
+
+// What weighs less than e^-CAND_SPAN of the largest token, as a multiple of 2^-50 (sixteen of them fit 32 bits; and a sum of
+// such in the unit above).
+__device__ __forceinline__ uint32_t to_fixed_rest(float w) { return (uint32_t)(w * 1125899906842624.0f); }
+__device__ __forceinline__ fixed_t fixed_of_rest(fixed_t rest) { return rest >> 10; }
 
 // Sum of whole numbers over the block; every thread gets it. wsum: CAND_WAVES words of LDS.
 __device__ __forceinline__ fixed_t block_sum_fixed(fixed_t v, fixed_t* wsum) {
@@ -330,7 +337,7 @@ __device__ __forceinline__ float wave_running_sum(float v, int lane) {
 #define PART_THREADS 256
 #define MAX_PARTS 64
 
-struct RowPart { float mx, se, mn; int arg, count; float rest; fixed_t mass; };
+struct RowPart { float mx, se, mn; int arg, count; fixed_t rest, mass; };
 struct RowState { uint32_t keep_key; int tie_limit, status, gathered; };
 enum { ROW_OPEN = 0, ROW_SETTLED = 1 };
 struct RowTop { float mx, se, mn; int arg; };
@@ -503,10 +510,10 @@ __global__ __launch_bounds__(PART_THREADS) void sample_span_kernel(
     for (int i = tid; i < HIST; i += PART_THREADS) h[i] = 0ull;
     __syncthreads();
     int count = 0;
-    float rest = 0.f;
-    fixed_t mass = 0ull;
+    fixed_t mass = 0ull, rest = 0ull;
     const PartRange r = part_range(V, part, parts);
     for_each_256(logits + (size_t)row * V, V, r, [&](int i, const float (&a)[4], int b) {
+        uint32_t rest4 = 0u;
         fixed_t mark = 0ull;
 #pragma unroll
         for (int c = 0; c < 4; ++c) {
@@ -522,9 +529,10 @@ __global__ __launch_bounds__(PART_THREADS) void sample_span_kernel(
                     atomicAdd(&h[at], f);
                     mass += in ? f : 0ull;
                 }
-                rest += in ? 0.f : weight;
+                rest4 += in ? 0u : to_fixed_rest(weight);
             }
         }
+        rest += rest4;
         if (lane < 4) ws.marks(row)[4 * (size_t)b + lane] = mark;
     });
 #pragma unroll
@@ -533,8 +541,7 @@ __global__ __launch_bounds__(PART_THREADS) void sample_span_kernel(
         mass += __shfl_xor(mass, o, 64);
     }
     __shared__ int wc[PART_THREADS / 64];
-    __shared__ float wr[PART_THREADS / 64];
-    __shared__ fixed_t wm[PART_THREADS / 64];
+    __shared__ fixed_t wr[PART_THREADS / 64], wm[PART_THREADS / 64];
     if (lane == 0) { wc[tid >> 6] = count; wr[tid >> 6] = rest; wm[tid >> 6] = mass; }
     __syncthreads();
     if (masses)
@@ -556,13 +563,13 @@ __device__ __forceinline__ bool row_is_flat(const RowPart* all, int parts, float
         for (int j = 0; j < parts; ++j) count += all[lane * parts + j].count;
     if (__ballot(count > CAND_PER_WAVE)) return true;
     fixed_t mass = lane < CAND_WAVES * parts ? all[lane].mass : 0ull;
-    float rest = lane < CAND_WAVES * parts ? all[lane].rest : 0.f;
+    fixed_t rest = lane < CAND_WAVES * parts ? all[lane].rest : 0ull;
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) {
         mass += __shfl_xor(mass, o, 64);
         rest += __shfl_xor(rest, o, 64);
     }
-    const fixed_t z = mass + (fixed_t)((double)rest * (double)FIXED_ONE_F);
+    const fixed_t z = mass + fixed_of_rest(rest);
     return mass <= (fixed_t)((double)top_p * (double)z);
 }
 
@@ -888,7 +895,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
         __syncthreads();
         {
             int have = 0;
-            float rest = 0.f;
+            fixed_t rest = 0ull;
             [[maybe_unused]] bool marked = false;
             if constexpr (PREPARED) marked = finite(gmax);
             if (marked) {
@@ -902,6 +909,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                     float v[4][4];
 #pragma unroll
                     for (int j = 0; j < 4; ++j) load4(i0 + 256 * j, v[j]);
+                    uint32_t rest16 = 0u;
 #pragma unroll
                     for (int j = 0; j < 4; ++j) {
                         int before = 0, all = 0;
@@ -929,16 +937,17 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                         }
                         if (sum_rest) {
 #pragma unroll
-                            for (int c = 0; c < 4; ++c) rest += in[c] ? 0.f : __expf((v[j][c] - gmax) * inv_t);
+                            for (int c = 0; c < 4; ++c) rest16 += in[c] ? 0u : to_fixed_rest(__expf((v[j][c] - gmax) * inv_t));
                         }
                     }
+                    rest += rest16;
                 }
             }
             if (lane == 0) {
                 cnt[wave] = min(have, CAND_PER_WAVE);
                 if (have > CAND_PER_WAVE) sh_over = 1;
             }
-            const float z_rest = sum_rest ? block_sum(rest, scratch) : 0.f;     // (with barriers of its own, or:)
+            const fixed_t z_rest = sum_rest ? block_sum_fixed(rest, wsum) : 0ull;       // (with barriers of its own, or:)
             __syncthreads();
             int total = 0;
             for (int w = 0; w < CAND_WAVES; ++w) total += cnt[w];
@@ -1013,7 +1022,7 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
                         run_of, weighed,
                         [&](fixed_t sum) {
                             zc = sum;
-                            const fixed_t z = sum + (fixed_t)((double)z_rest * (double)FIXED_ONE_F);
+                            const fixed_t z = sum + fixed_of_rest(z_rest);
                             return (fixed_t)((double)p * (double)z);
                         },
                         tid, fx, wsum, &few, keep_key, limit, above, at);
@@ -1304,10 +1313,10 @@ __global__ __launch_bounds__(SAMPLE_THREADS) void sample_kernel(
 // How many pieces a wave's run of the row is cut into for the kernels over several blocks a row; 0: one block a row.
 // The line, one block a row / several blocks, microseconds a call, logits near normal at T 0.7, greedy | top-p 0.9 with
 // 300 large logits | top-p 0.9, flat:
-//   vocabulary  65,536   1 row  10.3 / 13.1 | 29 / 32 |  60 / 37      32 rows 11.0 / 16.3 | 30 / 37 |  62 / 47
+//   vocabulary  65,536   1 row  10.5 / 13.1 | 30 / 32 |  56 / 37      32 rows 11.0 / 16.3 | 31 / 37 |  59 / 47
 //              128,256   1      16.4 / 13.8 | 41 / 33 |  99 / 42      32      16.9 / 18.0 | 41 / 41 | 101 / 62
 //              151,936   1      18.0 / 14.0 | 45 / 34 | 111 / 45      32      18.7 / 18.9 | 45 / 44 | 116 / 67
-//              151,936  64      20.5 / 23.6 | 52 / 54 | 123 / 84
+//              151,936  64      19.7 / 23.6 | 53 / 54 | 123 / 84
 // so that from about 100,000 tokens and up to 32 rows no kind of row loses; beyond SAMPLE_BLOCKS 256s a run the masses
 // have no room.
 static int sample_parts(int M, int V) {

@@ -139,3 +139,26 @@ def test_log_probabilities_of_masked_rows(ops, V, M):
             assert bool(chosen.isfinite().all()), tokens
             bound = (V / 1024 + 16) * 2.0 ** -24 + 2.0 ** -23 * (chosen.abs() + x.double().clamp(min=-100).abs().max())
             assert bool(((logs - chosen).abs() <= bound).all()), (logs, chosen)
+
+
+def test_a_row_draws_the_same_whatever_stands_beside_it(ops):
+    """Rows whose top-p boundary lies within a few roundings of a tie: K tokens of one value and a tail beyond the list, top-p
+    within a rounding of m / (K + tail), so that whether m or m + 1 of them stay hangs on the tail's sum. Every number of rows
+    (four, two, one workgroup a wave's run, and one block) keeps the same."""
+    V, R = 151936, 96
+    g = torch.Generator().manual_seed(7)
+    x = (-16.01 - 0.002 * torch.arange(R))[:, None].repeat(1, V)
+    m = 1.0 + torch.arange(R) % 3
+    for r in range(R):
+        x[r, torch.randperm(V, generator=g)[:2 + r % 3]] = 0.0       # (one more than m)
+    p = (m.double() / torch.exp(x.double()).sum(-1)).float()
+    assert bool((p < 1).all())
+    x, p = x.to(DEV), p.to(DEV)
+    t, k, u = torch.ones(R, device=DEV), torch.zeros(R, dtype=torch.int32, device=DEV), torch.full((R,), 0.999999, device=DEV)
+
+    def draw(M):
+        return [tok for i in range(0, R, M)
+                for tok in ops.sample(x[i:i + M].contiguous(), t[i:i + M], k[i:i + M], p[i:i + M].contiguous(), u[i:i + M])[:, 0].tolist()]
+    want = draw(1)
+    for M in (8, 12, 24, 32, 48):
+        assert draw(M) == want, M
