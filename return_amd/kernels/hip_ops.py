@@ -1509,9 +1509,9 @@ class HipOps:
             return (rows,) if rows == 64 else (rows, 64)
         return None
 
-    def _side_by_side(self, step, window):
-        """Whether a mixed step's two attention kernels go to two streams: from 512 Ki keys of decoded tokens on. A fork and
-        a join cost the host 30 us a layer and the device gaps as long, and the other kernel's workgroups disturb the
+    def _side_by_side(self, step, window, keep_first=0):
+        """Whether a mixed step's two attention kernels go to two streams: from 512 Ki keys on that its decoded tokens read
+        between them (counted once a step). A fork and a join cost the host 30 us a layer and the device gaps as long, and the other kernel's workgroups disturb the
         prefill kernel's order over the XCDs. Measured, a layer's attention between two products, microseconds, side
         by side / one after the other: heads 32 over 8 of 128, portions of 2,048 rows after 2,048: 8 requests of 1,024
         417 / 328, 64 of 4,096 519 / 502, 16 of 32,768 696 / 730, 128 of 16,384 1,748 / 1,798; portions of 512 after 16,384:
@@ -1519,8 +1519,13 @@ class HipOps:
         whole mixed step of the 4B shape (24 requests of about 450 tokens, a portion of 512) 11.0 / 8.7 ms."""
         if self.overlap_attention is not None:
             return self.overlap_attention
-        keys = min(step.max_decode_seq_len, window) if window > 0 else step.max_decode_seq_len
-        return step.n_decode * keys >= 1 << 19
+        if step.n_decode * step.max_decode_seq_len < 1 << 19:
+            return False
+        counted = step.__dict__.setdefault("keys_read_by_decoding", {})
+        if (window, keep_first) not in counted:
+            most = window + keep_first if window > 0 else step.max_decode_seq_len
+            counted[window, keep_first] = sum(min(start + 1, most) for q, start in zip(step.q_lens, step.q_starts) if q == 1)
+        return counted[window, keep_first] >= 1 << 19
 
     def attention(self, q, out, k_pool, v_pool, step, group, scale, window=0, head_scale=None, softcap=0.0,
                   keep_first=0, sink=False, sink_logit=None, out_scale=1.0, fine_weights=False):
@@ -1620,7 +1625,7 @@ class HipOps:
             # out, one is bound by memory and the other by the matrix cores and the latency inside its waves,
             # so where the decoding is long they run side by side on two streams (never while a graph is being
             # captured: such steps are not captured anyway, and a fork and join inside a graph costs more than it gives).
-            if self._side_by_side(step, window) and not torch.cuda.is_current_stream_capturing():
+            if self._side_by_side(step, window, keep_first) and not torch.cuda.is_current_stream_capturing():
                 main = torch.cuda.current_stream(self.device)
                 if self._side_stream is None:
                     self._side_stream = torch.cuda.Stream(self.device)      # (default priority, like every stream here)
