@@ -503,20 +503,23 @@ extern "C" int ra_moe_tile_rows(int n_pairs, int E, int n_rows, int K, int dtype
 }
 
 // x [rows][K]; w [E][N or 2N][K]; y [n_pairs][N]; the row of pair p in x is p / top_div (top_div = top: the
-// token's row; 1: the pair's own row). max_tiles: the grid's first dimension, at least the number of tiles
+// token's row; 1: the pair's own row). n_pairs: entries of order[]. max_tiles: the grid's first dimension, at least the number of tiles
 // the plan can have (n_pairs / rows + E); workgroups beyond meta[0] leave at once.
 // (act_kind, limit, slope, in_scale: what a gated product makes of its halves, see MoeAct)
 extern "C" int ra_moe_product_act(const void* x, const void* w, void* y, const int* order, const int* tiles,
-                                  const int* meta, int max_tiles, int tile_rows, int N, int K, int top_div, int gated,
+                                  const int* meta, int n_pairs, int max_tiles, int tile_rows, int N, int K, int top_div, int gated,
                                   int act_kind, float limit, float slope, const float* in_scale, int dtype,
                                   void* stream) {
     if (max_tiles <= 0) return RA_OK;
     if (N < 1 || K < 1 || top_div < 1 || act_kind < 0 || act_kind > 1 || (in_scale != nullptr && !gated)) return RA_ERR_ARG;
     const MoeAct act = {act_kind, limit, slope, in_scale};
     hipStream_t st = (hipStream_t)stream;
-    if (dtype == RA_DTYPE_BF16 && tile_rows == MOE_TILE_ROWS)
+    if (dtype == RA_DTYPE_BF16 && tile_rows == MOE_TILE_ROWS) {
+        // (32-bit offsets into an expert's matrix and into x: a caller that has not asked ra_moe_tile_rows is refused here)
+        if (!moe_tile_fits(n_pairs, gated ? 2ll * N : N, K)) return RA_ERR_ARG;
         return moe_tile_launch(st, (const bf16*)x, (const bf16*)w, (bf16*)y, order, tiles, meta, max_tiles, N, K, top_div, gated != 0,
                                act);
+    }
     if (dtype == RA_DTYPE_BF16 && K % 8 == 0 && tile_rows == MT_BM) {
         const int cn = gated ? 64 : 128;
         dim3 grid((N + cn - 1) / cn, max_tiles);
@@ -555,9 +558,9 @@ extern "C" int ra_moe_product_act(const void* x, const void* w, void* y, const i
 }
 
 extern "C" int ra_moe_product(const void* x, const void* w, void* y, const int* order, const int* tiles,
-                              const int* meta, int max_tiles, int tile_rows, int N, int K, int top_div, int gated,
+                              const int* meta, int n_pairs, int max_tiles, int tile_rows, int N, int K, int top_div, int gated,
                               int dtype, void* stream) {
-    return ra_moe_product_act(x, w, y, order, tiles, meta, max_tiles, tile_rows, N, K, top_div, gated, 0, 0.f, 0.f, nullptr, dtype,
+    return ra_moe_product_act(x, w, y, order, tiles, meta, n_pairs, max_tiles, tile_rows, N, K, top_div, gated, 0, 0.f, 0.f, nullptr, dtype,
                               stream);
 }
 

@@ -75,7 +75,7 @@ def _declare(lib):
         "ra_attention_latent_mfma_tile_tokens": [I],
         "ra_outer_rule": [P, L, P, L, P, L, P, F, P, F, P, P, P, P, P, I, I, I, P, P, L, I, I, I, I, P],
         "ra_moe_route_law": [P, L, P, I, I, I, I, I, F, P, P, I, P],
-        "ra_moe_product_act": [P, P, P, P, P, P, I, I, I, I, I, I, I, F, F, P, I, P],
+        "ra_moe_product_act": [P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, I, P],
         "ra_add_rmsnorm": [P, P, P, F, P, P, I, I, I, P],
         "ra_add_scaled_rmsnorm": [P, P, F, P, F, P, P, I, I, I, P],
         "ra_stream_pair_rows": [P, P, F, P, P, L, I, I, P],
@@ -87,7 +87,7 @@ def _declare(lib):
         "ra_moe_route": [P, P, I, I, I, I, I, F, P, P, P],
         "ra_moe_plan": [P, I, I, I, P, P, P, P],
         "ra_moe_tile_rows": [I, I, I, I, I],
-        "ra_moe_product": [P, P, P, P, P, P, I, I, I, I, I, I, I, P],
+        "ra_moe_product": [P, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
         "ra_moe_combine": [P, P, P, I, I, I, I, P],
         "ra_moe_combine_extra": [P, P, P, I, I, I, P, P, I, L, I, P],
         "ra_add_slabs_rmsnorm": [P, P, I, L, P, F, P, P, I, I, I, P],
@@ -2110,12 +2110,12 @@ class HipOps:
         down = up if rows_down == rows_up else plan(rows_down)
         order, tiles, meta, max_tiles, rows = up
         self._check(self.lib.ra_moe_product_act(_ptr(x), _ptr(w_gate_up), _ptr(mid), _ptr(order), _ptr(tiles), _ptr(meta),
-                                                max_tiles, rows, I, H, top, 1, act, float(limit), float(slope),
+                                                n_pairs, max_tiles, rows, I, H, top, 1, act, float(limit), float(slope),
                                                 _ptr(weights) if weigh == "input" else None, code,
                                                 self._stream()), "moe_product (gate-up)")
         order, tiles, meta, max_tiles, rows = down
         self._check(self.lib.ra_moe_product(_ptr(mid), _ptr(w_down), _ptr(y), _ptr(order), _ptr(tiles), _ptr(meta),
-                                            max_tiles, rows, H, I, 1, 0, code, self._stream()), "moe_product (down)")
+                                            n_pairs, max_tiles, rows, H, I, 1, 0, code, self._stream()), "moe_product (down)")
         sums = RowSums(y, top, weights if weigh == "output" else None, extra, extra_logits)
         return self.row_sums(sums) if combine else sums
 
