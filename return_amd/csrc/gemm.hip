@@ -129,7 +129,7 @@ __global__ __launch_bounds__(256) void gemv_f32_kernel(const float* __restrict__
 // together, and asks for the next 256 columns before it multiplies the last ones. A lane's sums are formed in the same order,
 // so the results are the same bits. Bound by the reading of W; microseconds with LDS / without, and rate of W: 4,096 x 12,288
 // at 1 row 46 / 32 (6.2 TB/s), 4 rows 61 / 35, 8 rows 84 / 46; 6,144 x 4,096 at 1 row 27 / 23, 4 rows 33 / 26, 8 rows 41 / 33;
-// 24,576 x 4,096 at 1 row 80 / 72, 4 rows 90 / 76. (512 columns ahead: the same to 8 % slower.)
+// 24,576 x 4,096 at 1 row 80 / 72, 4 rows 90 / 76 (where either is taken: ra_gemm_nt). (512 columns ahead: the same to 8 % slower.)
 template <int MR>
 __global__ __launch_bounds__(256) void gemv_f32_direct_kernel(const float* __restrict__ x, const float* __restrict__ W,
                                                               float* __restrict__ y, int M, int N, int K) {
@@ -204,10 +204,17 @@ extern "C" int ra_gemm_nt(const void* A, const void* W, void* C, int M, int N, i
         const dim3 g16((N + 15) / 16);
         const float *xa = (const float*)A, *wa = (const float*)W;
         float* ya = (float*)C;
-        // x from the cache up to 8 rows; from 5 rows on x is as much to load as W or more, which shows where W is long
-        // (151,936 x 4,096 at 5 rows 465 with LDS, 483 without) and beyond 8 rows wherever there are more workgroups than
-        // CUs (9 rows: 4,096 x 4,096 49 / 32, 6,144 x 4,096 53 / 58, 24,576 x 4,096 151 / 171)
-        if (M <= 4 || (M <= 8 && N < 65536) || N <= 4096) {
+        // x from the cache up to 4 rows; with more, x is as much to load as W or more, and that wins as long as all workgroups
+        // run at once: two a CU up to 8 rows, one beyond (registers), and with 8 rows over long rows of W for some rounds more.
+        // Microseconds with LDS / without, 256 CUs, K 2,560 | 4,096 | 12,288. 5 rows: N 8,192 27 / 22 | 46 / 37 | 95 / 78, 8,208
+        // 28 / 33 | 46 / 47 | 102 / 102, 24,576 60 / 61 | 99 / 94 | 234 / 216, 49,152 100 / 116 | 172 / 175 | 421 / 420. 8 rows:
+        // 8,192 28 / 25 | 48 / 38 | 106 / 89, 8,208 30 / 34 | 48 / 47 | 114 / 110, 24,576 63 / 66 | 103 / 97 | 250 / 244, 49,152
+        // 105 / 121 | 177 / 175 | 428 / 483. 9 rows: 4,096 34 / 26 | 47 / 32 | 107 / 62, 4,112 34 / 46 | 49 / 55 | 110 / 108
+        int dev = 0, cus = 0;
+        if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus <= 0)
+            cus = 256;
+        const long long per_cu = M <= 4 ? 0x7fffffff : M <= 8 ? (K >= 4096 ? 6 : 2) : 1;
+        if ((long long)g16.x <= per_cu * cus) {
             if (M <= 1) hipLaunchKernelGGL(gemv_f32_direct_kernel<1>, g16, block, 0, s, xa, wa, ya, M, N, K);
             else if (M <= 2) hipLaunchKernelGGL(gemv_f32_direct_kernel<2>, g16, block, 0, s, xa, wa, ya, M, N, K);
             else if (M <= 4) hipLaunchKernelGGL(gemv_f32_direct_kernel<4>, g16, block, 0, s, xa, wa, ya, M, N, K);
