@@ -48,6 +48,7 @@
 // a request and head that has one without asking for operands ahead.
 #include "common.h"
 #include "recurrence_chunks.h"
+#include <atomic>
 #include <type_traits>
 
 #define RC_C 32                       // rows of a chunk: two tiles of 16
@@ -864,9 +865,13 @@ static int rc_launch(hipStream_t st, const T* qkv, long long ld_qkv, const T* b,
     const int VT = (V + 15) / 16;
     const long long stride = rc_stride(DT, VT, delta);
     const size_t lds = rc_prepare_lds(DT);
-    if (lds > 64 * 1024 && hipFuncSetAttribute((const void*)recur_prepare_kernel<T, DT>, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                               (int)lds) != hipSuccess)
-        return RA_ERR_LAUNCH;
+    static std::atomic<unsigned long long> allowed{0};          // (devices on which the kernel may have so much LDS)
+    int dev = 0;
+    if (lds > 64 * 1024 && (hipGetDevice(&dev) != hipSuccess || dev > 63 || !(allowed.load() >> dev & 1))) {
+        if (hipFuncSetAttribute((const void*)recur_prepare_kernel<T, DT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
+            return RA_ERR_LAUNCH;
+        if (dev <= 63) allowed |= 1ull << dev;
+    }
     // 16-byte loads: a row's pieces and a head's begin at whole pieces
     const size_t per = 16 / sizeof(T);
     const bool vec = D % per == 0 && V % per == 0 && ld_qkv % per == 0 && ((size_t)qkv & 15) == 0 &&

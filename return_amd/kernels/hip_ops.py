@@ -766,15 +766,26 @@ class HipOps:
             "causal_conv")
         return out
 
-    def _recurrence_scratch(self, step, H, D, V, rule, dtype):
-        """(rows that every request brings, as a host array; scratch; its floats) for the recurrences' kernels by chunks
-        of rows, as the library's entries take them; nothing for a step of single tokens or in 32-bit."""
+    def _recurrence_room(self, step, T, H, D, V, rule, dtype):
+        """Device memory for a recurrence over the step's rows: (tensor that holds it, address of the read-outs, fp32
+        [T, H V]; rows that every request brings, as a host array; address and floats of the scratch of the kernels by chunks
+        of rows) as the library's entries take them. No scratch for a step of single tokens or in 32-bit. One allocation, and
+        what depends on the step alone is formed once a step: the layers of a short prompt wait for the host."""
+        read_outs = -(-T * H * V // 4) * 4                     # (16-byte pieces)
         if step.max_q_len <= 1 or dtype != torch.bfloat16:
-            return None, None, 0
+            room = torch.empty(read_outs, dtype=torch.float32, device=self.device)
+            return room, room.data_ptr(), None, None, 0
         cu = step.cu_q_host
-        rows = (_c_int * step.n_seqs)(*[cu[i + 1] - cu[i] for i in range(step.n_seqs)])
-        floats = self.lib.ra_recurrence_scratch(rows, step.n_seqs, H, D, V, rule)
-        return rows, torch.empty(floats, dtype=torch.float32, device=self.device) if floats > 0 else None, floats
+        known = step.__dict__.get("recurrence_rows")
+        if known is None or known[0] is not cu:
+            known = step.__dict__["recurrence_rows"] = (cu, (_c_int * step.n_seqs)(*[b - a for a, b in zip(cu, cu[1:])]), {})
+        _, rows, needs = known
+        floats = needs.get((H, D, V, rule))
+        if floats is None:
+            floats = needs[H, D, V, rule] = self.lib.ra_recurrence_scratch(rows, step.n_seqs, H, D, V, rule)
+        room = torch.empty(read_outs + floats, dtype=torch.float32, device=self.device)
+        at = room.data_ptr()
+        return room, at, rows, at + 4 * read_outs if floats else None, floats
 
     def delta_rule_fits(self, D, V):
         return bool(self.lib.ra_delta_rule_fits(int(D), int(V)))
@@ -804,12 +815,11 @@ class HipOps:
             raise KernelError("delta_rule: a request's slot lies beyond the state's rows")
         if not self.delta_rule_fits(D, V):
             raise KernelError(f"delta_rule: heads of {D} x {V} are beyond the kernel")
-        o_raw = torch.empty(T, H * V, dtype=torch.float32, device=self.device)
-        rows, scratch, floats = self._recurrence_scratch(step, H, D, V, 0, qkv.dtype)
+        room, o_raw, rows, scratch, floats = self._recurrence_room(step, T, H, D, V, 0, qkv.dtype)
         self._check(self.lib.ra_delta_rule(
             _ptr(qkv), ld_qkv, _ptr(beta), ld_b, _ptr(ag), ld_ag, _ptr(a_log), _ptr(dt_bias), _ptr(norm_w), float(eps),
-            _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), _ptr(o_raw), _ptr(out), step.n_seqs, T,
-            max(1, int(step.max_q_len)), rows, _ptr(scratch), floats, H, G, D, V,
+            _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), o_raw, _ptr(out), step.n_seqs, T,
+            max(1, int(step.max_q_len)), rows, scratch, floats, H, G, D, V,
             _code(qkv.dtype), self._stream()), "delta_rule")
         return out
 
@@ -839,12 +849,11 @@ class HipOps:
             raise KernelError("delta_rule_head: a request's slot lies beyond the state's rows")
         if not self.delta_rule_fits(D, V):
             raise KernelError(f"delta_rule_head: heads of {D} x {V} are beyond the kernel")
-        o_raw = torch.empty(T, H * V, dtype=torch.float32, device=self.device)
-        rows, scratch, floats = self._recurrence_scratch(step, H, D, V, 3, qkv.dtype)
+        room, o_raw, rows, scratch, floats = self._recurrence_room(step, T, H, D, V, 3, qkv.dtype)
         self._check(self.lib.ra_delta_rule_head(
             _ptr(qkv), ld_qkv, _ptr(beta), ld_b, _ptr(a), ld_a, _ptr(gate), ld_g, _ptr(a_log), _ptr(dt_bias), _ptr(norm_w),
-            float(eps), _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), _ptr(o_raw), _ptr(out), step.n_seqs, T,
-            max(1, int(step.max_q_len)), rows, _ptr(scratch), floats, H, G, D, V, _code(qkv.dtype),
+            float(eps), _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), o_raw, _ptr(out), step.n_seqs, T,
+            max(1, int(step.max_q_len)), rows, scratch, floats, H, G, D, V, _code(qkv.dtype),
             self._stream()), "delta_rule_head")
         return out
 
@@ -989,12 +998,11 @@ class HipOps:
             raise KernelError("outer_rule: a request's slot lies beyond the state's rows")
         if not self.delta_rule_fits(D, V) or not float(tau) > 0:
             raise KernelError(f"outer_rule: heads of {D} x {V} (tau {tau}) are beyond the kernel")
-        o_raw = torch.empty(T, H * V, dtype=torch.float32, device=self.device)
-        rows, scratch, floats = self._recurrence_scratch(step, H, D, V, 1, qkv.dtype)
+        room, o_raw, rows, scratch, floats = self._recurrence_room(step, T, H, D, V, 1, qkv.dtype)
         self._check(self.lib.ra_outer_rule(
             _ptr(qkv), ld_qkv, _ptr(a), ld_a, _ptr(gate), ld_g, _ptr(decay_bias), 1.0 / float(tau), _ptr(norm_w), float(eps),
-            _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), _ptr(o_raw), _ptr(out), step.n_seqs, T,
-            max(1, int(step.max_q_len)), rows, _ptr(scratch), floats, H, D, V, _code(qkv.dtype),
+            _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), o_raw, _ptr(out), step.n_seqs, T,
+            max(1, int(step.max_q_len)), rows, scratch, floats, H, D, V, _code(qkv.dtype),
             self._stream()), "outer_rule")
         return out
 
@@ -1025,12 +1033,11 @@ class HipOps:
             raise KernelError("scalar_rule: a request's slot lies beyond the state's rows")
         if not self.delta_rule_fits(D, V):
             raise KernelError(f"scalar_rule: heads of {D} x {V} are beyond the kernel")
-        o_raw = torch.empty(T, H * V, dtype=torch.float32, device=self.device)
-        rows, scratch, floats = self._recurrence_scratch(step, H, D, V, 2, qkv.dtype)
+        room, o_raw, rows, scratch, floats = self._recurrence_room(step, T, H, D, V, 2, qkv.dtype)
         self._check(self.lib.ra_scalar_rule(
             _ptr(qkv), ld_qkv, _ptr(dt), ld_dt, _ptr(gate), ld_g, _ptr(a_log), _ptr(dt_bias), _ptr(skip), _ptr(norm_w),
-            int(norm_groups), float(eps), _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), _ptr(o_raw), _ptr(out),
-            step.n_seqs, T, max(1, int(step.max_q_len)), rows, _ptr(scratch), floats, H, G, D, V,
+            int(norm_groups), float(eps), _ptr(state), _ptr(step.cu_q), _ptr(step.slot_ids), o_raw, _ptr(out),
+            step.n_seqs, T, max(1, int(step.max_q_len)), rows, scratch, floats, H, G, D, V,
             _code(qkv.dtype), self._stream()), "scalar_rule")
         return out
 
