@@ -99,6 +99,7 @@ def _declare(lib):
         "ra_qkv_prepare": [P, I, I, I, I, P, P, F, P, P, P, I, P, P, P, P, I, L, I, P],
         "ra_silu_mul": [P, P, I, I, I, P],
         "ra_gemm_nt": [P, P, P, I, I, I, I, I, P],
+        "ra_gemm_split_f32": [P, P, P, I, I, I, P, L, P],
         "ra_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, P],
         "ra_gemm_skinny_gated_bf16": [P, P, P, I, I, I, P],
         "ra_gemm_mfma_bf16": [P, P, P, I, I, I, I, P],
@@ -142,6 +143,8 @@ def _declare(lib):
         fn.restype = _c_int
     lib.ra_recurrence_scratch.argtypes = [P, I, I, I, I, I]
     lib.ra_recurrence_scratch.restype = _c_ll
+    lib.ra_gemm_split_scratch.argtypes = [I, I, I]
+    lib.ra_gemm_split_scratch.restype = _c_ll
     lib.ra_sample_scratch.argtypes = [I, I]
     lib.ra_sample_scratch.restype = _c_ll
 
@@ -1148,6 +1151,32 @@ class HipOps:
             return "skinny"
         return "two"
 
+    def use_split(self, M, N, K):
+        """Whether a float32 product is formed from the operands' bfloat16 parts (closer to 64 bits than the library's
+        float32 product). Measured on MI355X, microseconds by parts / the library: from 128 rows on it is the faster
+        one where there is work for the chip (128 rows of 4,096 x 12,288 99 / 123, 24,576 x 4,096 172 / 207; 633 rows
+        24,576 x 4,096 654 / 927, 4,096 x 4,096 126 / 167; 200 rows of 2,560 x 9,728 110 / 111), with fewer rows W's reading
+        decides (64 rows of 24,576 x 4,096 126 / 114) and on small products its three launches do (256 rows of 6,144 x
+        2,048 68 / 64, 1,000 rows of 1,024 x 1,024 37 / 22)."""
+        return M >= 128 and K % 32 == 0 and N % 4 == 0 and M * N * K >= 5e9 and not self.own_gemm
+
+    SPLIT_ROWS = 4096             # rows taken apart at a time: their parts are 6 bytes an element
+
+    def _linear_by_parts(self, x, w):
+        M, K = x.shape
+        N = w.shape[0]
+        y = torch.empty(M, N, dtype=torch.float32, device=self.device)
+        step = min(self.SPLIT_ROWS, max(128, (2 ** 31 - 1) // N // 128 * 128))
+        scratch, room = None, 0
+        for a in range(0, M, step):
+            m = min(step, M - a)
+            need = self.lib.ra_gemm_split_scratch(m, N, K)
+            if need > room:
+                scratch, room = torch.empty(need, dtype=torch.uint8, device=self.device), need
+            self._check(self.lib.ra_gemm_split_f32(x.data_ptr() + 4 * a * K, _ptr(w), y.data_ptr() + 4 * a * N, m, N, K,
+                                                   _ptr(scratch), room, self._stream()), "gemm_split")
+        return y
+
     def _linear_by(self, how, x, w, out_dtype):
         M, K = x.shape
         N = w.shape[0]
@@ -1320,6 +1349,9 @@ class HipOps:
         if w.shape[1] != K:
             raise KernelError(f"linear: x {tuple(x.shape)} times weight {tuple(w.shape)}^T")
         out_dtype = out_dtype or x.dtype
+        if x.dtype == torch.float32 and out_dtype == torch.float32 and self.use_split(M, N, K) \
+                and (x.data_ptr() | w.data_ptr()) % 16 == 0:
+            return self._linear_by_parts(x, w)
         if x.dtype == torch.float32 and out_dtype == torch.float32 and M > 16 and self._library_fp32_exact \
                 and not self.own_gemm:
             return torch.matmul(x, w.t())          # the library's float32 product: checked above to be 32-bit
