@@ -110,6 +110,9 @@ def _declare(lib):
         "ra_gemm_sweep_workgroups": [I, I],
         "ra_gemm_sweep_norm_bf16": [P, P, P, I, I, I, I, I, I, P, I, I, F, P, P, P, P],
         "ra_attention_plain": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, I, P, F, I, I, P, F, L, P],
+        "ra_attention_f32_fits": [I],
+        "ra_attention_prefill_f32": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, F, I, P, F, I, I, P, F, L, P],
+        "ra_attention_decode_f32": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, F, I, P, F, I, I, P, F, L, P],
         "ra_causal_conv": [P, L, P, P, P, P, P, L, I, I, I, I, I, I, P],
         "ra_delta_rule": [P, L, P, L, P, L, P, P, P, F, P, P, P, P, P, I, I, I, P, P, L, I, I, I, I, I, P],
         "ra_delta_rule_head": [P, L, P, L, P, L, P, L, P, P, P, F, P, P, P, P, P, I, I, I, P, P, L, I, I, I, I, I, P],
@@ -1546,6 +1549,8 @@ class HipOps:
         if dtype == torch.bfloat16 and D % 16 == 0 and D <= 256:
             rows = int(self.lib.ra_attention_prefill_tile_rows(D))
             return (rows,) if rows == 64 else (rows, 64)
+        if dtype == torch.float32 and self.lib.ra_attention_f32_fits(D):
+            return (64,)
         return None
 
     def _side_by_side(self, step, window, keep_first=0):
@@ -1652,6 +1657,21 @@ class HipOps:
                 split, n_q, n_kv, D, P, float(scale), window, _ptr(head_scale), softcap, keep_first,
                 1 if sink else 0, _ptr(sink_logit), out_scale, ld_out, 1 if fine_weights else 0, self._stream()),
                 "attention_prefill_bf16")
+
+        if q.dtype == torch.float32 and self.lib.ra_attention_f32_fits(D) and q.data_ptr() % 16 == 0 \
+                and (step.n_prefill_tokens == 0 or 64 in step.prefill_tiles) and (step.n_decode > 0 or step.n_prefill_tokens > 0):
+            more = (float(scale), window, _ptr(head_scale), softcap, keep_first, 1 if sink else 0, _ptr(sink_logit), out_scale,
+                    ld_out, self._stream())
+            if step.n_decode > 0:
+                self._check(self.lib.ra_attention_decode_f32(
+                    _ptr(q), _ptr(out), _ptr(k_pool), _ptr(v_pool), *tabs, _ptr(step.decode_segs), step.n_decode, n_q, n_kv, D, P,
+                    *more), "attention_decode_f32")
+            if step.n_prefill_tokens > 0:
+                tiles = step.prefill_tiles[64]
+                self._check(self.lib.ra_attention_prefill_f32(
+                    _ptr(q), _ptr(out), _ptr(k_pool), _ptr(v_pool), *tabs, _ptr(tiles), tiles.shape[0], n_q, n_kv, D, P,
+                    *more), "attention_prefill_f32")
+            return
 
         def plain_part(toks, n_tok):
             self._check(self.lib.ra_attention_plain(
