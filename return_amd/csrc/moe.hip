@@ -517,7 +517,7 @@ extern "C" int ra_moe_product_act(const void* x, const void* w, void* y, const i
     if (dtype == RA_DTYPE_BF16 && tile_rows == MOE_TILE_ROWS) {
         // (32-bit offsets into an expert's matrix and into x: a caller that has not asked ra_moe_tile_rows is refused here)
         if (!moe_tile_fits(n_pairs, gated ? 2ll * N : N, K)) return RA_ERR_ARG;
-        return moe_tile_launch(st, (const bf16*)x, (const bf16*)w, (bf16*)y, order, tiles, meta, max_tiles, N, K, top_div, gated != 0,
+        return moe_tile_launch(st, (const bf16*)x, (const bf16*)w, (bf16*)y, order, tiles, meta, max_tiles, (n_pairs - 1) / top_div + 1, N, K, top_div, gated != 0,
                                act);
     }
     if (dtype == RA_DTYPE_BF16 && K % 8 == 0 && tile_rows == MT_BM) {

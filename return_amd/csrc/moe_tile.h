@@ -28,7 +28,7 @@ static inline bool moe_tile_fits(long long n_pairs, long long n_rows, int K) {
     return K % 32 == 0 && n_pairs * K * 2 < 0x7fffff00ll && n_rows * K * 2 < 0x7fffff00ll;
 }
 int moe_tile_launch(hipStream_t st, const bf16* x, const bf16* w, bf16* y, const int* order, const int* tiles,
-                    const int* meta, int max_tiles, int N, int K, int top_div, bool gated, const MoeAct& act);
+                    const int* meta, int max_tiles, int x_rows, int N, int K, int top_div, bool gated, const MoeAct& act);
 
 // Few rows an expert: tiles of up to 16 rows.
 bool moe_sweep_fits(int K);

@@ -52,7 +52,7 @@ KINDS = ["silu", "clamped", "input"]
 @pytest.mark.parametrize("E,H,I,counts", [
     (4, 32, 32, [8, 9, 31, 33]), (3, 64, 96, [16, 20, 0]), (2, 224, 40, [64, 65]), (5, 256, 160, [128, 129, 144, 145, 0]),
     (3, 96, 300, [160, 192, 193]), (4, 160, 128, [224, 225, 256, 257]), (2, 1024, 224, [272, 700]), (1, 128, 64, [12]),
-    (6, 192, 2, [0, 0, 48, 0, 0, 500])])
+    (6, 192, 2, [0, 0, 48, 0, 0, 500]), (2, 352, 288, [15, 300]), (3, 416, 32, [64, 97, 513])])
 @pytest.mark.parametrize("kind", KINDS)
 def test_products_of_many_rows(ops, E, H, I, counts, kind):
     check(ops, 256, E, H, I, shuffled(counts), kind)
