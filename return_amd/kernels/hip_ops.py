@@ -100,6 +100,8 @@ def _declare(lib):
         "ra_silu_mul": [P, P, I, I, I, P],
         "ra_gemm_nt": [P, P, P, I, I, I, I, I, P],
         "ra_gemm_split_f32": [P, P, P, I, I, I, P, L, P],
+        "ra_gemm_rows_fits": [I, I, I],
+        "ra_gemm_rows_bf16": [P, P, P, I, I, I, I, I, I, I, P],
         "ra_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, P],
         "ra_gemm_skinny_gated_bf16": [P, P, P, I, I, I, P],
         "ra_gemm_mfma_bf16": [P, P, P, I, I, I, I, P],
@@ -253,6 +255,12 @@ class HipOps:
         if 1 <= M <= 8:
             return tiles >= 384
         return M > 8 and tiles >= 2048
+
+    def use_rows(self, M, N, K, gated):
+        """Whether the product of 17 to 64 rows that streams W through LDS is the rule's choice: where every CU has 64 rows of W
+        or more. Measured on MI355X, microseconds at 64 rows by it / by the library: gate-up of the 8B shape 39 / 50 and 5 for
+        the SiLU-mul, head 241 / 273; with fewer rows of W x is most of what a CU takes in (q/k/v 18.5 / 17.6)."""
+        return N * (2 if gated else 1) >= 64 * self.cu_count and bool(self.lib.ra_gemm_rows_fits(M, N, K)) and not self.own_gemm
 
     # ------------------------------------------------------------------ helpers
     def _stream(self):
@@ -1136,6 +1144,8 @@ class HipOps:
             return "sweep"
         if out_dtype in (torch.bfloat16, torch.float32) and self.use_resident(M, N, K, False):
             return "resident512" if M <= 8 else "resident256"
+        if out_dtype in (torch.bfloat16, torch.float32) and self.use_rows(M, N, K, False):
+            return "rows"
         if self.use_skinny(M, N, K, out_dtype):
             return "skinny"
         if not self.own_gemm and (out_dtype == torch.bfloat16 or self._library_fp32_out):
@@ -1146,6 +1156,8 @@ class HipOps:
         hit = self.product_plan.get((self._rows_step(M), I, K, True, torch.bfloat16))
         if hit is not None:
             return hit
+        if self.use_rows(M, I, K, True):
+            return "rows"
         if self.use_sweep(M, I, K, True):
             return "sweep"
         if self.use_resident(M, I, K, True):
@@ -1180,9 +1192,19 @@ class HipOps:
                                                    _ptr(scratch), room, self._stream()), "gemm_split")
         return y
 
+    def _rows_product(self, x, w, out, N, gated, pieces):
+        M, K = x.shape
+        self._check(self.lib.ra_gemm_rows_bf16(_ptr(x), _ptr(w), _ptr(out), M, N, K, 1 if gated else 0, pieces, _code(out.dtype),
+                                               self.cu_count, self._stream()), "gemm_rows")
+        return out
+
     def _linear_by(self, how, x, w, out_dtype):
         M, K = x.shape
         N = w.shape[0]
+        if how == "rows":
+            if (x.data_ptr() | w.data_ptr()) % 16 == 0:
+                return self._rows_product(x, w, torch.empty(M, N, dtype=out_dtype, device=self.device), N, False, 1)
+            how = "library" if out_dtype == torch.bfloat16 or self._library_fp32_out else "mfma"
         if how == "library":
             if out_dtype == torch.bfloat16:
                 return torch.matmul(x, w.t())          # library product, as the reference's F.linear
@@ -1312,10 +1334,13 @@ class HipOps:
         return ScaledRows(xw, psq, w.shape[0], eps)
 
     def _split_product(self, x, w, pieces):
-        """x @ w^T as `pieces` shares [pieces, M, N] fp32, share i from columns i*K/pieces .. of K: one batched
-        library product over strided views of x and w (nothing is copied)."""
+        """x @ w^T as `pieces` shares [pieces, M, N] fp32, share i from columns i*K/pieces .. of K: up to 64 rows by the
+        product that streams W through LDS (down and o of the 8B shape at 64 rows in four pieces 23 and 10.6 us, the library's
+        batch 27 and 13.6), else one batched library product over strided views of x and w (nothing is copied)."""
         M, K = x.shape
         N = w.shape[0]
+        if K % (128 * pieces) == 0 and self.lib.ra_gemm_rows_fits(M, N, K) and (x.data_ptr() | w.data_ptr()) % 16 == 0:
+            return Slabs(self._rows_product(x, w, torch.empty(pieces, M, N, dtype=torch.float32, device=self.device), N, False, pieces))
         xs = x.view(M, pieces, K // pieces).transpose(0, 1)
         wv = w.view(N, pieces, K // pieces).permute(1, 2, 0)
         return Slabs(torch.bmm(xs, wv, out_dtype=torch.float32))
@@ -1366,6 +1391,8 @@ class HipOps:
         M, K = x.shape
         I = w_gate_up.shape[0] // 2
         out = torch.empty(M, I, dtype=x.dtype, device=self.device)
+        if how == "rows" and (x.data_ptr() | w_gate_up.data_ptr()) % 16 == 0:
+            return self._rows_product(x, w_gate_up, out, I, True, 1)
         if how == "sweep":
             self._check(self.lib.ra_gemm_sweep_bf16(_ptr(x), _ptr(w_gate_up), _ptr(out), M, I, K, 1, _code(x.dtype),
                                                     self.cu_count, self._stream()), "gemm_sweep_gated")
@@ -1414,6 +1441,8 @@ class HipOps:
             c += ["resident256", "resident512"]
         if self.lib.ra_gemm_sweep_fits(M, K):
             c.append("sweep")
+        if self.lib.ra_gemm_rows_fits(M, N, K):
+            c.append("rows")
         if residual and self._library_bmm_fp32 and M > 16:
             c += [f"split{n}" for n in self.SPLITS if K % (8 * n) == 0]
         return c

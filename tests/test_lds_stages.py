@@ -105,7 +105,7 @@ def test_the_walk_finds_what_it_is_for():
 
 
 @pytest.mark.skipif(not (shutil.which("hipcc") or os.path.exists("/opt/rocm/bin/hipcc")), reason="no hipcc")
-@pytest.mark.parametrize("source", ["moe_tile.hip", "gemm_tile.hip"])
+@pytest.mark.parametrize("source", ["moe_tile.hip", "gemm_tile.hip", "gemm_rows.hip"])
 def test_no_stage_is_refilled_before_it_is_read(source, tmp_path):
     kernels = {n: b for n, b in _kernels(_compiled(source, tmp_path)).items() if any(" lds" in i for _, c in b for i in c)}
     assert kernels
@@ -116,8 +116,9 @@ def test_no_stage_is_refilled_before_it_is_read(source, tmp_path):
 
 
 @pytest.mark.skipif(not (shutil.which("hipcc") or os.path.exists("/opt/rocm/bin/hipcc")), reason="no hipcc")
-def test_stages_refilled_behind_the_barrier_they_are_read_before(tmp_path):
-    kernels = {n: b for n, b in _kernels(_compiled("moe_tile.hip", tmp_path)).items() if any(" lds" in i for _, c in b for i in c)}
+@pytest.mark.parametrize("source", ["moe_tile.hip", "gemm_rows.hip"])
+def test_stages_refilled_behind_the_barrier_they_are_read_before(source, tmp_path):
+    kernels = {n: b for n, b in _kernels(_compiled(source, tmp_path)).items() if any(" lds" in i for _, c in b for i in c)}
     for name, blocks in kernels.items():
         copies, bad = unfinished_reads(blocks, behind_same=True)
         assert copies > 0 and not bad, (name, bad[:8], len(bad))
