@@ -503,6 +503,35 @@ __global__ __launch_bounds__(256) void delta_out_kernel(const float* __restrict_
     }
 }
 
+// The same for bfloat16 with four neighbours a lane: L lanes to a (row, head) of V = 4 L (V 64, 128 or 256, gate, norm and result
+// in whole pieces of four). Bound by its rows: 2,048 rows of 32 heads of 128 32 -> 15 us.
+template <int L>
+__global__ __launch_bounds__(256) void delta_out_bf16x4_kernel(const float* __restrict__ o_raw, const bf16* __restrict__ gate,
+                                                               long long ld_gate, const float* __restrict__ norm_w, float eps,
+                                                               bf16* __restrict__ out, long long n_rows, int H, int silu_gate) {
+    const long long row = (long long)blockIdx.x * (256 / L) + threadIdx.x / L;
+    if (row >= n_rows) return;                         // (the L lanes of a row together)
+    const int c = (threadIdx.x & (L - 1)) * 4;
+    const long long t = row / H;
+    const int h = (int)(row - t * H);
+    const float4 o = *reinterpret_cast<const float4*>(o_raw + (size_t)row * (4 * L) + c);
+    const uint2 g2 = *reinterpret_cast<const uint2*>(gate + (size_t)t * ld_gate + (size_t)h * (4 * L) + c);
+    const float4 nw = *reinterpret_cast<const float4*>(norm_w + c);
+    float ss = fmaf(o.x, o.x, fmaf(o.y, o.y, fmaf(o.z, o.z, o.w * o.w)));
+#pragma unroll
+    for (int k = L / 2; k > 0; k >>= 1) ss += __shfl_xor(ss, k, 64);
+    const float rstd = 1.0f / sqrtf(ss / (float)(4 * L) + eps);
+    const float g[4] = {__uint_as_float(g2.x << 16), __uint_as_float(g2.x & 0xffff0000u), __uint_as_float(g2.y << 16),
+                        __uint_as_float(g2.y & 0xffff0000u)};
+    float y[4] = {o.x * rstd * nw.x, o.y * rstd * nw.y, o.z * rstd * nw.z, o.w * rstd * nw.w};
+#pragma unroll
+    for (int e = 0; e < 4; ++e) y[e] *= silu_gate ? g[e] * dr_sigmoid(g[e]) : dr_sigmoid(g[e]);
+    uint2 pk;
+    pk.x = (uint32_t)f2bf_bits(y[0]) | ((uint32_t)f2bf_bits(y[1]) << 16);
+    pk.y = (uint32_t)f2bf_bits(y[2]) | ((uint32_t)f2bf_bits(y[3]) << 16);
+    *reinterpret_cast<uint2*>(out + (size_t)row * (4 * L) + c) = pk;
+}
+
 // How a head's state is spread: RS lanes (a power of two) of DPT rows each to a column, VB columns a workgroup.
 static bool delta_rule_plan(int D, int V, int* RS_out, int* DPT_out, int* VB_out) {
     if (D < 1 || V < 1 || D > 512 || V > 4096) return false;
@@ -686,7 +715,15 @@ static int delta_rule_run(const void* qkv, long long ld_qkv, const void* b, long
     if (dtype == RA_DTYPE_F32)
         hipLaunchKernelGGL(delta_out_kernel<float>, ogrid, oblock, 0, st, o_raw, (const float*)gate, ld_gate, norm_w,
                            eps, (float*)out, n_rows, H, V, rule != 0);
-    else
+    else if ((V == 64 || V == 128 || V == 256) && ld_gate % 4 == 0 && (((uintptr_t)gate | (uintptr_t)out) & 7) == 0 &&
+             (((uintptr_t)o_raw | (uintptr_t)norm_w) & 15) == 0) {
+        const dim3 vgrid((unsigned)((n_rows + 1024 / V - 1) / (1024 / V)));
+#define DELTA_OUT(L_)                                                                                                            \
+    hipLaunchKernelGGL(delta_out_bf16x4_kernel<L_>, vgrid, oblock, 0, st, o_raw, (const bf16*)gate, ld_gate, norm_w, eps, (bf16*)out, \
+                       n_rows, H, rule != 0)
+        if (V == 64) DELTA_OUT(16); else if (V == 128) DELTA_OUT(32); else DELTA_OUT(64);
+#undef DELTA_OUT
+    } else
         hipLaunchKernelGGL(delta_out_kernel<bf16>, ogrid, oblock, 0, st, o_raw, (const bf16*)gate, ld_gate, norm_w,
                            eps, (bf16*)out, n_rows, H, V, rule != 0);
     return ra_launch_status();
@@ -775,6 +812,56 @@ __global__ __launch_bounds__(256) void scalar_out_kernel(const float* __restrict
     for (int e = lane; e < L; e += 64) out[(size_t)t * inner + c0 + e] = from_f<T>(value(c0 + e) * rstd * norm_w[c0 + e]);
 }
 
+// The same for bfloat16 with four neighbours a lane (L and V multiples of four, L at most 64 SO_KEEP, rows and addresses in whole
+// pieces of four): 2,000 rows of eight parts of 512 32 -> 16 us.
+__global__ __launch_bounds__(256) void scalar_out_bf16x4_kernel(const float* __restrict__ o_raw, const bf16* __restrict__ v,
+                                                                long long ld_v, const bf16* __restrict__ gate, long long ld_gate,
+                                                                const float* __restrict__ skip, const float* __restrict__ norm_w,
+                                                                float eps, bf16* __restrict__ out, long long n_units, int n_parts,
+                                                                int L, int V) {
+    const long long unit = (long long)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (unit >= n_units) return;
+    const int lane = threadIdx.x & 63;
+    const long long t = unit / n_parts;
+    const int c0 = (int)(unit - t * n_parts) * L;
+    const size_t at = (size_t)t * n_parts * L + c0;
+    float y[SO_KEEP / 4][4];
+    float ss = 0.f;
+#pragma unroll
+    for (int i = 0; i < SO_KEEP / 4; ++i) {
+        const int e = (lane + 64 * i) * 4;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) y[i][k] = 0.f;
+        if (e < L) {
+            const float4 o = *reinterpret_cast<const float4*>(o_raw + at + e);
+            const uint2 z2 = *reinterpret_cast<const uint2*>(gate + (size_t)t * ld_gate + c0 + e);
+            const uint2 v2 = *reinterpret_cast<const uint2*>(v + (size_t)t * ld_v + c0 + e);
+            const float sk = skip[(c0 + e) / V];
+            const float ov[4] = {o.x, o.y, o.z, o.w};
+            const float zv[4] = {__uint_as_float(z2.x << 16), __uint_as_float(z2.x & 0xffff0000u), __uint_as_float(z2.y << 16),
+                                 __uint_as_float(z2.y & 0xffff0000u)};
+            const float vv[4] = {__uint_as_float(v2.x << 16), __uint_as_float(v2.x & 0xffff0000u), __uint_as_float(v2.y << 16),
+                                 __uint_as_float(v2.y & 0xffff0000u)};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                y[i][k] = fmaf(sk, vv[k], ov[k]) * (zv[k] / (1.0f + expf(-zv[k])));
+                ss = fmaf(y[i][k], y[i][k], ss);
+            }
+        }
+    }
+    const float rstd = 1.0f / sqrtf(wave_sum(ss) / (float)L + eps);
+#pragma unroll
+    for (int i = 0; i < SO_KEEP / 4; ++i) {
+        const int e = (lane + 64 * i) * 4;
+        if (e >= L) continue;
+        const float4 nw = *reinterpret_cast<const float4*>(norm_w + c0 + e);
+        uint2 pk;
+        pk.x = (uint32_t)f2bf_bits(y[i][0] * rstd * nw.x) | ((uint32_t)f2bf_bits(y[i][1] * rstd * nw.y) << 16);
+        pk.y = (uint32_t)f2bf_bits(y[i][2] * rstd * nw.z) | ((uint32_t)f2bf_bits(y[i][3] * rstd * nw.w) << 16);
+        *reinterpret_cast<uint2*>(out + at + e) = pk;
+    }
+}
+
 // The scalar rule: qkv rows [q: G D | k: G D | v: H V]; d [T, H] the step before its bias and softplus; gate [T, H V];
 // S fp32 [slots, H, V, D]; out = groupnorm_{n_parts}((o + skip v) silu(gate)) norm_w, norm_w [H V], skip [H].
 extern "C" int ra_scalar_rule(const void* qkv, long long ld_qkv, const void* d, long long ld_d, const void* gate,
@@ -799,6 +886,10 @@ extern "C" int ra_scalar_rule(const void* qkv, long long ld_qkv, const void* d, 
     if (dtype == RA_DTYPE_F32)
         hipLaunchKernelGGL(scalar_out_kernel<float>, ogrid, oblock, 0, st, o_raw, (const float*)v, ld_qkv, (const float*)gate,
                            ld_gate, skip, norm_w, eps, (float*)out, n_units, n_parts, L, V);
+    else if (L % 4 == 0 && V % 4 == 0 && L <= 64 * SO_KEEP && ld_qkv % 4 == 0 && ld_gate % 4 == 0 &&
+             (((uintptr_t)v | (uintptr_t)gate | (uintptr_t)out) & 7) == 0 && (((uintptr_t)o_raw | (uintptr_t)norm_w) & 15) == 0)
+        hipLaunchKernelGGL(scalar_out_bf16x4_kernel, ogrid, oblock, 0, st, o_raw, (const bf16*)v, ld_qkv, (const bf16*)gate, ld_gate,
+                           skip, norm_w, eps, (bf16*)out, n_units, n_parts, L, V);
     else
         hipLaunchKernelGGL(scalar_out_kernel<bf16>, ogrid, oblock, 0, st, o_raw, (const bf16*)v, ld_qkv, (const bf16*)gate,
                            ld_gate, skip, norm_w, eps, (bf16*)out, n_units, n_parts, L, V);

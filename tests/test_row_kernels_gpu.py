@@ -1,0 +1,59 @@
+"""Kernels over rows that take 16-byte pieces where sizes and addresses allow: the same bits as element by element."""
+import pytest
+import torch
+
+from tests.test_kofipel_gpu import DEV, ops, ref, rnd, state_step  # noqa: F401
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+
+
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("C,q_lens", [(8, [8]), (1032, [1, 2, 3, 9]), (1024, [16, 7, 15]), (2056, [37, 1, 33])])
+@pytest.mark.parametrize("with_bias", [False, True])
+def test_convolution_by_pieces_has_the_bits_of_the_one_by_channels(ops, C, taps, q_lens, with_bias):
+    n, T = len(q_lens), sum(q_lens)
+    w = rnd(C, taps, seed=1, scale=0.5)
+    bias, in_bias = (rnd(C, seed=5), rnd(C, seed=6)) if with_bias else (None, None)
+    tails = [rnd(n + 1, taps - 1, C, dtype=BF, seed=2) for _ in range(2)]
+    slots = list(range(n, 0, -1))
+    for r in range(2):
+        x = rnd(T, C, dtype=BF, seed=3 + r)
+        wide = torch.zeros(T, C + 9, dtype=BF, device=DEV)
+        wide[:, 1:C + 1] = x                                     # an address that is no multiple of 16 bytes
+        outs = [torch.zeros(T, C, dtype=BF, device=DEV) for _ in range(2)]
+        for src, tail, out in zip((x, wide[:, 1:C + 1]), tails, outs):
+            ops.causal_conv(src, w, tail, state_step(q_lens, slots), out, add_input=r == 0, silu=True, bias=bias, in_bias=in_bias)
+        assert torch.equal(outs[0], outs[1]) and torch.equal(tails[0], tails[1])
+
+
+@pytest.mark.parametrize("T,N", [(1, 8), (3, 264), (130, 4096)])
+def test_rows_by_pieces(ops, T, N):
+    x, b = rnd(T, N, dtype=BF, seed=1, scale=3.0), rnd(N, seed=2)
+    r = torch.relu(x.float())
+    assert torch.equal(ops.relu_sq(x.clone()), (r * r).to(BF))
+    assert torch.equal(ops.add_bias(x.clone(), b), (x.float() + b).to(BF))
+    gu, b2 = rnd(T, 2 * N, dtype=BF, seed=3), rnd(2 * N, seed=4)
+    out = torch.empty(T, N, dtype=BF, device=DEV)
+    ops.silu_mul(gu, out, bias=b2)
+    g, u = (gu.double() + b2.double()).chunk(2, -1)
+    want = g * torch.sigmoid(g) * u
+    assert bool(((out.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5 * u.abs() + 1e-30).all())
+
+
+@pytest.mark.parametrize("V", [64, 128, 256])
+def test_read_outs_by_pieces(ops, V):
+    """The gated norm behind the recurrence: bfloat16 rows by pieces of four against the same rows at an odd place."""
+    H, D, T = 3, 64, 21
+    qkv = rnd(T, 2 * H * D + H * V, dtype=BF, seed=1)
+    beta, a_log, dt_bias, norm_w = rnd(T, H, dtype=BF, seed=2), rnd(H, seed=3), rnd(H * D, seed=4) - 1.0, 1 + rnd(V, seed=5, scale=0.1)
+    ag = rnd(T, H * D + H * V, dtype=BF, seed=6)
+    wide = torch.zeros(T, ag.shape[1] + 1, dtype=BF, device=DEV)
+    wide[:, :-1] = ag
+    got = []
+    for src in (ag, wide[:, :-1]):
+        state, out = rnd(2, H, V, D, seed=8, scale=0.3), torch.empty(T, H * V, dtype=BF, device=DEV)
+        ops.delta_rule(qkv, beta, src, a_log, dt_bias, norm_w, 1e-5, state, state_step([T], [1]), out, H, H, D, V)
+        got.append(out.float())
+    torch.testing.assert_close(got[0], got[1], atol=1e-6, rtol=2.0 ** -7)       # sums in another order: a rounding either way
+    assert float((got[0] != got[1]).float().mean()) < 0.02
