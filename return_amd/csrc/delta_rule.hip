@@ -503,8 +503,19 @@ __global__ __launch_bounds__(256) void delta_out_kernel(const float* __restrict_
     }
 }
 
+// The sum that wave_sum forms of 64 numbers, l = 4 (lane & 15) + k being v[k] of a lane, in the same order: the same bits. Every
+// group of 16 lanes gets its own.
+__device__ __forceinline__ float sum_of_quads(float (&v)[4]) {
+#pragma unroll
+    for (int o = 8; o > 0; o >>= 1)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) v[k] += __shfl_xor(v[k], o, 64);
+    return (v[0] + v[2]) + (v[1] + v[3]);
+}
+
 // The same for bfloat16 with four neighbours a lane: L lanes to a (row, head) of V = 4 L (V 64, 128 or 256, gate, norm and result
-// in whole pieces of four). Bound by its rows: 2,048 rows of 32 heads of 128 32 -> 15 us.
+// in whole pieces of four), the sum formed in the order of the kernel above: the same bits. Bound by its rows: 2,048 rows of 32
+// heads of 128 32 -> 17 us.
 template <int L>
 __global__ __launch_bounds__(256) void delta_out_bf16x4_kernel(const float* __restrict__ o_raw, const bf16* __restrict__ gate,
                                                                long long ld_gate, const float* __restrict__ norm_w, float eps,
@@ -517,10 +528,19 @@ __global__ __launch_bounds__(256) void delta_out_bf16x4_kernel(const float* __re
     const float4 o = *reinterpret_cast<const float4*>(o_raw + (size_t)row * (4 * L) + c);
     const uint2 g2 = *reinterpret_cast<const uint2*>(gate + (size_t)t * ld_gate + (size_t)h * (4 * L) + c);
     const float4 nw = *reinterpret_cast<const float4*>(norm_w + c);
-    float ss = fmaf(o.x, o.x, fmaf(o.y, o.y, fmaf(o.z, o.z, o.w * o.w)));
+    // elements l, l + 64, ... of a row lie 16 lanes apart; their squares are added first, in their order
+    const float ov[4] = {o.x, o.y, o.z, o.w};
+    float sq[4];
 #pragma unroll
-    for (int k = L / 2; k > 0; k >>= 1) ss += __shfl_xor(ss, k, 64);
-    const float rstd = 1.0f / sqrtf(ss / (float)(4 * L) + eps);
+    for (int k = 0; k < 4; ++k) {
+        sq[k] = 0.f;
+#pragma unroll
+        for (int i = 0; i < L / 16; ++i) {
+            const float x = L == 16 ? ov[k] : __shfl(ov[k], (threadIdx.x & (63 & ~(L - 1) | 15)) + 16 * i, 64);
+            sq[k] = fmaf(x, x, sq[k]);
+        }
+    }
+    const float rstd = 1.0f / sqrtf(sum_of_quads(sq) / (float)(4 * L) + eps);
     const float g[4] = {__uint_as_float(g2.x << 16), __uint_as_float(g2.x & 0xffff0000u), __uint_as_float(g2.y << 16),
                         __uint_as_float(g2.y & 0xffff0000u)};
     float y[4] = {o.x * rstd * nw.x, o.y * rstd * nw.y, o.z * rstd * nw.z, o.w * rstd * nw.w};
@@ -813,7 +833,7 @@ __global__ __launch_bounds__(256) void scalar_out_kernel(const float* __restrict
 }
 
 // The same for bfloat16 with four neighbours a lane (L and V multiples of four, L at most 64 SO_KEEP, rows and addresses in whole
-// pieces of four): 2,000 rows of eight parts of 512 32 -> 16 us.
+// pieces of four), the sum formed in the order of the kernel above: the same bits. 2,000 rows of eight parts of 512 32 -> 21 us.
 __global__ __launch_bounds__(256) void scalar_out_bf16x4_kernel(const float* __restrict__ o_raw, const bf16* __restrict__ v,
                                                                 long long ld_v, const bf16* __restrict__ gate, long long ld_gate,
                                                                 const float* __restrict__ skip, const float* __restrict__ norm_w,
@@ -825,10 +845,10 @@ __global__ __launch_bounds__(256) void scalar_out_bf16x4_kernel(const float* __r
     const long long t = unit / n_parts;
     const int c0 = (int)(unit - t * n_parts) * L;
     const size_t at = (size_t)t * n_parts * L + c0;
-    float y[SO_KEEP / 4][4];
-    float ss = 0.f;
+    float y[SO_KEEP / 4][4], sq[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < SO_KEEP / 4; ++i) {
+        if (256 * i >= L) break;                               // (the same in every lane)
         const int e = (lane + 64 * i) * 4;
 #pragma unroll
         for (int k = 0; k < 4; ++k) y[i][k] = 0.f;
@@ -845,13 +865,21 @@ __global__ __launch_bounds__(256) void scalar_out_bf16x4_kernel(const float* __r
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
                 y[i][k] = fmaf(sk, vv[k], ov[k]) * (zv[k] / (1.0f + expf(-zv[k])));
-                ss = fmaf(y[i][k], y[i][k], ss);
             }
         }
+        // elements l, l + 64, ... of the part lie 16 lanes apart
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const float x = __shfl(y[i][k], (lane & 15) + 16 * j, 64);
+                sq[k] = fmaf(x, x, sq[k]);
+            }
     }
-    const float rstd = 1.0f / sqrtf(wave_sum(ss) / (float)L + eps);
+    const float rstd = 1.0f / sqrtf(sum_of_quads(sq) / (float)L + eps);
 #pragma unroll
     for (int i = 0; i < SO_KEEP / 4; ++i) {
+        if (256 * i >= L) break;
         const int e = (lane + 64 * i) * 4;
         if (e >= L) continue;
         const float4 nw = *reinterpret_cast<const float4*>(norm_w + c0 + e);
