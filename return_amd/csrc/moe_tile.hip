@@ -40,6 +40,54 @@ __device__ __forceinline__ void mb_wait() {
     __builtin_amdgcn_s_waitcnt(0x0070 | COPIES | (READS << 8));        // (expcnt at its maximum)
 }
 
+// order between the LDS accesses of one wave: LDS serves a wave in order, the compiler must too
+#define MB_WAVE_SYNC()                                           \
+    do {                                                         \
+        __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");   \
+        __builtin_amdgcn_wave_barrier();                         \
+    } while (0)
+
+// The results of up to four groups of 16 rows of a wave, group, group + 2, ... of the tile, from LDS ([row][64 columns], rows of
+// MB_RS floats) to memory, in runs of 16 bytes.
+#define MB_RS 68
+typedef const mt_float4_t __attribute__((address_space(3)))* mb_lds_t;
+template <bool GATED>
+__device__ __forceinline__ void mb_store(uint32_t own, int lane, int group, int groups, int n_rows, const int* __restrict__ pairs,
+                                         bf16* __restrict__ y, int N, int col0, const MoeAct& act) {
+    constexpr int PER = GATED ? 4 : 8;                         // pieces of eight columns a row
+    const int r0 = lane / PER, c = (lane % PER) * 8;
+    if (col0 + c >= N) return;
+#pragma unroll 1
+    for (int r = r0; r < 16 * groups; r += 64 / PER) {
+        const int m = 16 * (group + 2 * (r >> 4)) + (r & 15);
+        if (m >= n_rows) continue;
+        const int p = pairs[m];
+        const uint32_t at = own + (r * MB_RS + c) * 4;
+        const mt_float4_t g0 = *(mb_lds_t)(uintptr_t)at, g1 = *(mb_lds_t)(uintptr_t)(at + 16);
+        float v[8];
+        if constexpr (GATED) {
+            const mt_float4_t u0 = *(mb_lds_t)(uintptr_t)(at + 128), u1 = *(mb_lds_t)(uintptr_t)(at + 144);
+            const float scale = act.in_scale != nullptr ? act.in_scale[p] : 1.0f;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = moe_gate<bf16>(k < 4 ? g0[k] : g1[k - 4], k < 4 ? u0[k] : u1[k - 4], act, scale);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = k < 4 ? g0[k] : g1[k - 4];
+        }
+        bf16* dst = y + (size_t)p * N + col0 + c;
+        if (((N & 7) | ((uintptr_t)y & 15)) == 0) {
+            uint32_t w[4];
+#pragma unroll
+            for (int k = 0; k < 4; ++k) w[k] = (uint32_t)f2bf_bits(v[2 * k]) | ((uint32_t)f2bf_bits(v[2 * k + 1]) << 16);
+            *reinterpret_cast<uint4*>(dst) = make_uint4(w[0], w[1], w[2], w[3]);
+        } else {
+#pragma unroll
+            for (int k = 0; k < 8; ++k)
+                if (col0 + c + k < N) dst[k] = from_f<bf16>(v[k]);
+        }
+    }
+}
+
 // A tile of 32 NB rows at most. xoff, woff: where this lane's rows begin (bytes), one for each of its copies.
 template <bool GATED, int NB>
 __device__ __forceinline__ void mb_tile(unsigned char* lds, const __amdgpu_buffer_rsrc_t xres, const __amdgpu_buffer_rsrc_t wres,
@@ -140,34 +188,25 @@ __device__ __forceinline__ void mb_tile(unsigned char* lds, const __amdgpu_buffe
     for (; it < nk; ++it) step(it, integral_constant<bool, false>{});
     MFMA_SETTLE();
 
-    // acc[a][b][c]: row 16 (wm + 2 b) + n of the tile, W row 64 wn + 16 a + 4 g + c of the workgroup's 256
+    // acc[a][b][c]: row 16 (wm + 2 b) + n of the tile, W row 64 wn + 16 a + 4 g + c of the workgroup's 256. A wave's results go through
+    // a part of LDS that is its own, four groups of rows at a time, so that what forms and stores them is a loop, and what is stored
+    // runs of 64 or 128 bytes. (Written out for all of a lane's results it was up to 30 KB of instructions for each count of groups,
+    // and a tile waited for them: 32 experts, 12,432 pairs, routed by a model, gate-up 764 -> 739 us, 8,000 pairs, down 288 -> 276.)
+    __syncthreads();                                           // every wave has read the last stage
+    const uint32_t own = lds0 + wave * (64 * MB_RS * 4);
+    typedef mt_float4_t __attribute__((address_space(3)))* put_t;
 #pragma unroll
-    for (int b = 0; b < NB; ++b) {
-        const int m = 16 * (wm + 2 * b) + n;
-        if (m >= n_rows) continue;
-        const int p = pairs[m];
-        bf16* yr = y + (size_t)p * N;
-        const float scale = GATED && act.in_scale != nullptr ? act.in_scale[p] : 1.0f;
+    for (int b0 = 0; b0 < NB; b0 += 4) {
+        constexpr int MOST = NB < 4 ? NB : 4;
+        const int groups = b0 + MOST < NB ? MOST : NB - b0;
 #pragma unroll
-        for (int a = 0; a < (GATED ? 2 : 4); ++a) {
-            const int col = GATED ? n0 + wn * 32 + a * 16 + 4 * g : n0 + wn * 64 + a * 16 + 4 * g;
-            float v[4];
+        for (int b = 0; b < MOST; ++b)
+            if (b0 + b < NB)
 #pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                v[c] = acc[a][b][c];
-                if constexpr (GATED) v[c] = moe_gate<bf16>(acc[a][b][c], acc[a + 2][b][c], act, scale);
-            }
-            if (col + 3 < N && (N & 3) == 0) {
-                uint2 pk;
-                pk.x = (uint32_t)f2bf_bits(v[0]) | ((uint32_t)f2bf_bits(v[1]) << 16);
-                pk.y = (uint32_t)f2bf_bits(v[2]) | ((uint32_t)f2bf_bits(v[3]) << 16);
-                *reinterpret_cast<uint2*>(yr + col) = pk;
-            } else {
-#pragma unroll
-                for (int c = 0; c < 4; ++c)
-                    if (col + c < N) yr[col + c] = from_f<bf16>(v[c]);
-            }
-        }
+                for (int a = 0; a < 4; ++a) *(put_t)(uintptr_t)(own + ((b * 16 + n) * MB_RS + 16 * a + 4 * g) * 4) = acc[a][b0 + b];
+        MB_WAVE_SYNC();
+        mb_store<GATED>(own, lane, wm + 2 * b0, groups, n_rows, pairs, y, N, GATED ? n0 + wn * 32 : n0 + wn * 64, act);
+        MB_WAVE_SYNC();
     }
 }
 
