@@ -182,6 +182,279 @@ __global__ __launch_bounds__(NTH) void token_side_bf16x8_kernel(
     }
 }
 
+// bfloat16 and S up to 32 (H, S as above): the same sums in the same order, with the reads asked for before what they wait behind.
+// (A loop over a row's runs of 512 columns waits for one load after the other, 1 us each where the matrices come from memory.)
+__device__ __forceinline__ void ts_unpack(const uint4& v, float (&f)[8]) {
+    const uint32_t p[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        f[2 * k] = __uint_as_float(p[k] << 16);
+        f[2 * k + 1] = __uint_as_float(p[k] & 0xffff0000u);
+    }
+}
+__device__ __forceinline__ float4 ts_row4(const float* h, const bf16* delta, size_t at) {
+    float4 v = *reinterpret_cast<const float4*>(h + at);
+    if (delta != nullptr) {
+        const uint2 d = *reinterpret_cast<const uint2*>(delta + at);
+        v.x += __uint_as_float(d.x << 16); v.y += __uint_as_float(d.x & 0xffff0000u);
+        v.z += __uint_as_float(d.y << 16); v.w += __uint_as_float(d.y & 0xffff0000u);
+    }
+    return v;
+}
+__device__ __forceinline__ float ts_gelu(float x) {
+    const float inner = 0.7978845608028654f * (x + 0.044715f * x * x * x);
+    return 0.5f * x * (1.f + tanhf(inner));
+}
+
+// One row a workgroup: a wave's gate rows (32 over WAVES waves), half of the projection and the token's entries are asked for beside
+// the row itself, the rest of the projection as the first half is used. RUNS: of 512 columns. H 4,096, S 32, matrices from memory:
+// 22 -> 17 us, which is one CU's reading of 512 KB (from the caches 14 -> 11).
+template <int RUNS, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void token_side_row_kernel(
+    float* __restrict__ h, const bf16* __restrict__ delta, const int* __restrict__ ids, const bf16* __restrict__ table,
+    long long ld_table, int off, const bf16* __restrict__ gate, const bf16* __restrict__ proj,
+    const float* __restrict__ w, float eps, int H, int S) {
+    constexpr int NT = 64 * WAVES, GATES = 32 / WAVES, COLS = 512 * RUNS / NT, QUADS = (128 * RUNS + NT - 1) / NT;
+    __shared__ __attribute__((aligned(16))) float x_s[512 * RUNS];
+    __shared__ float g_s[32], red[WAVES];
+    const int t = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const size_t row = (size_t)t * H;
+    const int id = ids[t];
+    // (what lies beyond H or S is read again from the last place, and meets zeros in x_s or g_s)
+    float4 xv[QUADS];
+    uint2 dv[QUADS];
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) {
+        const int c = min((tid + NT * i) * 4, H - 4);
+        xv[i] = *reinterpret_cast<const float4*>(h + row + c);
+        dv[i] = make_uint2(0u, 0u);
+        if (delta != nullptr) dv[i] = *reinterpret_cast<const uint2*>(delta + row + c);
+    }
+    uint4 gv[GATES][RUNS];
+#pragma unroll
+    for (int k = 0; k < GATES; ++k)
+#pragma unroll
+        for (int q = 0; q < RUNS; ++q) {
+            const int r = min(wave + WAVES * k, S - 1), c = min(lane * 8 + 512 * q, H - 8);
+            gv[k][q] = *reinterpret_cast<const uint4*>(gate + (unsigned)(r * H + c));
+        }
+    uint4 pv[COLS / 2][4];
+    auto ask = [&](int i, int half) {
+        const int c = min(tid + NT * (half * (COLS / 2) + i), H - 1);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) pv[i][q] = *reinterpret_cast<const uint4*>(proj + (unsigned)(c * S + min(8 * q, S - 8)));
+    };
+#pragma unroll
+    for (int i = 0; i < COLS / 2; ++i) ask(i, 0);
+    float e[GATES];
+#pragma unroll
+    for (int k = 0; k < GATES; ++k) e[k] = to_f(table[(size_t)id * ld_table + off + min(wave + WAVES * k, S - 1)]);
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) {
+        const int c = (tid + NT * i) * 4;
+        xv[i].x += __uint_as_float(dv[i].x << 16); xv[i].y += __uint_as_float(dv[i].x & 0xffff0000u);
+        xv[i].z += __uint_as_float(dv[i].y << 16); xv[i].w += __uint_as_float(dv[i].y & 0xffff0000u);
+        if (c < 512 * RUNS) *reinterpret_cast<float4*>(x_s + c) = c < H ? xv[i] : make_float4(0.f, 0.f, 0.f, 0.f);
+    }
+    __syncthreads();
+    float a[GATES];
+#pragma unroll
+    for (int k = 0; k < GATES; ++k) a[k] = 0.f;
+#pragma unroll
+    for (int q = 0; q < RUNS; ++q) {
+        const int c = lane * 8 + 512 * q;
+        const float4 x0 = *reinterpret_cast<const float4*>(x_s + c), x1 = *reinterpret_cast<const float4*>(x_s + c + 4);
+        const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+        for (int k = 0; k < GATES; ++k) {
+            float g[8];
+            ts_unpack(gv[k][q], g);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) a[k] = fmaf(g[i], x[i], a[k]);
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < GATES; ++k) {
+        const float x = wave_sum(a[k]);
+        const int r = wave + WAVES * k;
+        if (lane == k) g_s[r] = r < S ? ts_gelu(x) * e[k] : 0.f;
+    }
+    float wv[COLS];
+#pragma unroll
+    for (int i = 0; i < COLS; ++i) wv[i] = w[min(tid + NT * i, H - 1)];
+    __syncthreads();
+    float y[COLS], ss = 0.f;
+#pragma unroll
+    for (int half = 0; half < 2; ++half)
+#pragma unroll
+        for (int i = 0; i < COLS / 2; ++i) {
+            float v = 0.f;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                float p[8];
+                ts_unpack(pv[i][q], p);
+#pragma unroll
+                for (int k = 0; k < 8; ++k) v = fmaf(p[k], g_s[8 * q + k], v);
+            }
+            if (half == 0) ask(i, 1);
+            y[half * (COLS / 2) + i] = v;
+            ss = fmaf(v, tid + NT * (half * (COLS / 2) + i) < H ? v : 0.f, ss);
+        }
+    ss = wave_sum(ss);
+    if (lane == 0) red[wave] = ss;
+    __syncthreads();
+    float tot = 0.f;
+#pragma unroll
+    for (int v = 0; v < WAVES; ++v) tot += red[v];
+    const float rstd = 1.0f / sqrtf(tot / (float)H + eps);
+#pragma unroll
+    for (int i = 0; i < COLS; ++i) {
+        const int c = tid + NT * i;
+        if (c < H) h[row + c] = x_s[c] + y[i] * rstd * wv[i];
+    }
+}
+
+// Many rows, four a workgroup of four waves: a wave has the next two gate rows on their way while it multiplies two, by the rows
+// of the stream in LDS (in 32-bit); then y takes the rows' place there, a column a turn, the next one's projection on its way, and
+// the stream is read again at the end. Two workgroups a CU. H 4,096, S 32: 2,048 rows 91 -> 56 us.
+#define TR_ROWS 4
+// From three rounds of single rows over the CUs on (4,096 columns: 200 rows 12 us, 700 rows 34 either way).
+#define TR_FROM 768
+template <int RUNS>
+__global__ __launch_bounds__(256, 2) void token_side_rows_kernel(
+    float* __restrict__ h, const bf16* __restrict__ delta, const int* __restrict__ ids, const bf16* __restrict__ table,
+    long long ld_table, int off, const bf16* __restrict__ gate, const bf16* __restrict__ proj,
+    const float* __restrict__ w, float eps, int T_tokens, int H, int S) {
+    constexpr int HS = 512 * RUNS;
+    extern __shared__ __attribute__((aligned(16))) float x_s[];                       // [TR_ROWS][HS]: the stream, then y
+    __shared__ float g_s[TR_ROWS][32], red[TR_ROWS][4];
+    const int t0 = blockIdx.x * TR_ROWS, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const int rows = min(TR_ROWS, T_tokens - t0);
+    // piece (r0, first run): four runs of gate rows r0 and r0 + 4
+    uint4 next[2][4];
+    auto ask = [&](int r0, int q0) {
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const int r = min(r0 + 4 * k, S - 1), c = min(lane * 8 + 512 * (q0 + q), H - 8);
+                next[k][q] = *reinterpret_cast<const uint4*>(gate + (unsigned)(r * H + c));
+            }
+    };
+    ask(wave, 0);
+#pragma unroll 4
+    for (int c = tid * 4; c < TR_ROWS * HS; c += 1024) {
+        const int rr = c / HS, cc = c - rr * HS;
+        float4 v = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (rr < rows && cc < H) v = ts_row4(h, delta, (size_t)(t0 + rr) * H + cc);
+        *reinterpret_cast<float4*>(x_s + c) = v;
+    }
+    __syncthreads();
+    float a[2][TR_ROWS];
+#pragma unroll 1
+    for (int r0 = wave, q0 = 0; r0 < 32;) {
+        uint4 now[2][4];
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) now[k][q] = next[k][q];
+        const bool ends = q0 + 4 >= RUNS;
+        const int r1 = ends ? r0 + 8 : r0, q1 = ends ? 0 : q0 + 4;
+        ask(r1, q1);
+        if (q0 == 0) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k)
+#pragma unroll
+                for (int rr = 0; rr < TR_ROWS; ++rr) a[k][rr] = 0.f;
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float g[2][8];
+            ts_unpack(now[0][q], g[0]);
+            ts_unpack(now[1][q], g[1]);
+#pragma unroll
+            for (int rr = 0; rr < TR_ROWS; ++rr) {
+                const float* xr = x_s + rr * HS + lane * 8 + 512 * (q0 + q);
+                const float4 x0 = *reinterpret_cast<const float4*>(xr), x1 = *reinterpret_cast<const float4*>(xr + 4);
+                const float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+#pragma unroll
+                for (int k = 0; k < 2; ++k)
+#pragma unroll
+                    for (int i = 0; i < 8; ++i) a[k][rr] = fmaf(g[k][i], x[i], a[k][rr]);
+            }
+        }
+        if (ends) {
+#pragma unroll
+            for (int k = 0; k < 2; ++k) {
+                float mine = 0.f;                                                     // lane rr gets row rr's
+#pragma unroll
+                for (int rr = 0; rr < TR_ROWS; ++rr) {
+                    const float x = wave_sum(a[k][rr]);
+                    if (lane == rr) mine = x;
+                }
+                const int r = r0 + 4 * k;
+                if (lane < TR_ROWS) {
+                    const float e = r < S ? to_f(table[(size_t)ids[t0 + min(lane, rows - 1)] * ld_table + off + r]) : 0.f;
+                    g_s[lane][r] = r < S ? ts_gelu(mine) * e : 0.f;
+                }
+            }
+        }
+        r0 = r1;
+        q0 = q1;
+    }
+    __syncthreads();
+    // y of column tid + 256 i of every row, in place of the stream
+    float ss[TR_ROWS];
+#pragma unroll
+    for (int rr = 0; rr < TR_ROWS; ++rr) ss[rr] = 0.f;
+    uint4 pn[4];
+    auto column = [&](int c) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) pn[q] = *reinterpret_cast<const uint4*>(proj + (unsigned)(min(c, H - 1) * S + min(8 * q, S - 8)));
+    };
+    column(tid);
+#pragma unroll 1
+    for (int c = tid; c < H; c += 256) {
+        uint4 p4[4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) p4[q] = pn[q];
+        column(c + 256);
+        float y[TR_ROWS];
+#pragma unroll
+        for (int rr = 0; rr < TR_ROWS; ++rr) y[rr] = 0.f;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            float p[8];
+            ts_unpack(p4[q], p);
+#pragma unroll
+            for (int rr = 0; rr < TR_ROWS; ++rr)
+#pragma unroll
+                for (int k = 0; k < 8; ++k) y[rr] = fmaf(p[k], g_s[rr][8 * q + k], y[rr]);
+        }
+#pragma unroll
+        for (int rr = 0; rr < TR_ROWS; ++rr) {
+            ss[rr] = fmaf(y[rr], y[rr], ss[rr]);
+            x_s[rr * HS + c] = y[rr];
+        }
+    }
+#pragma unroll
+    for (int rr = 0; rr < TR_ROWS; ++rr) {
+        const float v = wave_sum(ss[rr]);
+        if (lane == 0) red[rr][wave] = v;
+    }
+    __syncthreads();
+#pragma unroll 4
+    for (int c = tid * 4; c < TR_ROWS * HS; c += 1024) {
+        const int rr = c / HS, cc = c - rr * HS;
+        if (rr >= rows || cc >= H) continue;
+        const size_t at = (size_t)(t0 + rr) * H + cc;
+        const float4 x = ts_row4(h, delta, at), y = *reinterpret_cast<const float4*>(x_s + c), wv = *reinterpret_cast<const float4*>(w + cc);
+        const float rstd = 1.0f / sqrtf((((red[rr][0] + red[rr][1]) + red[rr][2]) + red[rr][3]) / (float)H + eps);
+        *reinterpret_cast<float4*>(h + at) =
+            make_float4(x.x + y.x * rstd * wv.x, x.y + y.y * rstd * wv.y, x.z + y.z * rstd * wv.z, x.w + y.w * rstd * wv.w);
+    }
+}
+
 template <int R, int NTH>
 static int token_side_x8_launch(hipStream_t st, float* h, const void* delta, const int* ids, const void* table,
                                 long long ld_table, int off, const void* gate, const void* proj, const float* w, float eps,
@@ -204,6 +477,23 @@ extern "C" int ra_token_side(float* h, const void* delta, const int* ids, const 
     if (S < 1 || S > TS_MAX_S || H < 1 || H > TS_THREADS * TS_MAX_CPT || off < 0 || ld_table < off + S) return RA_ERR_ARG;
     dim3 grid(T_tokens), block(TS_THREADS);
     hipStream_t st = (hipStream_t)stream;
+    auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+    if (dtype == RA_DTYPE_BF16 && S <= 32 && S % 8 == 0 && H % 8 == 0 && H <= 4096 && al(h) && al(delta) && al(gate) && al(proj) && al(w)) {
+#define TS_ROW(RUNS_, WAVES_)                                                                                                      \
+    hipLaunchKernelGGL((token_side_row_kernel<RUNS_, WAVES_>), grid, dim3(64 * WAVES_), 0, st, h, (const bf16*)delta, ids, (const bf16*)table, ld_table, \
+                       off, (const bf16*)gate, (const bf16*)proj, w, eps, H, S)
+#define TS_ROWS(RUNS_)                                                                                                             \
+    hipLaunchKernelGGL(token_side_rows_kernel<RUNS_>, dim3((T_tokens + TR_ROWS - 1) / TR_ROWS), block, TR_ROWS * 2048 * RUNS_, st, h, \
+                       (const bf16*)delta, ids, (const bf16*)table, ld_table, off, (const bf16*)gate, (const bf16*)proj, w, eps, T_tokens, H, S)
+        if (T_tokens < TR_FROM) {
+            if (H <= 2048) TS_ROW(4, 16); else TS_ROW(8, 8);
+        } else {
+            if (H <= 2048) TS_ROWS(4); else TS_ROWS(8);
+        }
+#undef TS_ROW
+#undef TS_ROWS
+        return ra_launch_status();
+    }
     if (dtype == RA_DTYPE_BF16 && H % 8 == 0 && S % 8 == 0 && H <= 4096) {
         // many rows: four a workgroup, so that the two matrices are read once for four rows
         if (T_tokens >= 256)

@@ -73,3 +73,18 @@ def test_grouped_read_outs_by_pieces(ops, H, V, parts):
         ops.scalar_rule(qkv, dt, a_log, dt_bias, skip, src, norm_w, parts, 1e-5, state, state_step([T], [1]), out, H, G, D, V)
         got.append(out)
     assert torch.equal(got[0], got[1])
+
+
+@pytest.mark.parametrize("T,H,S", [(1, 8, 8), (3, 2048, 32), (5, 2056, 24), (2, 4096, 32), (7, 4088, 16),       # a row a workgroup
+                                   (768, 2048, 32), (769, 4096, 24), (770, 1000, 8), (771, 2056, 32)])          # four
+@pytest.mark.parametrize("with_delta", [False, True])
+def test_token_input_in_its_forms(ops, ref, T, H, S, with_delta):
+    table = rnd(50, 2 * S + 3, dtype=BF, seed=1)
+    gate, proj, w = rnd(S, H, dtype=BF, seed=2, scale=H ** -0.5), rnd(H, S, dtype=BF, seed=3), rnd(H, seed=4).abs()
+    ids = torch.randint(0, 50, (T,), generator=torch.Generator().manual_seed(5)).int().to(DEV)
+    delta = rnd(T, H, dtype=BF, seed=6) if with_delta else None
+    a = rnd(T, H, seed=7)
+    b = a.clone()
+    ops.token_side(a, delta, ids, table, S + 1, gate, proj, w, 1e-5)
+    ref.token_side(b, delta, ids, table, S + 1, gate, proj, w, 1e-5)
+    torch.testing.assert_close(a, b, atol=1e-4, rtol=1e-4)
