@@ -113,6 +113,9 @@ def _declare(lib):
         "ra_gemm_sweep_norm_bf16": [P, P, P, I, I, I, I, I, I, P, I, I, F, P, P, P, P],
         "ra_attention_plain": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, F, I, I, P, F, I, I, P, F, L, P],
         "ra_attention_f32_fits": [I],
+        "ra_latent_rows": [P, P, P, I, I, P],
+        "ra_attention_latent_prompt_fits": [I, I, I, I, I],
+        "ra_attention_latent_prompt": [P, L, P, L, P, P, P, P, P, P, I, I, I, I, I, F, P, P, L, P, P],
         "ra_attention_prefill_f32": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, F, I, P, F, I, I, P, F, L, P],
         "ra_attention_decode_f32": [P, P, P, P, P, P, P, P, P, P, I, I, I, I, I, F, I, P, F, I, I, P, F, L, P],
         "ra_causal_conv": [P, L, P, P, P, P, P, L, I, I, I, I, I, I, P],
@@ -2099,6 +2102,62 @@ class HipOps:
         self._check(self.lib.ra_attention_latent_plain_window(
             _ptr(qq), _ptr(out), _ptr(k_pool), _ptr(v_pool), *tabs, None, step.n_seqs, T, T, Hn, C, R, P, float(scale),
             _ptr(sink), 1 if step.all_decode else 0, window, _code(qq.dtype), self._stream()), "attention_latent_plain")
+
+    LATENT_PROMPT_ROWS = 128      # of a q tile of attention_latent_prompt
+
+    def latent_prompt_fits(self, n_heads, D, R, Dv, rotary_dim, C, scale, dtype):
+        """Whether attention_latent_prompt takes these sizes."""
+        return dtype == torch.bfloat16 and scale > 0 and C % 8 == 0 and \
+            bool(self.lib.ra_attention_latent_prompt_fits(int(n_heads), int(D), int(R), int(Dv), int(rotary_dim)))
+
+    def latent_rows(self, v_pool, slot_mapping, T):
+        """The value pool's rows that slot_mapping names, side by side: [T, C]."""
+        self._want(v_pool, "value pool", torch.bfloat16, 4)
+        self._want(slot_mapping, "slot mapping", torch.int32, 1)
+        C = v_pool.shape[3]
+        if slot_mapping.shape[0] != T or v_pool.shape[1] != 1:
+            raise KernelError(f"latent_rows: pool {tuple(v_pool.shape)}, {slot_mapping.shape[0]} slots for {T} rows")
+        rows = torch.empty(T, C, dtype=v_pool.dtype, device=self.device)
+        self._check(self.lib.ra_latent_rows(_ptr(v_pool), _ptr(slot_mapping), _ptr(rows), T, C, self._stream()), "latent_rows")
+        return rows
+
+    def attention_latent_prompt(self, q, kv, D, R, Dv, k_pool, slot_mapping, cos, sin, step, scale, sink, gate, out):
+        """Attention of whole prompts (every request of the step from position 0 on, two tokens or more) with formed keys
+        and values: q [T, H (D + R)], the rotated parts not yet turned (cos None: none turns), kv [T, H D + H Dv], the key
+        pool's rows of R (turned) by slot_mapping; softmax with exp(sink[h]) in its denominator (None: none); out
+        [T, H Dv] times sigmoid(gate [T, H]) (None: as it is). q and gate may be column slices of wider rows."""
+        ld_q, ld_kv = self._want_rows(q, "q", torch.bfloat16), self._want_rows(kv, "keys and values", torch.bfloat16)
+        self._want(out, "attention output", torch.bfloat16, 2)
+        self._want(slot_mapping, "slot mapping", torch.int32, 1)
+        T, Hn = q.shape[0], q.shape[1] // (D + R)
+        tiles = step.prefill_tiles.get(self.LATENT_PROMPT_ROWS) if getattr(step, "prefill_tiles", None) else None
+        if q.shape[1] != Hn * (D + R) or tuple(kv.shape) != (T, Hn * (D + Dv)) or tuple(out.shape) != (T, Hn * Dv) \
+                or T != step.n_tokens or slot_mapping.shape[0] != T or tiles is None or step.n_decode > 0 or max(step.q_starts) > 0:
+            raise KernelError(f"attention_latent_prompt: q {tuple(q.shape)}, kv {tuple(kv.shape)}, out {tuple(out.shape)}, "
+                              f"step of {step.n_tokens} tokens")
+        if R:
+            self._want(k_pool, "key pool", torch.bfloat16, 4)
+            if k_pool.shape[1] != 1 or k_pool.shape[3] != R:
+                raise KernelError(f"attention_latent_prompt: key pool {tuple(k_pool.shape)} for rotated parts of {R}")
+        if cos is not None:
+            self._want(cos, "cos table", torch.float32, 2)
+            self._want(sin, "sin table", torch.float32, 2)
+            if cos.shape[1] != R // 2 or sin.shape != cos.shape or cos.shape[0] < step.max_q_len:
+                raise KernelError(f"attention_latent_prompt: tables {tuple(cos.shape)} for rotated parts of {R}")
+        ld_gate = 0
+        if gate is not None:
+            ld_gate = self._want_rows(gate, "gate logits", torch.bfloat16)
+            if tuple(gate.shape) != (T, Hn):
+                raise KernelError(f"attention_latent_prompt: gate {tuple(gate.shape)}")
+        if sink is not None:
+            self._want(sink, "sink", torch.float32, 1)
+            if sink.shape[0] != Hn:
+                raise KernelError(f"attention_latent_prompt: sink {tuple(sink.shape)} for {Hn} heads")
+        self._check(self.lib.ra_attention_latent_prompt(
+            _ptr(q), ld_q, _ptr(kv), ld_kv, _ptr(k_pool) if R else None, _ptr(slot_mapping), _ptr(cos), _ptr(sin), _ptr(step.cu_q),
+            _ptr(tiles), tiles.shape[0], Hn, int(D), int(R), int(Dv), float(scale), _ptr(sink), _ptr(gate), ld_gate, _ptr(out),
+            self._stream()), "attention_latent_prompt")
+        return out
 
     def latent_prefill_tile_rows(self, n_heads, C, R, dtype):
         """Rows (tokens) per q tile of the lists that attention_latent reads from step.prefill_tiles, or None where

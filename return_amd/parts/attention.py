@@ -453,7 +453,9 @@ class LatentAttention:
     head. The products with W_uk and W_uv are moved to the query's side, where they cost one row per new token
     instead of one per key read:  q_h . (W_uk,h c) = (W_uk,h^T q_h) . c  and  sum_j p_j W_uv,h c_j = W_uv,h (sum_j p_j c_j),
     so every head reads the same rows [c | rot(k_r)] with a query of C + R elements, and one kernel serves
-    whole prompts, portions and single tokens. Both products write where their result is wanted: into the first C elements
+    prompts, portions and single tokens. (Where the kernel set can, a step of whole prompts, whose keys are all new and are read
+    by many queries each, forms the heads' keys and values instead: a score then costs D + R products and not C + R, its value Dv
+    and not C.) Both products write where their result is wanted: into the first C elements
     of every head's query, and (without a gate) into the heads' places side by side.
     With direct_q there is no query latent: q = W_q x (role q), whose rows ride in the first product, and one kernel turns
     q's rotated parts beside the token's key part.
@@ -533,6 +535,12 @@ class LatentAttention:
         self.w_uk = rt.matrix(tensors["uk"]).view(self.H, self.D, self.C).contiguous()
         self.w_uv_t = rt.matrix(tensors["uv"]).view(self.H, self.Dv, self.C).transpose(1, 2).contiguous()
         self.w_o = rt.product(rt.matrix(tensors["o"]))
+        # whole prompts: the heads' keys and values are formed, by [W_uk; W_uv] in one product
+        self.w_ukv = None
+        turned = self.position.tables()[2] if self.position is not None else 0
+        if hasattr(rt.ops, "latent_prompt_fits") and \
+                rt.ops.latent_prompt_fits(self.H, self.D, self.R, self.Dv, turned, self.C, self.scale, rt.dtype):
+            self.w_ukv = torch.cat([self.w_uk.view(self.H * self.D, self.C), rt.matrix(tensors["uv"])], dim=0).contiguous()
 
     def cache_spec(self):
         return PagedKVSpec(1, self.R, self.window, 0, self.C)
@@ -541,7 +549,16 @@ class LatentAttention:
         ops = self.rt.ops
         rows = ops.latent_prefill_tile_rows(self.H, self.C, self.R, self.rt.dtype) \
             if hasattr(ops, "latent_prefill_tile_rows") else None
-        return {"prefill_tile_rows": set(rows)} if rows else {}
+        rows = set(rows or ())
+        if self.w_ukv is not None:
+            rows.add(ops.LATENT_PROMPT_ROWS)
+        return {"prefill_tile_rows": rows} if rows else {}
+
+    def _whole_prompts(self, step):
+        """Whether every request brings all that its queries read: prompts from position 0 on, none beyond the window."""
+        return self.w_ukv is not None and step.n_decode == 0 and step.n_prefill_tokens == step.n_tokens and \
+            max(step.q_starts) == 0 and (not self.window or step.max_q_len <= self.window) and \
+            self.rt.ops.LATENT_PROMPT_ROWS in step.prefill_tiles
 
     def forward(self, x, step, cache, write_cache=True):
         rt, ops = self.rt, self.rt.ops
@@ -550,6 +567,20 @@ class LatentAttention:
         z = ops.linear(x, self.w_in)                                  # [T, H (D + R) or Q | C + R | H | pad]
         cos, sin, rot = self.position.tables() if self.position is not None else (None, None, 0)
         at, kv = self.at_kv, (cache.k_pool, cache.v_pool) if write_cache else (None, None)
+        if write_cache and self._whole_prompts(step):
+            if self.direct:
+                q = z[:, :at]
+                ops.latent_kv_prepare(z[:, at:at + C + R], 0, C, R, None, self.w_dkv_norm, self.eps, step.positions, cos, sin, rot,
+                                      None, *kv, tables.slot_mapping)
+            else:
+                cq = rt.empty(T, Q)
+                ops.latent_kv_prepare(z, Q, C, R, self.w_dq_norm, self.w_dkv_norm, self.eps, step.positions, cos, sin, rot, cq,
+                                      *kv, tables.slot_mapping)
+                q = ops.linear(cq, self.w_uq)
+            heads = ops.linear(ops.latent_rows(cache.v_pool, tables.slot_mapping, T), self.w_ukv)
+            y = ops.attention_latent_prompt(q, heads, D, R, Dv, cache.k_pool, tables.slot_mapping, cos, sin, step, self.scale,
+                                            self.sink, z[:, at + C + R:at + C + R + H] if self.gated else None, rt.empty(T, H * Dv))
+            return ops.linear(y, self.w_o)
         qq = rt.empty(T, H, C + R)
         if self.direct:
             q = z[:, :at]                                             # [T, H (D + R)], columns of z
