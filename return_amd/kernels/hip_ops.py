@@ -100,6 +100,8 @@ def _declare(lib):
         "ra_silu_mul": [P, P, I, I, I, P],
         "ra_gemm_nt": [P, P, P, I, I, I, I, I, P],
         "ra_gemm_split_f32": [P, P, P, I, I, I, P, L, P],
+        "ra_gemm_heads_fits": [I, I, I, I],
+        "ra_gemm_heads_bf16": [P, L, L, P, P, L, L, I, I, I, I, P],
         "ra_gemm_rows_fits": [I, I, I],
         "ra_gemm_rows_bf16": [P, P, P, I, I, I, I, I, I, I, P],
         "ra_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, P],
@@ -386,17 +388,28 @@ class HipOps:
                     "heads_gate")
 
     def batched_product(self, a, b, out=None):
-        """[B, M, K] x [B, K, N] -> [B, M, N] in a's dtype, by the library (32-bit operands: a true 32-bit product). out:
+        """[B, M, K] x [B, K, N] -> [B, M, N] in a's dtype (32-bit operands: a true 32-bit product): bfloat16 of up to 8 rows
+        and more of K than of N by the kernel that reads b once (heads of 512 x 128 at one row 5 us, the library's product
+        12; the other way round, 128 x 512, it is no faster), else by the library. out:
         where the result goes (rows of N elements side by side, apart by any distance: the rows of all b's batches may be
         columns of the same wider rows); None: a new tensor."""
         if a.dim() != 3 or b.dim() != 3 or a.shape[0] != b.shape[0] or a.shape[2] != b.shape[1] or a.dtype != b.dtype \
                 or not b.is_contiguous():
             raise KernelError(f"batched_product: {tuple(a.shape)} x {tuple(b.shape)}")
+        own = a.dtype == torch.bfloat16 and a.shape[2] > b.shape[2] and a.stride(2) == 1 and b.data_ptr() % 16 == 0 and \
+            a.data_ptr() % 16 == 0 and a.stride(0) % 8 == 0 and a.stride(1) % 8 == 0 and min(a.stride()) >= 0 and \
+            self.lib.ra_gemm_heads_fits(a.shape[0], a.shape[1], b.shape[2], a.shape[2])
         if out is None:
-            return torch.bmm(a, b)
+            if not own:
+                return torch.bmm(a, b)
+            out = torch.empty(a.shape[0], a.shape[1], b.shape[2], dtype=a.dtype, device=self.device)
         if tuple(out.shape) != (a.shape[0], a.shape[1], b.shape[2]) or out.dtype != a.dtype or (out.shape[2] > 1 and out.stride(2) != 1):
             raise KernelError(f"batched_product: {tuple(a.shape)} x {tuple(b.shape)} into {tuple(out.shape)}, strides {out.stride()}")
-        return torch.bmm(a, b, out=out)
+        if not own:
+            return torch.bmm(a, b, out=out)
+        self._check(self.lib.ra_gemm_heads_bf16(_ptr(a), a.stride(0), a.stride(1), _ptr(b), _ptr(out), out.stride(0), out.stride(1),
+                                                a.shape[0], a.shape[1], b.shape[2], a.shape[2], self._stream()), "gemm_heads")
+        return out
 
     def add_rmsnorm(self, h, delta, weight, eps, out, rows=None, delta_scale=1.0):
         """h += delta_scale * delta (in place, unless a row list is given); out = norm(h) * weight."""
