@@ -148,7 +148,9 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
                                                         int* __restrict__ meta) {
     __shared__ int place[MOE_MAX_EXPERTS > 16 * MOE_PLAN_EXPERTS ? MOE_MAX_EXPERTS : 16 * MOE_PLAN_EXPERTS];
     __shared__ unsigned long long wave_total[16];
+    __shared__ int sorted[MOE_MAX_EXPERTS];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const bool runs = rows == MOE_PANEL_ROWS;
     const int copies = E <= MOE_PLAN_EXPERTS ? 16 : 1;
     int* mine = place + (copies == 16 ? wave : 0) * E;
     for (int i = tid; i < copies * E; i += 1024) place[i] = 0;
@@ -162,10 +164,27 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
             if (id[j] >= 0) atomicAdd(&mine[id[j]], 1);
     }
     __syncthreads();
-    // thread e: its expert's pairs and tiles, and how many of both the experts before it have
+    int e = tid;
+    if (runs) {
+        // the experts with the largest tiles first: tiles go to the CUs in this order, and what is long must not come last
+        int n = 0, key = 0;
+        if (tid < E) {
+            for (int c = 0; c < copies; ++c) n += place[c * E + tid];
+            sorted[tid] = key = min(n, moe_rows_of_tile(n, rows));
+        }
+        __syncthreads();
+        int rank = 0;
+        if (tid < E)
+            for (int j = 0; j < E; ++j) rank += sorted[j] > key || (sorted[j] == key && j < tid);
+        __syncthreads();
+        if (tid < E) sorted[rank] = tid;
+        __syncthreads();
+        if (tid < E) e = sorted[tid];
+    }
+    // thread i: its expert's pairs and tiles, and how many of both the experts before it have
     int n = 0;
     if (tid < E)
-        for (int c = 0; c < copies; ++c) n += place[c * E + tid];
+        for (int c = 0; c < copies; ++c) n += place[c * E + e];
     const int own_tiles = tid < E && n > 0 ? moe_tiles_of(n, rows) : 0;
     unsigned long long sum = ((unsigned long long)n << 32) | (unsigned)own_tiles;
     const unsigned long long own = sum;
@@ -183,17 +202,18 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
     if (tid < E) {
         int tl = (int)(sum & 0xffffffffull);
         const int per = moe_rows_of_tile(n, rows);
-        for (int i = 0; i < n; i += per, ++tl) {
-            tiles[3 * tl] = tid;
+        for (int i = 0, j = 0; i < n; i += per, ++tl, ++j) {
+            tiles[3 * tl] = e;
             tiles[3 * tl + 1] = first + i;
-            tiles[3 * tl + 2] = min(per, n - i);
+            // (runs of up to four tiles of an expert: their number and the tile's place among them ride along)
+            tiles[3 * tl + 2] = min(per, n - i) | (runs ? (min(own_tiles - (j & ~3), 4) * 16 + (j & 3)) << 16 : 0);
         }
         // a pair's place among its expert's pairs is whatever the atomic gives: a row's result does not depend on its
         // place in a tile
         int at = first;
         for (int c = 0; c < copies; ++c) {
-            const int k = place[c * E + tid];
-            place[c * E + tid] = at;
+            const int k = place[c * E + e];
+            place[c * E + e] = at;
             at += k;
         }
     }
@@ -562,6 +582,31 @@ extern "C" int ra_moe_product(const void* x, const void* w, void* y, const int* 
                               int dtype, void* stream) {
     return ra_moe_product_act(x, w, y, order, tiles, meta, n_pairs, max_tiles, tile_rows, N, K, top_div, gated, 0, 0.f, 0.f, nullptr, dtype,
                               stream);
+}
+
+// The same with w laid out in panels (moe_tile.h). tile_rows: 16 or MOE_PANEL_ROWS, as ra_moe_panel_rows says: from two pairs an
+// expert on nearly every expert has one, and the tiles' longer reads are the faster ones; with fewer they are not enough tiles for
+// the CUs. 32 experts, gate-up and down, sweep / tiles, us: of 6,144 x 4,096, 8 tokens 188 + 101 / 211 + 103, 16 tokens 265 + 136 /
+// 249 + 128, 64 tokens 285 + 150 / 258 + 133; of 4,096 x 2,048, 8 tokens 67 + 34 / 73 + 36, 16 tokens 91 + 47 / 89 + 48, 64 tokens 102 +
+// 56 / 91 + 50.
+extern "C" int ra_moe_panel_rows(int n_pairs, int E) { return n_pairs >= 2 * E ? MOE_PANEL_ROWS : 16; }
+
+extern "C" int ra_moe_panel_product(const void* x, const void* w, void* y, const int* order, const int* tiles, const int* meta,
+                                    int n_pairs, int max_tiles, int tile_rows, int N, int K, int top_div, int gated, int act_kind,
+                                    float limit, float slope, const float* in_scale, void* stream) {
+    if (max_tiles <= 0) return RA_OK;
+    if (N < 16 || N % 16 || K < 64 || K % 64 || K > MOE_PANEL_K || top_div < 1 || act_kind < 0 || act_kind > 1 || (in_scale != nullptr && !gated))
+        return RA_ERR_ARG;
+    // (32-bit offsets into an expert's matrix and into x)
+    if (2ll * N * K * (gated ? 2 : 1) >= 0x7fffff00ll || 2ll * n_pairs * K >= 0x7fffff00ll) return RA_ERR_ARG;
+    const MoeAct act = {act_kind, limit, slope, in_scale};
+    const int x_rows = (n_pairs - 1) / top_div + 1;
+    if (tile_rows == MOE_PANEL_ROWS)
+        return moe_panel_tile_launch((hipStream_t)stream, (const bf16*)x, (const bf16*)w, (bf16*)y, order, tiles, meta, max_tiles, x_rows, N, K,
+                                     top_div, gated != 0, act);
+    if (tile_rows != 16) return RA_ERR_ARG;
+    return moe_panel_sweep_launch((hipStream_t)stream, (const bf16*)x, (const bf16*)w, (bf16*)y, order, tiles, meta, x_rows, N, K, top_div,
+                                  gated != 0, act);
 }
 
 // ------------------------------------------------------------------ combine

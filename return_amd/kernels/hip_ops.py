@@ -12,7 +12,7 @@ from typing import Optional
 
 import torch
 
-from ..parts.runtime import RowSums, ScaledRows, Slabs
+from ..parts.runtime import Panels, RowSums, ScaledRows, Slabs
 from . import build as _build
 
 _F32, _BF16 = 0, 1
@@ -87,6 +87,8 @@ def _declare(lib):
         "ra_moe_route": [P, P, I, I, I, I, I, F, P, P, P],
         "ra_moe_plan": [P, I, I, I, P, P, P, P],
         "ra_moe_tile_rows": [I, I, I, I, I],
+        "ra_moe_panel_rows": [I, I],
+        "ra_moe_panel_product": [P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, P],
         "ra_moe_product": [P, P, P, P, P, P, I, I, I, I, I, I, I, I, P],
         "ra_moe_combine": [P, P, P, I, I, I, I, P],
         "ra_moe_combine_extra": [P, P, P, I, I, I, P, P, I, L, I, P],
@@ -2234,10 +2236,64 @@ class HipOps:
                     "moe_route")
         return ids, weights
 
+    def expert_panels(self, matrix, experts, hidden, inter, gated, dtype):
+        """The experts' matrices (matrix(e): [2 inter, hidden], gate rows first, when gated, else [hidden, inter]) as Panels, laid out
+        as moe_tile.h says, or None for sizes that have no such layout (both products of a layer have it or neither)."""
+        if dtype != torch.bfloat16 or hidden % 64 or inter % 64 or not 64 <= min(hidden, inter) <= max(hidden, inter) <= 4096:
+            return None
+        R, K = (2 * inter, hidden) if gated else (hidden, inter)
+        out = torch.empty(experts, K // 64, R // 16, 2, 4, 16, 8, dtype=dtype, device=self.device)
+        for e in range(experts):
+            w = matrix(e).view(R // 16, 16, K // 64, 2, 4, 8)
+            if gated:
+                w = w.view(2, R // 32, 16, K // 64, 2, 4, 8).transpose(0, 1)         # panel of gate rows, panel of up rows
+                out[e].view(K // 64, R // 32, 2, 2, 4, 16, 8).copy_(w.permute(3, 0, 1, 4, 5, 2, 6))
+            else:
+                out[e].copy_(w.permute(2, 0, 3, 4, 1, 5))
+        return Panels(out, (experts, R, K))
+
+    def _moe_plan(self, ids, E, rows):
+        """(order, tiles, meta, tiles at most, rows): the step's pairs by expert, in tiles of at most so many rows."""
+        n_pairs = ids.numel()
+        max_tiles = min(n_pairs, n_pairs // rows + E)                  # (every expert may end in a tile that is not full)
+        order = torch.empty(n_pairs, dtype=torch.int32, device=self.device)
+        tiles = torch.empty(max_tiles, 3, dtype=torch.int32, device=self.device)
+        meta = torch.empty(1, dtype=torch.int32, device=self.device)
+        self._check(self.lib.ra_moe_plan(_ptr(ids), n_pairs, E, rows, _ptr(order), _ptr(tiles), _ptr(meta), self._stream()), "moe_plan")
+        return order, tiles, meta, max_tiles, rows
+
+    def _experts_panels(self, x, ids, in_scale, w_gate_up, w_down, y, act, limit, slope):
+        (T, H), (E, I2, _), top = x.shape, w_gate_up.shape, ids.shape[1]
+        n_pairs, I = T * top, I2 // 2
+        mid = torch.empty(n_pairs, I, dtype=x.dtype, device=self.device)
+        order, tiles, meta, max_tiles, rows = self._moe_plan(ids, E, int(self.lib.ra_moe_panel_rows(n_pairs, E)))
+        self._check(self.lib.ra_moe_panel_product(_ptr(x), _ptr(w_gate_up.tensor), _ptr(mid), _ptr(order), _ptr(tiles), _ptr(meta), n_pairs,
+                                                  max_tiles, rows, I, H, top, 1, act, float(limit), float(slope), _ptr(in_scale),
+                                                  self._stream()), "moe_panel_product (gate-up)")
+        self._check(self.lib.ra_moe_panel_product(_ptr(mid), _ptr(w_down.tensor), _ptr(y), _ptr(order), _ptr(tiles), _ptr(meta), n_pairs,
+                                                  max_tiles, rows, H, I, 1, 0, 0, 0.0, 0.0, None, self._stream()),
+                    "moe_panel_product (down)")
+
+    def _experts_plain(self, x, ids, in_scale, w_gate_up, w_down, y, act, limit, slope):
+        (T, H), (E, I2, _), top = x.shape, w_gate_up.shape, ids.shape[1]
+        n_pairs, I, code = T * top, I2 // 2, _code(x.dtype)
+        mid = torch.empty(n_pairs, I, dtype=x.dtype, device=self.device)
+        # the two products may take tiles of different heights (their K differ): a plan each where they do
+        rows_up, rows_down = (int(self.lib.ra_moe_tile_rows(n_pairs, E, N, K, code)) for N, K in ((I2, H), (H, I)))
+        up = self._moe_plan(ids, E, rows_up)
+        down = up if rows_down == rows_up else self._moe_plan(ids, E, rows_down)
+        order, tiles, meta, max_tiles, rows = up
+        self._check(self.lib.ra_moe_product_act(_ptr(x), _ptr(w_gate_up), _ptr(mid), _ptr(order), _ptr(tiles), _ptr(meta),
+                                                n_pairs, max_tiles, rows, I, H, top, 1, act, float(limit), float(slope),
+                                                _ptr(in_scale), code, self._stream()), "moe_product (gate-up)")
+        order, tiles, meta, max_tiles, rows = down
+        self._check(self.lib.ra_moe_product(_ptr(mid), _ptr(w_down), _ptr(y), _ptr(order), _ptr(tiles), _ptr(meta),
+                                            n_pairs, max_tiles, rows, H, I, 1, 0, code, self._stream()), "moe_product (down)")
+
     def moe_experts(self, x, ids, weights, w_gate_up, w_down, activation="silu", limit=0.0, slope=1.702, extra=None,
                     extra_logits=None, weigh="output", combine=True):
         """sum_k weights[t, k] * down_e(silu(gate_e x_t) * up_e x_t), e = ids[t, k]; w_gate_up [E, 2I, H] (gate
-        rows first), w_down [E, H, I]. The pairs are grouped by expert on the device. activation "clamped": an
+        rows first), w_down [E, H, I], or both as expert_panels gives them. The pairs are grouped by expert on the device. activation "clamped": an
         expert is down(g sigmoid(slope g) (u + 1)) with g = min(gate x, limit), u = clamp(up x, -limit, limit).
         extra [T, H] with extra_logits [T, 1] (possibly a column of wider rows): one more term of every token's sum,
         extra[t] * sigmoid(extra_logits[t]), added last in the same 32-bit sum (extra_logits in x's type or fp32).
@@ -2252,8 +2308,11 @@ class HipOps:
         self._want(x, "rows", dims=2)
         self._want(ids, "expert ids", torch.int32, 2)
         self._want(weights, "expert weights", torch.float32, 2)
-        self._want(w_gate_up, "gate-up matrices", x.dtype, 3)
-        self._want(w_down, "down matrices", x.dtype, 3)
+        panels = isinstance(w_gate_up, Panels)
+        if panels != isinstance(w_down, Panels):
+            raise KernelError("moe_experts: one product's matrices in panels and the other's not")
+        for w, name in ((w_gate_up, "gate-up matrices"), (w_down, "down matrices")):
+            self._want(w.tensor if panels else w, name, x.dtype, 7 if panels else 3)
         T, H = x.shape
         E, I2, _ = w_gate_up.shape
         top, I = ids.shape[1], I2 // 2
@@ -2261,44 +2320,31 @@ class HipOps:
                 or tuple(w_down.shape) != (E, H, I):
             raise KernelError(f"moe_experts: x {tuple(x.shape)}, ids {tuple(ids.shape)}, gate-up {tuple(w_gate_up.shape)}, "
                               f"down {tuple(w_down.shape)}")
-        n_pairs, code = T * top, _code(x.dtype)
-        ld_logits = 0
+        n_pairs = T * top
         if (extra is None) != (extra_logits is None):
             raise KernelError("moe_experts: a further term needs its rows and its gate logits")
         if extra is not None:
             self._want(extra, "further term", x.dtype, 2)
-            ld_logits = self._want_rows(extra_logits, "gate logits of the further term")
+            self._want_rows(extra_logits, "gate logits of the further term")
             if extra_logits.dtype not in (x.dtype, torch.float32) or (not combine and extra_logits.dtype != torch.float32):
                 raise KernelError(f"moe_experts: gate logits of the further term in {extra_logits.dtype}")
             if tuple(extra.shape) != (T, H) or tuple(extra_logits.shape) != (T, 1):
                 raise KernelError(f"moe_experts: further term {tuple(extra.shape)}, its logits {tuple(extra_logits.shape)}")
         if n_pairs == 0:
             return torch.empty(T, H, dtype=x.dtype, device=self.device)
-        mid = torch.empty(n_pairs, I, dtype=x.dtype, device=self.device)
         y = torch.empty(n_pairs, H, dtype=x.dtype, device=self.device)
-
-        def plan(rows):
-            # (every expert may end in a tile that is not full)
-            max_tiles = min(n_pairs, n_pairs // rows + E)
-            order = torch.empty(n_pairs, dtype=torch.int32, device=self.device)
-            tiles = torch.empty(max_tiles, 3, dtype=torch.int32, device=self.device)
-            meta = torch.empty(1, dtype=torch.int32, device=self.device)
-            self._check(self.lib.ra_moe_plan(_ptr(ids), n_pairs, E, rows, _ptr(order), _ptr(tiles), _ptr(meta),
-                                             self._stream()), "moe_plan")
-            return order, tiles, meta, max_tiles, rows
-
-        # the two products may take tiles of different heights (their K differ): a plan each where they do
-        rows_up, rows_down = (int(self.lib.ra_moe_tile_rows(n_pairs, E, N, K, code)) for N, K in ((I2, H), (H, I)))
-        up = plan(rows_up)
-        down = up if rows_down == rows_up else plan(rows_down)
-        order, tiles, meta, max_tiles, rows = up
-        self._check(self.lib.ra_moe_product_act(_ptr(x), _ptr(w_gate_up), _ptr(mid), _ptr(order), _ptr(tiles), _ptr(meta),
-                                                n_pairs, max_tiles, rows, I, H, top, 1, act, float(limit), float(slope),
-                                                _ptr(weights) if weigh == "input" else None, code,
-                                                self._stream()), "moe_product (gate-up)")
-        order, tiles, meta, max_tiles, rows = down
-        self._check(self.lib.ra_moe_product(_ptr(mid), _ptr(w_down), _ptr(y), _ptr(order), _ptr(tiles), _ptr(meta),
-                                            n_pairs, max_tiles, rows, H, I, 1, 0, code, self._stream()), "moe_product (down)")
+        in_scale = weights if weigh == "input" else None
+        if panels:
+            if x.data_ptr() % 16:
+                x = x.clone()
+            # (the kernels' offsets into their rows have 32 bits, a tile's number 15: a step beyond that goes in parts of its tokens)
+            part = max(1, min(0x7fffff00 // (2 * top * max(H, I)) - 1, 8_000_000 // top))
+            for t in range(0, T, part):
+                s = slice(t, min(t + part, T))
+                self._experts_panels(x[s], ids[s], None if in_scale is None else in_scale[s], w_gate_up, w_down, y[t * top:s.stop * top], act,
+                                     limit, slope)
+        else:
+            self._experts_plain(x, ids, in_scale, w_gate_up, w_down, y, act, limit, slope)
         sums = RowSums(y, top, weights if weigh == "output" else None, extra, extra_logits)
         return self.row_sums(sums) if combine else sums
 

@@ -25,7 +25,8 @@ expert_e(s_e x). With activation "silu" a shared expert has no limit. Params joi
 ride in the shared expert's first product, whose result then is 32-bit: one product for gate, up, the shared gate's one
 row and the router. Asked to (forward's combine False), the part leaves its sums to whatever forms the stream next.
 
-The experts' matrices are kept stacked ([E, 2 I, H] with gate rows first, [E, H, I]); a step's (token,
+The experts' matrices are kept stacked ([E, 2 I, H] with gate rows first, [E, H, I]), in the kernel set's own layout where it
+has one for these sizes (expert_panels; the plain stack is not kept beside it); a step's (token,
 choice) pairs are grouped by expert on the device and the products run over those groups, so nothing
 of a step's routing comes back to the host.
 """
@@ -100,9 +101,12 @@ class GroupedRoutedExperts:
         self.w_router = None
         second = "router_bias" if self.law == "softmax_top" else "correction"
         self.correction = rt.vector32(tensors[second]) if second in self.tensor_shapes(params) else None
-        self.w_gate_up = torch.stack([torch.cat([rt.matrix(tensors[f"gate_{e}"]), rt.matrix(tensors[f"up_{e}"])], dim=0)
-                                      for e in range(E)]).contiguous()                  # [E, 2I, H]
-        self.w_down = torch.stack([rt.matrix(tensors[f"down_{e}"]) for e in range(E)]).contiguous()   # [E, H, I]
+        def stacked(matrix, gated):
+            lay = getattr(rt.ops, "expert_panels", None)
+            panels = lay(matrix, E, self.hidden, self.inter, gated, rt.dtype) if lay is not None else None
+            return panels if panels is not None else torch.stack([matrix(e) for e in range(E)]).contiguous()
+        self.w_gate_up = stacked(lambda e: torch.cat([rt.matrix(tensors[f"gate_{e}"]), rt.matrix(tensors[f"up_{e}"])], dim=0), True)
+        self.w_down = stacked(lambda e: rt.matrix(tensors[f"down_{e}"]), False)       # [E, 2I, H] and [E, H, I]
         self.shared, self.joint = None, False
         if params.get("shared"):
             self.joint = bool(params.get("joint_router"))

@@ -112,6 +112,19 @@ class RowSums:
         return (self.rows.shape[0] // self.count, self.rows.shape[1])
 
 
+class Panels:
+    """Experts' matrices laid out for the matrix units (what the kernel set's expert_panels gives): the tensor, and the shape
+    [experts, rows, columns] of the matrices in it."""
+    __slots__ = ("tensor", "shape")
+
+    def __init__(self, tensor, shape):
+        self.tensor, self.shape = tensor, tuple(shape)
+
+    @property
+    def dtype(self):
+        return self.tensor.dtype
+
+
 def unscaled(delta):
     """(rows, factor) of a pending output, Scaled or plain (None stays None)."""
     if isinstance(delta, Scaled):

@@ -1,7 +1,9 @@
 """The experts' products on the matrix cores (bf16) against a 64-bit product of the same bfloat16 operands: tiles of up to 256
 rows in LDS (twelve pairs an expert and more) at every count of groups of 16 rows, few k-steps, experts without rows, widths
 that are no multiple of a tile; tiles of 16 rows with W read in whole runs (fewer pairs) at one to eight waves, columns shared
-out unevenly, more tiles than workgroups; both activations, factors on what an expert reads."""
+out unevenly, more tiles than workgroups; both activations, factors on what an expert reads. The same of matrices in panels: tiles of
+up to 320 rows at every count of groups, steps of K that are no multiple of four, W that ends inside a tile; few rows at one to eight steps a
+wave."""
 import pytest
 import torch
 
@@ -15,7 +17,7 @@ def ops():
     return HipOps(DEV)
 
 
-def check(ops, rows, E, H, I, ids, kind):
+def check(ops, rows, E, H, I, ids, kind, panels=False):
     """One expert a token, so that the counts are exact. A result is two bf16 roundings (2^-9 each of the halves and of the
     activation) away from the 64-bit one, grown by the product with them: 2^-6 of the largest."""
     g = torch.Generator().manual_seed(len(ids) + H)
@@ -24,8 +26,12 @@ def check(ops, rows, E, H, I, ids, kind):
     w_down = (torch.randn(E, H, I, generator=g) * I ** -0.5).bfloat16()
     factor = 0.5 + torch.rand(len(ids), 1, generator=g)
     kw = {"clamped": dict(activation="clamped", limit=1.0), "input": dict(weigh="input"), "silu": {}}[kind]
-    assert ops.lib.ra_moe_tile_rows(len(ids), E, 2 * I, H, 1) == rows        # (the kernel that this is about)
-    got = ops.moe_experts(x.to(DEV), ids.int()[:, None].to(DEV), factor.to(DEV), w_up.to(DEV), w_down.to(DEV), **kw)
+    # (the kernel that this is about)
+    assert (ops.lib.ra_moe_panel_rows(len(ids), E) if panels else ops.lib.ra_moe_tile_rows(len(ids), E, 2 * I, H, 1)) == rows
+    a, b = w_up.to(DEV), w_down.to(DEV)
+    if panels:
+        a, b = (ops.expert_panels(lambda e: w[e], E, H, I, gated, torch.bfloat16) for w, gated in ((a, True), (b, False)))
+    got = ops.moe_experts(x.to(DEV), ids.int()[:, None].to(DEV), factor.to(DEV), a, b, **kw)
     want = torch.zeros(len(ids), H, dtype=torch.float64)
     for e in ids.unique().tolist():
         t = (ids == e).nonzero()[:, 0]
@@ -64,3 +70,22 @@ def test_products_of_many_rows(ops, E, H, I, counts, kind):
 @pytest.mark.parametrize("kind", KINDS)
 def test_products_of_few_rows(ops, E, H, I, counts, kind):
     check(ops, 16, E, H, I, shuffled(counts), kind)
+
+
+@pytest.mark.parametrize("E,H,I,counts", [
+    (4, 64, 64, [1, 16, 17, 33]), (3, 128, 192, [48, 20, 0]), (2, 320, 64, [64, 65]), (5, 256, 192, [80, 96, 97, 112, 0]),
+    (3, 64, 448, [128, 144, 160]), (4, 192, 128, [176, 192, 208, 209]), (2, 1024, 576, [256, 700]), (1, 128, 64, [2]),
+    (6, 192, 64, [0, 0, 48, 0, 0, 500]), (2, 4096, 320, [15, 300]), (9, 448, 64, [64, 97, 0, 2, 5, 1, 1, 30, 1100]),
+    (40, 64, 128, [7] * 20 + [330] * 3 + [0] * 17), (2, 64, 64, [320, 321]), (3, 64, 320, [225, 241, 289])])
+@pytest.mark.parametrize("kind", KINDS)
+def test_panels_many_rows(ops, E, H, I, counts, kind):
+    check(ops, 320, E, H, I, shuffled(counts), kind, panels=True)
+
+
+@pytest.mark.parametrize("E,H,I,counts", [
+    (4, 64, 64, [1, 0, 2, 0]), (20, 576, 128, [5, 16, 7] + [0] * 17), (20, 1088, 192, [1, 20] + [0] * 18),
+    (40, 2048, 128, [1, 0, 0, 3, 17, 0, 33, 9] + [0] * 32), (16, 4096, 64, [15, 1] + [0] * 14), (4, 2624, 4096, [1, 1, 0, 0]), (8, 3136, 64, [11] + [0] * 7),
+    (700, 64, 64, [1] * 650 + [0] * 50), (5, 512, 1536, [0, 4, 0, 1, 0])])
+@pytest.mark.parametrize("kind", KINDS)
+def test_panels_few_rows(ops, E, H, I, counts, kind):
+    check(ops, 16, E, H, I, shuffled(counts), kind, panels=True)
