@@ -241,7 +241,7 @@ __host__ __device__ constexpr int dec_region_bytes(int D) {
 // per (request, kv head), wave w takes split w, and the waves' sums are merged through LDS here
 // (the same sums in the same order as the merge kernel), so that nothing goes through memory and
 // no second kernel runs; for requests whose splits fit one workgroup.
-template <int D16, bool FUSED, int XT>
+template <int D16, bool FUSED, int XT, bool AWAY>
 __global__ __launch_bounds__(D16 <= 8 ? 512 : 256) __attribute__((amdgpu_waves_per_eu(D16 <= 8 ? 2 : 1)))
 void attn_decode_kernel(
     const bf16* __restrict__ q, float* __restrict__ part_acc, float* __restrict__ part_ml,
@@ -307,17 +307,23 @@ void attn_decode_kernel(
     };
     int row_next = 0;
     [[maybe_unused]] int first_row = 0;          // FUSED: the rows of the first pass, whose keys are asked for before the loop
-    // the key tiles of a pass, straight into MFMA A operands
+    // the key tiles of a pass, straight into MFMA A operands. Keys and values are read once a step and go past the caches
+    // (AWAY, nontemporal): a layer of heads 32 over 8 of 128, 8 requests of 2,048 20.3 -> 18.7 us, 64 of 500 30.6 -> 28.1, 24 of 450 17.3 ->
+    // 16.0. Not where several waves share a kv head (32 heads over one: 29.8, past the caches 31.9), nor for smaller heads, whose rows
+    // the caches may still hold from the step before (8 over 2 of 64, 8 requests of 500 7.6, past them 7.9).
     bf16x8_t ak[4][D32 > 0 ? D32 : 1];
     bf16x8_t ak_tail[4];
+    auto take = [](const auto* p) {
+        if constexpr (AWAY) return __builtin_nontemporal_load(p);
+        else return *p;
+    };
     auto load_keys = [&](int row) {
 #pragma unroll
         for (int st = 0; st < 4; ++st) {
             const int r = __shfl(row, st * 16 + n, 64);
             const bf16* kp = k_pool + (size_t)r * D;
 #pragma unroll
-            for (int j = 0; j < D32; ++j)
-                ak[st][j] = *reinterpret_cast<const bf16x8_t*>(kp + 32 * j + 8 * g);
+            for (int j = 0; j < D32; ++j) ak[st][j] = take(reinterpret_cast<const bf16x8_t*>(kp + 32 * j + 8 * g));
             if constexpr (TAIL16) {
                 ak_tail[st] = z8;
                 if (g < 2) ak_tail[st] = *reinterpret_cast<const bf16x8_t*>(kp + (D - 16) + 8 * g);
@@ -421,7 +427,7 @@ void attn_decode_kernel(
         for (int i = 0; i < NVL; ++i) {
             const int e = min(lane + 64 * i, DEC_CHUNK * LPR - 1);
             const int r = __shfl(row, e / LPR, 64);
-            vv[i] = *reinterpret_cast<const uint4_t*>(v_pool + (size_t)r * D + (e % LPR) * 8);
+            vv[i] = take(reinterpret_cast<const uint4_t*>(v_pool + (size_t)r * D + (e % LPR) * 8));
         }
         WAVE_SYNC();                               // the previous pass has read its value tile
 #pragma unroll
@@ -622,8 +628,10 @@ static int dec_launch_one(dim3 grid, hipStream_t st, const bf16* q, float* pa, f
                           DecodeExtras ex) {
     constexpr int D = 16 * N;
     const size_t lds = (size_t)merge_waves * (dec_region_bytes(D) + (FUSED ? 4 * D : 0));
-    auto kern = attn_decode_kernel<N, FUSED, XT>;
-    static size_t allowed = 64 * 1024;                        // per instantiation: raised when needed
+    const bool away = N >= 8 && Hq <= DEC_MAX_GROUP * Hkv;
+    auto kern = away ? attn_decode_kernel<N, FUSED, XT, (N >= 8)> : attn_decode_kernel<N, FUSED, XT, false>;
+    static size_t allowed_by[2] = {64 * 1024, 64 * 1024};     // per kernel: raised when needed
+    size_t& allowed = allowed_by[away ? 1 : 0];
     if (lds > allowed) {
         if (lds > 160 * 1024 ||
             hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -14,6 +14,7 @@
 // library's product and the SiLU-mul behind it 55), at 32 rows 44.9 -> 37.1; head of 151,936 x 4,096 280 -> 241 (library 273);
 // down 4,096 x 12,288 in four pieces of K 24 -> 23 (library 27), o 4,096 x 4,096 in four 10.6 (13.6). With few columns a CU
 // (q/k/v 6,144 x 4,096: 24) x is most of what a CU takes in, and the library's product is as fast (18.5 / 17.6).
+// From 16 MB on W is read past the caches: gate-up 39.0 -> 36.9, head 243 -> 233.
 #include "common.h"
 #include <type_traits>
 
@@ -37,7 +38,7 @@ __device__ __forceinline__ void gr_wait() {
     __builtin_amdgcn_s_waitcnt(0x0070 | (COPIES & 15) | ((COPIES >> 4) << 14));        // (expcnt at its maximum)
 }
 
-template <int NB, int G, bool GATED, typename TO>
+template <int NB, int G, bool GATED, bool AWAY, typename TO>
 __device__ __forceinline__ void gr_tile(unsigned char* lds, const bf16* __restrict__ X, const bf16* __restrict__ W, TO* __restrict__ C,
                                         int M, int N, int K, int tiles, int k_steps) {
     constexpr int S = gr_stages(NB, G), STAGE = (NB + G) * 16 * GR_ROW, NC = NB + G;      // (copies a wave and step: NC)
@@ -69,8 +70,8 @@ __device__ __forceinline__ void gr_tile(unsigned char* lds, const bf16* __restri
             void __attribute__((address_space(3)))* to =
                 (void __attribute__((address_space(3)))*)(lds + stage * STAGE + (16 * i + 4 * wave) * GR_ROW);
             if (i < NB) __builtin_amdgcn_raw_ptr_buffer_load_lds(xres, to, 16, off[i], at, 0, 0);
-            else if (i < NB + H) __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, to, 16, off[i], at, 0, 0);
-            else __builtin_amdgcn_raw_ptr_buffer_load_lds(ures, to, 16, off[i], at, 0, 0);
+            else if (i < NB + H) __builtin_amdgcn_raw_ptr_buffer_load_lds(wres, to, 16, off[i], at, 0, AWAY ? 2 : 0);
+            else __builtin_amdgcn_raw_ptr_buffer_load_lds(ures, to, 16, off[i], at, 0, AWAY ? 2 : 0);
         }
     };
     gr_f4 acc[G][NB];
@@ -148,11 +149,11 @@ __device__ __forceinline__ void gr_tile(unsigned char* lds, const bf16* __restri
     }
 }
 
-template <int NB, int G, bool GATED, typename TO>
+template <int NB, int G, bool GATED, bool AWAY, typename TO>
 __global__ __launch_bounds__(256) void gemm_rows_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, TO* __restrict__ C, int M,
                                                         int N, int K, int tiles, int k_steps) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-    gr_tile<NB, G, GATED, TO>(lds, X, W, C, M, N, K, tiles, k_steps);
+    gr_tile<NB, G, GATED, AWAY, TO>(lds, X, W, C, M, N, K, tiles, k_steps);
 }
 
 // What the kernel takes: operands 16-byte aligned.
@@ -190,9 +191,11 @@ extern "C" int ra_gemm_rows_bf16(const void* X, const void* W, void* C, int M, i
     const dim3 grid((unsigned)(tiles * pieces)), block(256);
     const int lds = gr_stages(nb, G) * (nb + G) * 16 * GR_ROW;
     hipStream_t st = (hipStream_t)stream;
+    // (a small W may well lie in the caches from the step before, and stays there: 1,024 x 512 at 64 rows 4.1 us, read past them 4.6)
+    const bool away = 2ll * N * K * (gated ? 2 : 1) >= 16ll << 20;
 #define GR_GO(NB_, G_, GATED_, T_)                                                                                                      \
     do {                                                                                                                                \
-        const auto kern = gemm_rows_kernel<NB_, G_, GATED_, T_>;                                                                        \
+        const auto kern = away ? gemm_rows_kernel<NB_, G_, GATED_, true, T_> : gemm_rows_kernel<NB_, G_, GATED_, false, T_>;            \
         if (hipFuncSetAttribute(reinterpret_cast<const void*>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds) != hipSuccess)    \
             return RA_ERR_LAUNCH;                                                                                                       \
         hipLaunchKernelGGL(kern, grid, block, lds, st, (const bf16*)X, (const bf16*)W, (T_*)C, M, N, K, (int)tiles, k_steps);           \

@@ -14,6 +14,10 @@
 // 16x16x32 bf16 (lane (n, g): 16 bytes of row n at 32j + 8g); the wave's columns of x are B operands
 // that stay in registers for all tiles. The eight waves' partial tiles are added through LDS in wave
 // order, as in the x-resident product.
+// W is read past the caches (nontemporal loads), which hold nothing of it when the next step comes: at 8 rows 24,576 x 4,096 37.7 ->
+// 34.5 us (5.8 TB/s), 4,096 x 12,288 22.8 -> 21.5, 4,096 x 4,096 10.5 -> 9.8, 151,936 x 4,096 225 -> 206 (6.1; at one row 210 -> 187);
+// 1,024 x 512, which the caches could hold, 4.8 -> 4.5. The products that take operands of 64-byte pieces straight from memory
+// (x-resident, skinny) lose by it: a line goes when its first half has been read (head 221 -> 232, gate-up 48 -> 50).
 // Results: bfloat16 or fp32 [M, N]; GATED (W = [Wg; Wu], rollout/monkey_patch/qwen3.py:103): a tile
 // is 8 gate rows and the 8 up rows of the same columns, the result silu(g) * u as [M, N]
 // (rollout/fused.py:103-114).
@@ -119,7 +123,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
     auto fetch_row = [&](int t, int i) {
         const int col = b + G * (t * COLS + (GATED ? (i & 7) : i));
         const size_t row = (GATED && i >= 8) ? (size_t)N + col : (size_t)col;
-        wreg[i] = (k_in && col < N) ? *reinterpret_cast<const bf16x8_t*>(W + row * K + kb + lane * 8) : zero;
+        wreg[i] = (k_in && col < N) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + kb + lane * 8)) : zero;
     };
 #pragma unroll
     for (int i = 0; i < 16; ++i) fetch_row(0, i);
@@ -245,7 +249,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
         const int k = p * SW_SPAN + kb + lane * 8;
         const int col = b + G * (t * COLS + (GATED ? (i & 7) : i));
         const size_t row = (GATED && i >= 8) ? (size_t)N + col : (size_t)col;
-        wreg[i] = (k < K && col < N) ? *reinterpret_cast<const bf16x8_t*>(W + row * K + k) : zero;
+        wreg[i] = (k < K && col < N) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + k)) : zero;
     };
 #pragma unroll
     for (int i = 0; i < 16; ++i) fetch_row(0, 0, i);
@@ -370,7 +374,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_spans_kernel(
         const int k = p * SW_SPAN + kb + lane * 8;
         const int col = b + G * (t * COLS + (GATED ? (i & 7) : i));
         const size_t row = (GATED && i >= 8) ? (size_t)N + col : (size_t)col;
-        wreg[i] = (k < K && col < N) ? *reinterpret_cast<const bf16x8_t*>(W + row * K + k) : zero;
+        wreg[i] = (k < K && col < N) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + k)) : zero;
     };
 #pragma unroll
     for (int i = 0; i < 16; ++i) fetch_row(0, 0, i);

@@ -6,9 +6,9 @@
 // issued, so that 64 to 256 KB a CU are always on their way; its part of the tile's rows of x stays in registers. The waves'
 // results are added through LDS in wave order; the barrier for that waits for no load.
 //
-// Bound by the reading of W. Measured, gate-up and down of 32 experts, four a token, with rows of W through LDS (moe_sweep.hip) / this
-// kernel, us: of 6,144 x 4,096, 1 token 41 + 20 / 37 + 18, 8 tokens 194 + 102 / 188 + 101 (5.9 TB/s); of 4,096 x 2,048, 1 token 15 + 10 /
-// 15 + 9, 8 tokens 72 + 36 / 67 + 34.
+// Bound by the reading of W, which goes past the caches (nontemporal). Measured, gate-up and down of 32 experts, four a token, with rows
+// of W through LDS (moe_sweep.hip; caches / past them) / this kernel, us: of 6,144 x 4,096, 1 token 41 + 20, 37 + 22 / 34 + 19, 8
+// tokens 194 + 102, 169 + 90 / 167 + 87 (6.6 TB/s).
 #include "moe_tile.h"
 
 typedef __bf16 mq_bf16x8_t __attribute__((ext_vector_type(8)));
@@ -50,7 +50,7 @@ __global__ __launch_bounds__(64 * MQ_WAVES) __attribute__((amdgpu_waves_per_eu(K
 #pragma unroll
         for (int a = 0; a < NP; ++a)
             wf[j][h][a] = __builtin_bit_cast(mq_bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(
-                res, lane * 16 + a * 2048 + h * 1024, (k0 + j) * kstep + i * (NP * 2048), 0));
+                res, lane * 16 + a * 2048 + h * 1024, (k0 + j) * kstep + i * (NP * 2048), 2));
     };
 #pragma unroll
     for (int j = 0; j < KW; ++j)

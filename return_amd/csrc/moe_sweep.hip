@@ -14,6 +14,7 @@
 // came at 3.9 to 4.1 TB/s. Measured, gate-up and down of 32 experts, four a token: of 6,144 x 4,096, 1 token 61 us (65
 // before), 8 tokens 296 (391; 1.5 GB at 5.1 TB/s), 16 tokens 369 (408); of 4,096 x 2,048, 1 token 23 us (38), 8 tokens 108
 // (153), 64 tokens 155 (213).
+// W is read past the caches: 8 tokens of 6,144 x 4,096 194 -> 169 us, 16 tokens 271 -> 239.
 #include "moe_tile.h"
 
 typedef __bf16 ms_bf16x8_t __attribute__((ext_vector_type(8)));
@@ -61,7 +62,7 @@ __global__ __launch_bounds__(512) void moe_sweep_kernel(
         auto fetch_row = [&](int item, int i) {
             const int col = item * COLS + (GATED ? (i & 7) : i);
             const size_t row = (GATED && i >= 8) ? (size_t)N + col : (size_t)col;
-            wreg[i] = (k_in && col < N) ? *reinterpret_cast<const ms_bf16x8_t*>(we + row * K) : zero;
+            wreg[i] = (k_in && col < N) ? __builtin_nontemporal_load(reinterpret_cast<const ms_bf16x8_t*>(we + row * K)) : zero;
         };
 #pragma unroll
         for (int i = 0; i < 16; ++i) fetch_row(first, i);
