@@ -11,11 +11,11 @@
 //
 // The panels of a step lie side by side ([step][panel]), so that a workgroup reads 32 KB in a row: with [panel][step], runs a power of
 // two apart, gate-up of 32 experts of 6,144 x 4,096 took 697 instead of 658 us at 12,432 pairs. Measured there, W in rows through LDS /
-// this kernel, us: 256 pairs 298 / 258 (6.2 TB/s), 4,000 pairs 326 / 298, 8,000 pairs 501 / 393 (1.02 PFLOP/s), 12,432 pairs 627 /
-// 573, uneven counts (147 to 742) 698 / 609, 32,768 pairs 1,485 / 1,352 (1.22 PFLOP/s); down (4,096 x 3,072) 8,000 pairs 282 / 203,
-// 12,432 pairs 319 / 298; gate-up of 4,096 x 2,048, 256 pairs 127 / 91, 8,448 pairs 236 / 160. Bound, up to 100 rows an expert, by
-// the reading of W, beyond that by the matrix cores and the loads' way beside them: MFMAs alone take 0.6 to 0.7 of the time, with all
-// loads out of L2 it is 0.9. MFMA 32x32x16 instead of 16x16x32: 712 instead of 598 us at 12,432 pairs.
+// this kernel, us: 256 pairs 298 / 231 (7.0 TB/s), 4,000 pairs 326 / 283, 8,000 pairs 489 / 376 (1.07 PFLOP/s), 12,432 pairs 629 /
+// 550, uneven counts (147 to 742) 695 / 592, 32,768 pairs 1,486 / 1,285 (1.28 PFLOP/s); down (4,096 x 3,072) 8,000 pairs 281 / 193,
+// 12,432 pairs 325 / 279; gate-up of 4,096 x 2,048, 256 pairs 130 / 82, 8,448 pairs 226 / 150. Bound, up to 100 rows an expert, by
+// the reading of W, beyond that by the matrix cores and the loads' way beside them: MFMAs alone take 0.6 to 0.7 of the time. MFMA
+// 32x32x16 instead of 16x16x32: 712 instead of 598 us at 12,432 pairs (before the copies of x were spread).
 #include "moe_tile.h"
 #include <type_traits>
 
@@ -44,13 +44,17 @@ __device__ __forceinline__ void mp_tile(unsigned char* lds, const bf16* __restri
     // are read (above 16 groups the sums leave registers for no more)
     constexpr int ALL = 2 * NG, R = NG > 16 ? 4 : 8, MOST = NG > 16 ? 3 : 5, D = ALL < MOST ? ALL : MOST;
     constexpr int AHEAD = NG > 16 ? 2 : 3;                     // steps that W is asked for ahead (likewise)
+    // Large tiles spread the copies of x over a step, into the stage of two steps before: all at once behind the barrier they hold up the
+    // operand reads of all waves (32,768 pairs 1,352 -> 1,285 us, 10,240 even ones 482 -> 439). Small ones, whose steps are short, ask
+    // one step further ahead, behind the barrier.
+    constexpr bool SPREAD = NG >= 10;
     const int n = lane & 15, g = lane >> 4, nk = K / MP_BK, kstep = w_bytes / nk;
     // (a step beyond K reads from buffers of no length, which gives zeros: the loop has no branches)
-    auto copy_x = [&](int kk, auto stage_c) {
+    auto copy_x = [&](int kk, int stage, int from, int to) {
         const __amdgpu_buffer_rsrc_t res = __builtin_amdgcn_make_buffer_rsrc((void*)x, 0, kk < nk ? x_bytes : 0, 0x00020000);
-        unsigned char* base = lds + decltype(stage_c)::value * STAGE;
+        unsigned char* base = lds + stage * STAGE;
 #pragma unroll
-        for (int i = 0; i < NX; ++i)
+        for (int i = from; i < to; ++i)
             __builtin_amdgcn_raw_ptr_buffer_load_lds(res, (void __attribute__((address_space(3)))*)(base + (wave + 8 * i) * 1024), 16,
                                                      xoff[i], kk * (MP_BK * 2), 0, 0);
     };
@@ -89,17 +93,17 @@ __device__ __forceinline__ void mp_tile(unsigned char* lds, const bf16* __restri
     __builtin_amdgcn_sched_barrier(0);
     load_w(w[0], 0);
     __builtin_amdgcn_sched_barrier(0);
-    copy_x(0, integral_constant<int, 0>{});
+    copy_x(0, 0, 0, NX);
     __builtin_amdgcn_sched_barrier(0);
     load_w(w[1], 1);
     __builtin_amdgcn_sched_barrier(0);
-    copy_x(1, integral_constant<int, 1>{});
+    copy_x(1, 1, 0, NX);
     __builtin_amdgcn_sched_barrier(0);
     if constexpr (AHEAD > 2) load_w(w[2], 2);
     __builtin_amdgcn_sched_barrier(0);
-    copy_x(2, integral_constant<int, 2>{});
+    if constexpr (!SPREAD) copy_x(2, 2, 0, NX);
     __builtin_amdgcn_sched_barrier(0);
-    mp_wait<4 * (AHEAD - 1) + 2 * NX>();
+    mp_wait<4 * (AHEAD - 1) + (SPREAD ? 1 : 2) * NX>();
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
     mp_bf16x8_t xf[R];
@@ -117,11 +121,18 @@ __device__ __forceinline__ void mp_tile(unsigned char* lds, const bf16* __restri
         for (int i = 0; i < ALL; ++i) {
             if (i == ALL - D) {
                 // the next step's x has landed for everyone; everyone has read the step before this one, whose stage is refilled
-                mp_wait<8 + NX>();
+                mp_wait<(SPREAD ? 4 : 8) + NX>();
                 __builtin_amdgcn_s_barrier();
                 __builtin_amdgcn_sched_barrier(0);
-                copy_x(it + 3, refill);
+                if constexpr (!SPREAD) copy_x(it + 3, refill.value, 0, NX);
                 __builtin_amdgcn_sched_barrier(0);
+            }
+            if constexpr (SPREAD) {
+                constexpr int EACH = (ALL - D) / NX;           // operands between two copies
+                if (i % EACH == EACH - 1 && i / EACH < NX) {
+                    copy_x(it + 2, (slot + 2) & 3, i / EACH, i / EACH + 1);
+                    __builtin_amdgcn_sched_barrier(0);
+                }
             }
             xf[(at + i + D) % R] = i + D < ALL ? read_x(slot_c, i + D) : read_x(next, i + D - ALL);
 #pragma unroll
@@ -200,8 +211,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2))) void m
     // Items are pairs of a row tile and a column tile; workgroups go to the XCDs round-robin. Of every eight row tiles in the plan's
     // order an XCD has an eighth of the items, of what is left too: runs of columns, for all of the tiles of an expert that stand
     // together, so that these share W in L2. As the plan has the large tiles first, the XCDs have about the same work and end
-    // with small tiles: uneven counts (147 to 742), 12,432 pairs, gate-up 609 us; an eighth of all items in a row for each XCD 676,
-    // of all work 631, items taken from a counter of the XCD's 633 and 50 us more for a small product.
+    // with small tiles: uneven counts (147 to 742), 12,432 pairs, gate-up 609 us (592 now); an eighth of all items in a row for each
+    // XCD 676, of all work 631, items taken from a counter of the XCD's 633 and 50 us more for a small product.
     const int tiles_m = meta[0], xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, whole = tiles_m >> 3, rest = (tiles_m & 7) * tiles_n;
     int item;
     if (slot < whole * tiles_n) {
