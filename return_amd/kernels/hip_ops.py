@@ -239,18 +239,22 @@ class HipOps:
     def use_sweep(self, M, N, K, gated):
         """Whether the product that reads W as one sweep through memory (one workgroup per CU, column
         c with workgroup c % CUs) is the rule's choice for x [M, K] and N result columns. Measured on
-        MI355X at 1 to 16 rows: 12 against 15 µs (q/k/v of the 8B shape), 10 against 11 (o), 36 against
-        41 (gate-up), 100 against 118 (gate-up of the 32B shape, K = 5,120) for the x-resident and
-        skinny products; on the output head's 152 thousand rows the x-resident product is ahead (two
-        workgroups per CU hide each other's tile ends), and on few rows of many columns (down: one tile
-        a workgroup, K = 12,288) the library."""
+        MI355X, microseconds by it / by the best other product, at 1, 4, 8 and 16 rows: 151,936 x 4,096 188 / 209, 200 / 215, 206 / 222,
+        215 / 236; 32,000 x 4,096 42 / 49, 43 / 50, 44 / 52, 47 / 56; 6,144 x 4,096 12 / 15 at one row, 4,096 x 4,096 10 / 11; 2,048 x
+        2,048 5.0 / 5.0, 5.3 / 5.4, 5.6 / 5.8, 6.7 / 6.7; 1,024 x 4,096 5.6 / 7.0, 6.1 / 8.3, 6.6 / 9.0, 8.0 / 10.6 (3,072 x 512 4.5 / 2.9: too
+        little to stream). K beyond 4,096: 4,096 x 12,288 19 / 21, 20 / 23, 22 / 23, 26 / 23; 2,560 x 9,728 13 / 18, 13 / 18, 15 / 19,
+        18 / 19; 2,048 x 8,192 10 / 13, 11 / 13, 12 / 13, 15 / 13; 8,192 x 12,288 36 / 42, 37 / 44, 38 / 45, 40 / 44. Gated, 12,288 x
+        4,096 36 against 41 for the x-resident and skinny products, 25,600 x 5,120 100 against 118."""
         if not self.lib.ra_gemm_sweep_fits(M, K):
             return False
         if M > 16 and not gated:             # 17 to 32 rows: 41 to 44 µs against the library's 49 and the SiLU-mul's 5
             return False                     # for gate-up, but q/k/v 17 to 19 against 15, o 14 to 16 against 13
         rows = N * (2 if gated else 1)
-        least = 8 if K <= 4096 or M <= 2 else 32         # rows a workgroup, at least (down at 1 and 2 rows: 20 against 21 to 23 µs)
-        return least * self.cu_count <= rows <= 256 * self.cu_count
+        if gated:
+            return (8 if K <= 4096 or M <= 2 else 32) * self.cu_count <= rows <= 256 * self.cu_count
+        if K <= 4096:
+            return rows >= 4 * self.cu_count and rows * K >= 4 << 20
+        return rows >= (8 if M <= 8 else 32) * self.cu_count         # rows of W a workgroup, at least
 
     def use_resident(self, M, N, K, gated):
         """Whether the product with x resident in LDS beats the skinny product for x [M, K] and
