@@ -5,7 +5,7 @@ The reference fills pinned host arrays and copies them into persistent device
 tensors so that captured graphs replay on fixed addresses (rollout/cache.py:42-70,
 274-328). Here all integer tables of a step live in ONE pinned staging buffer and
 ONE device buffer of fixed layout; a step costs one host-to-device copy for the
-small tables and one per cache group for its page table, and the latter only when a
+small tables, its sampling options among them, and one per cache group for its page table, and the latter only when a
 page list has changed or other requests take part (rollout/cache.py:286-306).
 """
 from __future__ import annotations
@@ -87,6 +87,9 @@ def prefill_tiles(q_lens, q_starts=None, rows=64):
     return tiles
 
 
+FEW = ".few"              # tables by token of a step of one token a request
+
+
 class StepBuilder:
     """Fixed device buffers for the tables of a step, sized for the worst case."""
 
@@ -103,17 +106,23 @@ class StepBuilder:
         self.max_tokens = int(max_step_tokens)
         self.max_requests = int(max_requests)
         T, N, G = self.max_tokens, self.max_requests, len(cache.groups)
-        layout = [("token_ids", T), ("positions", T), ("logit_rows", T), ("cu_q", N + 1),
-                  ("q_start", N), ("seq_lens", N), ("slot_ids", N), ("decode_segs", N),
-                  ("prefill_toks", T)]
-        layout += [(f"prefill_tiles{rows}", 2 * (T // rows + N)) for rows in self.tile_rows]
-        layout += [(f"column_{name}", T) for name in self.token_columns]
+        # First what every step has, by request, with the sampling options, and the tables by token of a step of one token a
+        # request: such a step copies that much. Then the tables by token of any step, and the lists of prompts.
+        by_token = ["token_ids", "positions", "logit_rows"] + [f"column_{name}" for name in self.token_columns] + \
+            [f"slot_mapping{g}" for g in range(G)]
+        layout = [("sampling", 3 * N), ("top_k", N), ("cu_q", N + 1), ("q_start", N), ("seq_lens", N), ("slot_ids", N), ("decode_segs", N)]
         for g in range(G):
-            layout += [(f"slot_mapping{g}", T), (f"cu_pages{g}", N + 1), (f"kv_start{g}", N)]
-        self._small_end = None
+            layout += [(f"cu_pages{g}", N + 1), (f"kv_start{g}", N)]
+        layout += [(name + FEW, N) for name in by_token]
+        few = len(layout)
+        layout += [(name, T) for name in by_token + ["prefill_toks"]]
+        layout += [(f"prefill_tiles{rows}", 2 * (T // rows + N)) for rows in self.tile_rows]
+        self._few_end = self._small_end = None
         self._off = {}
         off = 0
-        for name, size in layout:
+        for i, (name, size) in enumerate(layout):
+            if i == few:
+                self._few_end = off
             self._off[name] = (off, size)
             off += -(-size // 4) * 4          # keep every table 16-byte aligned
         self._small_end = off
@@ -148,11 +157,17 @@ class StepBuilder:
         off, _ = self._off[name]
         return self._dev[off:off + k]
 
+    def sampling_options(self, m: int):
+        """The device's (temperature, top_k, top_p, uniforms) of the first m sampled places, as build() was last given them: views
+        that stay where they are."""
+        f = self._view("sampling", 3 * self.max_requests).view(torch.float32).view(3, self.max_requests)
+        return f[0, :m], self._view("top_k", m), f[1, :m], f[2, :m]
+
     def build(self, tables: StepTables, tokens: Sequence[Sequence[int]],
-              logit_rows: Sequence[int], columns: Optional[dict] = None) -> StepBatch:
+              logit_rows: Sequence[int], columns: Optional[dict] = None, sampling=None) -> StepBatch:
         """tokens[i] are the new tokens of request i; logit_rows index the step's flat token rows;
         columns: name -> T integers for the token columns the builder was made with (a name that is
-        missing gets the tokens' positions)."""
+        missing gets the tokens' positions); sampling: (temperature, top_k, top_p, uniforms), one of each per sampled place."""
         n = len(tables.request_ids)
         T = int(tables.cu_q[-1])
         if T > self.max_tokens:
@@ -165,19 +180,30 @@ class StepBuilder:
         flat = np.fromiter((t for seq in tokens for t in seq), dtype=np.int64, count=T)
         if len(tokens) != n or any(len(seq) != q for seq, q in zip(tokens, tables.q_lens)):
             raise ValueError("tokens do not match the step's q_lens")
-        self._put("token_ids", flat)
-        self._put("positions", tables.positions)
+        # (one token a request, no place wanted twice over: tables by token of max_requests places)
+        few = FEW if T == n and len(logit_rows) <= self.max_requests else ""
+        self._put("token_ids" + few, flat)
+        self._put("positions" + few, tables.positions)
         for name in self.token_columns:
             col = (columns or {}).get(name)
             col = tables.positions if col is None else np.asarray(col, dtype=np.int32)
             if len(col) != T:
                 raise ValueError(f"token column {name!r} has {len(col)} entries for {T} tokens")
-            self._put(f"column_{name}", col)
+            self._put(f"column_{name}{few}", col)
         unknown = set(columns or ()) - set(self.token_columns)
         if unknown:
             raise ValueError(f"token column(s) {sorted(unknown)} are not among those the model reads: "
                              f"{list(self.token_columns)}")
-        m = self._put("logit_rows", np.asarray(logit_rows, dtype=np.int32))
+        m = self._put("logit_rows" + few, np.asarray(logit_rows, dtype=np.int32))
+        if sampling is not None:
+            temperature, top_k, top_p, uniforms = sampling
+            off, N = self._off["sampling"][0], self.max_requests
+            if m > N or any(len(values) != m for values in sampling):
+                raise ValueError(f"sampling options of {[len(values) for values in sampling]} places for {m}, at most {N}")
+            f = self._host_np[off:off + 3 * N].view(np.float32).reshape(3, N)
+            for row, values in zip(f, (temperature, top_p, uniforms)):
+                row[:m] = values
+            self._put("top_k", np.asarray(top_k, dtype=np.int32))
         self._put("cu_q", tables.cu_q)
         self._put("q_start", tables.q_start)
         self._put("seq_lens", tables.seq_lens)
@@ -191,7 +217,7 @@ class StepBuilder:
             self._put("prefill_toks", np.concatenate(
                 [np.arange(tables.cu_q[i], tables.cu_q[i + 1], dtype=np.int32) for i in pre]))
         for g, gt in enumerate(tables.groups):
-            self._put(f"slot_mapping{g}", gt.slot_mapping)
+            self._put(f"slot_mapping{g}{few}", gt.slot_mapping)
             self._put(f"cu_pages{g}", gt.cu_pages)
             self._put(f"kv_start{g}", gt.kv_start)
         tables_there = tables.page_key is not None and tables.page_key == self._tables_on_device
@@ -204,7 +230,8 @@ class StepBuilder:
                 tiles[rows] = prefill_tiles(tables.q_lens, tables.q_start, rows)
                 self._put(f"prefill_tiles{rows}", np.asarray(tiles[rows], dtype=np.int32).reshape(-1))
         # one copy for the small tables, one per group for the used part of its page table
-        self._dev[:self._small_end].copy_(self._host[:self._small_end], non_blocking=True)
+        end = self._few_end if few else self._small_end
+        self._dev[:end].copy_(self._host[:end], non_blocking=True)
         groups = []
         for g, gt in enumerate(tables.groups):
             off, _ = self._off[f"page_table{g}"]
@@ -214,7 +241,7 @@ class StepBuilder:
                 self.page_table_copies += 1
             n_pages = np.diff(gt.cu_pages).tolist()
             groups.append(GroupOnDevice(
-                self._view(f"slot_mapping{g}", T), self._view(f"page_table{g}", k),
+                self._view(f"slot_mapping{g}{few}", T), self._view(f"page_table{g}", k),
                 self._view(f"cu_pages{g}", n + 1), self._view(f"kv_start{g}", n),
                 n_pages, max(n_pages) if n_pages else 0))
         self._tables_on_device = tables.page_key
@@ -223,10 +250,10 @@ class StepBuilder:
             self._copy_pending = True
         return StepBatch(
             n_seqs=n, n_tokens=T,
-            token_ids=self._view("token_ids", T), positions=self._view("positions", T),
+            token_ids=self._view("token_ids" + few, T), positions=self._view("positions" + few, T),
             cu_q=self._view("cu_q", n + 1), q_start=self._view("q_start", n),
             seq_lens=self._view("seq_lens", n), slot_ids=self._view("slot_ids", n),
-            logit_rows=self._view("logit_rows", m), n_logit_rows=m, groups=groups,
+            logit_rows=self._view("logit_rows" + few, m), n_logit_rows=m, groups=groups,
             request_ids=list(tables.request_ids), q_lens=list(tables.q_lens),
             q_starts=tables.q_start.tolist(), cu_q_host=tables.cu_q.tolist(),
             slot_ids_host=tables.slot_ids.tolist(),
@@ -240,4 +267,4 @@ class StepBuilder:
             prefill_segs=pre,
             prefill_tiles={rows: self._view(f"prefill_tiles{rows}", 2 * len(t)).view(-1, 2)
                            for rows, t in tiles.items()},
-            token_columns={name: self._view(f"column_{name}", T) for name in self.token_columns})
+            token_columns={name: self._view(f"column_{name}{few}", T) for name in self.token_columns})

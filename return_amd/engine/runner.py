@@ -81,11 +81,6 @@ class ModelRunner:
         self._graph_pool = None
         n = ec.max_reside
         pin = self.rt.device.type == "cuda"
-        self._samp_host_f = torch.zeros(3, n, dtype=torch.float32, pin_memory=pin)
-        self._samp_host_k = torch.zeros(n, dtype=torch.int32, pin_memory=pin)
-        self._samp_dev_f = torch.zeros(3, n, dtype=torch.float32, device=self.rt.device)
-        self._samp_dev_k = torch.zeros(n, dtype=torch.int32, device=self.rt.device)
-        self._samp_copied = torch.cuda.Event() if pin else None      # the staging above has left for the device
         # Launch and collection of a decode step are two calls, so that the next step can be
         # launched before this one's tokens are read: two pinned result buffers, the tokens of
         # the last launch kept on the device for the next one to pick up.
@@ -95,6 +90,7 @@ class ModelRunner:
         self._feed_dev = torch.zeros(n, dtype=torch.int64, device=self.rt.device)
         self._feed_at_host = torch.zeros(n, dtype=torch.int64, pin_memory=pin)
         self._feed_at_dev = torch.zeros(n, dtype=torch.int64, device=self.rt.device)
+        self._feed_copied = torch.cuda.Event() if pin else None      # the staging of what is fed has left for the device
         self._launches = 0
         self._last_picked: Optional[torch.Tensor] = None
 
@@ -161,9 +157,9 @@ class ModelRunner:
             return None
         return self._run(entries, None)[0]
 
-    def _run(self, entries: Sequence[StepEntry], after_build):
-        """Checks, cache tables, device tables, forward. after_build(batch) runs between the copy
-        of the tables and the model. Returns (logits or None, batch)."""
+    def _run(self, entries: Sequence[StepEntry], after_build, sampling=None):
+        """Checks, cache tables, device tables (with the sampling options, if there are), forward. after_build(batch) runs between
+        the copy of the tables and the model. Returns (logits or None, batch)."""
         rows: List[int] = []
         at = 0
         for e in entries:
@@ -185,7 +181,7 @@ class ModelRunner:
         tables = self.cache.begin_step([(e.request_id, len(e.tokens)) for e in entries])
         try:
             batch = self.builder.build(tables, [[0 if t is None else t for t in e.tokens] for e in entries], rows,
-                                       self._flat_columns([e.columns for e in entries], tables))
+                                       self._flat_columns([e.columns for e in entries], tables), sampling)
             if after_build is not None:
                 after_build(batch)
             with torch.no_grad():
@@ -218,22 +214,22 @@ class ModelRunner:
 
         def take_tokens(batch):
             if feed:
-                if self._samp_copied is not None:
-                    self._samp_copied.synchronize()      # the last launch's copies have left the staging buffers
+                if self._feed_copied is not None:
+                    self._feed_copied.synchronize()      # the last launch's copies have left the staging buffers
                 k = len(feed)
                 starts = batch.cu_q_host
                 self._feed_host[:k] = torch.as_tensor([int(r) for _, r in feed], dtype=torch.int64)
                 self._feed_at_host[:k] = torch.as_tensor([starts[i] for i, _ in feed], dtype=torch.int64)
                 self._feed_dev[:k].copy_(self._feed_host[:k], non_blocking=True)
                 self._feed_at_dev[:k].copy_(self._feed_at_host[:k], non_blocking=True)
+                if self._feed_copied is not None:
+                    self._feed_copied.record()
                 batch.token_ids.index_copy_(0, self._feed_at_dev[:k],
                                             self._last_picked[:, 0].index_select(0, self._feed_dev[:k]))
-            self._put_sampling(m, temperature, top_k, top_p, uniforms)
 
-        logits, _ = self._run(entries, take_tokens)
+        logits, _ = self._run(entries, take_tokens, (temperature, top_k, top_p, uniforms))
         with torch.no_grad():
-            picked = self.rt.ops.sample(logits, self._samp_dev_f[0, :m], self._samp_dev_k[:m],
-                                        self._samp_dev_f[1, :m], self._samp_dev_f[2, :m])
+            picked = self.rt.ops.sample(logits, *self.builder.sampling_options(m))
         return self._ticket(picked, m, logits)
 
     def _ticket(self, picked, n, logits):
@@ -246,24 +242,9 @@ class ModelRunner:
         return (slot, n, logits[:n])
 
     # ------------------------------------------------------------------ decode from a graph
-    def _put_sampling(self, m, temperature, top_k, top_p, uniforms):
-        if self._samp_copied is not None:
-            self._samp_copied.synchronize()          # the last launch's options have left the staging buffer
-        self._samp_host_f[0, :m] = torch.as_tensor(temperature, dtype=torch.float32)
-        self._samp_host_f[1, :m] = torch.as_tensor(top_p, dtype=torch.float32)
-        self._samp_host_f[2, :m] = torch.as_tensor(uniforms, dtype=torch.float32)
-        self._samp_host_k[:m] = torch.as_tensor(top_k, dtype=torch.int32)
-        self._samp_dev_f.copy_(self._samp_host_f, non_blocking=True)
-        self._samp_dev_k.copy_(self._samp_host_k, non_blocking=True)
-        if self._samp_copied is not None:
-            self._samp_copied.record()
-
     def _decode_body(self, batch):
         logits = self.model.forward(batch, self.cache)
-        m = batch.n_logit_rows
-        picked = self.rt.ops.sample(logits, self._samp_dev_f[0, :m], self._samp_dev_k[:m],
-                                    self._samp_dev_f[1, :m], self._samp_dev_f[2, :m])
-        return logits, picked
+        return logits, self.rt.ops.sample(logits, *self.builder.sampling_options(batch.n_logit_rows))
 
     def decode_launch(self, request_ids, tokens, temperature, top_k, top_p, uniforms, feed_rows=None,
                       columns=None):
@@ -303,19 +284,21 @@ class ModelRunner:
         try:
             tables = self.cache.pad_tables(tables, pad)
             host_tokens = [[0]] * rows if tokens is None else [[int(t)] for t in tokens] + [[0]] * pad
+            # (rows that only fill the batch up are chosen greedily and thrown away)
             batch = self.builder.build(tables, host_tokens, list(range(rows)),
-                                       self._flat_columns(list(columns) + [None] * pad, tables) if columns else None)
+                                       self._flat_columns(list(columns) + [None] * pad, tables) if columns else None,
+                                       (list(temperature) + [0.0] * pad, list(top_k) + [0] * pad, list(top_p) + [1.0] * pad,
+                                        list(uniforms) + [0.0] * pad))
             batch.decode_rule = key
             if tokens is None:
                 # after the tables' copy and before the step: the sampled tokens become the new tokens
-                if self._samp_copied is not None:
-                    self._samp_copied.synchronize()      # the last launch's copies have left the staging buffers
+                if self._feed_copied is not None:
+                    self._feed_copied.synchronize()      # the last launch's copies have left the staging buffers
                 self._feed_host[:n] = torch.as_tensor(list(feed_rows), dtype=torch.int64)
                 self._feed_dev[:n].copy_(self._feed_host[:n], non_blocking=True)
+                if self._feed_copied is not None:
+                    self._feed_copied.record()
                 batch.token_ids[:n].copy_(self._last_picked[:, 0].index_select(0, self._feed_dev[:n]))
-            # rows that only fill the batch up are chosen greedily and thrown away
-            self._put_sampling(rows, list(temperature) + [0.0] * pad, list(top_k) + [0] * pad,
-                               list(top_p) + [1.0] * pad, list(uniforms) + [0.0] * pad)
             with torch.no_grad():
                 if graphs:
                     logits, picked = self._replay(key)
