@@ -93,6 +93,46 @@ __device__ __forceinline__ void sweep_scales_make(const SweepNorm& nm, int rows,
     }
 }
 
+// A wave's 512 columns (from k0 on) of up to 16 rows of x, on their way as whole lines: a row is one load of 1 KB, like a row of W, and
+// rows from M on are not asked for. As operands straight from memory (16 rows by 64 bytes a load, once a tile and span) they kept
+// the address unit busy: 4,096 x 12,288 took 21.5 us at 8 rows and 26.0 at 16, now 19.2 and 22.2; 24,576 x 4,096, which reads them
+// once, 37.6 us at 16 rows, now 36.2; 2,048 x 8,192 at 16 rows 13.9, now 11.8. (The kernel of few tiles, which has no registers left
+// for it and reads x once a span, does not.)
+struct SweepX { bf16x8_t r[16]; };
+__device__ __forceinline__ void sweep_x_ask(SweepX& to, const bf16* __restrict__ x, int M, int K, int k0, int lane) {
+    const int k = k0 + lane * 8;
+    auto rows = [&](int from, int end) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (i >= from && i < end)
+                to.r[i] = k < K ? *reinterpret_cast<const bf16x8_t*>(x + (size_t)min(i, M - 1) * K + k) : bf16x8_t{0, 0, 0, 0, 0, 0, 0, 0};
+    };
+    rows(0, 1);
+    if (M > 1) rows(1, 2);
+    if (M > 2) rows(2, 4);
+    if (M > 4) rows(4, 8);
+    if (M > 8) rows(8, 16);
+}
+// Through the wave's part of LDS into B operands: lane (n, g) holds x[n][k0 + 32 j + 8 g ..]. (Rows that were not asked for are
+// whatever LDS held: the results' columns that they make are not used.)
+__device__ __forceinline__ void sweep_x_take(const SweepX& from, uint16_t* stage, int M, int lane, bf16x8_t (&bx)[SW_STEPS]) {
+    SW_WAVE_SYNC();
+    auto rows = [&](int a, int b) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i)
+            if (i >= a && i < b) *reinterpret_cast<bf16x8_t*>(&stage[i * SW_STRIDE + lane * 8]) = from.r[i];
+    };
+    rows(0, 1);
+    if (M > 1) rows(1, 2);
+    if (M > 2) rows(2, 4);
+    if (M > 4) rows(4, 8);
+    if (M > 8) rows(8, 16);
+    SW_WAVE_SYNC();
+#pragma unroll
+    for (int j = 0; j < SW_STEPS; ++j)
+        bx[j] = *reinterpret_cast<const bf16x8_t*>(&stage[(lane & 15) * SW_STRIDE + 32 * j + 8 * (lane >> 4)]);
+}
+
 // MB: blocks of 16 rows of x (1 or 2)
 template <int MB, bool GATED, typename TO, bool RESID = false>
 __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
@@ -125,18 +165,26 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
         const size_t row = (GATED && i >= 8) ? (size_t)N + col : (size_t)col;
         wreg[i] = (k_in && col < N) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + kb + lane * 8)) : zero;
     };
+    // (x first: it comes from nearby, and is made operands while the first rows of W are on their way)
+    [[maybe_unused]] SweepX xs;
+    if constexpr (MB == 1) sweep_x_ask(xs, x, M, K, kb, lane);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 16; ++i) fetch_row(0, i);
 
-    // the wave's columns of x as B operands: lane (n, g) holds x[n][kb + 32j + 8g ..], rows beyond M as zeros
+    // the wave's columns of x as B operands: lane (n, g) holds x[n][kb + 32j + 8g ..]
     bf16x8_t bx[MB][SW_STEPS];
+    if constexpr (MB == 1) {
+        sweep_x_take(xs, stage, M, lane, bx[0]);
+    } else {
 #pragma unroll
-    for (int mb = 0; mb < MB; ++mb)
+        for (int mb = 0; mb < MB; ++mb)
 #pragma unroll
-        for (int j = 0; j < SW_STEPS; ++j) {
-            const int k = kb + 32 * j + 8 * g, m = 16 * mb + n;
-            bx[mb][j] = (m < M && k < K) ? *reinterpret_cast<const bf16x8_t*>(x + (size_t)m * K + k) : zero;
-        }
+            for (int j = 0; j < SW_STEPS; ++j) {
+                const int k = kb + 32 * j + 8 * g, m = 16 * mb + n;
+                bx[mb][j] = (m < M && k < K) ? *reinterpret_cast<const bf16x8_t*>(x + (size_t)m * K + k) : zero;
+            }
+    }
 
     if (scaled) sweep_scales_make(nm, 16 * MB, share, rs);    // (read after the first tile's barrier)
     [[maybe_unused]] float sq = 0.f;                           // RESID: squares of this thread's row over its columns
@@ -251,17 +299,16 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
         const size_t row = (GATED && i >= 8) ? (size_t)N + col : (size_t)col;
         wreg[i] = (k < K && col < N) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + k)) : zero;
     };
+    SweepX xs;                                                 // of the span that comes next
+    sweep_x_ask(xs, x, M, K, kb, lane);
+    __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 16; ++i) fetch_row(0, 0, i);
     [[maybe_unused]] bf16x8_t held[HELD ? 2 : 1][SW_STEPS];
     if constexpr (HELD) {
-#pragma unroll
-        for (int p = 0; p < 2; ++p)
-#pragma unroll
-            for (int j = 0; j < SW_STEPS; ++j) {
-                const int k = p * SW_SPAN + kb + 32 * j + 8 * g;
-                held[p][j] = (n < M && k < K) ? *reinterpret_cast<const bf16x8_t*>(x + (size_t)n * K + k) : zero;
-            }
+        sweep_x_take(xs, stage, M, lane, held[0]);
+        sweep_x_ask(xs, x, M, K, SW_SPAN + kb, lane);
+        sweep_x_take(xs, stage, M, lane, held[1]);
     }
     if (scaled) sweep_scales_make(nm, 16, share, rs);
     [[maybe_unused]] float sq = 0.f;
@@ -277,18 +324,16 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
 #pragma unroll
         for (int p = 0; p < (HELD ? 2 : spans); ++p) {
             bf16x8_t bx[SW_STEPS];                              // the span's columns of x as B operands
-#pragma unroll
-            for (int j = 0; j < SW_STEPS; ++j) {
-                if constexpr (HELD) {
-                    bx[j] = held[p][j];
-                } else {
-                    const int k = p * SW_SPAN + kb + 32 * j + 8 * g;
-                    bx[j] = (n < M && k < K) ? *reinterpret_cast<const bf16x8_t*>(x + (size_t)n * K + k) : zero;
-                }
-            }
-            SW_WAVE_SYNC();
             const bool more = p + 1 < spans || t + 1 < n_tiles;
             const int t_next = p + 1 < spans ? t : t + 1, p_next = p + 1 < spans ? p + 1 : 0;
+            if constexpr (HELD) {
+#pragma unroll
+                for (int j = 0; j < SW_STEPS; ++j) bx[j] = held[p][j];
+            } else {
+                sweep_x_take(xs, stage, M, lane, bx);
+                if (more) sweep_x_ask(xs, x, M, K, p_next * SW_SPAN + kb, lane);     // (in front of the rows of W that it goes with)
+            }
+            SW_WAVE_SYNC();
 #pragma unroll
             for (int i = 0; i < 16; ++i) {
                 *reinterpret_cast<bf16x8_t*>(&stage[i * SW_STRIDE + lane * 8]) = wreg[i];
