@@ -3,8 +3,7 @@
 // Layout as in the reference's F.linear (rollout/monkey_patch/qwen3.py:21): x [M, K], W [N, K],
 // y [M, N].
 //
-// One workgroup of eight waves per CU. Result column c belongs to workgroup c % gridDim, so that at
-// any time the workgroups together read gridDim consecutive rows of W, one contiguous run of memory
+// One workgroup of eight waves per CU. At any time the workgroups together read one contiguous run of rows of W
 // (measured here: such a sweep reads 201 MB in 31 µs; the same bytes as 16 rows x 512 B per wave,
 // the order of an MFMA operand read straight from memory, take 35 µs). Wave w has columns
 // 512w .. 512w+511 of K: a row of W is one load of 1 KB per wave, sixteen rows (a tile) are on their
@@ -133,6 +132,33 @@ __device__ __forceinline__ void sweep_x_take(const SweepX& from, uint16_t* stage
         bx[j] = *reinterpret_cast<const bf16x8_t*>(&stage[(lane & 15) * SW_STRIDE + 32 * j + 8 * (lane >> 4)]);
 }
 
+// Which result columns a workgroup has.
+// NEAR (one span): of every whole round of G COLS columns its COLS neighbouring ones, and an even share of neighbouring ones (at most
+// COLS) of what is left; workgroups whose columns adjoin are on one XCD (workgroups go to the eight in turn), so that the lines
+// of y become whole in its L2. As every G-th column, y was written in pieces of one entry and every line by all XCDs: 151,936 x
+// 4,096 took 208 us at 8 rows and 220 at 16, now 191 and 197 (with neighbouring columns, but workgroups in plain order, 205
+// and 208); 24,576 x 4,096 at 16 rows 36.2, now 34.8; others the same within 0.2 us.
+// Otherwise (several spans, where a round is more of W and less of y) every G-th column: 4,096 x 12,288 18.3, 19.2 and 22.2 us at 1, 8 and
+// 16 rows, with the columns above 18.5, 19.6 and 22.4.
+template <int COLS, bool NEAR> struct SweepCols {
+    int N, G, b, n_tiles;
+    int full = 0, left = 0, share = 0;
+    __device__ __forceinline__ SweepCols(int N) : N(N), G(gridDim.x), b(blockIdx.x) {
+        if constexpr (NEAR) {
+            if (G % 8 == 0) b = (b & 7) * (G >> 3) + (b >> 3);
+            full = N / (G * COLS);
+            const int rest = N - full * G * COLS, each = rest / G, over = rest - each * G;
+            left = full * G * COLS + b * each + min(b, over);
+            share = each + (b < over);
+            n_tiles = full + (share > 0);
+        } else {
+            n_tiles = N > b ? ((N - 1 - b) / G + COLS) / COLS : 0;
+        }
+    }
+    __device__ __forceinline__ int at(int t, int i) const { return NEAR ? (t < full ? (t * G + b) * COLS : left) + i : b + G * (t * COLS + i); }
+    __device__ __forceinline__ bool has(int t, int i) const { return NEAR ? t < full || i < share : at(t, i) < N; }
+};
+
 // MB: blocks of 16 rows of x (1 or 2)
 template <int MB, bool GATED, typename TO, bool RESID = false>
 __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
@@ -146,9 +172,8 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
     uint16_t* stage = reinterpret_cast<uint16_t*>(lds_raw) + (size_t)wave * 16 * SW_STRIDE;
     float* red_both = reinterpret_cast<float*>(lds_raw + (size_t)SW_WAVES * 16 * SW_STRIDE * 2);   // [1 or 2][wave][16 rows][RS]
     float* rs = red_both + 2 * SW_WAVES * 16 * 17;            // [32] row scales, behind the result tiles
-    const int G = gridDim.x, b = blockIdx.x;
-    const int my_cols = N > b ? (N - 1 - b) / G + 1 : 0;
-    const int n_tiles = (my_cols + COLS - 1) / COLS;
+    const SweepCols<COLS, true> cols(N);
+    const int n_tiles = cols.n_tiles;
     if (n_tiles == 0) return;                                   // (the launch keeps the grid within N)
     const int kb = wave * SW_KW;
     const bool k_in = kb + lane * 8 < K;                        // K % 8 == 0: a lane's 8 columns are in or out together
@@ -158,12 +183,12 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
     float share[SW_SHARES];
     if (scaled) sweep_scales_ask(nm, M, share);
 
-    // row i of tile t: column b + G (COLS t + i % COLS), GATED: rows 8.. are the up rows
+    // row i of tile t: its column i % COLS, GATED: rows 8.. are the up rows
     bf16x8_t wreg[16];
     auto fetch_row = [&](int t, int i) {
-        const int col = b + G * (t * COLS + (GATED ? (i & 7) : i));
+        const int place = GATED ? (i & 7) : i, col = cols.at(t, place);
         const size_t row = (GATED && i >= 8) ? (size_t)N + col : (size_t)col;
-        wreg[i] = (k_in && col < N) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + kb + lane * 8)) : zero;
+        wreg[i] = (k_in && cols.has(t, place)) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + kb + lane * 8)) : zero;
     };
     // (x first: it comes from nearby, and is made operands while the first rows of W are on their way)
     [[maybe_unused]] SweepX xs;
@@ -196,7 +221,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
         // under no condition; what lies outside the result is not used.
         [[maybe_unused]] float h_old = 0.f, wn = 0.f;
         if constexpr (RESID) {
-            const int mm = min(tid / COLS, M - 1), col = min(b + G * (t * COLS + tid % COLS), N - 1);
+            const int mm = min(tid / COLS, M - 1), col = min(cols.at(t, tid % COLS), N - 1);
             h_old = nm.h[(size_t)mm * N + col];
             wn = nm.w_next[col];
         }
@@ -231,8 +256,8 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
         __syncthreads();
         if (tid < 16 * MB * COLS) {
             const int mm = tid / COLS, r = tid % COLS;        // r fastest: neighbours write neighbours' columns
-            const int col = b + G * (t * COLS + r);
-            if (mm < M && col < N) {
+            const int col = cols.at(t, r);
+            if (mm < M && cols.has(t, r)) {
                 float s = 0.f;
 #pragma unroll
                 for (int w = 0; w < SW_WAVES; ++w) s += red[(w * 16 + r) * RS + mm];
@@ -262,7 +287,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
         if (tid < 16 * COLS) {
 #pragma unroll
             for (int o = 8; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 16);
-            if ((tid & 15) == 0 && (tid >> 4) < M) nm.psq_out[(size_t)(tid >> 4) * G + b] = sq;
+            if ((tid & 15) == 0 && (tid >> 4) < M) nm.psq_out[(size_t)(tid >> 4) * cols.G + cols.b] = sq;
         }
     }
 }
@@ -281,10 +306,9 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
     uint16_t* stage = reinterpret_cast<uint16_t*>(lds_raw) + (size_t)wave * 16 * SW_STRIDE;
     float* red_both = reinterpret_cast<float*>(lds_raw + (size_t)SW_WAVES * 16 * SW_STRIDE * 2);
     float* rs = red_both + 2 * SW_WAVES * 16 * 17;
-    const int G = gridDim.x, b = blockIdx.x;
-    const int my_cols = N > b ? (N - 1 - b) / G + 1 : 0;
-    const int n_tiles = (my_cols + COLS - 1) / COLS;
-    if (n_tiles == 0) return;
+    const SweepCols<COLS, false> cols(N);
+    const int n_tiles = cols.n_tiles;
+    if (n_tiles == 0) return;                                   // (the launch keeps the grid within N)
     const int spans = (K + SW_SPAN - 1) / SW_SPAN;
     const int kb = wave * SW_KW;
     const bf16x8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -295,9 +319,9 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
     bf16x8_t wreg[16];
     auto fetch_row = [&](int t, int p, int i) {
         const int k = p * SW_SPAN + kb + lane * 8;
-        const int col = b + G * (t * COLS + (GATED ? (i & 7) : i));
+        const int place = GATED ? (i & 7) : i, col = cols.at(t, place);
         const size_t row = (GATED && i >= 8) ? (size_t)N + col : (size_t)col;
-        wreg[i] = (k < K && col < N) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + k)) : zero;
+        wreg[i] = (k < K && cols.has(t, place)) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + k)) : zero;
     };
     SweepX xs;                                                 // of the span that comes next
     sweep_x_ask(xs, x, M, K, kb, lane);
@@ -316,7 +340,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
     for (int t = 0; t < n_tiles; ++t) {
         [[maybe_unused]] float h_old = 0.f, wn = 0.f;          // (asked for before the tile's loads of W, as in the kernel above)
         if constexpr (RESID) {
-            const int mm = min(tid / COLS, M - 1), col = min(b + G * (t * COLS + tid % COLS), N - 1);
+            const int mm = min(tid / COLS, M - 1), col = min(cols.at(t, tid % COLS), N - 1);
             h_old = nm.h[(size_t)mm * N + col];
             wn = nm.w_next[col];
         }
@@ -353,8 +377,8 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
         __syncthreads();
         if (tid < 16 * COLS) {
             const int mm = tid / COLS, r = tid % COLS;
-            const int col = b + G * (t * COLS + r);
-            if (mm < M && col < N) {
+            const int col = cols.at(t, r);
+            if (mm < M && cols.has(t, r)) {
                 float s = 0.f;
 #pragma unroll
                 for (int w = 0; w < SW_WAVES; ++w) s += red[(w * 16 + r) * 17 + mm];
@@ -382,7 +406,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
         if (tid < 16 * COLS) {
 #pragma unroll
             for (int o = 8; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 16);
-            if ((tid & 15) == 0 && (tid >> 4) < M) nm.psq_out[(size_t)(tid >> 4) * G + b] = sq;
+            if ((tid & 15) == 0 && (tid >> 4) < M) nm.psq_out[(size_t)(tid >> 4) * cols.G + cols.b] = sq;
         }
     }
 }
@@ -403,10 +427,9 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_spans_kernel(
     uint16_t* stage = reinterpret_cast<uint16_t*>(lds_raw) + (size_t)wave * 16 * SW_STRIDE;
     float* red_both = reinterpret_cast<float*>(lds_raw + (size_t)SW_WAVES * 16 * SW_STRIDE * 2);
     float* rs = red_both + 2 * SW_WAVES * 16 * 17;
-    const int G = gridDim.x, b = blockIdx.x;
-    const int my_cols = N > b ? (N - 1 - b) / G + 1 : 0;
-    const int n_tiles = (my_cols + COLS - 1) / COLS;          // (the launch keeps it within SW_FEW_TILES)
-    if (n_tiles == 0) return;
+    const SweepCols<COLS, false> cols(N);
+    const int n_tiles = cols.n_tiles;                           // (the launch keeps it within SW_FEW_TILES)
+    if (n_tiles == 0) return;                                   // (the launch keeps the grid within N)
     const int spans = (K + SW_SPAN - 1) / SW_SPAN;
     const int kb = wave * SW_KW;
     const bf16x8_t zero = {0, 0, 0, 0, 0, 0, 0, 0};
@@ -417,9 +440,9 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_spans_kernel(
     bf16x8_t wreg[16];
     auto fetch_row = [&](int t, int p, int i) {
         const int k = p * SW_SPAN + kb + lane * 8;
-        const int col = b + G * (t * COLS + (GATED ? (i & 7) : i));
+        const int place = GATED ? (i & 7) : i, col = cols.at(t, place);
         const size_t row = (GATED && i >= 8) ? (size_t)N + col : (size_t)col;
-        wreg[i] = (k < K && col < N) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + k)) : zero;
+        wreg[i] = (k < K && cols.has(t, place)) ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8_t*>(W + row * K + k)) : zero;
     };
 #pragma unroll
     for (int i = 0; i < 16; ++i) fetch_row(0, 0, i);
@@ -436,7 +459,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_spans_kernel(
             if (p == spans - 1) {
 #pragma unroll
                 for (int t = 0; t < SW_FEW_TILES; ++t) {
-                    const int mm = min(tid / COLS, M - 1), col = min(b + G * (min(t, n_tiles - 1) * COLS + tid % COLS), N - 1);
+                    const int mm = min(tid / COLS, M - 1), col = min(cols.at(min(t, n_tiles - 1), tid % COLS), N - 1);
                     h_old[t] = nm.h[(size_t)mm * N + col];
                     wn[t] = nm.w_next[col];
                 }
@@ -478,8 +501,8 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_spans_kernel(
         __syncthreads();
         if (tid < 16 * COLS) {
             const int mm = tid / COLS, r = tid % COLS;
-            const int col = b + G * (t * COLS + r);
-            if (mm < M && col < N) {
+            const int col = cols.at(t, r);
+            if (mm < M && cols.has(t, r)) {
                 float s = 0.f;
 #pragma unroll
                 for (int w = 0; w < SW_WAVES; ++w) s += red[(w * 16 + r) * 17 + mm];
@@ -507,7 +530,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_spans_kernel(
         if (tid < 16 * COLS) {
 #pragma unroll
             for (int o = 8; o > 0; o >>= 1) sq += __shfl_xor(sq, o, 16);
-            if ((tid & 15) == 0 && (tid >> 4) < M) nm.psq_out[(size_t)(tid >> 4) * G + b] = sq;
+            if ((tid & 15) == 0 && (tid >> 4) < M) nm.psq_out[(size_t)(tid >> 4) * cols.G + cols.b] = sq;
         }
     }
 }

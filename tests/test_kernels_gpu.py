@@ -227,9 +227,11 @@ def test_resident_product(ops, ref, M, N, K, grid):
 
 @pytest.mark.parametrize("gated", [False, True])
 @pytest.mark.parametrize("N,K", [(6144, 4096), (2500, 2560), (700, 4096), (4099, 520), (37, 64), (4096, 12288), (300, 9728),
-                                 (5200, 4104), (1100, 5120), (300, 8192), (5120, 12288), (15000, 8200)])
+                                 (5200, 4104), (1100, 5120), (300, 8192), (5120, 12288), (15000, 8200),
+                                 (4096, 72), (4097, 72), (2303, 72)])
 def test_product_that_sweeps_the_weight(ops, N, K, gated):
-    """The product that reads W as one sweep (column c with workgroup c % CUs): widths that fill
+    """The product that reads W as one sweep (rounds of 16 columns a workgroup that end in whole ones,
+    one column over and part ones): widths that fill
     every wave's 512 columns and widths that leave waves idle, widths of several spans of 4,096 (whole
     ones and one that ends after 8 columns; up to two spans x stays in registers, beyond it is read
     per span, and once for all tiles where a workgroup has two to four of them), column counts that are no multiple of
