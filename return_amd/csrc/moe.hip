@@ -586,9 +586,8 @@ extern "C" int ra_moe_product(const void* x, const void* w, void* y, const int* 
 
 // The same with w laid out in panels (moe_tile.h). tile_rows: 16 or MOE_PANEL_ROWS, as ra_moe_panel_rows says: from two pairs an
 // expert on nearly every expert has one, and the tiles' longer reads are the faster ones; with fewer they are not enough tiles for
-// the CUs. 32 experts, gate-up and down, sweep / tiles, us: of 6,144 x 4,096, 8 tokens 188 + 101 / 211 + 103, 16 tokens 265 + 136 /
-// 249 + 128, 64 tokens 285 + 150 / 258 + 133; of 4,096 x 2,048, 8 tokens 67 + 34 / 73 + 36, 16 tokens 91 + 47 / 89 + 48, 64 tokens 102 +
-// 56 / 91 + 50.
+// the CUs. 32 experts of 6,144 x 4,096, four a token, gate-up and down, sweep / tiles, us: 8 tokens 167 + 87 / 193 + 94, 16 tokens 234 + 115 /
+// 222 + 114, 32 tokens 244 + 121 / 230 + 117; of 4,096 x 2,048, tiles, 16 tokens 80 + 42, 64 tokens 82 + 43.
 extern "C" int ra_moe_panel_rows(int n_pairs, int E) { return n_pairs >= 2 * E ? MOE_PANEL_ROWS : 16; }
 
 extern "C" int ra_moe_panel_product(const void* x, const void* w, void* y, const int* order, const int* tiles, const int* meta,

@@ -237,14 +237,14 @@ class HipOps:
         return M <= 4 or (M <= 16 and N * K <= (32 << 20)) or (M <= 32 and N * K <= (16 << 20))
 
     def use_sweep(self, M, N, K, gated):
-        """Whether the product that reads W as one sweep through memory (one workgroup per CU, column
-        c with workgroup c % CUs) is the rule's choice for x [M, K] and N result columns. Measured on
-        MI355X, microseconds by it / by the best other product, at 1, 4, 8 and 16 rows: 151,936 x 4,096 188 / 209, 200 / 215, 206 / 222,
-        215 / 236; 32,000 x 4,096 42 / 49, 43 / 50, 44 / 52, 47 / 56; 6,144 x 4,096 12 / 15 at one row, 4,096 x 4,096 10 / 11; 2,048 x
-        2,048 5.0 / 5.0, 5.3 / 5.4, 5.6 / 5.8, 6.7 / 6.7; 1,024 x 4,096 5.6 / 7.0, 6.1 / 8.3, 6.6 / 9.0, 8.0 / 10.6 (3,072 x 512 4.5 / 2.9: too
-        little to stream). K beyond 4,096: 4,096 x 12,288 19 / 21, 20 / 23, 22 / 23, 26 / 23; 2,560 x 9,728 13 / 18, 13 / 18, 15 / 19,
-        18 / 19; 2,048 x 8,192 10 / 13, 11 / 13, 12 / 13, 15 / 13; 8,192 x 12,288 36 / 42, 37 / 44, 38 / 45, 40 / 44. Gated, 12,288 x
-        4,096 36 against 41 for the x-resident and skinny products, 25,600 x 5,120 100 against 118."""
+        """Whether the product that reads W as one sweep through memory (one workgroup per CU) is the rule's
+        choice for x [M, K] and N result columns. Measured on MI355X, microseconds by it / by the best other product, at 1, 4, 8
+        and 16 rows: 151,936 x 4,096 188 / 209, 189 / 214, 192 / 221, 195 / 233; 32,000 x 4,096 43 / 48, 43 / 50, 43 / 51, 44 / 59; 6,144 x
+        4,096 11.3 / 14.2, 11.4 / 14.5, 11.8 / 15.2, 11.9 / 14.3; 4,096 x 4,096 8.7 / 9.1, 8.8 / 10.2, 8.5 / 10.6, 9.4 / 11.9; 2,048 x 2,048
+        4.8 / 5.0, 5.0 / 5.4, 5.2 / 5.8, 5.6 / 6.6; 1,024 x 4,096 5.2 / 6.9, 5.4 / 8.3, 6.0 / 9.0, 6.8 / 10.6 (3,072 x 512 4.5 / 2.9: too little to
+        stream). K beyond 4,096: 4,096 x 12,288 18.4 / 22.3, 17.7 / 21.2, 18.7 / 21.2, 21.3 / 21.7; 2,560 x 9,728 12.1 / 17.5, 12.8 / 15.6,
+        13.1 / 15.6, 15.6 / 16.0; 2,048 x 8,192 9.2 / 12.7, 9.2 / 12.6, 10.0 / 12.6, 11.6 / 12.9; 8,192 x 12,288 36 / 42, 36 / 43, 37 / 44,
+        41 / 44. Gated, 12,288 x 4,096 34 against 41 for the x-resident and skinny products, 25,600 x 5,120 100 against 118."""
         if not self.lib.ra_gemm_sweep_fits(M, K):
             return False
         if M > 16 and not gated:             # 17 to 32 rows: 41 to 44 µs against the library's 49 and the SiLU-mul's 5
@@ -254,7 +254,7 @@ class HipOps:
             return (8 if K <= 4096 or M <= 2 else 32) * self.cu_count <= rows <= 256 * self.cu_count
         if K <= 4096:
             return rows >= 4 * self.cu_count and rows * K >= 4 << 20
-        return rows >= (8 if M <= 8 else 32) * self.cu_count         # rows of W a workgroup, at least
+        return rows >= 8 * self.cu_count                      # rows of W a workgroup, at least
 
     def use_resident(self, M, N, K, gated):
         """Whether the product with x resident in LDS beats the skinny product for x [M, K] and
