@@ -167,7 +167,8 @@ class StepBuilder:
               logit_rows: Sequence[int], columns: Optional[dict] = None, sampling=None) -> StepBatch:
         """tokens[i] are the new tokens of request i; logit_rows index the step's flat token rows;
         columns: name -> T integers for the token columns the builder was made with (a name that is
-        missing gets the tokens' positions); sampling: (temperature, top_k, top_p, uniforms), one of each per sampled place."""
+        missing gets the tokens' positions); sampling: (temperature, top_k, top_p, uniforms), one of each per sampled place
+        or one for all of them."""
         n = len(tables.request_ids)
         T = int(tables.cu_q[-1])
         if T > self.max_tokens:
@@ -196,14 +197,17 @@ class StepBuilder:
                              f"{list(self.token_columns)}")
         m = self._put("logit_rows" + few, np.asarray(logit_rows, dtype=np.int32))
         if sampling is not None:
-            temperature, top_k, top_p, uniforms = sampling
+            # (whatever torch makes a tensor of, on any device)
+            options = [torch.as_tensor(values, dtype=torch.int32 if i == 1 else torch.float32).detach().cpu().numpy()
+                       for i, values in enumerate(sampling)]
             off, N = self._off["sampling"][0], self.max_requests
-            if m > N or any(len(values) != m for values in sampling):
-                raise ValueError(f"sampling options of {[len(values) for values in sampling]} places for {m}, at most {N}")
+            if m > N or any(o.size not in (1, m) for o in options):
+                raise ValueError(f"sampling options of {[o.size for o in options]} places for {m}, at most {N}")
+            temperature, top_k, top_p, uniforms = options
             f = self._host_np[off:off + 3 * N].view(np.float32).reshape(3, N)
-            for row, values in zip(f, (temperature, top_p, uniforms)):
-                row[:m] = values
-            self._put("top_k", np.asarray(top_k, dtype=np.int32))
+            for row, o in zip(f, (temperature, top_p, uniforms)):
+                row[:m] = o
+            self._put("top_k", np.broadcast_to(top_k, (m,)))
         self._put("cu_q", tables.cu_q)
         self._put("q_start", tables.q_start)
         self._put("seq_lens", tables.seq_lens)

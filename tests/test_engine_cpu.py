@@ -430,3 +430,25 @@ def test_the_engine_checks_the_cache_after_every_step_when_asked(folder_a):
                 runner.step([StepEntry("r", toks[10:12], [])])
         else:
             runner.step([StepEntry("r", toks[10:12], [])])
+
+
+def test_one_sampling_option_stands_for_all_places(folder_a):
+    """A launch takes options as numbers, arrays and tensors, and one for every place as one for all of them."""
+    reqs = {"a": tt.random_tokens(TINY_A["vocab_size"], 5, seed=1), "b": tt.random_tokens(TINY_A["vocab_size"], 9, seed=2)}
+
+    def run(of_step, of_decode):
+        runner = runner_for(folder_a, 128)
+        for rid in reqs:
+            runner.add_request(rid)
+        prompts = [StepEntry(rid, toks, [len(toks) - 1]) for rid, toks in reqs.items()]
+        first = runner.decode_collect(runner.step_launch(prompts, *of_step))
+        return first, runner.decode_collect(runner.decode_launch(list(reqs), first[0], *of_decode))
+
+    whole = ([0.7, 0.7], [5, 5], [0.9, 0.9], [0.3, 0.3])
+    want = run(whole, whole)
+    assert run(([0.7, 0.7], 5, 0.9, [0.3]), ([0.7], [5], [0.9], [0.3])) == want
+    arrays = (torch.tensor([0.7, 0.7], dtype=torch.float64).numpy(), torch.tensor([5]), torch.tensor(0.9), torch.tensor([0.3, 0.3]))
+    assert run(arrays, [torch.tensor(v) for v in whole]) == want
+    for wrong in (([0.7, 0.7], [5, 5, 5], [0.9, 0.9], [0.3, 0.3]), ([0.7], [5, 5], [0.9, 0.9], [0.3, 0.3])):
+        with pytest.raises(ValueError):
+            run(wrong, whole)
