@@ -449,6 +449,8 @@ def test_one_sampling_option_stands_for_all_places(folder_a):
     assert run(([0.7, 0.7], 5, 0.9, [0.3]), ([0.7], [5], [0.9], [0.3])) == want
     arrays = (torch.tensor([0.7, 0.7], dtype=torch.float64).numpy(), torch.tensor([5]), torch.tensor(0.9), torch.tensor([0.3, 0.3]))
     assert run(arrays, [torch.tensor(v) for v in whole]) == want
+    half = (torch.tensor([0.5, 0.5], dtype=torch.bfloat16), torch.tensor([5, 5]), torch.tensor(0.75, requires_grad=True), [0.25] * 2)
+    assert run(half, whole) == run(([0.5] * 2, [5] * 2, [0.75] * 2, [0.25] * 2), whole)
     for wrong in (([0.7, 0.7], [5, 5, 5], [0.9, 0.9], [0.3, 0.3]), ([0.7], [5, 5], [0.9, 0.9], [0.3, 0.3])):
         with pytest.raises(ValueError):
             run(wrong, whole)
