@@ -201,8 +201,12 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
     const int first = (int)(sum >> 32);
     if (tid < E) {
         int tl = (int)(sum & 0xffffffffull);
-        const int per = moe_rows_of_tile(n, rows);
+        // runs: of an expert's groups of 16 rows every tile has as many, or one fewer, so that where there are several tiles none has
+        // fewer than ten groups (of 3,649 rows the last of twelve had nine; it read W, which the others share, past the caches)
+        int per = moe_rows_of_tile(n, rows);
+        const int full = runs && own_tiles > 1 ? ((n + 15) >> 4) - (per / 16 - 1) * own_tiles : own_tiles;
         for (int i = 0, j = 0; i < n; i += per, ++tl, ++j) {
+            if (j == full) per -= 16;
             tiles[3 * tl] = e;
             tiles[3 * tl + 1] = first + i;
             // (runs of up to four tiles of an expert: their number and the tile's place among them ride along)

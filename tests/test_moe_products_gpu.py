@@ -89,3 +89,33 @@ def test_panels_many_rows(ops, E, H, I, counts, kind):
 @pytest.mark.parametrize("kind", KINDS)
 def test_panels_few_rows(ops, E, H, I, counts, kind):
     check(ops, 16, E, H, I, shuffled(counts), kind, panels=True)
+
+
+@pytest.mark.parametrize("E,counts", [
+    (3, [3649, 40, 0]), (1, [6081]), (2, [321, 320]), (4, [1700, 3300, 1281, 640]), (130, [1] * 60 + [700, 0, 1601] + [17] * 67),
+    (200, [330, 0, 2, 16] * 50), (1024, [0] * 1000 + [400] * 24)])
+def test_plan_of_tiles_of_panels(ops, E, counts):
+    """Every pair stands once, with its expert's; an expert's tiles are as few as 320 rows allow, even within a group of 16 rows, so
+    that of several none has fewer than ten groups; the largest tiles come first; runs of up to four of an expert's tiles are numbered."""
+    ids = shuffled(counts)
+    order, tiles, meta, most, _ = ops._moe_plan(ids.int().to(DEV), E, 320)
+    n = int(meta)
+    order, tiles = order.cpu(), tiles[:n].cpu().tolist()
+    assert n == sum(-(-c // 320) for c in counts) <= most and order.sort().values.tolist() == list(range(len(ids)))
+    at, first_of = 0, []
+    while tiles:
+        e = tiles[0][0]
+        of_e = [t for t in tiles if t[0] == e]
+        assert tiles[:len(of_e)] == of_e and len(of_e) == -(-counts[e] // 320)
+        first_of.append(of_e[0][2] & 0xffff)
+        groups = []
+        for j, (_, start, packed) in enumerate(of_e):
+            rows = packed & 0xffff
+            assert start == at and packed >> 16 == min(len(of_e) - (j & ~3), 4) * 16 + (j & 3)
+            assert (ids[order[at:at + rows].long()] == e).all()
+            at += rows
+            groups.append(-(-rows // 16))
+        assert at - of_e[0][1] == counts[e] and max(groups) <= 20
+        assert max(groups) - min(groups) <= 1 and (len(of_e) == 1 or min(groups) >= 10), (counts[e], groups)
+        tiles = tiles[len(of_e):]
+    assert at == len(ids) and first_of == sorted(first_of, reverse=True)
