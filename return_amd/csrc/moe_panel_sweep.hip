@@ -3,7 +3,8 @@
 // An item is 16 result columns of a tile of up to 16 pairs of one expert: a panel of W, or one of gate and one of up rows. All items
 // stand in a row and every workgroup has an equal share of them, across tiles. Wave w has an eighth of K: its part of an item
 // comes straight into MFMA operands, 1 KB a load, and a register is asked for again for the next item as soon as its MFMA has been
-// issued, so that 64 to 256 KB a CU are always on their way; its part of the tile's rows of x stays in registers. The waves'
+// issued, so that a workgroup has a whole item, 64 K bytes gated and 32 K not, always on its way (of one workgroup a CU, up to K of
+// 2,048 of two: 256 KB a CU at K of 2,048 and 4,096 gated, 32 KB at K of 512 not gated); its part of the tile's rows of x stays in registers. The waves'
 // results are added through LDS in wave order; the barrier for that waits for no load.
 //
 // Bound by the reading of W, which goes past the caches (nontemporal). Measured, gate-up and down of 32 experts, four a token, with rows
@@ -37,13 +38,22 @@ __global__ __launch_bounds__(64 * MQ_WAVES) __attribute__((amdgpu_waves_per_eu(K
     const int items = N >> 4, nk = K >> 6, w_bytes = NP * N * K * 2, kstep = NP * N * 128, x_bytes = x_rows * K * 2;
     const int k0 = wave * nk / MQ_WAVES, k_n = (wave + 1) * nk / MQ_WAVES - k0;
     const long long total = (long long)meta[0] * items;
-    long long at = total * blockIdx.x / gridDim.x;
-    const long long end = total * (blockIdx.x + 1) / gridDim.x;
+    // Of fewer items than workgroups every eighth share, say, has one, and as workgroups go to the XCDs in turn, all of them would be
+    // on one XCD (the 64 items of gate-up of 8 experts of 1,024 x 2,048, 2 pairs: both products and the plan 19.5 us, with the shares
+    // in an XCD's order 17.2). With more items plain order is up to 5 % the faster one.
+    const int G = gridDim.x, b = total < G && G % 8 == 0 ? (blockIdx.x & 7) * (G >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+    long long at = total * b / G;
+    const long long end = total * (b + 1) / G;
     if (at >= end) return;                                     // (the same in every thread)
     int tile = (int)(at / items), item = (int)(at - (long long)tile * items);
     mq_bf16x8_t wf[KW][2][NP], xf[KW][2];
     const size_t w_size = (size_t)NP * N * K;
     const bf16* wt = w + (size_t)tiles[3 * tile] * w_size;     // W of the tile that is read from
+    // (the first tile's pairs are asked for before its W: loads come back in order, and the rows of x that they name would wait for all
+    // of W: 0.3 to 0.5 us a product where a workgroup has an item or two)
+    auto pairs_of = [&](int t) { return order[tiles[3 * t + 1] + (n < tiles[3 * t + 2] ? n : 0)]; };
+    int pair = pairs_of(tile);
+    __builtin_amdgcn_sched_barrier(0);
     // (steps that the wave does not have, and what lies behind the last item, are read from buffers of no length: zeros)
     auto fetch = [&](int j, int h, int i, bool in) {
         const __amdgpu_buffer_rsrc_t res = __builtin_amdgcn_make_buffer_rsrc((void*)wt, 0, in && j < k_n ? w_bytes : 0, 0x00020000);
@@ -64,9 +74,10 @@ __global__ __launch_bounds__(64 * MQ_WAVES) __attribute__((amdgpu_waves_per_eu(K
         if (tile != have) {
             // lane (n, g) holds x[row n][64 (k0 + j) + 32 h + 8 g ..]; lanes of rows that the tile does not have hold its first
             // row, whose results are not used
+            if (have >= 0) pair = pairs_of(tile);
             have = tile;
             n_rows = tiles[3 * tile + 2];
-            const int pair = order[tiles[3 * tile + 1] + (n < n_rows ? n : 0)], row = pair / top_div;
+            const int row = pair / top_div;
             pairs_in ^= 1;                                     // (the tile before: its last results may still be read)
             if (tid < 16) {
                 pair_both[pairs_in][tid] = pair;
