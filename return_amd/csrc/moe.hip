@@ -126,9 +126,13 @@ extern "C" int ra_moe_route(const float* z, const float* bias, int T, int E, int
 }
 
 // ------------------------------------------------------------------ plan: one workgroup
+// Tiles of matrices in panels are 320, 160 or 80 rows at most; no other tiles are.
+__host__ __device__ __forceinline__ bool moe_panel_height(int rows) {
+    return rows == MOE_PANEL_ROWS || rows == MOE_PANEL_ROWS / 2 || rows == MOE_PANEL_ROWS / 4;
+}
 // Rows of an expert's tiles, and how many tiles its n rows make.
 __device__ __forceinline__ int moe_rows_of_tile(int n, int rows) {
-    if (rows < MOE_TILE_ROWS) return rows;
+    if (rows < MOE_TILE_ROWS && !moe_panel_height(rows)) return rows;
     const int t = (n + rows - 1) / rows;
     return t > 1 ? min(rows, ((n + t - 1) / t + 15) & ~15) : rows;
 }
@@ -150,7 +154,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
     __shared__ unsigned long long wave_total[16];
     __shared__ int sorted[MOE_MAX_EXPERTS];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const bool runs = rows == MOE_PANEL_ROWS;
+    const bool runs = moe_panel_height(rows);
     const int copies = E <= MOE_PLAN_EXPERTS ? 16 : 1;
     int* mine = place + (copies == 16 ? wave : 0) * E;
     for (int i = tid; i < copies * E; i += 1024) place[i] = 0;
@@ -588,10 +592,10 @@ extern "C" int ra_moe_product(const void* x, const void* w, void* y, const int* 
                               stream);
 }
 
-// The same with w laid out in panels (moe_tile.h). tile_rows: 16 or MOE_PANEL_ROWS, as ra_moe_panel_rows says: from two pairs an
-// expert on nearly every expert has one, and the tiles' longer reads are the faster ones; with fewer they are not enough tiles for
-// the CUs. 32 experts of 6,144 x 4,096, four a token, gate-up and down, sweep / tiles, us: 8 tokens 167 + 87 / 193 + 94, 16 tokens 234 + 115 /
-// 222 + 114, 32 tokens 244 + 121 / 230 + 117; of 4,096 x 2,048, tiles, 16 tokens 80 + 42, 64 tokens 82 + 43.
+// The same with w laid out in panels (moe_tile.h). tile_rows: 16, or 320, 160 or 80 (moe_panel_height). ra_moe_panel_rows: which of 16 and
+// 320 where the tiles of 320 rows are enough for the CUs: from two pairs an expert on nearly every expert has one, and the tiles'
+// longer reads are the faster ones. 32 experts of 6,144 x 4,096, four a token, gate-up and down, sweep / tiles, us: 8 tokens 167 + 87 /
+// 193 + 94, 16 tokens 234 + 115 / 222 + 114, 32 tokens 244 + 121 / 230 + 117; of 4,096 x 2,048, tiles, 16 tokens 80 + 42, 64 tokens 82 + 43.
 extern "C" int ra_moe_panel_rows(int n_pairs, int E) { return n_pairs >= 2 * E ? MOE_PANEL_ROWS : 16; }
 
 extern "C" int ra_moe_panel_product(const void* x, const void* w, void* y, const int* order, const int* tiles, const int* meta,
@@ -604,7 +608,7 @@ extern "C" int ra_moe_panel_product(const void* x, const void* w, void* y, const
     if (2ll * N * K * (gated ? 2 : 1) >= 0x7fffff00ll || 2ll * n_pairs * K >= 0x7fffff00ll) return RA_ERR_ARG;
     const MoeAct act = {act_kind, limit, slope, in_scale};
     const int x_rows = (n_pairs - 1) / top_div + 1;
-    if (tile_rows == MOE_PANEL_ROWS)
+    if (moe_panel_height(tile_rows))
         return moe_panel_tile_launch((hipStream_t)stream, (const bf16*)x, (const bf16*)w, (bf16*)y, order, tiles, meta, max_tiles, x_rows, N, K,
                                      top_div, gated != 0, act);
     if (tile_rows != 16) return RA_ERR_ARG;

@@ -66,8 +66,9 @@ __device__ __forceinline__ void mp_tile(unsigned char* lds, const bf16* __restri
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int a = 0; a < 2; ++a)
-                // (a tile of up to nine groups is its expert's only one, as the plan has it: W, which nothing shares then, is read past the caches. 64
-                // tokens 258 -> 231 us, 7.0 TB/s; with W that tiles share 605 -> 626)
+                // (of tiles of 320 rows one of up to nine groups is its expert's only one, as the plan has it: W, which nothing shares then, is read
+                // past the caches. 64 tokens 258 -> 231 us, 7.0 TB/s; with W that tiles share 605 -> 626. Shorter tiles, of steps that would leave
+                // CUs idle, share it and read it so all the same: their matrices are small)
                 to.f[a][h] = __builtin_bit_cast(mp_bf16x8_t, __builtin_amdgcn_raw_buffer_load_b128(res, woff + a * 2048 + h * 1024, kk * kstep, NG <= 9 ? 2 : 0));
     };
     // Piece c of row r of a stage lies at piece c ^ ((r >> 1) & 7); lane (n, g) reads row n of a group, piece 4 h + g

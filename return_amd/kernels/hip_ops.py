@@ -195,6 +195,7 @@ class HipOps:
         self._side_stream = None
         self.skinny_max_grid = 0             # 0: one workgroup per 16 weight rows
         self.gated_skinny_rows = 8           # up to this many rows gate-up and SiLU-mul are one kernel
+        self.panel_tile_rows = 0             # rows of the tiles of experts' matrices in panels; 0: by the step's sizes
         self.own_gemm = False                # True: bf16 products of many rows use the hand-written MFMA kernel
         self.defer_norms = True              # finish RMSNorms inside the products around them where the sweep takes both
         try:                                 # whether the library multiplies bf16 operands into fp32 results
@@ -2266,11 +2267,35 @@ class HipOps:
         self._check(self.lib.ra_moe_plan(_ptr(ids), n_pairs, E, rows, _ptr(order), _ptr(tiles), _ptr(meta), self._stream()), "moe_plan")
         return order, tiles, meta, max_tiles, rows
 
+    def use_panel_rows(self, n_pairs, E, H, I):
+        """Rows of the tiles that matrices in panels are multiplied by: 16 (a sweep over W that all CUs share evenly), or up to 320, 160 or 80,
+        a workgroup for each tile and 128 columns of I. Where those are fewer than the CUs the sweep is the faster one for longer, and
+        shorter tiles make more workgroups. Measured on MI355X, microseconds of plan and both products, sweep / tiles of 320 / with rows of W
+        through LDS (moe_sweep.hip, moe_tile.hip), at 4, 16, 32 and 64 pairs an expert: 4 experts of 2,048 x 1,024 (32 workgroups) 17 / 33 / 21,
+        20 / 34 / 29, 26 / 37 / 31, 33 / 42 / 39; 8 of 2,048 x 2,048 (64) 28 / 45 / 31, 39 / 46 / 53, 53 / 49 / 56, 84 / 56 / 63; 32 of 1,024 x 1,024
+        (128) 27 / 33 / 41, 36 / 34 / 36, 52 / 37 / 40, 86 / 43 / 47; 16 of 2,048 x 4,096 (128) 80 / 79 / 84, 94 / 82 / 103, 159 / 86 / 107, 307 / 93 /
+        116; 64 of 1,024 x 2,048 (256) 78 / 73 / 91, 103 / 77 / 104, 174 / 81 / 109. Tiles of 320 / 160 / 80 at 128 and 160 at 256 pairs: 8 of
+        2,048 x 2,048 67 / 67 / 54 and 98 / 68 (rows through LDS 73 and 97); 32 of 1,024 x 1,024 54 / 54 / 47 and 80 / 63 (55 and 75); 64 of
+        1,024 x 2,048, which have the workgroups, 108 / 106 / 129 and 161 / 182. Slower than rows through LDS only experts of 512 columns: 32 of
+        512 x 512 at 24 to 64 pairs 20.5, 26 and 31 where those took 20, 22.5 and 28, at 48 of 1,024 x 512 and 512 pairs 111 for 103 (at one to 16
+        pairs they are 5 to 20 % faster)."""
+        if self.panel_tile_rows:
+            return self.panel_tile_rows
+        rows = int(self.lib.ra_moe_panel_rows(n_pairs, E))
+        groups = E * -(-I // 128)                               # workgroups of gate-up, a tile an expert
+        if rows == 16 or groups >= self.cu_count:
+            return rows
+        if n_pairs < E * (12 if 2 * groups >= self.cu_count else 32 if 4 * groups >= self.cu_count else 96):
+            return 16
+        while rows > 80 and 2 * groups * -(-n_pairs // (E * rows)) <= self.cu_count:
+            rows //= 2
+        return rows
+
     def _experts_panels(self, x, ids, in_scale, w_gate_up, w_down, y, act, limit, slope):
         (T, H), (E, I2, _), top = x.shape, w_gate_up.shape, ids.shape[1]
         n_pairs, I = T * top, I2 // 2
         mid = torch.empty(n_pairs, I, dtype=x.dtype, device=self.device)
-        order, tiles, meta, max_tiles, rows = self._moe_plan(ids, E, int(self.lib.ra_moe_panel_rows(n_pairs, E)))
+        order, tiles, meta, max_tiles, rows = self._moe_plan(ids, E, self.use_panel_rows(n_pairs, E, H, I))
         self._check(self.lib.ra_moe_panel_product(_ptr(x), _ptr(w_gate_up.tensor), _ptr(mid), _ptr(order), _ptr(tiles), _ptr(meta), n_pairs,
                                                   max_tiles, rows, I, H, top, 1, act, float(limit), float(slope), _ptr(in_scale),
                                                   self._stream()), "moe_panel_product (gate-up)")

@@ -91,22 +91,37 @@ def test_panels_few_rows(ops, E, H, I, counts, kind):
     check(ops, 16, E, H, I, shuffled(counts), kind, panels=True)
 
 
+@pytest.mark.parametrize("rows", [16, 80, 160, 320])
+@pytest.mark.parametrize("E,H,I,counts", [
+    (4, 64, 64, [1, 16, 17, 33]), (2, 320, 64, [80, 81]), (3, 192, 448, [159, 160, 161]), (4, 448, 128, [176, 0, 320, 321]), (1, 1024, 192, [1700]),
+    (2, 128, 320, [3300, 15]), (130, 128, 64, [1] * 60 + [700, 0, 161] + [17] * 67)])
+@pytest.mark.parametrize("kind", KINDS)
+def test_panels_by_tiles_of_every_height(ops, rows, E, H, I, counts, kind):
+    """At the edges of the heights, with more than four tiles of an expert, whatever the rule would take for these sizes."""
+    ops.panel_tile_rows = rows
+    try:
+        check(ops, ops.lib.ra_moe_panel_rows(sum(counts), E), E, H, I, shuffled(counts), kind, panels=True)
+    finally:
+        ops.panel_tile_rows = 0
+
+
 @pytest.mark.parametrize("E,counts", [
     (3, [3649, 40, 0]), (1, [6081]), (2, [321, 320]), (4, [1700, 3300, 1281, 640]), (130, [1] * 60 + [700, 0, 1601] + [17] * 67),
     (200, [330, 0, 2, 16] * 50), (1024, [0] * 1000 + [400] * 24)])
-def test_plan_of_tiles_of_panels(ops, E, counts):
-    """Every pair stands once, with its expert's; an expert's tiles are as few as 320 rows allow, even within a group of 16 rows, so
-    that of several none has fewer than ten groups; the largest tiles come first; runs of up to four of an expert's tiles are numbered."""
+@pytest.mark.parametrize("most_rows", [320, 160, 80])
+def test_plan_of_tiles_of_panels(ops, E, counts, most_rows):
+    """Every pair stands once, with its expert's; an expert's tiles are as few as their height allows, even within a group of 16 rows, so
+    that of several of 320 rows none has fewer than ten groups; the largest tiles come first; runs of up to four of an expert's tiles are numbered."""
     ids = shuffled(counts)
-    order, tiles, meta, most, _ = ops._moe_plan(ids.int().to(DEV), E, 320)
+    order, tiles, meta, most, _ = ops._moe_plan(ids.int().to(DEV), E, most_rows)
     n = int(meta)
     order, tiles = order.cpu(), tiles[:n].cpu().tolist()
-    assert n == sum(-(-c // 320) for c in counts) <= most and order.sort().values.tolist() == list(range(len(ids)))
+    assert n == sum(-(-c // most_rows) for c in counts) <= most and order.sort().values.tolist() == list(range(len(ids)))
     at, first_of = 0, []
     while tiles:
         e = tiles[0][0]
         of_e = [t for t in tiles if t[0] == e]
-        assert tiles[:len(of_e)] == of_e and len(of_e) == -(-counts[e] // 320)
+        assert tiles[:len(of_e)] == of_e and len(of_e) == -(-counts[e] // most_rows)
         first_of.append(of_e[0][2] & 0xffff)
         groups = []
         for j, (_, start, packed) in enumerate(of_e):
@@ -115,7 +130,7 @@ def test_plan_of_tiles_of_panels(ops, E, counts):
             assert (ids[order[at:at + rows].long()] == e).all()
             at += rows
             groups.append(-(-rows // 16))
-        assert at - of_e[0][1] == counts[e] and max(groups) <= 20
-        assert max(groups) - min(groups) <= 1 and (len(of_e) == 1 or min(groups) >= 10), (counts[e], groups)
+        assert at - of_e[0][1] == counts[e] and 16 * max(groups) <= most_rows
+        assert max(groups) - min(groups) <= 1 and (len(of_e) == 1 or 32 * min(groups) >= most_rows), (counts[e], groups)
         tiles = tiles[len(of_e):]
     assert at == len(ids) and first_of == sorted(first_of, reverse=True)
