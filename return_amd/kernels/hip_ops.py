@@ -2274,9 +2274,10 @@ class HipOps:
         through LDS (moe_sweep.hip, moe_tile.hip), at 4, 16, 32 and 64 pairs an expert: 4 experts of 2,048 x 1,024 (32 workgroups) 17 / 33 / 21,
         20 / 34 / 29, 26 / 37 / 31, 33 / 42 / 39; 8 of 2,048 x 2,048 (64) 28 / 45 / 31, 39 / 46 / 53, 53 / 49 / 56, 84 / 56 / 63; 32 of 1,024 x 1,024
         (128) 27 / 33 / 41, 36 / 34 / 36, 52 / 37 / 40, 86 / 43 / 47; 16 of 2,048 x 4,096 (128) 80 / 79 / 84, 94 / 82 / 103, 159 / 86 / 107, 307 / 93 /
-        116; 64 of 1,024 x 2,048 (256) 78 / 73 / 91, 103 / 77 / 104, 174 / 81 / 109. Tiles of 320 / 160 / 80 at 128 and 160 at 256 pairs: 8 of
-        2,048 x 2,048 67 / 67 / 54 and 98 / 68 (rows through LDS 73 and 97); 32 of 1,024 x 1,024 54 / 54 / 47 and 80 / 63 (55 and 75); 64 of
-        1,024 x 2,048, which have the workgroups, 108 / 106 / 129 and 161 / 182. Slower than rows through LDS only experts of 512 columns: 32 of
+        116; 64 of 1,024 x 2,048 (256) 78 / 73 / 91, 103 / 77 / 104, 174 / 81 / 109. Tiles of 320 / 160 / 80 at 128 and 256 pairs: 8 of 2,048
+        x 2,048 67 / 67 / 54 and 98 / 67 / 61 (rows through LDS 73 and 97); 32 of 1,024 x 1,024 54 / 54 / 47 and 79 / 60 / 77 (55 and 75); 64 of
+        1,024 x 2,048, which have the workgroups, 108 / 106 / 129 and 161 / 182; at 64 pairs, where shorter ones are not more of them but for an
+        expert with many, 32 of 1,024 x 2,048 62 / 62 / 69. Slower than rows through LDS only experts of 512 columns: 32 of
         512 x 512 at 24 to 64 pairs 20.5, 26 and 31 where those took 20, 22.5 and 28, at 48 of 1,024 x 512 and 512 pairs 111 for 103 (at one to 16
         pairs they are 5 to 20 % faster)."""
         if self.panel_tile_rows:
@@ -2287,9 +2288,10 @@ class HipOps:
             return rows
         if n_pairs < E * (12 if 2 * groups >= self.cu_count else 32 if 4 * groups >= self.cu_count else 96):
             return 16
-        while rows > 80 and 2 * groups * -(-n_pairs // (E * rows)) <= self.cu_count:
-            rows //= 2
-        return rows
+        heights = (rows, rows // 2, rows // 4)
+        tiles = [-(-n_pairs // (E * h)) for h in heights]       # of an expert
+        least = next((t for t in tiles if 2 * groups * t > self.cu_count), tiles[-1])
+        return heights[tiles.index(least)]                      # the tallest that make as many
 
     def _experts_panels(self, x, ids, in_scale, w_gate_up, w_down, y, act, limit, slope):
         (T, H), (E, I2, _), top = x.shape, w_gate_up.shape, ids.shape[1]

@@ -137,10 +137,10 @@ def test_experts_in_panels_go_by_the_sweep_while_their_tiles_are_too_few():
     """(pairs, experts, hidden, inner) on either side of the rule's lines at 256 CUs: the sweep's 16 rows, or tiles of up to 320, 160 or 80."""
     ops = kernel_set("cpu", ra_moe_panel_rows=lambda n, E: 320 if n >= 2 * E else 16)
     ops.cu_count, ops.panel_tile_rows = 256, 0
-    for n, E, H, I, want in [(128, 8, 2048, 1024, 16), (255, 8, 2048, 1024, 16), (256, 8, 2048, 1024, 80), (8 * 161, 8, 2048, 1024, 80), (8 * 240, 8, 2048, 1024, 80),
-                             (8 * 320, 8, 2048, 1024, 80), (8 * 321, 8, 2048, 1024, 160), (383, 32, 1024, 512, 16), (384, 32, 1024, 512, 80),
+    for n, E, H, I, want in [(128, 8, 2048, 1024, 16), (255, 8, 2048, 1024, 16), (256, 8, 2048, 1024, 320), (8 * 80, 8, 2048, 1024, 320), (8 * 81, 8, 2048, 1024, 80), (8 * 161, 8, 2048, 1024, 80), (8 * 240, 8, 2048, 1024, 80),
+                             (8 * 320, 8, 2048, 1024, 80), (8 * 321, 8, 2048, 1024, 160), (383, 32, 1024, 512, 16), (384, 32, 1024, 512, 320), (32 * 80, 32, 1024, 512, 320), (32 * 81, 32, 1024, 512, 80),
                              (32 * 160, 32, 1024, 512, 80), (32 * 161, 32, 1024, 512, 160), (32 * 321, 32, 1024, 512, 320), (127, 64, 2048, 512, 16),
-                             (128, 64, 2048, 512, 320), (64, 32, 4096, 3072, 320), (63, 32, 4096, 3072, 16), (383, 4, 1024, 1024, 16), (384, 4, 1024, 1024, 80),
+                             (128, 64, 2048, 512, 320), (64, 32, 4096, 3072, 320), (63, 32, 4096, 3072, 16), (383, 4, 1024, 1024, 16), (384, 4, 1024, 1024, 80), (4 * 700, 4, 1024, 1024, 160),
                              (40 * 128, 40, 1536, 512, 320), (16 * 12, 16, 1024, 1408, 320), (16, 8, 4096, 4096, 320), (15, 8, 4096, 4096, 16)]:
         assert ops.use_panel_rows(n, E, H, I) == want, (n, E, H, I)
         tiles = min(n, n // want + E)                          # (the plan's places; a tile's number has 15 bits)
