@@ -242,8 +242,11 @@ class HipOps:
         choice for x [M, K] and N result columns. Measured on MI355X, microseconds by it / by the best other product, at 1, 4, 8
         and 16 rows: 151,936 x 4,096 188 / 209, 189 / 214, 192 / 221, 195 / 233; 32,000 x 4,096 43 / 48, 43 / 50, 43 / 51, 44 / 59; 6,144 x
         4,096 11.3 / 14.2, 11.4 / 14.5, 11.8 / 15.2, 11.9 / 14.3; 4,096 x 4,096 8.7 / 9.1, 8.8 / 10.2, 8.5 / 10.6, 9.4 / 11.9; 2,048 x 2,048
-        4.8 / 5.0, 5.0 / 5.4, 5.2 / 5.8, 5.6 / 6.6; 1,024 x 4,096 5.2 / 6.9, 5.4 / 8.3, 6.0 / 9.0, 6.8 / 10.6 (3,072 x 512 4.5 / 2.9: too little to
-        stream). K beyond 4,096: 4,096 x 12,288 18.4 / 22.3, 17.7 / 21.2, 18.7 / 21.2, 21.3 / 21.7; 2,560 x 9,728 12.1 / 17.5, 12.8 / 15.6,
+        4.8 / 5.0, 5.0 / 5.4, 5.2 / 5.8, 5.6 / 6.6; 1,024 x 4,096 5.2 / 6.9, 5.4 / 8.3, 6.0 / 9.0, 6.8 / 10.6. A wave has 512 columns of K, so
+        with narrow W most waves have none: 3,072 x 512 4.5 / 2.9, and beyond 256 columns of the result a CU, where the x-resident product
+        is the other one (sweep / that, at 1, 8 and 16 rows, its rule's form), 151,936 x 512 65 / 41, 65 / 44, 67 / 61; x 768 73 / 44, 66 / 52, 68 /
+        74; x 1,024 77 / 56, 69 / 58, 71 / 85; x 1,280 79 / 70, 77 / 74, 72 / 103; x 1,536 80 / 86, 81 / 92, 76 / 116; with wide W (the library
+        at 16 rows) x 5,120 235 / 284, 252 / 289, 262 / 311; x 8,192 395 / 455, 417 / 473, 433 / 444; x 9,728 445 / 495, 466 / 504, 560 / 543. K beyond 4,096: 4,096 x 12,288 18.4 / 22.3, 17.7 / 21.2, 18.7 / 21.2, 21.3 / 21.7; 2,560 x 9,728 12.1 / 17.5, 12.8 / 15.6,
         13.1 / 15.6, 15.6 / 16.0; 2,048 x 8,192 9.2 / 12.7, 9.2 / 12.6, 10.0 / 12.6, 11.6 / 12.9; 8,192 x 12,288 36 / 42, 36 / 43, 37 / 44,
         41 / 44. Gated, 12,288 x 4,096 34 against 41 for the x-resident and skinny products, 25,600 x 5,120 100 against 118."""
         if not self.lib.ra_gemm_sweep_fits(M, K):
@@ -253,6 +256,8 @@ class HipOps:
         rows = N * (2 if gated else 1)
         if gated:
             return (8 if K <= 4096 or M <= 2 else 32) * self.cu_count <= rows <= 256 * self.cu_count
+        if rows > 256 * self.cu_count and not (K >= 1536 if M <= 8 else 768 <= K <= 8192):
+            return False
         if K <= 4096:
             return rows >= 4 * self.cu_count and rows * K >= 4 << 20
         return rows >= 8 * self.cu_count                      # rows of W a workgroup, at least

@@ -147,3 +147,17 @@ def test_experts_in_panels_go_by_the_sweep_while_their_tiles_are_too_few():
         assert tiles <= 0x7fff
     ops.panel_tile_rows = 160
     assert ops.use_panel_rows(16, 8, 2048, 1024) == 160
+
+
+def test_products_of_up_to_16_rows_that_the_sweep_forms_more_slowly_are_not_its():
+    """(rows, result columns, K) on either side of the rule's lines at 256 CUs: beyond 256 result columns a CU narrow W leaves most of
+    its waves without columns of K."""
+    from return_amd.kernels.hip_ops import load_library
+    lib = load_library()
+    ops = kernel_set("cpu", ra_gemm_sweep_fits=lib.ra_gemm_sweep_fits)
+    ops.cu_count = 256
+    for M, N, K, want in [(1, 65536, 1024, True), (1, 65537, 1024, False), (8, 151936, 512, False), (8, 151936, 1528, False), (8, 151936, 1536, True),
+                          (9, 151936, 760, False), (9, 151936, 768, True), (16, 151936, 4096, True), (16, 151936, 5120, True), (16, 151936, 8192, True),
+                          (16, 151936, 9728, False), (8, 151936, 9728, True), (16, 65536, 12288, True), (1, 1024, 4096, True), (1, 1023, 4096, False),
+                          (4, 3072, 512, False), (16, 2048, 8192, True), (16, 2047, 8192, False)]:
+        assert ops.use_sweep(M, N, K, False) == want, (M, N, K)
