@@ -159,11 +159,12 @@ template <int COLS, bool NEAR> struct SweepCols {
     __device__ __forceinline__ bool has(int t, int i) const { return NEAR ? t < full || i < share : at(t, i) < N; }
 };
 
-// MB: blocks of 16 rows of x (1 or 2)
-template <int MB, bool GATED, typename TO, bool RESID = false>
+// MB: blocks of 16 rows of x (1 or 2). LINES: x as whole lines (SweepX), else as operands straight from memory.
+template <int MB, bool GATED, typename TO, bool RESID, bool LINES>
 __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ W, TO* __restrict__ out, int M, int N, int K, SweepNorm nm) {
     static_assert(!RESID || (!GATED && MB == 1), "the residual epilogue belongs to the plain product of up to 16 rows");
+    static_assert(!LINES || MB == 1, "32 rows as lines are more registers than there are");
     constexpr int COLS = GATED ? 8 : 16;                        // result columns of a tile
     constexpr int RS = 16 * MB + 1;                             // row stride of the waves' tiles in LDS (floats)
     constexpr bool TWO_BUFFERS = MB == 1;                       // of those tiles (LDS has room for one set with MB == 2)
@@ -192,14 +193,14 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
     };
     // (x first: it comes from nearby, and is made operands while the first rows of W are on their way)
     [[maybe_unused]] SweepX xs;
-    if constexpr (MB == 1) sweep_x_ask(xs, x, M, K, kb, lane);
+    if constexpr (LINES) sweep_x_ask(xs, x, M, K, kb, lane);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int i = 0; i < 16; ++i) fetch_row(0, i);
 
     // the wave's columns of x as B operands: lane (n, g) holds x[n][kb + 32j + 8g ..]
     bf16x8_t bx[MB][SW_STEPS];
-    if constexpr (MB == 1) {
+    if constexpr (LINES) {
         sweep_x_take(xs, stage, M, lane, bx[0]);
     } else {
 #pragma unroll
@@ -578,11 +579,17 @@ static int launch_sweep(int grid, hipStream_t st, const bf16* x, const bf16* W, 
     if constexpr (!RESID) {
         if (M > 16) {
             static bool allowed = false;
-            return launch_sweep_kernel(gemm_sweep_kernel<2, GATED, TO, false>, allowed, grid, st, x, W, out, M, N, K, nm);
+            return launch_sweep_kernel(gemm_sweep_kernel<2, GATED, TO, false, false>, allowed, grid, st, x, W, out, M, N, K, nm);
         }
     }
+    // K up to 1,024 and one tile a workgroup: two waves load x, once, and the way through LDS is longer than their address units'
+    // time (gated 1,024 x 512, as lines / straight, us: 8 rows 4.7 / 4.5, 16 rows 5.1 / 4.6)
+    if (M > 4 && K <= 2 * SW_KW && N <= grid * (GATED ? 8 : 16)) {
+        static bool allowed = false;
+        return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, false>, allowed, grid, st, x, W, out, M, N, K, nm);
+    }
     static bool allowed = false;
-    return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID>, allowed, grid, st, x, W, out, M, N, K, nm);
+    return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, true>, allowed, grid, st, x, W, out, M, N, K, nm);
 }
 
 static int sweep_dispatch(const void* x, const void* W, void* out, int M, int N, int K, int gated, int out_dtype,
