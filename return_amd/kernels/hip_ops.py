@@ -275,13 +275,14 @@ class HipOps:
 
     def use_rows(self, M, N, K, gated):
         """Whether the product of 17 to 64 rows that streams W through LDS is the rule's choice: where every CU has 64 rows of W
-        or more, gated up to one round of workgroups. Measured on MI355X, microseconds by it / by the library (gated: with the
+        or more, gated up to one round of workgroups, or of K up to 1,024. Measured on MI355X, microseconds by it / by the library (gated: with the
         SiLU-mul) / by the sweep, at 17, 32 and 64 rows: gate-up 12,288 x 4,096 36 / 51 / 40, 36 / 50 / 44, 38 / 51; 8,192 x 1,024 9.4 / 16
-        / 14, 9.4 / 16 / 15, 11 / 17; 13,824 x 5,120 51 / 56, 51 / 54, 58 / 58; 25,600 x 5,120 104 / 98, 106 / 101, 112 / 105; plain
+        / 14, 9.4 / 16 / 15, 11 / 17; 13,824 x 5,120 51 / 56, 51 / 54, 58 / 58; 25,600 x 5,120 104 / 98, 106 / 101, 112 / 105; 28,672 x
+        1,024 26 / 28 / 38, 27 / 29 / 39, 30 / 36; x 512 17 / 20 / 35, 16 / 21 / 35, 20 / 26 (x 2,048 at 17 rows 42 / 45 / 44, 16,640 x 2,048 32 / 35 / 31); plain
         151,936 x 4,096 223 / 264, 216 / 272, 234 / 261; 16,384 x 4,096 25 / 33, 25 / 32, 27 / 33; 24,576 x 1,024 13 / 32, 13 / 32, 14 /
         16; 151,936 x 5,120 274 / 335, 269 / 357, 303 / 300. With fewer rows of W x is most of what a CU takes in (6,144 x 4,096 at 64
         rows 18.5 / 17.6)."""
-        if N * (2 if gated else 1) < 64 * self.cu_count or (gated and N > 64 * self.cu_count):
+        if N * (2 if gated else 1) < 64 * self.cu_count or (gated and N > 64 * self.cu_count and K > 1024):
             return False
         return bool(self.lib.ra_gemm_rows_fits(M, N, K)) and not self.own_gemm
 

@@ -119,6 +119,8 @@ def test_products_of_17_to_64_rows_that_the_library_forms_faster_are_its():
     for N, gated, want in [(12288, True, True), (8192, True, True), (16384, True, True), (25600, True, False), (27648, True, False), (6144, True, False),
                            (16384, False, True), (151936, False, True), (6144, False, False)]:
         assert ops.use_rows(64, N, 5120, gated) == want, (N, gated)
+    for N, K, want in [(16385, 1024, True), (28672, 512, True), (16385, 1032, False), (28672, 1280, False), (16384, 4096, True), (8191, 1024, False)]:
+        assert ops.use_rows(17, N, K, True) == want, (N, K)
 
 
 def test_many_very_short_prompts_go_over_the_latents():
