@@ -628,8 +628,14 @@ static int dec_launch_one(dim3 grid, hipStream_t st, const bf16* q, float* pa, f
                           DecodeExtras ex) {
     constexpr int D = 16 * N;
     const size_t lds = (size_t)merge_waves * (dec_region_bytes(D) + (FUSED ? 4 * D : 0));
-    const bool away = N >= 8 && Hq <= DEC_MAX_GROUP * Hkv;
-    auto kern = away ? attn_decode_kernel<N, FUSED, XT, (N >= 8)> : attn_decode_kernel<N, FUSED, XT, false>;
+    // Past the caches (see the kernel's loads): heads of 128 and more whose rows are whole lines or halves; with rows that begin inside
+    // a 64-byte piece, an odd N, what two rows share goes between them: 32 requests of 4,096, 16 heads over 2 of 240 65 us, past
+    // the caches 76, 64 of 144 at 2,048 1.15 of the time; of 160 and 224 0.85 to 1. Heads of 256 not where few waves walk long splits:
+    // 16 over 2, one request of 65,536 80.8 us, past the caches 84.5; 8 of them, 1,024 waves, 0.91 of the time.
+    constexpr bool CAN = N >= 8 && N % 2 == 0;
+    const bool few = N == 16 && split_tokens >= 256 && (long long)grid.x * grid.y * grid.z * merge_waves < 1024;
+    const bool away = CAN && !few && Hq <= DEC_MAX_GROUP * Hkv;
+    auto kern = away ? attn_decode_kernel<N, FUSED, XT, CAN> : attn_decode_kernel<N, FUSED, XT, false>;
     static size_t allowed_by[2] = {64 * 1024, 64 * 1024};     // per kernel: raised when needed
     size_t& allowed = allowed_by[away ? 1 : 0];
     if (lds > allowed) {
