@@ -95,8 +95,8 @@ __device__ __forceinline__ void sweep_scales_make(const SweepNorm& nm, int rows,
 // A wave's 512 columns (from k0 on) of up to 16 rows of x, on their way as whole lines: a row is one load of 1 KB, like a row of W, and
 // rows from M on are not asked for. As operands straight from memory (16 rows by 64 bytes a load, once a tile and span) they kept
 // the address unit busy: 4,096 x 12,288 took 21.5 us at 8 rows and 26.0 at 16, now 19.2 and 22.2; 24,576 x 4,096, which reads them
-// once, 37.6 us at 16 rows, now 36.2; 2,048 x 8,192 at 16 rows 13.9, now 11.8. (The kernel of few tiles, which has no registers left
-// for it and reads x once a span, does not.)
+// once, 37.6 us at 16 rows, now 36.2; 2,048 x 8,192 at 16 rows 13.9, now 11.8. (The kernel of few tiles, which reads x once a span, does
+// not: with these rows as well the compiler keeps 80 to 105 of its registers in scratch, though by count they would fit.)
 struct SweepX { bf16x8_t r[16]; };
 __device__ __forceinline__ void sweep_x_ask(SweepX& to, const bf16* __restrict__ x, int M, int K, int k0, int lane) {
     const int k = k0 + lane * 8;
@@ -582,9 +582,11 @@ static int launch_sweep(int grid, hipStream_t st, const bf16* x, const bf16* W, 
             return launch_sweep_kernel(gemm_sweep_kernel<2, GATED, TO, false, false>, allowed, grid, st, x, W, out, M, N, K, nm);
         }
     }
-    // K up to 1,024 and one tile a workgroup: two waves load x, once, and the way through LDS is longer than their address units'
-    // time (gated 1,024 x 512, as lines / straight, us: 8 rows 4.7 / 4.5, 16 rows 5.1 / 4.6)
-    if (M > 4 && K <= 2 * SW_KW && N <= grid * (GATED ? 8 : 16)) {
+    // One tile a workgroup, so that x is read once, and narrow W, where few waves load it, or rows of x that are no whole lines: the way
+    // through LDS is longer than the address units' time. 1,024 gated columns, straight / as lines, us: K of 512 4.5 / 4.7 at 8 rows and 4.6 /
+    // 5.1 at 16; of the time as lines, at 8 and 16 rows, K of 1,280 0.96 and 0.97, 1,536 1.01 and 1.03, 2,048 1.05 and 1.09, 4,096 1.09 and 1.13, but
+    // 1,544 0.92 and 0.91, 2,056 0.94 and 0.90, 3,080 0.95 and 0.96.
+    if (M > 4 && (K < 3 * SW_KW || K % 64 != 0) && N <= grid * (GATED ? 8 : 16)) {
         static bool allowed = false;
         return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, false>, allowed, grid, st, x, W, out, M, N, K, nm);
     }
