@@ -152,7 +152,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
                                                         int* __restrict__ meta) {
     __shared__ int place[MOE_MAX_EXPERTS > 16 * MOE_PLAN_EXPERTS ? MOE_MAX_EXPERTS : 16 * MOE_PLAN_EXPERTS];
     __shared__ unsigned long long wave_total[16];
-    __shared__ int sorted[MOE_MAX_EXPERTS];
+    __shared__ int sorted[MOE_MAX_EXPERTS], of_wave[MOE_PANEL_ROWS / 16 + 1][16], of_all[MOE_PANEL_ROWS / 16 + 1];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const bool runs = moe_panel_height(rows);
     const int copies = E <= MOE_PLAN_EXPERTS ? 16 : 1;
@@ -170,18 +170,39 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
     __syncthreads();
     int e = tid;
     if (runs) {
-        // the experts with the largest tiles first: tiles go to the CUs in this order, and what is long must not come last
-        int n = 0, key = 0;
-        if (tid < E) {
+        // the experts with the largest tiles first, by groups of 16 rows: tiles go to the CUs in this order, and what is long must not come
+        // last. Up to 64 experts each looks at all. Of more that took 5.5 of the plan's 10.5 us (256 experts) and 38 of 44 (1,024): a
+        // counting sort, how many experts of a wave have as many groups, by ballots, and sums of those, 6.7 and 8.5 us in all (3.9 and 5.2 without the order).
+        int n = 0, ahead = 0;
+        if (tid < E)
             for (int c = 0; c < copies; ++c) n += place[c * E + tid];
-            sorted[tid] = key = min(n, moe_rows_of_tile(n, rows));
+        const int groups = tid < E ? (min(n, moe_rows_of_tile(n, rows)) + 15) >> 4 : -1;
+        if (E <= 64) {
+            if (tid < E) sorted[tid] = groups;
+            __syncthreads();
+            if (tid < E)
+                for (int j = 0; j < E; ++j) ahead += sorted[j] > groups || (sorted[j] == groups && j < tid);
+        } else {
+#pragma unroll
+            for (int k = 0; k <= MOE_PANEL_ROWS / 16; ++k) {
+                const unsigned long long same = __ballot(groups == k);
+                if (groups == k) ahead = __popcll(same & ((1ull << lane) - 1));
+                if (lane == 0) of_wave[k][wave] = __popcll(same);
+            }
+            __syncthreads();
+            if (tid <= MOE_PANEL_ROWS / 16) {
+                int sum = 0;
+                for (int v = 0; v < 16; ++v) sum += of_wave[tid][v];
+                of_all[tid] = sum;
+            }
+            __syncthreads();
+            if (tid < E) {
+                for (int k = MOE_PANEL_ROWS / 16; k > groups; --k) ahead += of_all[k];
+                for (int v = 0; v < wave; ++v) ahead += of_wave[groups][v];
+            }
         }
         __syncthreads();
-        int rank = 0;
-        if (tid < E)
-            for (int j = 0; j < E; ++j) rank += sorted[j] > key || (sorted[j] == key && j < tid);
-        __syncthreads();
-        if (tid < E) sorted[rank] = tid;
+        if (tid < E) sorted[ahead] = tid;
         __syncthreads();
         if (tid < E) e = sorted[tid];
     }

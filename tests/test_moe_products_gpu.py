@@ -111,7 +111,7 @@ def test_panels_by_tiles_of_every_height(ops, rows, E, H, I, counts, kind):
 @pytest.mark.parametrize("most_rows", [320, 160, 80])
 def test_plan_of_tiles_of_panels(ops, E, counts, most_rows):
     """Every pair stands once, with its expert's; an expert's tiles are as few as their height allows, even within a group of 16 rows, so
-    that of several of 320 rows none has fewer than ten groups; the largest tiles come first; runs of up to four of an expert's tiles are numbered."""
+    that of several of 320 rows none has fewer than ten groups; the largest tiles, by groups, come first; runs of up to four of an expert's tiles are numbered."""
     ids = shuffled(counts)
     order, tiles, meta, most, _ = ops._moe_plan(ids.int().to(DEV), E, most_rows)
     n = int(meta)
@@ -122,7 +122,7 @@ def test_plan_of_tiles_of_panels(ops, E, counts, most_rows):
         e = tiles[0][0]
         of_e = [t for t in tiles if t[0] == e]
         assert tiles[:len(of_e)] == of_e and len(of_e) == -(-counts[e] // most_rows)
-        first_of.append(of_e[0][2] & 0xffff)
+        first_of.append(((of_e[0][2] & 0xffff) + 15) // 16)
         groups = []
         for j, (_, start, packed) in enumerate(of_e):
             rows = packed & 0xffff
