@@ -2299,6 +2299,8 @@ class HipOps:
         least = next((t for t in tiles if 2 * groups * t > self.cu_count), tiles[-1])
         return heights[tiles.index(least)]                      # the tallest that make as many
 
+    PANEL_STEP_BYTES = 0x7fffff00 # rows of a step's products by panels, at most
+
     def _experts_panels(self, x, ids, in_scale, w_gate_up, w_down, y, act, limit, slope):
         (T, H), (E, I2, _), top = x.shape, w_gate_up.shape, ids.shape[1]
         n_pairs, I = T * top, I2 // 2
@@ -2375,7 +2377,7 @@ class HipOps:
             if x.data_ptr() % 16:
                 x = x.clone()
             # (the kernels' offsets into their rows have 32 bits, a tile's number 15: a step beyond that goes in parts of its tokens)
-            part = max(1, min(0x7fffff00 // (2 * top * max(H, I)) - 1, 8_000_000 // top))
+            part = max(1, min(self.PANEL_STEP_BYTES // (2 * top * max(H, I)) - 1, 8_000_000 // top))
             for t in range(0, T, part):
                 s = slice(t, min(t + part, T))
                 self._experts_panels(x[s], ids[s], None if in_scale is None else in_scale[s], w_gate_up, w_down, y[t * top:s.stop * top], act,

@@ -298,3 +298,52 @@ def test_page_tables_are_copied_only_when_a_page_list_changed():
             assert batch.groups[0].cu_pages.tolist()[-1] == len(batch.groups[0].page_table)
             cm.end_step()
         cm.check_invariants()
+
+
+def test_tables_of_steps_of_one_token_a_request_and_back():
+    """Such a step copies small tables of its own; prompts, mixed steps and steps that want more places than there are requests have
+    the full ones: every table of every step is right, whatever kind the one before was, and so are the sampling options."""
+    from return_amd.engine.batch import StepBuilder
+    rng = random.Random(3)
+    cm = manager(page=4, max_token=400, max_requests=4, window=6)
+    sb = StepBuilder(cm, 64, 4, "cpu", tile_rows=(16, 64), token_columns=("kind",))
+    small = few = 0
+    for step in range(200):
+        for rid in [r for r in list(cm.live) if cm.seq_len(r) > 60]:
+            cm.free_request(rid)
+        while len(cm.live) < 4:
+            cm.add_request(f"r{step}.{len(cm.live)}")
+        ids = rng.sample(sorted(cm.live), rng.randint(1, 4))
+        one = rng.random() < 0.5
+        lens = [1 if one or rng.random() < 0.4 else rng.randint(2, 9) for _ in ids]
+        starts = [cm.seq_len(r) for r in ids]
+        t = cm.begin_step(list(zip(ids, lens)))
+        total = sum(lens)
+        tokens = [[rng.randrange(1000) for _ in range(n)] for n in lens]
+        kind = [rng.randrange(9) for _ in range(total)]
+        rows = [rng.randrange(total) for _ in range(rng.choice([0, 1, len(ids), 4, 6]))]
+        m = len(rows)
+        options = None if m > 4 or rng.random() < 0.3 else tuple([rng.random() for _ in rows] if i != 1 else [rng.randrange(50) for _ in rows] for i in range(4))
+        b = sb.build(t, tokens, rows, {"kind": kind}, options)
+        small += total == len(ids) and m <= 4
+        few += total == len(ids)
+        assert b.token_ids.tolist() == [v for seq in tokens for v in seq] and b.token_columns["kind"].tolist() == kind
+        assert b.positions.tolist() == [s + i for s, n in zip(starts, lens) for i in range(n)]
+        assert b.logit_rows.tolist() == rows and b.cu_q.tolist() == np.cumsum([0] + lens).tolist()
+        assert b.q_start.tolist() == starts and b.seq_lens.tolist() == [s + n for s, n in zip(starts, lens)]
+        for g, gt in enumerate(t.groups):
+            assert b.groups[g].slot_mapping.tolist() == gt.slot_mapping.tolist() and b.groups[g].page_table.tolist() == gt.page_table.tolist()
+            assert b.groups[g].cu_pages.tolist() == gt.cu_pages.tolist() and b.groups[g].kv_start.tolist() == gt.kv_start.tolist()
+        long = [i for i, n in enumerate(lens) if n > 1]
+        for height in (16, 64) if long else ():
+            assert sorted(map(tuple, b.prefill_tiles[height].tolist())) == sorted((i, o) for i in long for o in range(0, lens[i], height))
+        if long and len(long) < len(ids):
+            assert b.decode_segs.tolist() == [i for i, n in enumerate(lens) if n == 1]
+            assert b.prefill_toks.tolist() == [r for i in long for r in range(int(t.cu_q[i]), int(t.cu_q[i + 1]))]
+        if options is not None:
+            temperature, top_k, top_p, uniforms = sb.sampling_options(m)
+            assert top_k.tolist() == options[1]
+            for got, want in ((temperature, options[0]), (top_p, options[2]), (uniforms, options[3])):
+                assert torch.equal(got, torch.tensor(want, dtype=torch.float32))
+        cm.end_step()
+    assert few - small > 5 and small > 50 and few < 180

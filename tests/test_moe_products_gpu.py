@@ -134,3 +134,27 @@ def test_plan_of_tiles_of_panels(ops, E, counts, most_rows):
         assert max(groups) - min(groups) <= 1 and (len(of_e) == 1 or 32 * min(groups) >= most_rows), (counts[e], groups)
         tiles = tiles[len(of_e):]
     assert at == len(ids) and first_of == sorted(first_of, reverse=True)
+
+
+@pytest.mark.parametrize("weigh", ["input", "output"])
+@pytest.mark.parametrize("tokens", [1, 7, 8, 9, 61, 64])
+def test_panels_of_steps_in_parts_and_of_rows_at_odd_places(ops, tokens, weigh):
+    """A step whose rows are beyond what an offset of 32 bits reaches goes in parts of its tokens (eight of them here), and rows that are not
+    16-byte aligned are copied: the same bits. Tiles of one height, whose sums have one order whatever the step's size."""
+    E, H, I, top = 5, 128, 192, 3
+    g = torch.Generator().manual_seed(tokens)
+    w_up, w_down = (torch.randn(*s, generator=g).bfloat16().to(DEV) * 0.1 for s in ((E, 2 * I, H), (E, H, I)))
+    a, b = ops.expert_panels(lambda e: w_up[e], E, H, I, True, torch.bfloat16), ops.expert_panels(lambda e: w_down[e], E, H, I, False, torch.bfloat16)
+    x = torch.randn(tokens, H, generator=g).bfloat16().to(DEV)
+    ids = torch.rand(tokens, E, generator=g).argsort(1)[:, :top].int().to(DEV)
+    weights = torch.rand(tokens, top, generator=g).to(DEV)
+    ops.panel_tile_rows = 320
+    try:
+        want = ops.moe_experts(x, ids, weights, a, b, weigh=weigh)
+        odd = torch.empty(tokens * H + 1, dtype=torch.bfloat16, device=DEV)[1:].view(tokens, H).copy_(x)
+        assert odd.data_ptr() % 16 and torch.equal(ops.moe_experts(odd, ids, weights, a, b, weigh=weigh), want)
+        ops.PANEL_STEP_BYTES = 9 * 2 * top * I
+        assert torch.equal(ops.moe_experts(x, ids, weights, a, b, weigh=weigh), want)
+    finally:
+        ops.panel_tile_rows = 0
+        ops.__dict__.pop("PANEL_STEP_BYTES", None)
