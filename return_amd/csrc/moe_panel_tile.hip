@@ -14,8 +14,9 @@
 // this kernel, us: 256 pairs 298 / 231 (7.0 TB/s), 4,000 pairs 326 / 283, 8,000 pairs 489 / 376 (1.07 PFLOP/s), 12,432 pairs 629 /
 // 550, uneven counts (147 to 742) 695 / 592, 32,768 pairs 1,486 / 1,285 (1.28 PFLOP/s); down (4,096 x 3,072) 8,000 pairs 281 / 193,
 // 12,432 pairs 325 / 279; gate-up of 4,096 x 2,048, 256 pairs 130 / 82, 8,448 pairs 226 / 150. Bound, up to 100 rows an expert, by
-// the reading of W, beyond that by the matrix cores and the loads' way beside them: MFMAs alone take 0.6 to 0.7 of the time. MFMA
-// 32x32x16 instead of 16x16x32: 712 instead of 598 us at 12,432 pairs (before the copies of x were spread).
+// the reading of W, beyond that by LDS as much as by the matrix cores: all eight waves read all of x, 320 KB a step of 320 rows beside the
+// 40 KB that are copied in, 2,880 clocks at 128 bytes a clock where the step's MFMAs take 2,560. MFMAs alone take 0.6 to 0.7 of the
+// time. MFMA 32x32x16 instead of 16x16x32: 712 instead of 598 us at 12,432 pairs (before the copies of x were spread).
 #include "moe_tile.h"
 #include <type_traits>
 
@@ -73,7 +74,9 @@ __device__ __forceinline__ void mp_tile(unsigned char* lds, const bf16* __restri
     };
     // Piece c of row r of a stage lies at piece c ^ ((r >> 1) & 7); lane (n, g) reads row n of a group, piece 4 h + g
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lds);
-    uint32_t rd[2][2];                                         // [64 KB base: offsets fit the instruction's 16 bits][h]
+    // [pair of stages][h]. The instruction's offset has 16 bits: up to 16 groups a pair's reads end at 63,488; beyond, a stage is 40 KB and
+    // those of an odd one from group 12 on lie further, an addition each (32 beside the 320 MFMAs of four steps of 20 groups)
+    uint32_t rd[2][2];
 #pragma unroll
     for (int v = 0; v < 2; ++v)
 #pragma unroll

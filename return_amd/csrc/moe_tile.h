@@ -35,8 +35,9 @@ bool moe_sweep_fits(int K);
 int moe_sweep_launch(hipStream_t st, const bf16* x, const bf16* w, bf16* y, const int* order, const int* tiles,
                      const int* meta, int N, int K, int top_div, bool gated, const MoeAct& act);
 
-// Experts' matrices laid out in panels when they are loaded, for sizes that allow it (bfloat16, K % 64 == 0 and at most 4,096, rows
-// % 16 == 0): [step of 64 columns][panel of 16 rows][half of the step][lane][8 elements], lane (n, g) of a half with row n, columns
+// Experts' matrices laid out in panels when they are loaded, for sizes that allow it (bfloat16, rows % 16 == 0, K % 64 == 0 and at most
+// 4,096, for which the sweep over panels has a wave's eight steps in registers; the tiles have no such limit):
+// [step of 64 columns][panel of 16 rows][half of the step][lane][8 elements], lane (n, g) of a half with row n, columns
 // 8 g ... 8 g + 7: what a lane of MFMA 16x16x32 takes, so that a wave reads an operand as 1 KB in a row, and needs no LDS for it.
 // Gated matrices have a panel of gate rows and the one of the up rows of the same columns side by side.
 #define MOE_PANEL_ROWS 320                        // rows of a tile at most

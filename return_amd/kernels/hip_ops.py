@@ -265,7 +265,9 @@ class HipOps:
     def use_resident(self, M, N, K, gated):
         """Whether the product with x resident in LDS beats the skinny product for x [M, K] and
         N result columns (measured on MI355X): when there are tiles of 16 columns enough for
-        every workgroup (two per CU); few tiles are the skinny product's."""
+        every workgroup (two per CU); few tiles are the skinny product's. Asked after use_sweep, which leaves it (at 256 CUs) W below
+        4 Mi elements (6,129 columns and more, so K below 685), more than 65,536 columns of K below 1,536 up to 8 rows and below 768
+        up to 16, and gated products of more than 32,768 columns; measuring at load may choose it elsewhere."""
         if not self.lib.ra_gemm_resident_fits(M, K, 1 if gated else 0):
             return False
         tiles = -(-N // 16)
