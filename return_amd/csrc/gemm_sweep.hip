@@ -138,8 +138,10 @@ __device__ __forceinline__ void sweep_x_take(const SweepX& from, uint16_t* stage
 // of y become whole in its L2. As every G-th column, y was written in pieces of one entry and every line by all XCDs: 151,936 x
 // 4,096 took 208 us at 8 rows and 220 at 16, now 191 and 197 (with neighbouring columns, but workgroups in plain order, 205
 // and 208); 24,576 x 4,096 at 16 rows 36.2, now 34.8; others the same within 0.2 us.
-// Otherwise (several spans, where a round is more of W and less of y) every G-th column: 4,096 x 12,288 18.3, 19.2 and 22.2 us at 1, 8 and
-// 16 rows, with the columns above 18.5, 19.6 and 22.4.
+// Otherwise every G-th column. Several spans, where a round is more of W and less of y: 4,096 x 12,288 18.3, 19.2 and 22.2 us at 1, 8 and
+// 16 rows, with the columns above 18.5, 19.6 and 22.4. And gated products of 17 to 32 rows with more than two tiles a workgroup: 31,872 x
+// 1,280 at 17 rows 38.3 us (41.9 with the columns above), 17,344 x 1,448 24.6 (26.3), 21,184 x 2,080 34.9 (36.9); over 45 shapes 0.98 of
+// the time, the slowest 1.03 (25,744 x 2,048 at 32 rows); with up to two tiles 1.02.
 template <int COLS, bool NEAR> struct SweepCols {
     int N, G, b, n_tiles;
     int full = 0, left = 0, share = 0;
@@ -159,8 +161,8 @@ template <int COLS, bool NEAR> struct SweepCols {
     __device__ __forceinline__ bool has(int t, int i) const { return NEAR ? t < full || i < share : at(t, i) < N; }
 };
 
-// MB: blocks of 16 rows of x (1 or 2). LINES: x as whole lines (SweepX), else as operands straight from memory.
-template <int MB, bool GATED, typename TO, bool RESID, bool LINES>
+// MB: blocks of 16 rows of x (1 or 2). LINES: x as whole lines (SweepX), else as operands straight from memory. NEAR: see SweepCols.
+template <int MB, bool GATED, typename TO, bool RESID, bool LINES, bool NEAR>
 __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ W, TO* __restrict__ out, int M, int N, int K, SweepNorm nm) {
     static_assert(!RESID || (!GATED && MB == 1), "the residual epilogue belongs to the plain product of up to 16 rows");
@@ -173,7 +175,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
     uint16_t* stage = reinterpret_cast<uint16_t*>(lds_raw) + (size_t)wave * 16 * SW_STRIDE;
     float* red_both = reinterpret_cast<float*>(lds_raw + (size_t)SW_WAVES * 16 * SW_STRIDE * 2);   // [1 or 2][wave][16 rows][RS]
     float* rs = red_both + 2 * SW_WAVES * 16 * 17;            // [32] row scales, behind the result tiles
-    const SweepCols<COLS, true> cols(N);
+    const SweepCols<COLS, NEAR> cols(N);
     const int n_tiles = cols.n_tiles;
     if (n_tiles == 0) return;                                   // (the launch keeps the grid within N)
     const int kb = wave * SW_KW;
@@ -578,8 +580,12 @@ static int launch_sweep(int grid, hipStream_t st, const bf16* x, const bf16* W, 
     }
     if constexpr (!RESID) {
         if (M > 16) {
+            if (GATED && N > 2 * grid * 8) {
+                static bool allowed = false;
+                return launch_sweep_kernel(gemm_sweep_kernel<2, GATED, TO, false, false, !GATED>, allowed, grid, st, x, W, out, M, N, K, nm);
+            }
             static bool allowed = false;
-            return launch_sweep_kernel(gemm_sweep_kernel<2, GATED, TO, false, false>, allowed, grid, st, x, W, out, M, N, K, nm);
+            return launch_sweep_kernel(gemm_sweep_kernel<2, GATED, TO, false, false, true>, allowed, grid, st, x, W, out, M, N, K, nm);
         }
     }
     // One tile a workgroup, so that x is read once, and narrow W, where few waves load it, or rows of x that are no whole lines: the way
@@ -588,10 +594,10 @@ static int launch_sweep(int grid, hipStream_t st, const bf16* x, const bf16* W, 
     // 1,544 0.92 and 0.91, 2,056 0.94 and 0.90, 3,080 0.95 and 0.96.
     if (M > 4 && (K < 3 * SW_KW || K % 64 != 0) && N <= grid * (GATED ? 8 : 16)) {
         static bool allowed = false;
-        return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, false>, allowed, grid, st, x, W, out, M, N, K, nm);
+        return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, false, true>, allowed, grid, st, x, W, out, M, N, K, nm);
     }
     static bool allowed = false;
-    return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, true>, allowed, grid, st, x, W, out, M, N, K, nm);
+    return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, true, true>, allowed, grid, st, x, W, out, M, N, K, nm);
 }
 
 static int sweep_dispatch(const void* x, const void* W, void* out, int M, int N, int K, int gated, int out_dtype,
