@@ -248,7 +248,9 @@ class HipOps:
         74; x 1,024 77 / 56, 69 / 58, 71 / 85; x 1,280 79 / 70, 77 / 74, 72 / 103; x 1,536 80 / 86, 81 / 92, 76 / 116; with wide W (the library
         at 16 rows) x 5,120 235 / 284, 252 / 289, 262 / 311; x 8,192 395 / 455, 417 / 473, 433 / 444; x 9,728 445 / 495, 466 / 504, 560 / 543. K beyond 4,096: 4,096 x 12,288 18.4 / 22.3, 17.7 / 21.2, 18.7 / 21.2, 21.3 / 21.7; 2,560 x 9,728 12.1 / 17.5, 12.8 / 15.6,
         13.1 / 15.6, 15.6 / 16.0; 2,048 x 8,192 9.2 / 12.7, 9.2 / 12.6, 10.0 / 12.6, 11.6 / 12.9; 8,192 x 12,288 36 / 42, 36 / 43, 37 / 44,
-        41 / 44. Gated, 12,288 x 4,096 34 against 41 for the x-resident and skinny products, 25,600 x 5,120 100 against 118."""
+        41 / 44; just beyond 4,096 the second span of eight waves is nearly empty, and with one tile a workgroup that is half of the time: 2,048 x 4,104
+        8.2 / 6.2, 8.5 / 6.6, 9.0 / 7.1, 10.5 / 8.1; 4,096 x 4,224 10.1 / 9.1, 10.5 / 9.6, 11.0 / 10.4, 12.5 / 12.0; 4,096 x 4,608 10.2 / 9.4, 10.5 / 9.9, 11.1 / 10.6,
+        12.4 / 12.7; 2,112 x 5,024 9.2 / 7.0 at 6 rows (5,120 x 4,224 13.3 / 13.4, 13.5 / 14.1, 14.1 / 15.3, 15.7 / 19.2; 4,096 x 5,120 10.3 / 10.5, 10.6 / 11.0, 11.1 / 12.1, 12.4 / 14.8). Gated, 12,288 x 4,096 34 against 41 for the x-resident and skinny products, 25,600 x 5,120 100 against 118."""
         if not self.lib.ra_gemm_sweep_fits(M, K):
             return False
         if M > 16 and not gated:             # 17 to 32 rows: 41 to 44 µs against the library's 49 and the SiLU-mul's 5
@@ -260,7 +262,7 @@ class HipOps:
             return False
         if K <= 4096:
             return rows >= 4 * self.cu_count and rows * K >= 4 << 20
-        return rows >= 8 * self.cu_count                      # rows of W a workgroup, at least
+        return rows >= (8 if K >= 5120 else 17) * self.cu_count                # rows of W a workgroup, at least
 
     def use_resident(self, M, N, K, gated):
         """Whether the product with x resident in LDS beats the skinny product for x [M, K] and

@@ -161,5 +161,6 @@ def test_products_of_up_to_16_rows_that_the_sweep_forms_more_slowly_are_not_its(
     for M, N, K, want in [(1, 65536, 1024, True), (1, 65537, 1024, False), (8, 151936, 512, False), (8, 151936, 1528, False), (8, 151936, 1536, True),
                           (9, 151936, 760, False), (9, 151936, 768, True), (16, 151936, 4096, True), (16, 151936, 5120, True), (16, 151936, 8192, True),
                           (16, 151936, 9728, False), (8, 151936, 9728, True), (16, 65536, 12288, True), (1, 1024, 4096, True), (1, 1023, 4096, False),
-                          (4, 3072, 512, False), (16, 2048, 8192, True), (16, 2047, 8192, False)]:
+                          (4, 3072, 512, False), (16, 2048, 8192, True), (16, 2047, 8192, False), (1, 4096, 4104, False), (16, 4351, 5112, False),
+                          (8, 4352, 4104, True), (8, 2048, 5120, True), (8, 2047, 5120, False)]:
         assert ops.use_sweep(M, N, K, False) == want, (M, N, K)
