@@ -264,6 +264,17 @@ class HipOps:
             return rows >= 4 * self.cu_count and rows * K >= 4 << 20
         return rows >= (8 if K >= 5120 else 17) * self.cu_count                # rows of W a workgroup, at least
 
+    def library_over_sweep(self, M, N, K):
+        """Whether a product that use_sweep would take is the library's, whose tiles are at their best where K is whole 512s (elsewhere it
+        takes up to twice as long): K beyond two spans of the sweep and up to 12,288, matrices beyond 32 Mi elements, columns for more than one tile a
+        workgroup but few rounds of them. Measured on MI355X, microseconds by the sweep / by the library, at 5, 8 and 16 rows: 5,120 x 8,704 22.3 /
+        20.2, 22.8 / 20.6, 25.3 / 22.0; 6,144 x 9,216 24.4 / 22.5, 25.1 / 22.7, 28.2 / 24.1; 7,168 x 9,728 27.4 / 26.8, 28.5 / 26.9, 31.5 / 27.3; 5,120 x 10,240
+        24.2 / 26.8, 25.0 / 27.2, 28.6 / 28.3; 6,144 x 11,264 26.5 / 26.4, 27.5 / 27.1, 30.6 / 28.6; 4,096 x 9,216 16.0 / 16.6, 16.3 / 16.6, 18.1 / 17.0; 5,120
+        x 8,448 22.2 / 28.0, 22.6 / 28.6, 25.1 / 30.2; 6,144 x 8,192 19.7 / 21.4, 19.9 / 21.9, 21.1 / 22.5; 6,144 x 12,288 27.5 / 30.3, 28.4 / 32.7, 32.2 / 34.3."""
+        if self.own_gemm or K % 512 or not 8192 < K < 12288 or N * K <= 32 << 20 or N >= 32 * self.cu_count:
+            return False
+        return M > 8 or (M > 4 and K < 10240 and N > 16 * self.cu_count)
+
     def use_resident(self, M, N, K, gated):
         """Whether the product with x resident in LDS beats the skinny product for x [M, K] and
         N result columns (measured on MI355X): when there are tiles of 16 columns enough for
@@ -1192,7 +1203,7 @@ class HipOps:
                 return "split4"
             out_dtype = torch.bfloat16
         if out_dtype in (torch.bfloat16, torch.float32) and self.use_sweep(M, N, K, False):
-            return "sweep"
+            return "library" if out_dtype == torch.bfloat16 and self.library_over_sweep(M, N, K) else "sweep"
         if out_dtype in (torch.bfloat16, torch.float32) and self.use_resident(M, N, K, False):
             return "resident512" if M <= 8 else "resident256"
         if out_dtype in (torch.bfloat16, torch.float32) and self.use_rows(M, N, K, False):

@@ -164,3 +164,16 @@ def test_products_of_up_to_16_rows_that_the_sweep_forms_more_slowly_are_not_its(
                           (4, 3072, 512, False), (16, 2048, 8192, True), (16, 2047, 8192, False), (1, 4096, 4104, False), (16, 4351, 5112, False),
                           (8, 4352, 4104, True), (8, 2048, 5120, True), (8, 2047, 5120, False)]:
         assert ops.use_sweep(M, N, K, False) == want, (M, N, K)
+
+
+def test_products_of_long_rows_that_the_library_forms_faster_are_its():
+    """(rows, result columns, K) on either side of the rule's lines at 256 CUs; only bfloat16 results are the library's."""
+    from return_amd.kernels.hip_ops import load_library
+    lib = load_library()
+    ops = kernel_set("cpu", ra_gemm_sweep_fits=lib.ra_gemm_sweep_fits)
+    ops.cu_count, ops.product_plan, ops.own_gemm = 256, {}, False
+    for M, N, K, want in [(5, 5120, 8704, "library"), (4, 5120, 8704, "sweep"), (8, 4096, 8704, "sweep"), (8, 4097, 8704, "library"), (9, 4096, 8704, "library"),
+                          (8, 8191, 9728, "library"), (8, 8192, 9728, "sweep"), (8, 5120, 10240, "sweep"), (16, 5120, 10240, "library"),
+                          (16, 5120, 12288, "sweep"), (16, 5120, 8448, "sweep"), (16, 6144, 8192, "sweep"), (16, 3072, 10240, "sweep")]:
+        assert ops.route_linear(M, N, K, BF) == want, (M, N, K)
+        assert ops.route_linear(M, N, K, torch.float32) == "sweep", (M, N, K)
