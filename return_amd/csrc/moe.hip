@@ -130,14 +130,14 @@ extern "C" int ra_moe_route(const float* z, const float* bias, int T, int E, int
 __host__ __device__ __forceinline__ bool moe_panel_height(int rows) {
     return rows == MOE_PANEL_ROWS || rows == MOE_PANEL_ROWS / 2 || rows == MOE_PANEL_ROWS / 4;
 }
-// Rows of an expert's tiles, and how many tiles its n rows make.
-__device__ __forceinline__ int moe_rows_of_tile(int n, int rows) {
-    if (rows < MOE_TILE_ROWS && !moe_panel_height(rows)) return rows;
+// Rows of an expert's tiles, and how many tiles its n rows make. PANEL: rows is one of those heights.
+template <bool PANEL> __device__ __forceinline__ int moe_rows_of_tile(int n, int rows) {
+    if (!PANEL && rows < MOE_TILE_ROWS) return rows;
     const int t = (n + rows - 1) / rows;
     return t > 1 ? min(rows, ((n + t - 1) / t + 15) & ~15) : rows;
 }
-__device__ __forceinline__ int moe_tiles_of(int n, int rows) {
-    const int per = moe_rows_of_tile(n, rows);
+template <bool PANEL> __device__ __forceinline__ int moe_tiles_of(int n, int rows) {
+    const int per = moe_rows_of_tile<PANEL>(n, rows);
     return (n + per - 1) / per;
 }
 // meta[0] = number of tiles. order [n_pairs], tiles [max_tiles][3].
@@ -146,15 +146,15 @@ __device__ __forceinline__ int moe_tiles_of(int n, int rows) {
 // sixteen waves would queue at the same few LDS words); and the sums over the experts are a scan over the threads, not a
 // loop of one of them (32 experts: 32 pairs 5.4 -> 4.0 us, 12,432 pairs 18.8 -> 9.9; 1,024
 // experts, 1,200 pairs 108 -> 4.4).
+// Tiles of panels (RUNS) have a kernel of their own: as a branch they cost every plan 0.1 to 0.3 us (32 experts 3.40 us, 3.28 without; 1,024 4.43 and 4.16; panels of
+// 32 experts 4.75 and 4.60).
 #define MOE_PLAN_EXPERTS 128
-__global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ ids, int n_pairs, int E, int rows,
+template <bool RUNS> __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ ids, int n_pairs, int E, int rows,
                                                         int* __restrict__ order, int* __restrict__ tiles,
                                                         int* __restrict__ meta) {
     __shared__ int place[MOE_MAX_EXPERTS > 16 * MOE_PLAN_EXPERTS ? MOE_MAX_EXPERTS : 16 * MOE_PLAN_EXPERTS];
     __shared__ unsigned long long wave_total[16];
-    __shared__ int sorted[MOE_MAX_EXPERTS], of_wave[MOE_PANEL_ROWS / 16 + 1][16], of_all[MOE_PANEL_ROWS / 16 + 1];
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
-    const bool runs = moe_panel_height(rows);
     const int copies = E <= MOE_PLAN_EXPERTS ? 16 : 1;
     int* mine = place + (copies == 16 ? wave : 0) * E;
     for (int i = tid; i < copies * E; i += 1024) place[i] = 0;
@@ -169,14 +169,15 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
     }
     __syncthreads();
     int e = tid;
-    if (runs) {
+    if constexpr (RUNS) {
+        __shared__ int sorted[MOE_MAX_EXPERTS], of_wave[MOE_PANEL_ROWS / 16 + 1][16], of_all[MOE_PANEL_ROWS / 16 + 1];
         // the experts with the largest tiles first, by groups of 16 rows: tiles go to the CUs in this order, and what is long must not come
         // last. Up to 64 experts each looks at all. Of more that took 5.5 of the plan's 10.5 us (256 experts) and 38 of 44 (1,024): a
         // counting sort, how many experts of a wave have as many groups, by ballots, and sums of those, 6.7 and 8.5 us in all (3.9 and 5.2 without the order).
         int n = 0, ahead = 0;
         if (tid < E)
             for (int c = 0; c < copies; ++c) n += place[c * E + tid];
-        const int groups = tid < E ? (min(n, moe_rows_of_tile(n, rows)) + 15) >> 4 : -1;
+        const int groups = tid < E ? (min(n, moe_rows_of_tile<RUNS>(n, rows)) + 15) >> 4 : -1;
         if (E <= 64) {
             if (tid < E) sorted[tid] = groups;
             __syncthreads();
@@ -210,7 +211,7 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
     int n = 0;
     if (tid < E)
         for (int c = 0; c < copies; ++c) n += place[c * E + e];
-    const int own_tiles = tid < E && n > 0 ? moe_tiles_of(n, rows) : 0;
+    const int own_tiles = tid < E && n > 0 ? moe_tiles_of<RUNS>(n, rows) : 0;
     unsigned long long sum = ((unsigned long long)n << 32) | (unsigned)own_tiles;
     const unsigned long long own = sum;
 #pragma unroll
@@ -226,16 +227,16 @@ __global__ __launch_bounds__(1024) void moe_plan_kernel(const int* __restrict__ 
     const int first = (int)(sum >> 32);
     if (tid < E) {
         int tl = (int)(sum & 0xffffffffull);
-        // runs: of an expert's groups of 16 rows every tile has as many, or one fewer, so that where there are several tiles none has
+        // RUNS: of an expert's groups of 16 rows every tile has as many, or one fewer, so that where there are several tiles none has
         // fewer than ten groups (of 3,649 rows the last of twelve had nine; it read W, which the others share, past the caches)
-        int per = moe_rows_of_tile(n, rows);
-        const int full = runs && own_tiles > 1 ? ((n + 15) >> 4) - (per / 16 - 1) * own_tiles : own_tiles;
+        int per = moe_rows_of_tile<RUNS>(n, rows);
+        const int full = RUNS && own_tiles > 1 ? ((n + 15) >> 4) - (per / 16 - 1) * own_tiles : own_tiles;
         for (int i = 0, j = 0; i < n; i += per, ++tl, ++j) {
-            if (j == full) per -= 16;
+            if (RUNS && j == full) per -= 16;
             tiles[3 * tl] = e;
             tiles[3 * tl + 1] = first + i;
             // (runs of up to four tiles of an expert: their number and the tile's place among them ride along)
-            tiles[3 * tl + 2] = min(per, n - i) | (runs ? (min(own_tiles - (j & ~3), 4) * 16 + (j & 3)) << 16 : 0);
+            tiles[3 * tl + 2] = min(per, n - i) | (RUNS ? (min(own_tiles - (j & ~3), 4) * 16 + (j & 3)) << 16 : 0);
         }
         // a pair's place among its expert's pairs is whatever the atomic gives: a row's result does not depend on its
         // place in a tile
@@ -261,8 +262,10 @@ extern "C" int ra_moe_plan(const int* ids, int n_pairs, int E, int rows, int* or
                            void* stream) {
     if (n_pairs <= 0) return RA_OK;
     if (E < 1 || E > MOE_MAX_EXPERTS || rows < 1) return RA_ERR_ARG;
-    hipLaunchKernelGGL(moe_plan_kernel, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, n_pairs, E, rows, order,
-                       tiles, meta);
+    if (moe_panel_height(rows))
+        hipLaunchKernelGGL(moe_plan_kernel<true>, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, n_pairs, E, rows, order, tiles, meta);
+    else
+        hipLaunchKernelGGL(moe_plan_kernel<false>, dim3(1), dim3(1024), 0, (hipStream_t)stream, ids, n_pairs, E, rows, order, tiles, meta);
     return ra_launch_status();
 }
 
