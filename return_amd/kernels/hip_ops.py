@@ -8,6 +8,7 @@ built or loaded, constructing HipOps raises.
 from __future__ import annotations
 
 import ctypes
+import functools
 from typing import Optional
 
 import torch
@@ -104,6 +105,8 @@ def _declare(lib):
         "ra_gemm_split_f32": [P, P, P, I, I, I, P, L, P],
         "ra_gemm_heads_fits": [I, I, I, I],
         "ra_gemm_heads_bf16": [P, L, L, P, P, L, L, I, I, I, I, P],
+        "ra_gemm_block_plan": [I, I, I, I, I, I, P, P],
+        "ra_gemm_block_bf16": [P, P, P, I, I, I, I, I, I, P],
         "ra_gemm_rows_fits": [I, I, I],
         "ra_gemm_rows_bf16": [P, P, P, I, I, I, I, I, I, I, P],
         "ra_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, P],
@@ -170,6 +173,13 @@ def _ptr(t: Optional[torch.Tensor]):
 _PRODUCTS_MEASURED = {}
 _PRODUCT_TIMES = {}        # the same keys -> {way: seconds}, as measured
 _NORM_PAIRS_MEASURED = {}  # (row step, shape of the product before a norm, of the one after, gated) -> the norm inside them is faster
+
+
+@functools.lru_cache(maxsize=4096)
+def _block_plan(M, N, K, gated, pieces, cus):
+    tiles, us = ctypes.c_int(), ctypes.c_float()
+    plan = load_library().ra_gemm_block_plan(M, N, K, gated, pieces, cus, ctypes.byref(tiles), ctypes.byref(us))
+    return None if plan < 0 else (plan, tiles.value, us.value)
 
 
 class HipOps:
@@ -1191,7 +1201,7 @@ class HipOps:
         """How linear() forms a bfloat16 product of M rows: the measured choice if there is one, else the rule.
         out_dtype "residual": the product whose result goes into the residual stream (linear_residual), bfloat16
         rows or, "split<n>", n shares of 32-bit sums over n pieces of K (up to 64 rows by the product that streams W through
-        LDS where it takes the pieces, else by the library's batched product)."""
+        LDS, beyond by the tiled one, where these take the pieces, else by the library's batched product)."""
         hit = self.product_plan.get((self._rows_step(M, out_dtype == "residual"), N, K, False, out_dtype))
         if hit is not None:
             return hit
@@ -1201,6 +1211,9 @@ class HipOps:
             # take 20 to 23 with W streamed through LDS, 22 to 24 as the library's batch
             if 16 < M <= 64 and K >= 8192 and N * 2 <= K and K % 32 == 0 and self._library_bmm_fp32:
                 return "split4"
+            pieces = self.use_block_residual(M, N, K)
+            if pieces:
+                return "block" if pieces == 1 else f"split{pieces}"
             out_dtype = torch.bfloat16
         if out_dtype in (torch.bfloat16, torch.float32) and self.use_sweep(M, N, K, False):
             return "library" if out_dtype == torch.bfloat16 and self.library_over_sweep(M, N, K) else "sweep"
@@ -1210,6 +1223,8 @@ class HipOps:
             return "rows"
         if self.use_skinny(M, N, K, out_dtype):
             return "skinny"
+        if out_dtype == torch.bfloat16 and self.use_block(M, N, K):
+            return "block"
         if not self.own_gemm and (out_dtype == torch.bfloat16 or self._library_fp32_out):
             return "library"
         return "mfma" if K % 8 == 0 else "plain"
@@ -1224,6 +1239,8 @@ class HipOps:
             return "sweep"
         if self.use_resident(M, I, K, True):
             return "resident512" if M <= 8 else "resident256"
+        if self.use_block_gated(M, I, K):
+            return "block"
         if 0 < M <= self.gated_skinny_rows and K % 8 == 0:
             return "skinny"
         return "two"
@@ -1258,6 +1275,59 @@ class HipOps:
                                                    _ptr(scratch), room, self._stream()), "gemm_split")
         return y
 
+    BLOCK_PIECES = 8              # pieces of K that a product for the residual stream is cut into, at most
+
+    def block_plan(self, M, N, K, gated, pieces=1):
+        """What the tiled product for more than 64 rows does with x [M, K] and N rows of W: (its plan, the number of its tiles,
+        the microseconds that it reckons with), K in up to `pieces` pieces (negative: exactly so many); None where it does not take
+        the sizes."""
+        return _block_plan(M, N, K, 1 if gated else 0, pieces, self.cu_count)
+
+    def use_block(self, M, N, K):
+        """Whether the tiled product forms a bfloat16 result of more than 64 rows. The library cuts K where tiles do not fill the chip,
+        this product has tiles of 64 x 128 at least: from 0.8 tiles a CU on. Beyond 1,536 rows of more than 4,096 columns the library has tiles
+        that fit multiples of 256 rows, and is the faster one on W of 40 Mi elements and more. Measured on MI355X, microseconds by it / by
+        the library, W from memory: 4,096 x 4,096 at 256, 420, 480, 800, 1,100 and 2,048 rows 29.2 / 22.8, 28.1 / 27.2, 27.9 / 28.7, 31.8 / 38.3,
+        42 / 48, 57.7 / 59.4; 6,144 x 2,560 at 256, 536, 1,200, 1,999 and 2,048 22.9 / 30.7, 24.6 / 29.4, 38.9 / 45.7, 57.6 / 57.5, 58.3 / 55.9; 6,144 x
+        4,096 at 2,048, 2,304, 2,804 and 3,000 87 / 82, 92 / 85, 132 / 212, 133 / 143; 10,496 x 4,096 at 1,999 and 2,112 146 / 202, 146 / 206; 12,288 x
+        4,096 at 256, 536, 1,400, 1,999 and 4,096 43.6 / 49.9, 58.8 / 57.3, 129 / 140, 170 / 162, 297 / 274; 1,536 x 512 5.5 to 12 / 6.4 to 15."""
+        if M <= 64 or self.own_gemm:
+            return False
+        if M > 1536 and N > 4096 and (M % 256 == 0 or N * K >= 40 << 20):
+            return False
+        plan = self.block_plan(M, N, K, False)
+        return plan is not None and plan[1] * 5 >= 4 * self.cu_count
+
+    def use_block_gated(self, M, I, K):
+        """Whether the tiled product forms silu(gate) * up of more than 64 rows (one kernel where the library's product and the SiLU-mul
+        are two): up to 128 rows from 48 rows of W a CU on. Measured on MI355X, microseconds by it / by the two: 12,288 x 4,096 at 90, 256,
+        536, 1,400, 2,048 and 2,804 rows 51 / 56, 69 / 72, 120 / 121, 242 / 261, 313 / 312, 458 / 521; 9,728 x 2,560 at 90, 536 and 2,048 34 / 36, 57 / 63, 192 /
+        226; 8,192 x 2,048 22 / 25, 42 / 48, 121 / 125; 3,072 x 4,096 28 / 26, 34 / 43, 93 / 92; 1,536 x 512 6.6 / 10, 7.1 / 13, 13 / 23."""
+        if M <= 64 or self.own_gemm or (M <= 128 and 2 * I < 48 * self.cu_count and K > 1024):
+            return False
+        return self.block_plan(M, 2 * I, K, True) is not None
+
+    def use_block_residual(self, M, N, K):
+        """The pieces of K that the tiled product takes for the residual stream (1: a bfloat16 result), or 0 where another is the rule's.
+        Measured on MI355X with the norm that takes the result, microseconds by it / by the best of the library's one product and its
+        batch over two or four pieces: 2,560 x 9,728 at 90, 256, 536, 1,024, 2,048 and 4,096 rows 24 / 25, 30 / 38, 42 / 50, 62 / 63, 105 / 105, 190 / 191; 2,560 x
+        4,096 17 / 17, 20 / 26, 27 / 31, 36 / 40, 58 / 62, 97 / 98; 4,096 x 4,096 18 / 20, 23 / 25, 33 / 36, 50 / 49, 77 / 79, 132 / 132; 4,096 x 12,288 32 / 33,
+        42 / 48, 67 / 69, 100 / 104, 178 / 178, 323 / 315. Rows of fewer than 2,048 columns are added up too slowly for shares (512 x 1,536
+        at 333 rows 13 / 10): they go as plain results do."""
+        if M <= 64 or self.own_gemm or N < 2048:
+            return 0
+        plan = self.block_plan(M, N, K, False, self.BLOCK_PIECES)
+        return 0 if plan is None else plan[0] >> 4
+
+    def _block_product(self, x, w, gated, plan, out_dtype):
+        M, K = x.shape
+        N, pieces = w.shape[0], plan >> 4
+        shape = (M, N // 2) if gated else (M, N) if pieces == 1 else (pieces, M, N)
+        out = torch.empty(shape, dtype=out_dtype, device=self.device)
+        self._check(self.lib.ra_gemm_block_bf16(_ptr(x), _ptr(w), _ptr(out), M, N, K, 1 if gated else 0, plan, _code(out_dtype),
+                                                self._stream()), "gemm_block")
+        return out
+
     def _rows_product(self, x, w, out, N, gated, pieces):
         M, K = x.shape
         self._check(self.lib.ra_gemm_rows_bf16(_ptr(x), _ptr(w), _ptr(out), M, N, K, 1 if gated else 0, pieces, _code(out.dtype),
@@ -1271,6 +1341,10 @@ class HipOps:
             if (x.data_ptr() | w.data_ptr()) % 16 == 0:
                 return self._rows_product(x, w, torch.empty(M, N, dtype=out_dtype, device=self.device), N, False, 1)
             how = "library" if out_dtype == torch.bfloat16 or self._library_fp32_out else "mfma"
+        if how == "block":
+            if (x.data_ptr() | w.data_ptr()) % 16 == 0:
+                return self._block_product(x, w, False, self.block_plan(M, N, K, False)[0], torch.bfloat16)
+            how = "library"
         if how == "library":
             if out_dtype == torch.bfloat16:
                 return torch.matmul(x, w.t())          # library product, as the reference's F.linear
@@ -1402,9 +1476,14 @@ class HipOps:
     def _split_product(self, x, w, pieces):
         """x @ w^T as `pieces` shares [pieces, M, N] fp32, share i from columns i*K/pieces .. of K: up to 64 rows by the
         product that streams W through LDS (down and o of the 8B shape at 64 rows in four pieces 23 and 10.6 us, the library's
-        batch 27 and 13.6), else one batched library product over strided views of x and w (nothing is copied)."""
+        batch 27 and 13.6), beyond by the tiled product (use_block_residual), else one batched library product over strided views of x
+        and w (nothing is copied)."""
         M, K = x.shape
         N = w.shape[0]
+        if M > 64 and not self.own_gemm and (x.data_ptr() | w.data_ptr()) % 16 == 0:
+            plan = self.block_plan(M, N, K, False, -pieces)
+            if plan is not None:
+                return Slabs(self._block_product(x, w, False, plan[0], torch.float32))
         if K % (128 * pieces) == 0 and self.lib.ra_gemm_rows_fits(M, N, K) and (x.data_ptr() | w.data_ptr()) % 16 == 0:
             return Slabs(self._rows_product(x, w, torch.empty(pieces, M, N, dtype=torch.float32, device=self.device), N, False, pieces))
         xs = x.view(M, pieces, K // pieces).transpose(0, 1)
@@ -1456,6 +1535,8 @@ class HipOps:
     def _gated_by(self, how, x, w_gate_up):
         M, K = x.shape
         I = w_gate_up.shape[0] // 2
+        if how == "block" and (x.data_ptr() | w_gate_up.data_ptr()) % 16 == 0:
+            return self._block_product(x, w_gate_up, True, self.block_plan(M, 2 * I, K, True)[0], x.dtype)
         out = torch.empty(M, I, dtype=x.dtype, device=self.device)
         if how == "rows" and (x.data_ptr() | w_gate_up.data_ptr()) % 16 == 0:
             return self._rows_product(x, w_gate_up, out, I, True, 1)
