@@ -29,6 +29,15 @@ typedef unsigned blk_u4 __attribute__((ext_vector_type(4)));
 
 enum { BLK_PLAIN = 0, BLK_GATED = 1, BLK_SHARES = 2 };
 
+// What a kernel behind the product would make of its results, which are rounded to bfloat16 first, bit for bit: bias added (gated: N
+// of them, gate and up halves; null: none); plain: act 2 max(y, 0)^2; gated: act 0 silu(g) u, 1 g sigmoid(slope g) (u + 1) with g = min(gate, limit),
+// u = clamp(up, -limit, limit). 2,048 rows of 12,288 squared by a kernel of their own 17 us, 2,333 of 8,192 columns biased and gated 30.
+struct BlockAct {
+    int kind;
+    float limit, slope;
+    const float* bias;
+};
+
 // Waits until at most COPIES of the wave's copies are on their way, and for its LDS reads.
 template <int COPIES>
 __device__ __forceinline__ void blk_wait() {
@@ -59,7 +68,7 @@ struct BlockTile {
 // up to 8 tiles, else 4), so that what its tiles share is read out of one L2.
 template <typename T, int MODE>
 __device__ __forceinline__ void block_tile(const bf16* __restrict__ X, const bf16* __restrict__ W, void* __restrict__ C, int M, int N, int K,
-                                           int tiles_m, int tiles_n, int k_piece) {
+                                           int tiles_m, int tiles_n, int k_piece, const BlockAct& act) {
     constexpr int NW = T::NW, TM = T::TM, TN = T::TN, SX = T::SX, SW = T::SW, XS = T::BM * 128, WS = T::BN * 128;
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, n = lane & 15, g = lane >> 4;
@@ -207,6 +216,13 @@ __device__ __forceinline__ void block_tile(const bf16* __restrict__ X, const bf1
         const int NO = MODE == BLK_GATED ? N >> 1 : N, c0 = (MODE == BLK_GATED ? n0 >> 1 : n0) + wn * COLS;
         __syncthreads();                                     // (everyone's copies have landed)
         const uint32_t mine = lds0 + wave * (2 * 16 * ROW);
+        blk_f4 bias[TN];                                     // of the wave's rows of W
+#pragma unroll
+        for (int a = 0; a < TN; ++a) {
+            const int col = c0 + (MODE == BLK_GATED ? a / 2 : a) * 16 + 4 * g;
+            bias[a] = blk_f4{0.f, 0.f, 0.f, 0.f};
+            if (act.bias != nullptr && col < NO) bias[a] = *reinterpret_cast<const blk_f4*>(act.bias + (MODE == BLK_GATED && (a & 1) ? NO : 0) + col);
+        }
 #pragma unroll
         for (int b = 0; b < TM; ++b) {
             const uint32_t buf = mine + (b & 1) * 16 * ROW;
@@ -216,10 +232,24 @@ __device__ __forceinline__ void block_tile(const bf16* __restrict__ X, const bf1
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
                     if constexpr (MODE == BLK_GATED) {
-                        const float gate = round_to<bf16>(acc[a][b][e]), up = round_to<bf16>(acc[a + 1][b][e]);
-                        v[e] = gate / (1.0f + expf(-gate)) * up;
+                        float gate = round_to<bf16>(acc[a][b][e]), up = round_to<bf16>(acc[a + 1][b][e]);
+                        if (act.bias != nullptr) {
+                            gate += bias[a][e];
+                            up += bias[a + 1][e];
+                        }
+                        if (act.kind == 1) {
+                            const float x = fminf(gate, act.limit), u = fminf(fmaxf(up, -act.limit), act.limit);
+                            v[e] = x / (1.0f + expf(-act.slope * x)) * (u + 1.0f);
+                        } else {
+                            v[e] = gate / (1.0f + expf(-gate)) * up;
+                        }
                     } else {
-                        v[e] = acc[a][b][e];
+                        v[e] = round_to<bf16>(acc[a][b][e]);
+                        if (act.bias != nullptr) v[e] += bias[a][e];
+                        if (act.kind == 2) {
+                            v[e] = fmaxf(v[e], 0.f);
+                            v[e] *= v[e];
+                        }
                     }
                 }
                 *(blk_u2 __attribute__((address_space(3)))*)(uintptr_t)(buf + n * ROW + (MODE == BLK_GATED ? a / 2 : a) * 32 + g * 8) =
@@ -241,8 +271,8 @@ __device__ __forceinline__ void block_tile(const bf16* __restrict__ X, const bf1
 
 template <typename T, int MODE>
 __global__ __launch_bounds__(512, 1) void gemm_block_kernel(const bf16* __restrict__ X, const bf16* __restrict__ W, void* __restrict__ C, int M, int N,
-                                                            int K, int tiles_m, int tiles_n, int k_piece) {
-    block_tile<T, MODE>(X, W, C, M, N, K, tiles_m, tiles_n, k_piece);
+                                                            int K, int tiles_m, int tiles_n, int k_piece, const BlockAct act) {
+    block_tile<T, MODE>(X, W, C, M, N, K, tiles_m, tiles_n, k_piece, act);
 }
 
 // The tiles: rows of x, rows of W, microseconds a step of 64 columns and what start and end of a tile take, fitted to 4,700 measurements
@@ -299,12 +329,12 @@ extern "C" int ra_gemm_block_plan(int M, int N, int K, int gated, int pieces, in
 }
 
 template <typename T>
-static int block_go(hipStream_t st, const void* X, const void* W, void* C, int M, int N, int K, int mode, int pieces) {
+static int block_go(hipStream_t st, const void* X, const void* W, void* C, int M, int N, int K, int mode, int pieces, const BlockAct& act) {
     const int tm = (M + T::BM - 1) / T::BM, tn = (N + T::BN - 1) / T::BN;
     const dim3 grid((unsigned)((long long)tm * tn * pieces)), block(512);
     auto go = [&](auto kernel) {
         if (hipFuncSetAttribute((const void*)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, T::LDS) != hipSuccess) return RA_ERR_LAUNCH;
-        hipLaunchKernelGGL(kernel, grid, block, T::LDS, st, (const bf16*)X, (const bf16*)W, C, M, N, K, tm, tn, K / pieces);
+        hipLaunchKernelGGL(kernel, grid, block, T::LDS, st, (const bf16*)X, (const bf16*)W, C, M, N, K, tm, tn, K / pieces, act);
         return ra_launch_status();
     };
     return mode == BLK_PLAIN ? go(gemm_block_kernel<T, BLK_PLAIN>) : mode == BLK_GATED ? go(gemm_block_kernel<T, BLK_GATED>)
@@ -312,8 +342,9 @@ static int block_go(hipStream_t st, const void* X, const void* W, void* C, int M
 }
 
 // plan: what ra_gemm_block_plan gave for these sizes. gated: N rows of W are gate and up halves, C [M, N / 2] bfloat16. Else C [M, N]
-// bfloat16 (one piece) or 32-bit [pieces, M, N]. x, W and C 16-byte aligned.
-extern "C" int ra_gemm_block_bf16(const void* X, const void* W, void* C, int M, int N, int K, int gated, int plan, int out_dtype, void* stream) {
+// bfloat16 (one piece) or 32-bit [pieces, M, N]. x, W, C and bias 16-byte aligned. act, limit, slope, bias: BlockAct, for bfloat16 results.
+extern "C" int ra_gemm_block_bf16(const void* X, const void* W, void* C, int M, int N, int K, int gated, int plan, int out_dtype, int act, float limit,
+                                  float slope, const float* bias, void* stream) {
     const int tile = plan & 15, pieces = plan >> 4;
     if (plan < 0 || M <= 0 || N <= 0 || K <= 0 || pieces < 1 || pieces > BLK_PIECES || K % (64 * pieces) != 0 || N % (gated ? 16 : 8) != 0)
         return RA_ERR_ARG;
@@ -321,11 +352,14 @@ extern "C" int ra_gemm_block_bf16(const void* X, const void* W, void* C, int M, 
         return RA_ERR_ARG;
     if ((gated || out_dtype != RA_DTYPE_F32) && (pieces != 1 || out_dtype != RA_DTYPE_BF16)) return RA_ERR_ARG;
     if ((long long)((M + 63) / 64) * ((N + 127) / 128) * pieces > 0x7fffffff) return RA_ERR_ARG;
+    if (act < 0 || act > 2 || (act == 2 && gated) || (act == 1 && (!gated || !(limit > 0.f))) || ((uintptr_t)bias & 15) != 0) return RA_ERR_ARG;
+    if (out_dtype == RA_DTYPE_F32 && (act != 0 || bias != nullptr)) return RA_ERR_ARG;
+    const BlockAct with = {act, limit, slope, bias};
     const int mode = gated ? BLK_GATED : out_dtype == RA_DTYPE_F32 ? BLK_SHARES : BLK_PLAIN;
     hipStream_t st = (hipStream_t)stream;
     switch (tile) {
 #define BLK_CASE(ID, BM, BN, WM, WN, SX, SW, STEP, ENDS) \
-    case ID: return block_go<BlockTile<BM, BN, WM, WN, SX, SW>>(st, X, W, C, M, N, K, mode, pieces);
+    case ID: return block_go<BlockTile<BM, BN, WM, WN, SX, SW>>(st, X, W, C, M, N, K, mode, pieces, with);
         BLK_TILES(BLK_CASE)
     }
     return RA_ERR_ARG;

@@ -63,7 +63,33 @@ struct SweepNorm {
     float* h;                  // RESID: residual stream [M, N], updated in place
     const float* w_next;       // RESID: weight [N] of the norm that follows
     float* psq_out;            // RESID: [M, gridDim.x]
+    const float* bias;         // ACT: added to the sums, which are rounded to bfloat16 first ([N], gated [2N]; null: none)
+    int act;                   // ACT: plain 0 nothing, 2 max(y, 0)^2; gated 0 silu(g) u, 1 clamped: g sigmoid(slope g) (u + 1) with
+    float limit, slope;        //      g = min(gate, limit), u = clamp(up, -limit, limit)
 };
+
+// ACT: what a kernel behind the product would make of a result (of a gate and an up result), whose sums are s (and up), bit for bit. As kernels
+// of their own these were 4.6 us each in a decode step (a squared ReLU of 12,288 columns, biases, a gated product of its biased halves): start and end
+// of a kernel.
+template <bool GATED>
+__device__ __forceinline__ float sweep_act(float s, float up, float b, float b_up, const SweepNorm& nm) {
+    s = round_to<bf16>(s);
+    if (nm.bias != nullptr) s += b;
+    if constexpr (GATED) {
+        up = round_to<bf16>(up);
+        if (nm.bias != nullptr) up += b_up;
+        if (nm.act == 1) {
+            const float g = fminf(s, nm.limit), u = fminf(fmaxf(up, -nm.limit), nm.limit);
+            return g / (1.0f + expf(-nm.slope * g)) * (u + 1.0f);
+        }
+        return s / (1.0f + expf(-s)) * up;
+    }
+    if (nm.act == 2) {
+        const float v = fmaxf(s, 0.f);
+        return v * v;
+    }
+    return s;
+}
 
 // rstd of up to 16 * MB rows into LDS (rs), from the partial sums: thread (row, j) adds partials j,
 // j + 16, ..., the sixteen threads of a row are then added in a fixed tree.
@@ -162,11 +188,12 @@ template <int COLS, bool NEAR> struct SweepCols {
 };
 
 // MB: blocks of 16 rows of x (1 or 2). LINES: x as whole lines (SweepX), else as operands straight from memory. NEAR: see SweepCols.
-template <int MB, bool GATED, typename TO, bool RESID, bool LINES, bool NEAR>
+template <int MB, bool GATED, typename TO, bool RESID, bool LINES, bool NEAR, bool ACT = false>
 __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ W, TO* __restrict__ out, int M, int N, int K, SweepNorm nm) {
     static_assert(!RESID || (!GATED && MB == 1), "the residual epilogue belongs to the plain product of up to 16 rows");
     static_assert(!LINES || MB == 1, "32 rows as lines are more registers than there are");
+    static_assert(!ACT || (!RESID && MB == 1), "an activation belongs to results of up to 16 rows that are stored as they are");
     constexpr int COLS = GATED ? 8 : 16;                        // result columns of a tile
     constexpr int RS = 16 * MB + 1;                             // row stride of the waves' tiles in LDS (floats)
     constexpr bool TWO_BUFFERS = MB == 1;                       // of those tiles (LDS has room for one set with MB == 2)
@@ -228,6 +255,14 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
             h_old = nm.h[(size_t)mm * N + col];
             wn = nm.w_next[col];
         }
+        [[maybe_unused]] float bias = 0.f, bias_up = 0.f;      // (likewise)
+        if constexpr (ACT) {
+            if (nm.bias != nullptr) {
+                const int col = min(cols.at(t, tid % COLS), N - 1);
+                bias = nm.bias[col];
+                if constexpr (GATED) bias_up = nm.bias[N + col];
+            }
+        }
         SW_WAVE_SYNC();                                         // the tile before has been read out of the wave's LDS
         // row by row: as soon as a row has arrived and gone into LDS, the same row of the next tile is
         // asked for, so that the loads on their way never run out at a tile's end
@@ -270,7 +305,10 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
                     float up = 0.f;
 #pragma unroll
                     for (int w = 0; w < SW_WAVES; ++w) up += red[(w * 16 + 8 + r) * RS + mm];
-                    s = s / (1.0f + expf(-s)) * (up * scale); // gate and up stay 32-bit until here
+                    if constexpr (ACT) s = sweep_act<true>(s, up * scale, bias, bias_up, nm);
+                    else s = s / (1.0f + expf(-s)) * (up * scale); // gate and up stay 32-bit until here
+                } else if constexpr (ACT) {
+                    s = sweep_act<false>(s, 0.f, bias, 0.f, nm);
                 }
                 if constexpr (RESID) {
                     const size_t at = (size_t)mm * N + col;
@@ -299,7 +337,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_kernel(
 #define SW_SPAN (SW_WAVES * SW_KW)        // columns of K that the eight waves cover at once
 
 // HELD: K is at most two spans, and the columns of x of both stay in registers for all tiles.
-template <bool GATED, typename TO, bool RESID = false, bool HELD = false>
+template <bool GATED, typename TO, bool RESID = false, bool HELD = false, bool ACT = false>
 __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ W, TO* __restrict__ out, int M, int N, int K, SweepNorm nm) {
     static_assert(!RESID || !GATED, "the residual epilogue belongs to the plain product");
@@ -347,6 +385,14 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
             h_old = nm.h[(size_t)mm * N + col];
             wn = nm.w_next[col];
         }
+        [[maybe_unused]] float bias = 0.f, bias_up = 0.f;      // (likewise)
+        if constexpr (ACT) {
+            if (nm.bias != nullptr) {
+                const int col = min(cols.at(t, tid % COLS), N - 1);
+                bias = nm.bias[col];
+                if constexpr (GATED) bias_up = nm.bias[N + col];
+            }
+        }
         float4_t c = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int p = 0; p < (HELD ? 2 : spans); ++p) {
@@ -391,7 +437,10 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
                     float up = 0.f;
 #pragma unroll
                     for (int w = 0; w < SW_WAVES; ++w) up += red[(w * 16 + 8 + r) * 17 + mm];
-                    s = s / (1.0f + expf(-s)) * (up * scale);
+                    if constexpr (ACT) s = sweep_act<true>(s, up * scale, bias, bias_up, nm);
+                    else s = s / (1.0f + expf(-s)) * (up * scale);
+                } else if constexpr (ACT) {
+                    s = sweep_act<false>(s, 0.f, bias, 0.f, nm);
                 }
                 if constexpr (RESID) {
                     const size_t at = (size_t)mm * N + col;
@@ -420,7 +469,7 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_long_kernel(
 // projection): span by span, so that a span's columns of x are read once and serve every tile; the tiles'
 // sums stay in registers until the last span. (gemm_sweep_long_kernel reads x again for every tile, as many
 // bytes as the tile of W.)
-template <bool GATED, typename TO, bool RESID = false>
+template <bool GATED, typename TO, bool RESID = false, bool ACT = false>
 __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_spans_kernel(
     const bf16* __restrict__ x, const bf16* __restrict__ W, TO* __restrict__ out, int M, int N, int K, SweepNorm nm) {
     static_assert(!RESID || !GATED, "the residual epilogue belongs to the plain product");
@@ -457,6 +506,15 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_spans_kernel(
     // RESID: the tiles' entries of h and of the next norm's weight are asked for at the start of the last
     // span, before its rows of W (asked for in the epilogue they would be waited for; see the kernel above)
     [[maybe_unused]] float h_old[SW_FEW_TILES], wn[SW_FEW_TILES];
+    [[maybe_unused]] float bias[SW_FEW_TILES], bias_up[SW_FEW_TILES];
+    if constexpr (ACT) {
+#pragma unroll
+        for (int t = 0; t < SW_FEW_TILES; ++t) {
+            const int col = min(cols.at(min(t, n_tiles - 1), tid % COLS), N - 1);
+            bias[t] = nm.bias != nullptr ? nm.bias[col] : 0.f;
+            bias_up[t] = GATED && nm.bias != nullptr ? nm.bias[N + col] : 0.f;
+        }
+    }
     for (int p = 0; p < spans; ++p) {
         if constexpr (RESID) {
             if (p == spans - 1) {
@@ -515,7 +573,10 @@ __global__ __launch_bounds__(SW_THREADS) void gemm_sweep_spans_kernel(
                     float up = 0.f;
 #pragma unroll
                     for (int w = 0; w < SW_WAVES; ++w) up += red[(w * 16 + 8 + r) * 17 + mm];
-                    s = s / (1.0f + expf(-s)) * (up * scale);
+                    if constexpr (ACT) s = sweep_act<true>(s, up * scale, bias[t], bias_up[t], nm);
+                    else s = s / (1.0f + expf(-s)) * (up * scale);
+                } else if constexpr (ACT) {
+                    s = sweep_act<false>(s, 0.f, bias[t], 0.f, nm);
                 }
                 if constexpr (RESID) {
                     const size_t at = (size_t)mm * N + col;
@@ -561,24 +622,24 @@ static int launch_sweep_kernel(KERN kern, bool& allowed, int grid, hipStream_t s
     return RA_OK;
 }
 
-template <bool GATED, typename TO, bool RESID>
+template <bool GATED, typename TO, bool RESID, bool ACT = false>
 static int launch_sweep(int grid, hipStream_t st, const bf16* x, const bf16* W, TO* out, int M, int N, int K,
                         const SweepNorm& nm) {
     if (K > SW_SPAN) {
         if (K <= 2 * SW_SPAN) {
             static bool allowed = false;
-            return launch_sweep_kernel(gemm_sweep_long_kernel<GATED, TO, RESID, true>, allowed, grid, st, x, W, out, M, N, K, nm);
+            return launch_sweep_kernel(gemm_sweep_long_kernel<GATED, TO, RESID, true, ACT>, allowed, grid, st, x, W, out, M, N, K, nm);
         }
         const int cols = GATED ? 8 : 16, workgroups = grid < N ? grid : N;
         const int most_tiles = ((N + workgroups - 1) / workgroups + cols - 1) / cols;
         if (most_tiles >= 2 && most_tiles <= SW_FEW_TILES) {    // (with one tile the two orders are the same, and this one a little slower)
             static bool allowed = false;
-            return launch_sweep_kernel(gemm_sweep_spans_kernel<GATED, TO, RESID>, allowed, grid, st, x, W, out, M, N, K, nm);
+            return launch_sweep_kernel(gemm_sweep_spans_kernel<GATED, TO, RESID, ACT>, allowed, grid, st, x, W, out, M, N, K, nm);
         }
         static bool allowed = false;
-        return launch_sweep_kernel(gemm_sweep_long_kernel<GATED, TO, RESID, false>, allowed, grid, st, x, W, out, M, N, K, nm);
+        return launch_sweep_kernel(gemm_sweep_long_kernel<GATED, TO, RESID, false, ACT>, allowed, grid, st, x, W, out, M, N, K, nm);
     }
-    if constexpr (!RESID) {
+    if constexpr (!RESID && !ACT) {
         if (M > 16) {
             if (GATED && N > 2 * grid * 8) {
                 static bool allowed = false;
@@ -594,10 +655,10 @@ static int launch_sweep(int grid, hipStream_t st, const bf16* x, const bf16* W, 
     // 1,544 0.92 and 0.91, 2,056 0.94 and 0.90, 3,080 0.95 and 0.96.
     if (M > 4 && (K < 3 * SW_KW || K % 64 != 0) && N <= grid * (GATED ? 8 : 16)) {
         static bool allowed = false;
-        return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, false, true>, allowed, grid, st, x, W, out, M, N, K, nm);
+        return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, false, true, ACT>, allowed, grid, st, x, W, out, M, N, K, nm);
     }
     static bool allowed = false;
-    return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, true, true>, allowed, grid, st, x, W, out, M, N, K, nm);
+    return launch_sweep_kernel(gemm_sweep_kernel<1, GATED, TO, RESID, true, true, ACT>, allowed, grid, st, x, W, out, M, N, K, nm);
 }
 
 static int sweep_dispatch(const void* x, const void* W, void* out, int M, int N, int K, int gated, int out_dtype,
@@ -646,6 +707,24 @@ extern "C" int ra_gemm_sweep_norm_bf16(const void* x, const void* W, void* out, 
     if ((h == nullptr) != (w_next == nullptr) || (h == nullptr) != (psq_out == nullptr)) return RA_ERR_ARG;
     if (psq_in != nullptr && (n_in <= 0 || n_in > 16 * SW_SHARES || norm_cols <= 0)) return RA_ERR_ARG;
     if (M > 32) return RA_ERR_ARG;                            // the row scales of a workgroup are at most 32
-    SweepNorm nm = {psq_in, n_in, norm_cols > 0 ? 1.0f / (float)norm_cols : 0.f, eps, h, w_next, psq_out};
+    SweepNorm nm = {psq_in, n_in, norm_cols > 0 ? 1.0f / (float)norm_cols : 0.f, eps, h, w_next, psq_out, nullptr, 0, 0.f, 0.f};
     return sweep_dispatch(x, W, out, M, N, K, gated, out_dtype, grid, nm, stream);
+}
+
+// The plain bfloat16 product of up to 16 rows, or the gated one, with what a kernel behind it would make of its results (sweep_act): act, limit,
+// slope and bias as SweepNorm has them.
+extern "C" int ra_gemm_sweep_act_bf16(const void* x, const void* W, void* out, int M, int N, int K, int gated, int grid, int act, float limit,
+                                      float slope, const float* bias, void* stream) {
+    if (M <= 0 || N <= 0) return RA_OK;
+    if (M > 16 || !ra_gemm_sweep_fits(M, K) || grid <= 0 || act < 0 || act > 2 || (act == 2 && gated) || (act == 1 && (!gated || !(limit > 0.f))))
+        return RA_ERR_ARG;
+    if (grid > N) grid = N;
+    SweepNorm nm = {};
+    nm.bias = bias;
+    nm.act = act;
+    nm.limit = limit;
+    nm.slope = slope;
+    const int rc = gated ? launch_sweep<true, bf16, false, true>(grid, (hipStream_t)stream, (const bf16*)x, (const bf16*)W, (bf16*)out, M, N, K, nm)
+                         : launch_sweep<false, bf16, false, true>(grid, (hipStream_t)stream, (const bf16*)x, (const bf16*)W, (bf16*)out, M, N, K, nm);
+    return rc != RA_OK ? rc : ra_launch_status();
 }

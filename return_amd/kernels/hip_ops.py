@@ -106,7 +106,8 @@ def _declare(lib):
         "ra_gemm_heads_fits": [I, I, I, I],
         "ra_gemm_heads_bf16": [P, L, L, P, P, L, L, I, I, I, I, P],
         "ra_gemm_block_plan": [I, I, I, I, I, I, P, P],
-        "ra_gemm_block_bf16": [P, P, P, I, I, I, I, I, I, P],
+        "ra_gemm_block_bf16": [P, P, P, I, I, I, I, I, I, I, F, F, P, P],
+        "ra_gemm_sweep_act_bf16": [P, P, P, I, I, I, I, I, I, F, F, P, P],
         "ra_gemm_rows_fits": [I, I, I],
         "ra_gemm_rows_bf16": [P, P, P, I, I, I, I, I, I, I, P],
         "ra_gemm_skinny_bf16": [P, P, P, I, I, I, I, I, P],
@@ -1319,13 +1320,13 @@ class HipOps:
         plan = self.block_plan(M, N, K, False, self.BLOCK_PIECES)
         return 0 if plan is None else plan[0] >> 4
 
-    def _block_product(self, x, w, gated, plan, out_dtype):
+    def _block_product(self, x, w, gated, plan, out_dtype, act=0, limit=0.0, slope=0.0, bias=None):
         M, K = x.shape
         N, pieces = w.shape[0], plan >> 4
         shape = (M, N // 2) if gated else (M, N) if pieces == 1 else (pieces, M, N)
         out = torch.empty(shape, dtype=out_dtype, device=self.device)
         self._check(self.lib.ra_gemm_block_bf16(_ptr(x), _ptr(w), _ptr(out), M, N, K, 1 if gated else 0, plan, _code(out_dtype),
-                                                self._stream()), "gemm_block")
+                                                act, limit, slope, _ptr(bias), self._stream()), "gemm_block")
         return out
 
     def _rows_product(self, x, w, out, N, gated, pieces):
@@ -1570,6 +1571,61 @@ class HipOps:
             raise KernelError(f"linear_silu_mul: x {tuple(x.shape)}, weight {tuple(w_gate_up.shape)}")
         how = self.route_gated(M, I, K) if x.dtype == torch.bfloat16 and M > 0 else "two"
         return self._gated_by(how, x, w_gate_up)
+
+    # ---- a product and the row kernel behind it in one (the same bits): where the sweep or the tiled product forms it
+    def _act_by(self, x, w, gated, act, limit, slope, bias):
+        """The product with its activation or bias, or None where it is formed by a way that has none."""
+        if isinstance(x, ScaledRows) or x.dtype != torch.bfloat16 or x.shape[0] == 0 or x.shape[1] != w.shape[1] or w.dtype != x.dtype:
+            return None
+        self._want(x, "x", dims=2)
+        self._want(w, "weight", dims=2)
+        M, K = x.shape
+        N = w.shape[0] // 2 if gated else w.shape[0]
+        if bias is not None:
+            self._want(bias, "bias", torch.float32, 1)
+            if bias.shape[0] != w.shape[0]:
+                raise KernelError(f"product: bias {tuple(bias.shape)} for weight {tuple(w.shape)}")
+        if M <= 16 and (self.use_sweep(M, N, K, True) if gated else self.route_linear(M, N, K, torch.bfloat16) == "sweep"):
+            out = torch.empty(M, N, dtype=x.dtype, device=self.device)
+            self._check(self.lib.ra_gemm_sweep_act_bf16(_ptr(x), _ptr(w), _ptr(out), M, N, K, 1 if gated else 0, self.cu_count, act, limit, slope,
+                                                        _ptr(bias), self._stream()), "gemm_sweep_act")
+            return out
+        # (the row kernel's time is in the bargain, so the library's large tiles have no edge: use_block's lines for many rows do not count)
+        if M > 64 and not self.own_gemm and (x.data_ptr() | w.data_ptr() | (bias.data_ptr() if bias is not None else 0)) % 16 == 0:
+            plan = self.block_plan(M, w.shape[0], K, gated)
+            if plan is not None and (self.use_block_gated(M, N, K) if gated else plan[1] * 5 >= 4 * self.cu_count):
+                return self._block_product(x, w, gated, plan[0], x.dtype, act, limit, slope, bias)
+        return None
+
+    def linear_bias(self, x, w, bias):
+        """add_bias(linear(x, w), bias)."""
+        y = self._act_by(x, w, False, 0, 0.0, 0.0, bias)
+        return self.add_bias(self.linear(x, w), bias) if y is None else y
+
+    def linear_relu_sq(self, x, w):
+        """relu_sq(linear(x, w))."""
+        y = self._act_by(x, w, False, 2, 0.0, 0.0, None)
+        return self.relu_sq(self.linear(x, w)) if y is None else y
+
+    def linear_gated_bias(self, x, w_gate_up, bias):
+        """silu_mul(linear(x, w_gate_up), bias=bias)."""
+        y = self._act_by(x, w_gate_up, True, 0, 0.0, 0.0, bias)
+        if y is None:
+            gu = self.linear(x, w_gate_up)
+            y = torch.empty(gu.shape[0], gu.shape[1] // 2, dtype=gu.dtype, device=self.device)
+            self.silu_mul(gu, y, bias=bias)
+        return y
+
+    def linear_clamped(self, x, w_gate_up, limit, slope=1.702):
+        """gated_rows(linear(x, w_gate_up), "clamped", limit, slope)."""
+        if not limit > 0:
+            raise KernelError(f"linear_clamped: limit {limit} must be positive")
+        y = self._act_by(x, w_gate_up, True, 1, float(limit), float(slope), None)
+        if y is None:
+            gu = self.linear(x, w_gate_up)
+            y = torch.empty(gu.shape[0], gu.shape[1] // 2, dtype=gu.dtype, device=self.device)
+            self.gated_rows(gu, y, "clamped", limit, slope)
+        return y
 
     def _candidates(self, M, N, K, gated, out_dtype):
         """The ways that can form this product at all."""

@@ -127,6 +127,8 @@ class PagedAttention:
             o = rt.empty(T, Hq, D)
             ops.attention(q, o, cache.k_pool, cache.v_pool, step, cache.group, self.scale,
                           int(self.window) if self.window else 0, **self.extras)
+            if self.bias_o is not None and sink is None and hasattr(ops, "linear_bias"):
+                return ops.linear_bias(o.view(T, Hq * D), self.w_o, self.bias_o)
             y = project(o.view(T, Hq * D), self.w_o)
             return ops.add_bias(y, self.bias_o) if self.bias_o is not None else y
         if self._fusable and not self.extras and write_cache and hasattr(ops, "attention_qkv"):

@@ -41,6 +41,8 @@ class SwiGLU:
     def forward(self, x, step=None, sink=None):
         ops = self.rt.ops
         if self.bias_in is not None:
+            if hasattr(ops, "linear_gated_bias"):          # (a kernel set that has the two as one)
+                return ops.linear_bias(ops.linear_gated_bias(x, self.w_gate_up, self.bias_in), self.w_down, self.bias_out)
             gu = ops.linear(x, self.w_gate_up)             # [T, 2 I], gate columns first
             a = self.rt.empty(x.shape[0], self.inter)
             ops.silu_mul(gu, a, bias=self.bias_in)         # silu(gate + b_g) * (up + b_u)
@@ -71,7 +73,8 @@ class SquaredReLU:
 
     def forward(self, x, step=None):
         ops = self.rt.ops
-        return ops.linear(ops.relu_sq(ops.linear(x, self.w_up)), self.w_down)
+        up = ops.linear_relu_sq(x, self.w_up) if hasattr(ops, "linear_relu_sq") else ops.relu_sq(ops.linear(x, self.w_up))
+        return ops.linear(up, self.w_down)
 
 
 register_part("feed_forward", "relu2", SquaredReLU)
@@ -102,6 +105,8 @@ class ClampedGLU:
 
     def forward(self, x, step=None):
         ops = self.rt.ops
+        if hasattr(ops, "linear_clamped"):
+            return ops.linear(ops.linear_clamped(x, self.w_gate_up, self.limit, self.slope), self.w_down)
         a = self.rt.empty(x.shape[0], self.inter)
         ops.gated_rows(ops.linear(x, self.w_gate_up), a, "clamped", self.limit, self.slope)
         return ops.linear(a, self.w_down)

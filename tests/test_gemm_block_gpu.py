@@ -32,7 +32,8 @@ def test_every_tile_at_its_edges(ops, tile, K):
         assert bool(((y.double() - want).abs() <= bound(K, want)).all()), (M, N)
         for pieces in (1, 2) if K > 64 and K % 128 == 0 else (1,):
             y = torch.full((pieces, M, N), float("nan"), device=x.device)
-            ops._check(ops.lib.ra_gemm_block_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, 0, tile + 16 * pieces, 0, ops._stream()), "")
+            ops._check(ops.lib.ra_gemm_block_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, 0, tile + 16 * pieces, 0, 0, 0.0, 0.0, None,
+                                                   ops._stream()), "")
             torch.testing.assert_close(y.double().sum(0), want, atol=2.0 ** -22 * K, rtol=1e-6)
     for M, I in [(bm + 1, bn // 2 + 8), (65, 8)]:
         x, w = rnd(M, K, dtype=BF, seed=M), rnd(2 * I, K, dtype=BF, seed=I, scale=0.2)
@@ -100,7 +101,7 @@ def test_plans_and_calls_that_are_refused():
     for plan, M, N, K, gated, dtype, at in [(-1, 64, 64, 64, 0, 1, 0), (12 + 16, 64, 64, 64, 0, 1, 0), (0, 64, 64, 64, 0, 1, 0), (9 + 32, 64, 64, 64, 0, 0, 0),
                                             (9 + 32, 64, 64, 128, 0, 1, 0), (9 + 16, 64, 64, 64, 1, 0, 0), (9 + 16, 64, 60, 64, 0, 1, 0),
                                             (9 + 16, 64, 64, 64, 0, 1, 8), (9 + 16 * 9, 64, 64, 576, 0, 0, 0)]:
-        assert lib.ra_gemm_block_bf16(16 + at, 16, 16, M, N, K, gated, plan, dtype, None) != 0, plan
+        assert lib.ra_gemm_block_bf16(16 + at, 16, 16, M, N, K, gated, plan, dtype, 0, 0.0, 0.0, None, None) != 0, plan
 
 
 @pytest.mark.skipif(not (shutil.which("hipcc") or os.path.exists("/opt/rocm/bin/hipcc")), reason="no hipcc")
