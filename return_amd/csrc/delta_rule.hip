@@ -20,7 +20,8 @@
 // long pole, and it is as long for 16 columns as for 128. The output kernel norms a head's read-out
 // over all its columns, weighs and gates it: a wave per (row, head). In bf16 requests of rc_min_rows rows and
 // more go by chunks on the matrix cores (recurrence_chunks.hip) if a head has at most 128 channels; other requests of eight
-// rows and more take the recurrence kernel with feeder waves (below); single tokens and short portions the plain one, which
+// rows and more take the recurrence kernel with feeder waves (below); steps of single tokens a kernel of their own (delta_one_kernel) where
+// the sizes allow it; other single tokens and short portions the plain one, which
 // needs half the threads, few registers and little LDS, so that many workgroups share a CU.
 //
 // A second rule runs on the same kernels (rule 1, "outer"): the gated outer-product memory of a linear attention,
@@ -516,18 +517,9 @@ __device__ __forceinline__ float sum_of_quads(float (&v)[4]) {
 // The same for bfloat16 with four neighbours a lane: L lanes to a (row, head) of V = 4 L (V 64, 128 or 256, gate, norm and result
 // in whole pieces of four), the sum formed in the order of the kernel above: the same bits. Bound by its rows: 2,048 rows of 32
 // heads of 128 32 -> 17 us.
+// (o, gate and norm: of this lane's four columns)
 template <int L>
-__global__ __launch_bounds__(256) void delta_out_bf16x4_kernel(const float* __restrict__ o_raw, const bf16* __restrict__ gate,
-                                                               long long ld_gate, const float* __restrict__ norm_w, float eps,
-                                                               bf16* __restrict__ out, long long n_rows, int H, int silu_gate) {
-    const long long row = (long long)blockIdx.x * (256 / L) + threadIdx.x / L;
-    if (row >= n_rows) return;                         // (the L lanes of a row together)
-    const int c = (threadIdx.x & (L - 1)) * 4;
-    const long long t = row / H;
-    const int h = (int)(row - t * H);
-    const float4 o = *reinterpret_cast<const float4*>(o_raw + (size_t)row * (4 * L) + c);
-    const uint2 g2 = *reinterpret_cast<const uint2*>(gate + (size_t)t * ld_gate + (size_t)h * (4 * L) + c);
-    const float4 nw = *reinterpret_cast<const float4*>(norm_w + c);
+__device__ __forceinline__ void delta_out_quad(float4 o, uint2 g2, float4 nw, float eps, int silu_gate, bf16* to) {
     // elements l, l + 64, ... of a row lie 16 lanes apart; their squares are added first, in their order
     const float ov[4] = {o.x, o.y, o.z, o.w};
     float sq[4];
@@ -549,7 +541,121 @@ __global__ __launch_bounds__(256) void delta_out_bf16x4_kernel(const float* __re
     uint2 pk;
     pk.x = (uint32_t)f2bf_bits(y[0]) | ((uint32_t)f2bf_bits(y[1]) << 16);
     pk.y = (uint32_t)f2bf_bits(y[2]) | ((uint32_t)f2bf_bits(y[3]) << 16);
-    *reinterpret_cast<uint2*>(out + (size_t)row * (4 * L) + c) = pk;
+    *reinterpret_cast<uint2*>(to) = pk;
+}
+template <int L>
+__global__ __launch_bounds__(256) void delta_out_bf16x4_kernel(const float* __restrict__ o_raw, const bf16* __restrict__ gate,
+                                                               long long ld_gate, const float* __restrict__ norm_w, float eps,
+                                                               bf16* __restrict__ out, long long n_rows, int H, int silu_gate) {
+    const long long row = (long long)blockIdx.x * (256 / L) + threadIdx.x / L;
+    if (row >= n_rows) return;                         // (the L lanes of a row together)
+    const int c = (threadIdx.x & (L - 1)) * 4;
+    const long long t = row / H;
+    const int h = (int)(row - t * H);
+    delta_out_quad<L>(*reinterpret_cast<const float4*>(o_raw + (size_t)row * (4 * L) + c),
+                      *reinterpret_cast<const uint2*>(gate + (size_t)t * ld_gate + (size_t)h * (4 * L) + c),
+                      *reinterpret_cast<const float4*>(norm_w + c), eps, silu_gate, out + (size_t)row * (4 * L) + c);
+}
+
+// Steps in which every request brings one token, bfloat16: a workgroup per (request, head) with all V = 4 L columns of the state. Rules 0,
+// 1 and 3: the read-out is normed, gated and stored here, with the bits of the two kernels; rule 2: as it is. Few requests are bound by
+// the chain from the slot to the state and back, many by reading and writing the states. The walk's workgroups of 16 columns each
+// prepared the head's whole row (decays, unit vectors) for themselves, and had one row of a chunk of four. Microseconds, walk and
+// read-out / this, 32 heads of 128 x 128, rule 0, at 1, 8, 16 and 64 requests: 9.4 / 7.2, 24.7 / 13.3, 38 / 24, 120 / 86 (3.1 of the
+// 6.5 TB/s that a plain read reaches, read and written); 64 heads of 64 x 64 8.0 / 5.0, 18.5 / 7.4, 27.8 / 11.4, 93.6 / 35.4.
+template <int DPT, int L>
+__global__ __launch_bounds__(1024) void delta_one_kernel(
+    const bf16* __restrict__ qkv, long long ld_qkv, const bf16* __restrict__ b, long long ld_b, const bf16* __restrict__ ag, long long ld_ag,
+    const bf16* __restrict__ gate, long long ld_gate, const float* __restrict__ A_log, const float* __restrict__ dt_bias,
+    const float* __restrict__ norm_w, float eps, float* __restrict__ S, const int* __restrict__ slot_ids, bf16* __restrict__ out,
+    float* __restrict__ o_raw, int H, int G, int D, int RS, int rule, float rate) {
+    constexpr int V = 4 * L, PS = DPT + DR_PAD;
+    __shared__ __attribute__((aligned(16))) float k_s[8 * PS], q_s[8 * PS], g_s[8 * PS], o_s[V];
+    __shared__ float sums[2];
+    const int tid = threadIdx.x, NT = blockDim.x, lane = tid & 63, wave = tid >> 6, h = blockIdx.x, s = blockIdx.y, kvh = h / (H / G);
+    const int j = tid / RS, rp = tid % RS;
+    float* Sc = S + (((size_t)slot_ids[s] * H + h) * V + j) * D;
+    const bf16* row = qkv + (size_t)s * ld_qkv;
+    float st[DPT];
+#pragma unroll
+    for (int ii = 0; ii < DPT; ii += 4) {                      // (D % 4 == 0)
+        float4 v4 = make_float4(0.f, 0.f, 0.f, 0.f);
+        if (rp * DPT + ii < D) v4 = *reinterpret_cast<const float4*>(Sc + rp * DPT + ii);
+        st[ii] = v4.x; st[ii + 1] = v4.y; st[ii + 2] = v4.z; st[ii + 3] = v4.w;
+    }
+    const float vv = to_f(row[2 * G * D + h * V + j]);
+    const float neg_a = rule == 1 ? -rate : -expf(A_log[h]);
+    const float step = rule >= 2 ? dr_softplus_exact(to_f(ag[(size_t)s * ld_ag + h]) + dt_bias[h]) : 0.f;
+    const float beta = rule == 1 ? 1.f : rule == 2 ? step : dr_sigmoid(to_f(b[(size_t)s * ld_b + h]));
+    const float dec = rule >= 2 ? expf(neg_a * step) : 1.f;
+    const float q_scale = rule == 2 ? 1.f : 1.0f / sqrtf((float)D);
+    uint2 g2 = make_uint2(0, 0);
+    float4 nw = make_float4(0.f, 0.f, 0.f, 0.f);
+    if (rule != 2 && tid < L) {
+        g2 = *reinterpret_cast<const uint2*>(gate + (size_t)s * ld_gate + (size_t)h * V + 4 * tid);
+        nw = *reinterpret_cast<const float4*>(norm_w + 4 * tid);
+    }
+    for (int idx = tid; idx < 3 * RS * DPT; idx += NT) {
+        const int what = idx / (RS * DPT), i = idx - what * (RS * DPT), at = (i / DPT) * PS + (i % DPT);
+        if (what == 2) {
+            const float a_sign = rule == 1 ? -1.f : 1.f;
+            g_s[at] = rule >= 2 ? (i < D || rule == 3 ? dec : 1.f)
+                      : i < D ? dr_decay(neg_a, a_sign * (to_f(ag[(size_t)s * ld_ag + h * D + i]) + dt_bias[h * D + i])) : 1.f;
+        } else {
+            (what ? k_s : q_s)[at] = i < D ? to_f(row[(what ? G * D : 0) + kvh * D + i]) : 0.f;
+        }
+    }
+    __syncthreads();
+    if (wave < 2 && rule != 2) {                               // what makes k and q unit vectors
+        const float* x = wave ? q_s : k_s;
+        float ss = 0.f;
+        for (int i = lane; i < D; i += 64) {
+            const float v = x[(i / DPT) * PS + (i % DPT)];
+            ss = fmaf(v, v, ss);
+        }
+        ss = wave_sum(ss);
+        if (lane == 0) sums[wave] = wave ? (rule == 1 ? q_scale : q_scale / sqrtf(ss + 1e-6f)) : (rule == 1 ? 1.f : 1.0f / sqrtf(ss + 1e-6f));
+    }
+    __syncthreads();
+    const float sk = rule == 2 ? 1.f : sums[0], sq = rule == 2 ? 1.f : sums[1];
+    float kreg[DPT], a0 = 0.f, a1 = 0.f, a2 = 0.f, a3 = 0.f;
+#pragma unroll
+    for (int ii = 0; ii < DPT; ii += 4) {
+        const float4 k4 = *reinterpret_cast<const float4*>(k_s + rp * PS + ii), g4 = *reinterpret_cast<const float4*>(g_s + rp * PS + ii);
+        kreg[ii] = k4.x * sk; kreg[ii + 1] = k4.y * sk; kreg[ii + 2] = k4.z * sk; kreg[ii + 3] = k4.w * sk;
+        st[ii] *= g4.x; st[ii + 1] *= g4.y; st[ii + 2] *= g4.z; st[ii + 3] *= g4.w;
+        a0 = fmaf(st[ii], kreg[ii], a0);
+        a1 = fmaf(st[ii + 1], kreg[ii + 1], a1);
+        a2 = fmaf(st[ii + 2], kreg[ii + 2], a2);
+        a3 = fmaf(st[ii + 3], kreg[ii + 3], a3);
+    }
+    const float acc = rule == 1 || rule == 2 ? 0.f : dr_group_sum((a0 + a1) + (a2 + a3), RS);
+    const float u = beta * (vv - acc);
+    float o0 = 0.f, o1 = 0.f, o2 = 0.f, o3 = 0.f;
+#pragma unroll
+    for (int ii = 0; ii < DPT; ii += 4) {
+        const float4 q4 = *reinterpret_cast<const float4*>(q_s + rp * PS + ii);
+        st[ii] = fmaf(kreg[ii], u, st[ii]);
+        st[ii + 1] = fmaf(kreg[ii + 1], u, st[ii + 1]);
+        st[ii + 2] = fmaf(kreg[ii + 2], u, st[ii + 2]);
+        st[ii + 3] = fmaf(kreg[ii + 3], u, st[ii + 3]);
+        o0 = fmaf(st[ii], q4.x * sq, o0);
+        o1 = fmaf(st[ii + 1], q4.y * sq, o1);
+        o2 = fmaf(st[ii + 2], q4.z * sq, o2);
+        o3 = fmaf(st[ii + 3], q4.w * sq, o3);
+    }
+    const float o = dr_group_sum((o0 + o1) + (o2 + o3), RS);
+    if (rp == 0) {
+        if (rule == 2) o_raw[((size_t)s * H + h) * V + j] = o;
+        else o_s[j] = o;
+    }
+#pragma unroll
+    for (int ii = 0; ii < DPT; ii += 4)
+        if (rp * DPT + ii < D) *reinterpret_cast<float4*>(Sc + rp * DPT + ii) = make_float4(st[ii], st[ii + 1], st[ii + 2], st[ii + 3]);
+    if (rule == 2) return;                                     // (its read-outs are normed over other parts of a row)
+    __syncthreads();
+    if (tid < L)
+        delta_out_quad<L>(*reinterpret_cast<const float4*>(o_s + 4 * tid), g2, nw, eps, rule != 0, out + (size_t)s * H * V + (size_t)h * V + 4 * tid);
 }
 
 // How a head's state is spread: RS lanes (a power of two) of DPT rows each to a column, VB columns a workgroup.
@@ -656,6 +762,16 @@ static int delta_rule_launch(hipStream_t st, int DPT, dim3 grid, dim3 block, siz
     return ra_launch_status();
 }
 
+// Whether a step goes by delta_one_kernel: single tokens, heads of 64 or 128 columns.
+static bool delta_one_fits(int n_seqs, int T_tokens, int max_q_len, int D, int V, int RS, int DPT, int dtype) {
+    return dtype == RA_DTYPE_BF16 && max_q_len == 1 && T_tokens == n_seqs && D % 4 == 0 && RS == 8 && (DPT == 8 || DPT == 16) && (V == 64 || V == 128);
+}
+// 1: steps of single tokens go by delta_one_kernel, 0: by the kernels for any requests.
+extern "C" int ra_delta_rule_form(int D, int V, int dtype) {
+    int RS, DPT, VB;
+    return delta_rule_plan(D, V, &RS, &DPT, &VB) && delta_one_fits(1, 1, 1, D, V, RS, DPT, dtype);
+}
+
 // qkv [T, 2 G D + H V] rows; b: rows whose first H columns are the heads' beta (before the sigmoid); ag [T, H D + H V];
 // S fp32 [slots, H, V, D] (column by column); o_raw fp32 [T, H V] scratch; out [T, H V]; max_q_len: the longest request's rows.
 // (ag: the decay's projection, H D columns of rows ld_ag apart; gate: the output gate's, H V columns of rows ld_gate
@@ -676,6 +792,16 @@ static int delta_rule_run(const void* qkv, long long ld_qkv, const void* b, long
     if (TC <= 0 || max_q_len < 1) return RA_ERR_ARG;
     hipStream_t st = (hipStream_t)stream;
     int rc;
+    if (delta_one_fits(n_seqs, T_tokens, max_q_len, D, V, RS, DPT, dtype) && ((uintptr_t)S & 15) == 0 &&
+        (rule == 2 || (ld_gate % 4 == 0 && (((uintptr_t)gate | (uintptr_t)out) & 7) == 0 && ((uintptr_t)norm_w & 15) == 0))) {
+#define DELTA_ONE(DPT_, L_)                                                                                                                \
+    hipLaunchKernelGGL((delta_one_kernel<DPT_, L_>), dim3(H, n_seqs), dim3(V * RS), 0, st, (const bf16*)qkv, ld_qkv, (const bf16*)b, ld_b, \
+                       (const bf16*)ag, ld_ag, (const bf16*)gate, ld_gate, A_log, dt_bias, norm_w, eps, S, slot_ids, (bf16*)out, o_raw, H, G, D, RS, rule, rate)
+        if (DPT == 8) { if (V == 64) DELTA_ONE(8, 16); else DELTA_ONE(8, 32); }
+        else { if (V == 64) DELTA_ONE(16, 16); else DELTA_ONE(16, 32); }
+#undef DELTA_ONE
+        return ra_launch_status();
+    }
     // Requests of rc_min_rows rows and more go by chunks on the matrix cores, as far as the heads fit those kernels (in bf16;
     // the 32-bit mode, which checks are run in, keeps its one order of sums);
     // the others of the step, if there are any, walk their rows here.

@@ -137,6 +137,7 @@ def _declare(lib):
         "ra_stream_rows": [P, P, L, I, P],
         "ra_softcap": [P, F, L, P],
         "ra_delta_rule_fits": [I, I],
+        "ra_delta_rule_form": [I, I, I],
         "ra_token_side": [P, P, P, P, L, I, P, P, P, F, I, I, I, I, P],
         "ra_relu_sq": [P, L, I, P],
         "ra_add_bias": [P, P, L, I, I, P],
