@@ -296,3 +296,89 @@ extern "C" int ra_causal_conv_bias(const void* x, long long ld_x, const float* i
     return causal_conv_run(x, ld_x, in_bias, w, bias, tail, cu_q, slot_ids, out, ld_out, T_tokens, n_seqs, max_q_len, C, taps, flags,
                            dtype, stream);
 }
+
+// A pre-norm and the convolution behind it for steps in which every request brings one token, bfloat16: h += delta, x = h / rms(h) w rounded
+// to bfloat16, out = x + filter(x), one workgroup a request, four channels a thread; bit for bit what the norm's kernel (its thread
+// count, order of sums and rounding) and the one above give. Both are bound by their start and end (4.6 us each in a decode step); the tail and
+// the filter are asked for before the norm's sum is formed. Four taps, two kernels / this in a graph: a row of 2,048 5.6 / 3.7 us, of 4,096
+// 6.3 / 5.0, 64 rows of 4,096 7.5 / 5.6. Several tokens a request need the rows before a token's own normed, so they stay with two kernels.
+template <int TAPS>
+__global__ __launch_bounds__(1024) void norm_conv_one_kernel(float* __restrict__ h, const bf16* __restrict__ delta, const float* __restrict__ norm_w,
+                                                             float eps, const float* __restrict__ w, bf16* __restrict__ tail,
+                                                             const int* __restrict__ slot_ids, bf16* __restrict__ out, int H) {
+    __shared__ float scratch[16];
+    const int r = blockIdx.x, c = 4 * threadIdx.x;
+    const bool in = c < H;
+    float4 v = make_float4(0.f, 0.f, 0.f, 0.f), nw = v;
+    float taps[4][TAPS], win[TAPS - 1][4], ss = 0.f;
+    bf16* my_tail = tail + (size_t)slot_ids[r] * (TAPS - 1) * H + c;
+    if (in) {
+        float4* hr = reinterpret_cast<float4*>(h + (size_t)r * H + c);
+        v = *hr;
+        if (delta != nullptr) {
+            const uint2 d = *reinterpret_cast<const uint2*>(delta + (size_t)r * H + c);
+            v.x += __uint_as_float(d.x << 16);
+            v.y += __uint_as_float(d.x & 0xffff0000u);
+            v.z += __uint_as_float(d.y << 16);
+            v.w += __uint_as_float(d.y & 0xffff0000u);
+            *hr = v;
+        }
+        nw = *reinterpret_cast<const float4*>(norm_w + c);
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j) {
+            const uint2 t = *reinterpret_cast<const uint2*>(my_tail + (size_t)j * H);
+            win[j][0] = __uint_as_float(t.x << 16);
+            win[j][1] = __uint_as_float(t.x & 0xffff0000u);
+            win[j][2] = __uint_as_float(t.y << 16);
+            win[j][3] = __uint_as_float(t.y & 0xffff0000u);
+        }
+#pragma unroll
+        for (int i = 0; i < TAPS; ++i) {                       // four channels' filters lie side by side
+            const float4 t = reinterpret_cast<const float4*>(w + (size_t)c * TAPS)[i];
+            const float f[4] = {t.x, t.y, t.z, t.w};
+#pragma unroll
+            for (int k = 0; k < 4; ++k) taps[(4 * i + k) / TAPS][(4 * i + k) % TAPS] = f[k];
+        }
+        ss += v.x * v.x + v.y * v.y + v.z * v.z + v.w * v.w;
+    }
+    ss = block_sum(ss, scratch);
+    const float rstd = 1.0f / sqrtf(ss / (float)H + eps);
+    if (!in) return;
+    const float x[4] = {round_to<bf16>(v.x * rstd * nw.x), round_to<bf16>(v.y * rstd * nw.y), round_to<bf16>(v.z * rstd * nw.z),
+                        round_to<bf16>(v.w * rstd * nw.w)};
+    float y[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+        y[k] = 0.f;
+#pragma unroll
+        for (int j = 0; j < TAPS - 1; ++j) y[k] = fmaf(taps[k][j], win[j][k], y[k]);
+        y[k] = fmaf(taps[k][TAPS - 1], x[k], y[k]);
+        y[k] += x[k];
+    }
+    auto pack = [](const float (&f)[4]) {
+        return make_uint2((uint32_t)f2bf_bits(f[0]) | ((uint32_t)f2bf_bits(f[1]) << 16), (uint32_t)f2bf_bits(f[2]) | ((uint32_t)f2bf_bits(f[3]) << 16));
+    };
+    *reinterpret_cast<uint2*>(out + (size_t)r * H + c) = pack(y);
+#pragma unroll
+    for (int j = 0; j + 1 < TAPS - 1; ++j) *reinterpret_cast<uint2*>(my_tail + (size_t)j * H) = pack(win[j + 1]);
+    *reinterpret_cast<uint2*>(my_tail + (size_t)(TAPS - 2) * H) = pack(x);
+}
+
+extern "C" int ra_norm_conv_fits(int H, int taps) { return H > 0 && H % 4 == 0 && H <= 4096 && taps >= 2 && taps <= 4; }
+
+// h fp32 [rows, H], delta (may be null) and out bfloat16 [rows, H], w [H, taps], tail [slots, taps - 1, H]; row r is request r's one token.
+// h, norm_w and w 16-byte aligned, the others 8.
+extern "C" int ra_norm_conv_one(float* h, const void* delta, const float* norm_w, float eps, const float* w, void* tail, const int* slot_ids, void* out,
+                                int rows, int H, int taps, void* stream) {
+    if (rows <= 0) return RA_OK;
+    if (!ra_norm_conv_fits(H, taps) || (((uintptr_t)h | (uintptr_t)norm_w | (uintptr_t)w) & 15) != 0 ||
+        (((uintptr_t)delta | (uintptr_t)tail | (uintptr_t)out) & 7) != 0)
+        return RA_ERR_ARG;
+    const dim3 block(H <= 1024 ? 256 : H <= 2048 ? 512 : 1024);
+#define NORM_CONV(TAPS_)                                                                                                               \
+    hipLaunchKernelGGL(norm_conv_one_kernel<TAPS_>, dim3(rows), block, 0, (hipStream_t)stream, h, (const bf16*)delta, norm_w, eps, w,  \
+                       (bf16*)tail, slot_ids, (bf16*)out, H)
+    if (taps == 2) NORM_CONV(2); else if (taps == 3) NORM_CONV(3); else NORM_CONV(4);
+#undef NORM_CONV
+    return ra_launch_status();
+}

@@ -137,6 +137,8 @@ def _declare(lib):
         "ra_stream_rows": [P, P, L, I, P],
         "ra_softcap": [P, F, L, P],
         "ra_delta_rule_fits": [I, I],
+        "ra_norm_conv_fits": [I, I],
+        "ra_norm_conv_one": [P, P, P, F, P, P, P, P, I, I, I, P],
         "ra_delta_rule_form": [I, I, I],
         "ra_token_side": [P, P, P, P, L, I, P, P, P, F, I, I, I, I, P],
         "ra_relu_sq": [P, L, I, P],
@@ -851,6 +853,33 @@ class HipOps:
             _ptr(x), ld_x, _ptr(w), _ptr(tail), _ptr(step.cu_q), _ptr(step.slot_ids), _ptr(out), ld_out, T, step.n_seqs,
             step.max_q_len, C, taps, (1 if add_input else 0) | (2 if silu else 0), _code(x.dtype), self._stream()),
             "causal_conv")
+        return out
+
+    def norm_conv(self, h, delta, weight, eps, w, tail, step):
+        """causal_conv(add_rmsnorm(h, delta, weight, eps), w, tail, step, add_input=True) in one kernel, or None where the step or the sizes
+        are not its own: one token of every request, bfloat16 rows of up to 4,096, two to four taps."""
+        if tail.dtype != torch.bfloat16 or step.max_q_len != 1 or step.n_tokens != step.n_seqs or h.dim() != 2 or \
+                not self.lib.ra_norm_conv_fits(h.shape[1], w.shape[1]) or \
+                (h.data_ptr() | weight.data_ptr() | w.data_ptr()) % 16 or (tail.data_ptr() | (0 if delta is None else delta.data_ptr())) % 8:
+            return None
+        self._want(h, "residual stream", torch.float32, 2)
+        self._want(weight, "norm weight", torch.float32, 1)
+        self._want(w, "conv weight", torch.float32, 2)
+        self._want(tail, "conv tail", dims=3)
+        T, H = h.shape
+        taps = w.shape[1]
+        if delta is not None:
+            self._want(delta, "delta", torch.bfloat16, 2)
+            if tuple(delta.shape) != (T, H):
+                raise KernelError(f"norm_conv: delta {tuple(delta.shape)} does not match h {tuple(h.shape)}")
+        if T != step.n_tokens or weight.shape[0] != H or w.shape[0] != H or tuple(tail.shape[1:]) != (taps - 1, H):
+            raise KernelError(f"norm_conv: h {tuple(h.shape)}, norm weight {tuple(weight.shape)}, w {tuple(w.shape)}, tail {tuple(tail.shape)}, "
+                              f"step of {step.n_tokens}")
+        if max(step.slot_ids_host, default=0) >= tail.shape[0]:
+            raise KernelError("norm_conv: a request's slot lies beyond the tail's rows")
+        out = torch.empty(T, H, dtype=tail.dtype, device=self.device)
+        self._check(self.lib.ra_norm_conv_one(_ptr(h), _ptr(delta), _ptr(weight), float(eps), _ptr(w), _ptr(tail), _ptr(step.slot_ids), _ptr(out),
+                                              T, H, taps, self._stream()), "norm_conv")
         return out
 
     def _recurrence_room(self, step, T, H, D, V, rule, dtype):

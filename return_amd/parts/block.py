@@ -20,6 +20,7 @@ from __future__ import annotations
 
 import inspect
 
+from .conv import ResidualCausalConv
 from .runtime import Normed, NormSink, Pair, ResidualSink, Scaled, StreamRows, enter_stream
 
 
@@ -140,6 +141,10 @@ class ConvSideBlock:
     def _normed(norm, conv, h, pending, step, tails, tail_name):
         """What a sublayer reads: the norm of the stream (pending added first) and, if there is one, the
         convolution behind it."""
+        if conv is not None and type(conv) is ResidualCausalConv and hasattr(norm, "forward_conv"):
+            x = norm.forward_conv(h, pending, conv, step, tails[tail_name])
+            if x is not None:
+                return x
         x = norm.forward(h, pending)
         return x if conv is None else conv.forward(x, step, tails[tail_name])
 

@@ -66,6 +66,13 @@ class RMSNorm:
             self.rt.ops.add_rmsnorm(h, delta, self.weight, self.eps, out, out_rows)
         return out
 
+    def forward_conv(self, h, delta, conv, step, tail):
+        """conv.forward(self.forward(h, delta), step, tail) where the kernel set forms both at once, else None."""
+        ops = self.rt.ops
+        if not hasattr(ops, "norm_conv") or not (delta is None or isinstance(delta, torch.Tensor)):
+            return None
+        return ops.norm_conv(h, delta, self.weight, self.eps, conv.weight, tail, step)
+
 
 class LayerNorm:
     """y = (x - mean) / sqrt(variance + eps) * w (+ b with params bias: role "bias") over the last axis, the variance the
