@@ -186,17 +186,22 @@ __global__ __launch_bounds__(256 * KSPLIT) __attribute__((amdgpu_waves_per_eu(2)
     // what each thread moves per tile: its key row's pieces my_sub, my_sub + TPK, ... of K and of V
     uint4_t kreg[NLD], vreg[NLD];                        // native vectors: they stay in registers
     const int my_key = tid / TPK, my_sub = tid % TPK;
-    // cache row of key position kp (clamped into what this tile may read, so every address is valid)
+    // Where the row of key position kp (clamped into what this tile may read, so every address is valid) lies: its page's
+    // entry of the table, which is only asked for here, and what comes to it (row = page Hkv P + off). The entry is used a
+    // pass later: a use beside the load would wait for it there and with it for every load asked for before it, the rows of
+    // the tile after the next (32 heads of 128, 512 rows after 3,584: 73.3 us with that wait, 70.9 without).
     const int p_shift = (P & (P - 1)) == 0 ? __builtin_ctz(P) : -1;
-#define ROW_OF(kp)                                                                  \
-    ([&]() {                                                                        \
+    int page_next, off_next;
+#define LOOK_UP(kp)                                                                 \
+    {                                                                               \
         const int idx_ = min(max((kp), low_key), tile_last_pos) - start;            \
         const int pi_ = p_shift >= 0 ? (idx_ >> p_shift) : (idx_ / P);              \
-        return (pt[pi_] * Hkv + kvh) * P + (idx_ - pi_ * P);                        \
-    }())
-#define FETCH_ROW(row_)                                                             \
+        page_next = pt[pi_];                                                        \
+        off_next = kvh * P + (idx_ - pi_ * P);                                      \
+    }
+#define FETCH_ROW()                                                                 \
     {                                                                               \
-        const size_t base_ = (size_t)(row_) * D;                                    \
+        const size_t base_ = (size_t)(page_next * Hkv * P + off_next) * D;          \
         _Pragma("unroll") for (int i = 0; i < NLD; ++i) {                           \
             const int p_ = my_sub + TPK * i;                                        \
             if (p_ < LPR) {                                                         \
@@ -215,15 +220,14 @@ __global__ __launch_bounds__(256 * KSPLIT) __attribute__((amdgpu_waves_per_eu(2)
     }
     // group grp takes the key tiles grp, grp + KSPLIT, grp + 2 KSPLIT, ... counted from c_first
     constexpr int STEP = KSPLIT * BN;                    // from one tile of a group to its next
-    int row_next;                                        // row of this thread's key in the tile fetched next
     {
         const int u_mine = u_first + grp * BN;
-        const int r0 = ROW_OF(POS_OF(u_mine) + my_key);
-        row_next = ROW_OF(POS_OF(u_mine + STEP) + my_key);
-        FETCH_ROW(r0)
+        LOOK_UP(POS_OF(u_mine) + my_key)
+        FETCH_ROW()
+        LOOK_UP(POS_OF(u_mine + STEP) + my_key)
         STAGE_TO(0)
-        FETCH_ROW(row_next)                              // the group's second tile (or a repeat of valid rows if there is none)
-        row_next = ROW_OF(POS_OF(u_mine + 2 * STEP) + my_key);
+        FETCH_ROW()                                      // the group's second tile (or a repeat of valid rows if there is none)
+        LOOK_UP(POS_OF(u_mine + 2 * STEP) + my_key)
     }
     __syncthreads();
 
@@ -239,8 +243,8 @@ __global__ __launch_bounds__(256 * KSPLIT) __attribute__((amdgpu_waves_per_eu(2)
             // at the last barrier); then the tile after it is asked for
             STAGE_TO(cur ^ 1)
             if (POS_OF(u0 + 2 * STEP) <= tile_last_pos) {
-                FETCH_ROW(row_next)
-                row_next = ROW_OF(POS_OF(u0 + 3 * STEP) + my_key);
+                FETCH_ROW()
+                LOOK_UP(POS_OF(u0 + 3 * STEP) + my_key)
             }
         }
 
@@ -268,6 +272,21 @@ __global__ __launch_bounds__(256 * KSPLIT) __attribute__((amdgpu_waves_per_eu(2)
                     cs[qg][st] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, bq_tail[qg], cs[qg][st], 0, 0, 0);
             }
         }
+        // The first 32 keys' values come out of LDS while the softmax is formed: with two waves a SIMD a wave's own chain,
+        // products, softmax, products, is what takes the time (512 rows after 1,024 30.3 us without, 29.6 so; head size 256
+        // after 3,584 201 before all three of these, 167 now). No gain: the next tile's way into LDS between the products and
+        // the softmax, writes without bank conflicts, the two groups half a pass apart (15 % slower), tiles of 64 rows as four
+        // groups of two waves over 32 keys each (10 % slower).
+        auto values = [&](int b, int dt) {
+            // this lane's address as lane l' = n of its group: key 32b + 4g + n/4, columns 4(n%4)..+3
+            const uint16_t* vr = &v_cur[(32 * b + 4 * g + (n >> 2)) * VS + 4 * (n & 3)];
+            const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(vr + dt * 16));
+            const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(vr + 16 * VS + dt * 16));
+            return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+        };
+        short8_t v_first[D16];
+#pragma unroll
+        for (int dt = 0; dt < D16; ++dt) v_first[dt] = values(0, dt);
         MFMA_SETTLE();
         // p = 2^((s - m) * scale * log2(e)) with s the raw score and m the raw maximum of the row: one fused
         // multiply-add and one exponential a score (the scale is positive, so the maximum may be taken first).
@@ -300,17 +319,17 @@ __global__ __launch_bounds__(256 * KSPLIT) __attribute__((amdgpu_waves_per_eu(2)
             float s[BN / 16][4];
             float mx = -INFINITY;
             if (need_mask) {
+                // a row sees the keys from its window's first one to its own, and the kept ones up to itself; both bounds are
+                // formed once a row (a look at the window for every score made the prompt of 2,048 69.1 us in place of 65.7)
+                const int lowest = window > 0 ? max(low_key, pos_q[qg] - window + 1) : low_key;
+                [[maybe_unused]] const int kept_end = window > 0 ? min(keep_first, pos_q[qg] + 1) : 0;
 #pragma unroll
                 for (int st = 0; st < BN / 16; ++st) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         const int kpos = c0 + st * 16 + 4 * g + i;
-                        bool ok = kpos >= low_key && kpos <= pos_q[qg];
-                        if constexpr (XT != 0) {
-                            if (window > 0) ok = ok && (kpos > pos_q[qg] - window || kpos < keep_first);
-                        } else {
-                            if (window > 0) ok = ok && kpos > pos_q[qg] - window;
-                        }
+                        bool ok = kpos >= lowest && kpos <= pos_q[qg];
+                        if constexpr (XT != 0) ok = ok || (kpos >= low_key && kpos < kept_end);
                         s[st][i] = ok ? cs[qg][st][i] : -INFINITY;
                         mx = fmaxf(mx, s[st][i]);
                     }
@@ -371,13 +390,9 @@ __global__ __launch_bounds__(256 * KSPLIT) __attribute__((amdgpu_waves_per_eu(2)
         // ---- O^T += V^T P^T, 32 keys per MFMA; V^T through the transposing LDS read, once for every group
 #pragma unroll
         for (int b = 0; b < BN / 32; ++b) {
-            // this lane's address as lane l' = n of its group: key 32b + 4g + n/4, columns 4(n%4)..+3
-            const uint16_t* vr = &v_cur[(32 * b + 4 * g + (n >> 2)) * VS + 4 * (n & 3)];
 #pragma unroll
             for (int dt = 0; dt < D16; ++dt) {
-                const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(vr + dt * 16));
-                const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_short4_ptr)(vr + 16 * VS + dt * 16));
-                const short8_t both = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+                const short8_t both = b == 0 ? v_first[dt] : values(b, dt);
 #pragma unroll
                 for (int qg = 0; qg < QG; ++qg) {
                     acc[qg][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
@@ -394,7 +409,7 @@ __global__ __launch_bounds__(256 * KSPLIT) __attribute__((amdgpu_waves_per_eu(2)
 
 #undef FETCH_ROW
 #undef STAGE_TO
-#undef ROW_OF
+#undef LOOK_UP
 #undef POS_OF
 #undef K_S
 #undef V_S
