@@ -1333,8 +1333,12 @@ class HipOps:
         """Whether the tiled product forms silu(gate) * up of more than 64 rows (one kernel where the library's product and the SiLU-mul
         are two): up to 128 rows from 48 rows of W a CU on. Measured on MI355X, microseconds by it / by the two: 12,288 x 4,096 at 90, 256,
         536, 1,400, 2,048 and 2,804 rows 51 / 56, 69 / 72, 120 / 121, 242 / 261, 313 / 312, 458 / 521; 9,728 x 2,560 at 90, 536 and 2,048 34 / 36, 57 / 63, 192 /
-        226; 8,192 x 2,048 22 / 25, 42 / 48, 121 / 125; 3,072 x 4,096 28 / 26, 34 / 43, 93 / 92; 1,536 x 512 6.6 / 10, 7.1 / 13, 13 / 23."""
+        226; 8,192 x 2,048 22 / 25, 42 / 48, 121 / 125; 3,072 x 4,096 28 / 26, 34 / 43, 93 / 92; 1,536 x 512 6.6 / 10, 7.1 / 13, 13 / 23. Where the library's
+        tiles of 256 x 256 come to whole rounds over the CUs and K is long the two are at par here and the library ahead in a model, whose
+        products the card's power bounds (36 layers of 12,288 x 4,096 at 2,048 rows, the whole prompt: 27.35 ms / 27.03)."""
         if M <= 64 or self.own_gemm or (M <= 128 and 2 * I < 48 * self.cu_count and K > 1024):
+            return False
+        if K >= 4096 and M % 256 == 0 and I % 128 == 0 and (M // 256) * (I // 128) % self.cu_count == 0:
             return False
         return self.block_plan(M, 2 * I, K, True) is not None
 

@@ -82,6 +82,7 @@ def test_which_products_go_by_the_tiles():
                           (536, 32, 4096, False)]:
         assert ops.use_block(M, N, K) == want, (M, N, K)
     for M, I, K, want in [(64, 12288, 4096, False), (65, 12288, 4096, True), (128, 3072, 4096, False), (129, 3072, 4096, True), (65, 1536, 512, True),
+                          (2048, 12288, 4096, False), (2049, 12288, 4096, True), (2048, 12416, 4096, True), (2048, 8192, 2048, True),
                           (300, 100, 4096, False), (300, 104, 4096, True), (300, 104, 4104, False)]:
         assert ops.use_block_gated(M, I, K) == want, (M, I, K)
     for M, N, K, want in [(64, 2560, 9728, 0), (536, 2560, 9728, 4), (2048, 4096, 4096, 1), (536, 2047, 4096, 0), (536, 2048, 4100, 0)]:
