@@ -78,6 +78,12 @@ __global__ __launch_bounds__(256 * KSPLIT) __attribute__((amdgpu_waves_per_eu(2)
     constexpr int LPR = D / 8;                          // 16-byte pieces in one row
     constexpr int TPK = 256 / BN;                       // threads that share the loading of one key row
     constexpr int NLD = (LPR + TPK - 1) / TPK;          // pieces of K (and of V) per thread per tile
+    // Whether the first 32 keys' values leave LDS before the softmax (below): they are 4 D16 registers, held while it is formed. Not where
+    // they are a workgroup a CU less. Microseconds before there was any such hold / held / not held, 32 heads over 8: four requests of 1,024 after
+    // 1,024, head size 192 261 / 275 / 250, 176 295 / 327 / 296, 144 with capped scores 259 / 274 / 255; a prompt of 2,048, capped, windows of 300,
+    // head size 32 28.6 / 36.3 / 28.1. Nor at 208 (the four requests 355 / 335 / 326). 224 and 240 are 1 to 5 % faster held than not.
+    constexpr bool VALUES_EARLY =
+        !((D16 == 2 && QG == 2 && KSPLIT == 2 && XT != 2) || (D16 == 9 && XT != 0) || (D16 >= 11 && D16 <= 13));
 
     // Per group of four waves two tiles of K and of V: one is used while the next is written. With
     // KSPLIT == 2 a second group of four waves works on the same query rows and takes every other
@@ -285,8 +291,10 @@ __global__ __launch_bounds__(256 * KSPLIT) __attribute__((amdgpu_waves_per_eu(2)
             return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
         };
         short8_t v_first[D16];
+        if constexpr (VALUES_EARLY) {
 #pragma unroll
-        for (int dt = 0; dt < D16; ++dt) v_first[dt] = values(0, dt);
+            for (int dt = 0; dt < D16; ++dt) v_first[dt] = values(0, dt);
+        }
         MFMA_SETTLE();
         // p = 2^((s - m) * scale * log2(e)) with s the raw score and m the raw maximum of the row: one fused
         // multiply-add and one exponential a score (the scale is positive, so the maximum may be taken first).
@@ -392,7 +400,7 @@ __global__ __launch_bounds__(256 * KSPLIT) __attribute__((amdgpu_waves_per_eu(2)
         for (int b = 0; b < BN / 32; ++b) {
 #pragma unroll
             for (int dt = 0; dt < D16; ++dt) {
-                const short8_t both = b == 0 ? v_first[dt] : values(b, dt);
+                const short8_t both = VALUES_EARLY && b == 0 ? v_first[dt] : values(b, dt);
 #pragma unroll
                 for (int qg = 0; qg < QG; ++qg) {
                     acc[qg][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
