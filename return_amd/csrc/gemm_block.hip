@@ -292,7 +292,10 @@ static const BlockCost block_costs[] = {BLK_TILES(BLK_COST)};
 #define BLK_PIECES 8
 
 // The tile and the pieces of K (`least` to `most`) with the least time by the figures above: rounds of tiles over the CUs, a part-filled one
-// at 0.83 to 1 of a full one; several shares cost the kernel that adds them 0.64 us a million values each, written and read.
+// at 0.83 to 1 of a full one; several shares cost the kernel that adds them 0.64 us a million values each, written and read. One, two, four or
+// eight pieces: for these that kernel reads whole 16-byte pieces of all shares at once, other numbers go by one that reads 4 bytes after 4 (with the norm,
+// three pieces / the best of these, 1,200 rows of 4,096 x 12,288 129 / 120 us, 2,048 x 6,144 49 / 45; five / these 66 rows of 5,120 x 5,120 28.1 / 25.2, but
+// 256 rows of 5,120 x 25,600 98 / 107).
 // Returns tile + 16 pieces and the time, or -1 for what the kernel does not take.
 static int block_plan(int M, int N, int K, bool gated, int least, int most, int cus, int* workgroups, float* us) {
     if (M <= 0 || N <= 0 || K <= 0 || K % 64 != 0 || N % (gated ? 16 : 8) != 0 || cus <= 0) return -1;
@@ -302,7 +305,7 @@ static int block_plan(int M, int N, int K, bool gated, int least, int most, int 
         const BlockCost& k = block_costs[c];
         const long long tiles = (long long)((M + k.bm - 1) / k.bm) * ((N + k.bn - 1) / k.bn);
         for (int p = least; p <= most; ++p) {
-            if (K % (64 * p) != 0 || tiles * p > 0x7ffffff) continue;
+            if ((p & (p - 1)) != 0 || K % (64 * p) != 0 || tiles * p > 0x7ffffff) continue;
             const long long full = tiles * p / cus, rest = tiles * p % cus;
             const float rounds = (float)full + (rest ? 0.83f + 0.17f * (float)rest / (float)cus : 0.0f);
             const float t = 5.0f + rounds * ((float)(K / 64 / p) * k.step + k.ends) + (p > 1 ? 0.64e-6f * (2 * p - 1) * (float)M * (float)N : 0.0f);
@@ -317,7 +320,7 @@ static int block_plan(int M, int N, int K, bool gated, int least, int most, int 
 }
 
 // The choice for a product of these sizes: tile + 16 pieces, -1 where the kernel does not take it; its workgroups and its time as it is
-// reckoned (either may be null). pieces: of K, at most so many, or exactly so many where it is negative.
+// reckoned (either may be null). pieces: of K, at most so many, or exactly so many where it is negative (none but powers of two have a plan).
 extern "C" int ra_gemm_block_plan(int M, int N, int K, int gated, int pieces, int cus, int* workgroups, float* us) {
     float t = 0.0f;
     int n = 0;

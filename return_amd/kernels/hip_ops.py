@@ -1343,7 +1343,8 @@ class HipOps:
         return self.block_plan(M, 2 * I, K, True) is not None
 
     def use_block_residual(self, M, N, K):
-        """The pieces of K that the tiled product takes for the residual stream (1: a bfloat16 result), or 0 where another is the rule's.
+        """The pieces of K that the tiled product takes for the residual stream (1: a bfloat16 result; else 2, 4 or 8, which the norm's kernel has
+        forms for), or 0 where another is the rule's.
         Measured on MI355X with the norm that takes the result, microseconds by it / by the best of the library's one product and its
         batch over two or four pieces: 2,560 x 9,728 at 90, 256, 536, 1,024, 2,048 and 4,096 rows 24 / 25, 30 / 38, 42 / 50, 62 / 63, 105 / 105, 190 / 191; 2,560 x
         4,096 17 / 17, 20 / 26, 27 / 31, 36 / 40, 58 / 62, 97 / 98; 4,096 x 4,096 18 / 20, 23 / 25, 33 / 36, 50 / 49, 77 / 79, 132 / 132; 4,096 x 12,288 32 / 33,
