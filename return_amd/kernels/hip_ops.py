@@ -1215,9 +1215,11 @@ class HipOps:
     # rule's choice, tune_products replaces it where a measurement at load time says otherwise.
     ROW_STEPS = (1, 2, 4, 8, 12, 16, 24, 32, 48, 64)     # row counts at which products are measured
     # ... and beyond them the products for the residual stream only: with a few hundred rows (portions of
-    # prompts beside decoded tokens) the library gives a product with few result columns and many of K too
-    # few workgroups, and a batch over pieces of K is up to twice as fast (measured on MI355X, 512 rows:
-    # 8B down 84 -> 55 µs, 32B down 272 -> 122 µs)
+    # prompts beside decoded tokens) a product with few result columns and many of K makes too few tiles,
+    # and shares of it over pieces of K are up to twice as fast. Which number of pieces, and from where on the one
+    # product (by tiles or by the library) is the faster one, the rule tells to about 10 %: with the norm that takes the
+    # result, the rule's choice / the best one, 4,096 rows of 4,096 x 4,096 138 / 130 µs (library), of 8,192 x 8,192 462 / 422
+    # (library), 800 of 5,120 x 5,120 70 / 64 (two pieces), 90 of 2,560 x 4,096 17.4 / 15.6 (four), of 8,192 x 8,192 46 / 42 (eight)
     ROW_STEPS_RESIDUAL = (96, 128, 192, 256, 384, 512, 640, 768, 1024, 1536, 2048, 3072, 4096)
 
     def _rows_step(self, M, residual=False):
@@ -1681,8 +1683,12 @@ class HipOps:
             c.append("sweep")
         if self.lib.ra_gemm_rows_fits(M, N, K):
             c.append("rows")
-        if residual and self._library_bmm_fp32 and M > 16:
-            c += [f"split{n}" for n in self.SPLITS if K % (8 * n) == 0]
+        tiles = M > 64 and not self.own_gemm
+        if tiles and self.block_plan(M, 2 * N if gated else N, K, gated) is not None:
+            c.append("block")
+        if residual and M > 16:
+            c += [f"split{n}" for n in self.SPLITS if (self._library_bmm_fp32 and K % (8 * n) == 0) or
+                  (tiles and self.block_plan(M, N, K, False, -n) is not None)]
         return c
 
     def tune_products(self, products, max_rows=64, margin=0.93, max_rows_residual=0):

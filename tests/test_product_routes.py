@@ -177,3 +177,50 @@ def test_products_of_long_rows_that_the_library_forms_faster_are_its():
                           (16, 5120, 12288, "sweep"), (16, 5120, 8448, "sweep"), (16, 6144, 8192, "sweep"), (16, 3072, 10240, "sweep")]:
         assert ops.route_linear(M, N, K, BF) == want, (M, N, K)
         assert ops.route_linear(M, N, K, torch.float32) == "sweep", (M, N, K)
+
+
+def product_routes():
+    """The rules and candidates of products, on the host."""
+    from return_amd.kernels.hip_ops import load_library
+    ops = kernel_set("cpu")
+    ops.lib, ops.cu_count, ops.own_gemm, ops.product_plan = load_library(), 256, False, {}
+    ops._library_fp32_out = ops._library_bmm_fp32 = True
+    ops.gated_skinny_rows, ops._times = 8, {}
+    return ops
+
+
+@pytest.mark.parametrize("batches", [True, False])
+def test_the_rule_for_a_residual_product_is_among_what_is_measured(batches):
+    """Else nothing is measured, and the rule's choice stays whatever the other ways take."""
+    ops = product_routes()
+    ops._library_bmm_fp32 = batches                              # (whether the library has a batch with 32-bit results)
+    for N, K in [(4096, 12288), (4096, 4096), (2560, 9728), (2560, 4096), (5120, 25600), (5120, 5120), (5120, 8192), (2048, 2048), (2048, 8192),
+                 (1024, 3072), (512, 1536), (4096, 4160), (2048, 6152)]:
+        for rows in ops.ROW_STEPS + ops.ROW_STEPS_RESIDUAL:
+            ways = ops._candidates(rows, N, K, False, "residual")
+            assert ops.route_linear(rows, N, K, "residual") in ways and len(ways) == len(set(ways)), (rows, N, K, ways)
+            if rows > 64:
+                assert "library" in ways and ("block" in ways) == (K % 64 == 0), (rows, N, K, ways)
+    ops.own_gemm = True
+    assert not any(w == "block" for w in ops._candidates(512, 4096, 4096, False, "residual"))
+    # what a measurement has said is what is done, the one tiled product too
+    ops.own_gemm = False
+    for how in ("block", "library", "split8"):
+        ops.product_plan = {(512, 4096, 4096, False, "residual"): how}
+        assert ops.route_linear(400, 4096, 4096, "residual") == how
+    assert ops.route_linear(513, 4096, 4096, "residual") != "split8"
+
+
+def test_ways_of_many_rows_are_measured_beside_the_rule():
+    """Which ways _measure times, and that it follows them: here the tiled product in one piece takes half as long as all others."""
+    ops = product_routes()
+    seen = []
+
+    def fake(runs, weights, launches):
+        seen.append(sorted(runs))
+        return {how: 1.0 if how == "block" else 2.0 for how in runs}
+    ops._time_ways = fake
+    key = (512, 2048, 8192, False, "residual")
+    assert ops.route_linear(512, 2048, 8192, "residual").startswith("split")
+    assert ops._measure(key, [torch.zeros(2048, 8192, dtype=BF)], 1, 0.93) == "block"
+    assert seen == [["block", "library", "split2", "split4", "split8"]]
