@@ -1541,6 +1541,8 @@ class HipOps:
         if M == 0:
             return self.linear(x, w)
         how = self.route_linear(M, w.shape[0], K, "residual")
+        if how.startswith("split") and M > 64 and (x.data_ptr() | w.data_ptr()) % 16 and self.block_plan(M, w.shape[0], K, False) is not None:
+            how = "library"                       # (the rule cuts K for the tiled product, which wants whole 16 bytes: the one product then)
         if how.startswith("split"):
             return self._split_product(x, w, int(how[5:]))
         return self._linear_by(how, x, w, torch.bfloat16)

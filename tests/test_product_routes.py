@@ -224,3 +224,19 @@ def test_ways_of_many_rows_are_measured_beside_the_rule():
     assert ops.route_linear(512, 2048, 8192, "residual").startswith("split")
     assert ops._measure(key, [torch.zeros(2048, 8192, dtype=BF)], 1, 0.93) == "block"
     assert seen == [["block", "library", "split2", "split4", "split8"]]
+
+
+@pytest.mark.parametrize("batches", [True, False])
+@pytest.mark.parametrize("M,K", [(300, 1024), (100, 2048), (65, 8192)])
+def test_residual_products_of_operands_at_odd_places_are_the_librarys_one_product(batches, M, K):
+    """Sizes that the rule cuts into pieces of K, x 2 bytes off: also on a library without batches of 32-bit results."""
+    ops = product_routes()
+    ops._library_bmm_fp32 = batches
+    w = torch.randn(2048, K).to(BF)
+    x = torch.empty(M * K + 1, dtype=BF)[1:].view(M, K).copy_(torch.randn(M, K))
+    assert ops.route_linear(M, 2048, K, "residual").startswith("split") and x.data_ptr() % 16
+    y = ops.linear_residual(x, w)
+    assert torch.equal(y, x @ w.t())
+    ops.lib = types.SimpleNamespace(ra_gemm_block_bf16=lambda *a: ops.launched.append(a) or 0)
+    shares = ops._split_product(x[:, :].clone(), w, 2)           # (operands in place: by tiles)
+    assert len(ops.launched) == 1 and tuple(shares.tensor.shape) == (2, M, 2048)
