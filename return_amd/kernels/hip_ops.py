@@ -1316,20 +1316,44 @@ class HipOps:
         the sizes."""
         return _block_plan(M, N, K, 1 if gated else 0, pieces, self.cu_count)
 
+    def library_us(self, M, N, K):
+        """What the library's product of more than 64 rows takes by a reckoning that the rules below compare plans with: rounds of tiles of 256 x 256
+        over the CUs, a begun one at half and half of its share of a full one, 1.2 us a step of 64 columns, columns that are no whole 256s 15 %
+        more. Fitted to 5,157 products (66 to 4,096 rows, 46 widths of 512 to 24,576, K of 512 to 12,288, W from memory): the middle of what the library
+        takes over this is 1.1 to 1.2 (as it is for plans and what the tiled product takes), but now and then it takes 1.7 times as much as at a neighbouring
+        size (2,804 rows of 6,144 x 4,096 212 us, 3,000 rows 149; 2,804 of 10,240 181 and of 10,304 308), which no rule of sizes tells."""
+        tiles = -(-M // 256) * -(-N // 256)
+        begun = tiles % self.cu_count
+        rounds = tiles // self.cu_count + (0.5 + 0.5 * begun / self.cu_count if begun else 0.0)
+        return (K / 64 * 1.2 + 8.0) * rounds * (1.15 if N % 256 else 1.0)
+
+    def block_over_library(self, plan, M, N, K, share=0.95, behind=0.0):
+        """Whether a plan of the tiled product is taken in place of the library's product and a kernel behind it of `behind` microseconds: by what
+        both are reckoned with, the library's times `share`. A round of the library's of which at most a tenth is there counts for more (it is
+        0.65 of a full one: 264 tiles, the 2,804 rows above, 135 by the tiles here). With K of 8,192 and more and few tiles the library cuts K, which this
+        product does not: from 0.3 tiles of 256 x 256 a CU on (1,536 rows of 2,048 x 12,288 98 us, the library 87)."""
+        tiles = -(-M // 256) * -(-N // 256)
+        begun = tiles % self.cu_count
+        if K >= 8192 and tiles * 10 < 3 * self.cu_count:
+            return False
+        if tiles > self.cu_count and 0 < begun * 10 <= self.cu_count and K >= 2048:
+            share = 1.1
+        return plan[2] < share * self.library_us(M, N, K) + behind
+
     def use_block(self, M, N, K):
-        """Whether the tiled product forms a bfloat16 result of more than 64 rows. The library cuts K where tiles do not fill the chip,
-        this product has tiles of 64 x 128 at least: from 0.8 tiles a CU on. Beyond 1,536 rows of more than 4,096 columns the library has tiles
-        that fit multiples of 256 rows, and is the faster one on W of 40 Mi elements and more. Measured on MI355X, microseconds by it / by
-        the library, W from memory: 4,096 x 4,096 at 256, 420, 480, 800, 1,100 and 2,048 rows 29.2 / 22.8, 28.1 / 27.2, 27.9 / 28.7, 31.8 / 38.3,
-        42 / 48, 57.7 / 59.4; 6,144 x 2,560 at 256, 536, 1,200, 1,999 and 2,048 22.9 / 30.7, 24.6 / 29.4, 38.9 / 45.7, 57.6 / 57.5, 58.3 / 55.9; 6,144 x
-        4,096 at 2,048, 2,304, 2,804 and 3,000 87 / 82, 92 / 85, 132 / 212, 133 / 143; 10,496 x 4,096 at 1,999 and 2,112 146 / 202, 146 / 206; 12,288 x
-        4,096 at 256, 536, 1,400, 1,999 and 4,096 43.6 / 49.9, 58.8 / 57.3, 129 / 140, 170 / 162, 297 / 274; 1,536 x 512 5.5 to 12 / 6.4 to 15."""
+        """Whether the tiled product forms a bfloat16 result of more than 64 rows: where it has 0.8 tiles a CU (the library cuts K where its tiles are
+        fewer) and is the faster one by the reckoning. Over those 5,157 products this takes 2.1 % less time than the library alone (geometric mean); 246 are more
+        than 3 % slower by it and 22 more than 10 (by the number of rows, columns and elements alone 744 and 260). Measured on MI355X, microseconds
+        by the tiles / by the library, W from memory, those it takes: 6,144 x 2,560 at 536 and 1,280 rows 26 / 30, 43 / 46; 6,144 x 4,096 at 536 and 2,804
+        35 / 39, 135 / 212; 4,096 x 4,096 at 800 and 1,100 32 / 38, 42 / 48; 8,192 x 2,048 at 256 19 / 25; 8,256 x 2,048 at 2,804 93 / 100; 10,304 x 4,096 at 256
+        and 1,999 38 / 50, 156 / 197. Those it leaves: 8,192 x 2,048 at 1,280, 1,999 and 3,072 43 / 40, 62 / 52, 97 / 88; 12,288 x 2,048 at 1,280 61 / 52;
+        6,144 x 4,096 at 1,999 and 2,048 92 / 84, 95 / 84; 12,288 x 4,096 at 1,280, 2,048 and 3,072 111 / 96, 187 / 168, 250 / 240; 24,576 x 1,024 at 1,280 79 /
+        60. Left though faster here: 10,304 x 4,096 at 2,804 198 / 308, 8,192 x 4,096 158 / 267, 10,496 x
+        4,096 at 1,999 165 / 202, 256 rows of 6,144 x 4,096 32 / 41; taken though slower: 12,288 x 2,048 at 2,804 138 / 126."""
         if M <= 64 or self.own_gemm:
             return False
-        if M > 1536 and N > 4096 and (M % 256 == 0 or N * K >= 40 << 20):
-            return False
         plan = self.block_plan(M, N, K, False)
-        return plan is not None and plan[1] * 5 >= 4 * self.cu_count
+        return plan is not None and plan[1] * 5 >= 4 * self.cu_count and self.block_over_library(plan, M, N, K)
 
     def use_block_gated(self, M, I, K):
         """Whether the tiled product forms silu(gate) * up of more than 64 rows (one kernel where the library's product and the SiLU-mul
