@@ -1371,15 +1371,17 @@ class HipOps:
     def use_block_residual(self, M, N, K):
         """The pieces of K that the tiled product takes for the residual stream (1: a bfloat16 result; else 2, 4 or 8, which the norm's kernel has
         forms for), or 0 where another is the rule's.
-        Measured on MI355X with the norm that takes the result, microseconds by it / by the best of the library's one product and its
-        batch over two or four pieces: 2,560 x 9,728 at 90, 256, 536, 1,024, 2,048 and 4,096 rows 24 / 25, 30 / 38, 42 / 50, 62 / 63, 105 / 105, 190 / 191; 2,560 x
-        4,096 17 / 17, 20 / 26, 27 / 31, 36 / 40, 58 / 62, 97 / 98; 4,096 x 4,096 18 / 20, 23 / 25, 33 / 36, 50 / 49, 77 / 79, 132 / 132; 4,096 x 12,288 32 / 33,
-        42 / 48, 67 / 69, 100 / 104, 178 / 178, 323 / 315. Rows of fewer than 2,048 columns are added up too slowly for shares (512 x 1,536
+        Where the library's one product is the faster one by the reckoning it is taken: microseconds with the norm, by the tiles / by the library, 4,096 rows
+        of 4,096 x 4,096 138 / 130, of 8,192 x 8,192 462 / 422, 2,048 of 5,120 x 25,600 475 / 439, of 8,192 x 8,192 234 / 218 (now and then the library is far
+        off there: 2,804 of 8,192 x 8,192 340 / 553); measuring at load corrects both sides. Measured on MI355X with the norm that takes the result, microseconds by it / by the best of the library's one product and its
+        batch over two or four pieces: 2,560 x 9,728 at 90, 256, 536, 1,024 and 2,048 rows 24 / 25, 30 / 38, 42 / 50, 62 / 63, 105 / 105; 2,560 x
+        4,096 17 / 17, 20 / 26, 27 / 31, 36 / 40, 58 / 62; 4,096 x 4,096 18 / 20, 23 / 25, 33 / 36, 50 / 49, 77 / 79; 4,096 x 12,288 32 / 33,
+        42 / 48, 67 / 69, 100 / 104, 178 / 178. Rows of fewer than 2,048 columns are added up too slowly for shares (512 x 1,536
         at 333 rows 13 / 10): they go as plain results do."""
         if M <= 64 or self.own_gemm or N < 2048:
             return 0
         plan = self.block_plan(M, N, K, False, self.BLOCK_PIECES)
-        return 0 if plan is None else plan[0] >> 4
+        return 0 if plan is None or plan[2] >= self.library_us(M, N, K) else plan[0] >> 4
 
     def _block_product(self, x, w, gated, plan, out_dtype, act=0, limit=0.0, slope=0.0, bias=None):
         M, K = x.shape

@@ -89,7 +89,8 @@ def test_which_products_go_by_the_tiles():
                           (2048, 12288, 4096, False), (2049, 12288, 4096, True), (2048, 12416, 4096, True), (2048, 8192, 2048, True),
                           (300, 100, 4096, False), (300, 104, 4096, True), (300, 104, 4104, False)]:
         assert ops.use_block_gated(M, I, K) == want, (M, I, K)
-    for M, N, K, want in [(64, 2560, 9728, 0), (536, 2560, 9728, 4), (2048, 4096, 4096, 1), (536, 2047, 4096, 0), (536, 2048, 4100, 0)]:
+    for M, N, K, want in [(64, 2560, 9728, 0), (536, 2560, 9728, 4), (2048, 4096, 4096, 1), (536, 2047, 4096, 0), (536, 2048, 4100, 0),
+                          (2048, 4096, 12288, 1), (4096, 4096, 4096, 0), (2048, 8192, 8192, 0), (4096, 8192, 8192, 0), (2048, 5120, 25600, 0)]:
         assert ops.use_block_residual(M, N, K) == want, (M, N, K)
     ops.own_gemm = True
     assert not ops.use_block(536, 6144, 2560) and not ops.use_block_gated(536, 9728, 2560) and not ops.use_block_residual(536, 2560, 9728)
