@@ -1356,24 +1356,29 @@ class HipOps:
         return plan is not None and plan[1] * 5 >= 4 * self.cu_count and self.block_over_library(plan, M, N, K)
 
     def use_block_gated(self, M, I, K):
-        """Whether the tiled product forms silu(gate) * up of more than 64 rows (one kernel where the library's product and the SiLU-mul
-        are two): up to 128 rows from 48 rows of W a CU on. Measured on MI355X, microseconds by it / by the two: 12,288 x 4,096 at 90, 256,
-        536, 1,400, 2,048 and 2,804 rows 51 / 56, 69 / 72, 120 / 121, 242 / 261, 313 / 312, 458 / 521; 9,728 x 2,560 at 90, 536 and 2,048 34 / 36, 57 / 63, 192 /
-        226; 8,192 x 2,048 22 / 25, 42 / 48, 121 / 125; 3,072 x 4,096 28 / 26, 34 / 43, 93 / 92; 1,536 x 512 6.6 / 10, 7.1 / 13, 13 / 23. Where the library's
-        tiles of 256 x 256 come to whole rounds over the CUs and K is long the two are at par here and the library ahead in a model, whose
-        products the card's power bounds (36 layers of 12,288 x 4,096 at 2,048 rows, the whole prompt: 27.35 ms / 27.03)."""
-        if M <= 64 or self.own_gemm or (M <= 128 and 2 * I < 48 * self.cu_count and K > 1024):
+        """Whether the tiled product forms silu(gate) * up of more than 64 rows, one kernel where the library's product and the SiLU-mul are two
+        (the latter 8 us and 6 bytes an element at 8 TB/s): by the reckoning, and with K beyond 1,024 only from 0.6 tiles a CU on, for a gated product's K is
+        never cut. Measured on MI355X, microseconds by it / by the two, W from memory, those it takes: 12,288 x 4,096 at 300, 1,024, 1,400 and 2,804 rows 80 / 78,
+        194 / 185, 265 / 278, 505 / 514 (another day 449 / 504); 9,728 x 2,560 at 300, 536 and 2,804 49 / 53, 60 / 65, 265 / 278; 3,072 x 4,096 at 2,804 136 / 224; 8,192 x 2,048 at 300 and 2,804 32 / 36,
+        181 / 198; 3,072 x 4,096 at 536 35 / 44; 1,024 x 4,096 at 1,000 29 / 31; 256 x 512 and 256 x 1,024 at 300 7.0 / 9.2, 9.1 / 11. Those it leaves: 104 x
+        4,096 at 300 20 / 14; 512 x 12,288 at 300 82 / 42; 1,024 x 4,096 at 300 28 / 24; 768 x 8,192 at 300 50 / 29; 3,072 x 12,288 at 2,048 260 / 240. Of 2,719
+        products measured 91 are more than 3 % slower by it and two more than 10, and 11 % of the time is saved (geometric mean).
+        2,048 rows of 12,288 x 4,096, where the library's tiles of 256 x 256 come to whole rounds, are at par alone (313 / 312; 4,096 669 / 602), and in
+        a model, whose products the card's power bounds, the library is ahead: whole prompts, the two in turn, 14 times each, 36 layers at 2,048 rows 27.05 to
+        27.24 ms / 26.53 to 26.82, 12 layers at 4,096 18.03 to 18.24 / 17.74 to 17.97, at 2,048 9.26 to 9.34 / 9.12 to 9.37."""
+        if M <= 64 or self.own_gemm:
             return False
-        if K >= 4096 and M % 256 == 0 and I % 128 == 0 and (M // 256) * (I // 128) % self.cu_count == 0:
+        plan = self.block_plan(M, 2 * I, K, True)
+        if plan is None or (K > 1024 and plan[1] * 5 < 3 * self.cu_count):
             return False
-        return self.block_plan(M, 2 * I, K, True) is not None
+        return self.block_over_library(plan, M, 2 * I, K, share=1.0, behind=8.0 + 6e-6 / 8 * M * I)
 
     def use_block_residual(self, M, N, K):
         """The pieces of K that the tiled product takes for the residual stream (1: a bfloat16 result; else 2, 4 or 8, which the norm's kernel has
         forms for), or 0 where another is the rule's.
         Where the library's one product is the faster one by the reckoning it is taken: microseconds with the norm, by the tiles / by the library, 4,096 rows
         of 4,096 x 4,096 138 / 130, of 8,192 x 8,192 462 / 422, 2,048 of 5,120 x 25,600 475 / 439, of 8,192 x 8,192 234 / 218 (now and then the library is far
-        off there: 2,804 of 8,192 x 8,192 340 / 553); measuring at load corrects both sides. Measured on MI355X with the norm that takes the result, microseconds by it / by the best of the library's one product and its
+        off there: 2,804 of 8,192 x 8,192 340 / 553); measuring at load corrects both sides. By it / by the best of the library's one product and its
         batch over two or four pieces: 2,560 x 9,728 at 90, 256, 536, 1,024 and 2,048 rows 24 / 25, 30 / 38, 42 / 50, 62 / 63, 105 / 105; 2,560 x
         4,096 17 / 17, 20 / 26, 27 / 31, 36 / 40, 58 / 62; 4,096 x 4,096 18 / 20, 23 / 25, 33 / 36, 50 / 49, 77 / 79; 4,096 x 12,288 32 / 33,
         42 / 48, 67 / 69, 100 / 104, 178 / 178. Rows of fewer than 2,048 columns are added up too slowly for shares (512 x 1,536

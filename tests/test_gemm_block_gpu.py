@@ -85,9 +85,11 @@ def test_which_products_go_by_the_tiles():
                           (2804, 8256, 2048, True), (256, 10304, 4096, True), (1999, 10304, 4096, True), (1999, 10240, 4096, False),
                           (1536, 2048, 12288, False), (1536, 2048, 8184, False), (536, 6144, 2568, False), (536, 6140, 2560, False), (536, 32, 4096, False)]:
         assert ops.use_block(M, N, K) == want, (M, N, K)
-    for M, I, K, want in [(64, 12288, 4096, False), (65, 12288, 4096, True), (128, 3072, 4096, False), (129, 3072, 4096, True), (65, 1536, 512, True),
-                          (2048, 12288, 4096, False), (2049, 12288, 4096, True), (2048, 12416, 4096, True), (2048, 8192, 2048, True),
-                          (300, 100, 4096, False), (300, 104, 4096, True), (300, 104, 4104, False)]:
+    for M, I, K, want in [(64, 12288, 4096, False), (65, 1536, 512, True), (300, 12288, 4096, True), (1024, 12288, 4096, True), (1400, 12288, 4096, True),
+                          (2048, 12288, 4096, False), (4096, 12288, 4096, False), (2804, 12288, 4096, True), (536, 9728, 2560, True), (2804, 9728, 2560, True),
+                          (300, 8192, 2048, True), (2804, 8192, 2048, True), (128, 3072, 4096, False), (536, 3072, 4096, True), (1000, 1024, 4096, True),
+                          (300, 256, 512, True), (300, 256, 1024, True), (300, 104, 4096, False), (300, 512, 12288, False), (300, 1024, 4096, False),
+                          (300, 768, 8192, False), (2048, 3072, 12288, False), (300, 104, 512, True), (300, 100, 512, False), (300, 104, 520, False)]:
         assert ops.use_block_gated(M, I, K) == want, (M, I, K)
     for M, N, K, want in [(64, 2560, 9728, 0), (536, 2560, 9728, 4), (2048, 4096, 4096, 1), (536, 2047, 4096, 0), (536, 2048, 4100, 0),
                           (2048, 4096, 12288, 1), (4096, 4096, 4096, 0), (2048, 8192, 8192, 0), (4096, 8192, 8192, 0), (2048, 5120, 25600, 0)]:
