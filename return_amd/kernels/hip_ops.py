@@ -1660,10 +1660,13 @@ class HipOps:
             self._check(self.lib.ra_gemm_sweep_act_bf16(_ptr(x), _ptr(w), _ptr(out), M, N, K, 1 if gated else 0, self.cu_count, act, limit, slope,
                                                         _ptr(bias), self._stream()), "gemm_sweep_act")
             return out
-        # (the row kernel's time is in the bargain, so the library's large tiles have no edge: use_block's lines for many rows do not count)
+        # The row kernel's time is in the bargain, 3 us and 4 bytes an element at 6 TB/s. Microseconds of the tiles / of the library's product and squared
+        # ReLU, 12,288 x 4,096 at 300, 1,500, 2,304 and 3,072 rows 49 / 58, 147 / 164, 204 / 191, 251 / 264; 4,096 x 12,288 at 512 and 1,024 89 / 85, 114 / 121; 8,192 x
+        # 2,048 at 256 and 2,048 19 / 29, 63 / 65: of 144 measured (with biases too) none that is taken is more than 3 % slower, by the number of tiles alone seven.
         if M > 64 and not self.own_gemm and (x.data_ptr() | w.data_ptr() | (bias.data_ptr() if bias is not None else 0)) % 16 == 0:
             plan = self.block_plan(M, w.shape[0], K, gated)
-            if plan is not None and (self.use_block_gated(M, N, K) if gated else plan[1] * 5 >= 4 * self.cu_count):
+            if plan is not None and (self.use_block_gated(M, N, K) if gated else plan[1] * 5 >= 4 * self.cu_count and
+                                     self.block_over_library(plan, M, N, K, behind=3.0 + 4e-6 / 6 * M * N)):
                 return self._block_product(x, w, gated, plan[0], x.dtype, act, limit, slope, bias)
         return None
 

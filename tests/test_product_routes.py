@@ -240,3 +240,26 @@ def test_residual_products_of_operands_at_odd_places_are_the_librarys_one_produc
     ops.lib = types.SimpleNamespace(ra_gemm_block_bf16=lambda *a: ops.launched.append(a) or 0)
     shares = ops._split_product(x[:, :].clone(), w, 2)           # (operands in place: by tiles)
     assert len(ops.launched) == 1 and tuple(shares.tensor.shape) == (2, M, 2048)
+
+
+class Noted:
+    """The library with entries that note their calls in place of launching."""
+
+    def __init__(self, *entries):
+        from return_amd.kernels.hip_ops import load_library
+        self.lib, self.entries, self.calls = load_library(), entries, []
+
+    def __getattr__(self, name):
+        if name in self.entries:
+            return lambda *a: self.calls.append(name) or 0
+        return getattr(self.lib, name)
+
+
+def test_products_with_a_row_kernel_behind_go_by_the_tiles_where_the_two_kernels_take_longer():
+    """(rows, columns, K) on either side of the line; the figures stand at the rule."""
+    ops = product_routes()
+    for M, N, K, one in [(1500, 12288, 4096, True), (3072, 12288, 4096, True), (2304, 12288, 4096, False), (256, 8192, 2048, True), (2048, 8192, 2048, True),
+                         (512, 4096, 12288, False), (256, 12288, 4096, False)]:
+        ops.lib = Noted("ra_gemm_block_bf16")
+        x, w = torch.empty(M, K, dtype=BF), torch.empty(N, K, dtype=BF)
+        assert (ops._act_by(x, w, False, 2, 0.0, 0.0, None) is not None) == one == (ops.lib.calls == ["ra_gemm_block_bf16"]), (M, N, K)
