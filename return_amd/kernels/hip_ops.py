@@ -1655,7 +1655,8 @@ class HipOps:
             self._want(bias, "bias", torch.float32, 1)
             if bias.shape[0] != w.shape[0]:
                 raise KernelError(f"product: bias {tuple(bias.shape)} for weight {tuple(w.shape)}")
-        if M <= 16 and (self.use_sweep(M, N, K, True) if gated else self.route_linear(M, N, K, torch.bfloat16) == "sweep"):
+        if M <= 16 and (self.use_sweep(M, N, K, True) and self._sweep_measured(M, w.shape[0], K) if gated
+                        else self.route_linear(M, N, K, torch.bfloat16) == "sweep"):
             out = torch.empty(M, N, dtype=x.dtype, device=self.device)
             self._check(self.lib.ra_gemm_sweep_act_bf16(_ptr(x), _ptr(w), _ptr(out), M, N, K, 1 if gated else 0, self.cu_count, act, limit, slope,
                                                         _ptr(bias), self._stream()), "gemm_sweep_act")
@@ -1669,6 +1670,13 @@ class HipOps:
                                      self.block_over_library(plan, M, N, K, behind=3.0 + 4e-6 / 6 * M * N)):
                 return self._block_product(x, w, gated, plan[0], x.dtype, act, limit, slope, bias)
         return None
+
+    def _sweep_measured(self, M, N, K):
+        """Whether a measurement of the plain product leaves the sweep, with the row kernel inside, the faster way: another one may be ahead by what
+        that kernel takes of its own (4.6 us in a decode step), no more."""
+        key = (self._rows_step(M), N, K, False, torch.bfloat16)
+        how, times = self.product_plan.get(key), self._times.get(key, {})
+        return how in (None, "sweep") or (how in times and "sweep" in times and times["sweep"] - times[how] < 4.6e-6)
 
     def linear_bias(self, x, w, bias):
         """add_bias(linear(x, w), bias)."""

@@ -263,3 +263,15 @@ def test_products_with_a_row_kernel_behind_go_by_the_tiles_where_the_two_kernels
         ops.lib = Noted("ra_gemm_block_bf16")
         x, w = torch.empty(M, K, dtype=BF), torch.empty(N, K, dtype=BF)
         assert (ops._act_by(x, w, False, 2, 0.0, 0.0, None) is not None) == one == (ops.lib.calls == ["ra_gemm_block_bf16"]), (M, N, K)
+
+
+def test_a_measured_way_is_left_only_where_the_row_kernel_makes_up_for_it():
+    """Gated products of few rows with a bias or a clamp behind: the plain product as it was measured, its times in microseconds."""
+    key, x, w = (8, 24576, 4096, False, BF), torch.empty(6, 4096, dtype=BF), torch.empty(24576, 4096, dtype=BF)
+    for plan, times, one in [({}, {}, True), ({key: "sweep"}, {}, True), ({key: "library"}, {"sweep": 40.0, "library": 30.0}, False),
+                             ({key: "library"}, {"sweep": 40.0, "library": 36.5}, True), ({key: "library"}, {"library": 30.0}, False),
+                             ({key: "library"}, {}, False)]:
+        ops = product_routes()
+        ops.lib, ops.product_plan, ops._times = Noted("ra_gemm_sweep_act_bf16"), plan, {key: {how: t * 1e-6 for how, t in times.items()}}
+        for act, bias in ((1, None), (0, torch.empty(24576))):
+            assert (ops._act_by(x, w, True, act, 7.0, 1.702, bias) is not None) == one, (plan, times)
