@@ -21,6 +21,7 @@ from __future__ import annotations
 import inspect
 
 from .conv import ResidualCausalConv
+from .norm import RMSNorm
 from .runtime import Normed, NormSink, Pair, ResidualSink, Scaled, StreamRows, enter_stream
 
 
@@ -141,7 +142,7 @@ class ConvSideBlock:
     def _normed(norm, conv, h, pending, step, tails, tail_name):
         """What a sublayer reads: the norm of the stream (pending added first) and, if there is one, the
         convolution behind it."""
-        if conv is not None and type(conv) is ResidualCausalConv and hasattr(norm, "forward_conv"):
+        if type(conv) is ResidualCausalConv and type(norm) is RMSNorm:       # (not a part derived from one, which may form something else)
             x = norm.forward_conv(h, pending, conv, step, tails[tail_name])
             if x is not None:
                 return x

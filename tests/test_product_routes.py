@@ -275,3 +275,31 @@ def test_a_measured_way_is_left_only_where_the_row_kernel_makes_up_for_it():
         ops.lib, ops.product_plan, ops._times = Noted("ra_gemm_sweep_act_bf16"), plan, {key: {how: t * 1e-6 for how, t in times.items()}}
         for act, bias in ((1, None), (0, torch.empty(24576))):
             assert (ops._act_by(x, w, True, act, 7.0, 1.702, bias) is not None) == one, (plan, times)
+
+
+def test_a_norm_derived_from_the_rms_norm_forms_its_own_rows_before_a_convolution():
+    """The one kernel for a norm and the convolution behind it stands for these two parts, not for parts derived from them."""
+    from return_amd.parts.block import ConvSideBlock
+    from return_amd.parts.conv import ResidualCausalConv
+    from return_amd.parts.norm import RMSNorm
+    both = torch.zeros(2, 8)
+    rt = types.SimpleNamespace(vector32=lambda t: t, ops=types.SimpleNamespace(norm_conv=lambda *a: both))
+
+    class Doubled(RMSNorm):
+        def forward(self, h, delta=None, out_rows=None):
+            return 2 * h
+
+    class Shifted(ResidualCausalConv):
+        def forward(self, x, step, tail):
+            return x + 1
+
+    h, params = torch.randn(2, 8), {"size": 8, "eps": 1e-6, "taps": 4}
+    part = {cls: cls(params, {"weight": torch.ones(8, 4) if issubclass(cls, ResidualCausalConv) else torch.ones(8)}, rt)
+            for cls in (RMSNorm, Doubled, ResidualCausalConv, Shifted)}
+
+    def formed(norm, conv):
+        return ConvSideBlock._normed(part[norm], part[conv] if conv else None, h, None, None, {"tail": None}, "tail")
+    assert formed(RMSNorm, ResidualCausalConv) is both
+    assert torch.equal(formed(Doubled, Shifted), 2 * h + 1) and torch.equal(formed(Doubled, None), 2 * h)
+    part[ResidualCausalConv].forward = lambda x, step, tail: x - 1
+    assert torch.equal(formed(Doubled, ResidualCausalConv), 2 * h - 1)
