@@ -46,6 +46,35 @@ def test_every_tile_at_its_edges(ops, tile, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("tile,M,N", [(11, 64 * 13 - 5, 128 * 5 + 8), (11, 64 * 9, 128 * 3), (10, 96 * 11 - 1, 128 * 4 - 8), (6, 256 * 9 - 7, 128 * 2 + 16),
+                                      (5, 96 * 14 - 90, 256 + 8), (0, 256 * 10 - 255, 256 * 2), (11, 64 * 8, 128 * 3 + 8)])
+def test_every_tile_of_many_is_formed_once(ops, tile, M, N):
+    """Up to eight tiles of rows, and more, which go by fours with a shorter last run; the workgroups no whole number an XCD; one, three and five
+    pieces of K of several steps each, fewer and more than the stages. Results are written over what is no number."""
+    K = 64 * 3 * 5
+    x, w = rnd(M, K, dtype=BF, seed=M), rnd(N, K, dtype=BF, seed=N, scale=0.3)
+    want = x.double() @ w.double().t()
+
+    def run(gated, pieces, dtype):
+        y = torch.full((M, N // 2) if gated else (M, N) if dtype == 1 else (pieces, M, N), float("nan"), dtype=BF if dtype == 1 else torch.float32, device=x.device)
+        ops._check(ops.lib.ra_gemm_block_bf16(x.data_ptr(), w.data_ptr(), y.data_ptr(), M, N, K, gated, tile + 16 * pieces, dtype, 0, 0.0, 0.0, None,
+                                              ops._stream()), "")
+        return y.double()
+    assert bool(((run(0, 1, 1) - want).abs() <= bound(K, want)).all())
+    for pieces in (1, 3, 5):
+        y, step = run(0, pieces, 0), K // pieces
+        for i in range(pieces):
+            part = x[:, i * step:(i + 1) * step].double() @ w[:, i * step:(i + 1) * step].double().t()
+            torch.testing.assert_close(y[i], part, atol=2.0 ** -22 * step, rtol=1e-6)
+    if N % 16 == 0:
+        gu = want.float().to(BF).double()
+        g, u = gu[:, :N // 2], gu[:, N // 2:]
+        silu = g * torch.sigmoid(g)
+        lax = (g.abs() * 1.1 * u.abs() + (silu * u).abs()) * 2.0 ** -8 + (silu * u).abs() * 2.0 ** -8 + 2.0 ** -20 * K
+        assert bool(((run(1, 1, 1) - silu * u).abs() <= lax).all())
+
+
+@pytest.mark.gpu
 def test_products_go_by_the_tiles_and_stay_the_products(ops):
     """The public entries at sizes that the rules give to the tiled product; operands at odd places go to the library as before."""
     from return_amd.parts.runtime import Slabs
