@@ -1318,42 +1318,42 @@ class HipOps:
 
     def library_us(self, M, N, K):
         """What the library's product of more than 64 rows takes by a reckoning that the rules below compare plans with: rounds of tiles of 256 x 256
-        over the CUs, a begun one at half and half of its share of a full one, 1.2 us a step of 64 columns, columns that are no whole 256s 15 %
-        more. Fitted to 5,157 products (66 to 4,096 rows, 46 widths of 512 to 24,576, K of 512 to 12,288, W from memory): the middle of what the library
-        takes over this is 1.1 to 1.2 (as it is for plans and what the tiled product takes), but now and then it takes 1.7 times as much as at a neighbouring
-        size (2,804 rows of 6,144 x 4,096 212 us, 3,000 rows 149; 2,804 of 10,240 181 and of 10,304 308), which no rule of sizes tells."""
+        over the CUs, a begun one at half and half of its share of a full one, 1.2 us a step of 64 columns; where columns are no whole 256s, 1 us a million
+        results more. Fitted to 5,493 products (66 to 8,192 rows, 47 widths of 512 to 24,576, K of 64 to 12,288, W from memory): what the library takes
+        over this is 1.1 to 1.2 as a rule (as it is for plans and what the tiled product takes), but now and then it takes 1.7 times as much as at a
+        neighbouring size (2,804 rows of 6,144 x 4,096 212 us, 3,000 rows 149; 2,804 of 10,240 181 and of 10,304 308), which no rule of sizes tells."""
         tiles = -(-M // 256) * -(-N // 256)
         begun = tiles % self.cu_count
         rounds = tiles // self.cu_count + (0.5 + 0.5 * begun / self.cu_count if begun else 0.0)
-        return (K / 64 * 1.2 + 8.0) * rounds * (1.15 if N % 256 else 1.0)
+        return (K / 64 * 1.2 + 8.0) * rounds + (1e-6 * M * N if N % 256 else 0.0)
 
-    def block_over_library(self, plan, M, N, K, share=0.95, behind=0.0):
-        """Whether a plan of the tiled product is taken in place of the library's product and a kernel behind it of `behind` microseconds: by what
-        both are reckoned with, the library's times `share`. A round of the library's of which at most a tenth is there counts for more (it is
-        0.65 of a full one: 264 tiles, the 2,804 rows above, 135 by the tiles here). With K of 8,192 and more and few tiles the library cuts K, which this
-        product does not: from 0.2 tiles of 256 x 256 a CU on (1,536 rows of 2,048 x 12,288 98 us, the library 87)."""
+    def block_over_library(self, plan, M, N, K, behind):
+        """Whether a plan of the tiled product is taken in place of the library's product, by what both are reckoned with; `behind`: microseconds that the
+        library's way takes beside. A round of the library's of which at most a tenth is there counts for more (it is 0.65 of a full one: 264
+        tiles, the 2,804 rows above, 135 by the tiles here). With K of 8,192 and more and few tiles the library cuts K, which this product does
+        not: from 0.2 tiles of 256 x 256 a CU on (1,536 rows of 2,048 x 12,288 98 us, the library 87)."""
         tiles = -(-M // 256) * -(-N // 256)
         begun = tiles % self.cu_count
         if K >= 8192 and tiles * 5 < self.cu_count:
             return False
-        if tiles > self.cu_count and 0 < begun * 10 <= self.cu_count and K >= 2048:
-            share = 1.1
-        return plan[2] < share * self.library_us(M, N, K) + behind
+        more = 1.15 if tiles > self.cu_count and 0 < begun * 10 <= self.cu_count and K >= 2048 else 1.0
+        return plan[2] < more * self.library_us(M, N, K) + behind
 
     def use_block(self, M, N, K):
         """Whether the tiled product forms a bfloat16 result of more than 64 rows: where it has 0.8 tiles a CU (the library cuts K where its tiles are
-        fewer) and is the faster one by the reckoning. Over those 5,157 products this takes 2.2 % less time than the library alone (geometric mean); 262 are more
-        than 3 % slower by it and 27 more than 10 (by the number of rows, columns and elements alone 744 and 260). Measured on MI355X, microseconds
-        by the tiles / by the library, W from memory, those it takes: 6,144 x 2,560 at 536 and 1,280 rows 26 / 30, 43 / 46; 6,144 x 4,096 at 536 and 2,804
-        35 / 39, 135 / 212; 4,096 x 4,096 at 800 and 1,100 32 / 38, 42 / 48; 8,192 x 2,048 at 256 19 / 25; 8,256 x 2,048 at 2,804 93 / 100; 10,304 x 4,096 at 256
-        and 1,999 38 / 50, 156 / 197. Those it leaves: 8,192 x 2,048 at 1,280, 1,999 and 3,072 43 / 40, 62 / 52, 97 / 88; 12,288 x 2,048 at 1,280 61 / 52;
-        6,144 x 4,096 at 1,999 and 2,048 92 / 84, 95 / 84; 12,288 x 4,096 at 1,280, 2,048 and 3,072 111 / 96, 187 / 168, 250 / 240; 24,576 x 1,024 at 1,280 79 /
-        60. Left though faster here: 10,304 x 4,096 at 2,804 198 / 308, 8,192 x 4,096 158 / 267, 10,496 x
-        4,096 at 1,999 165 / 202, 256 rows of 6,144 x 4,096 32 / 41; taken though slower: 12,288 x 2,048 at 2,804 138 / 126."""
+        fewer) and is the faster one by the reckoning, its results stored at 0.6 us a million more than the library's. Over those 5,493 products this takes
+        2.2 % less time than the library alone (geometric mean); 215 are more than 3 % slower by it and 20 more than 10 (by the number of rows, columns
+        and elements alone 817 and 319). Measured on MI355X, microseconds by the tiles / by the library, W from memory, those it takes: 6,144 x 2,560 at 536
+        rows 26 / 30; 6,144 x 4,096 at 536 and 2,804 35 / 39, 135 / 212; 4,096 x 4,096 at 800 and 1,100 32 / 38, 42 / 48; 8,192 x 2,048 at 256 19 / 25; 8,256 x
+        2,048 at 2,804 93 / 100, x 256 at 1,024 14 / 20, x 128 at 2,048 22 / 31; 10,304 x 4,096 at 256 and 1,999 38 / 50, 156 / 197. Those it leaves: 8,192 x
+        2,048 at 1,280, 1,999 and 3,072 43 / 40, 62 / 52, 97 / 88, x 128 at 2,048 18 / 13; 12,288 x 2,048 at 1,280 and 2,804 61 / 52, 138 / 126; 16,384 x 64 at 4,096 52 /
+        33; 6,144 x 4,096 at 1,999 and 2,048 92 / 84, 95 / 84; 12,288 x 4,096 at 1,280, 2,048 and 3,072 111 / 96, 187 / 168, 250 / 240; 24,576 x 1,024 at 1,280 79 /
+        60. Left though faster here: 10,304 x 4,096 at 2,804 198 / 308, 8,192 x 4,096 158 / 267, 10,496 x 4,096 at 1,999 165 / 202, 256 rows of 6,144 x 4,096
+        32 / 41; 6,144 x 2,560 at 1,280 43 / 46."""
         if M <= 64 or self.own_gemm:
             return False
         plan = self.block_plan(M, N, K, False)
-        return plan is not None and plan[1] * 5 >= 4 * self.cu_count and self.block_over_library(plan, M, N, K)
+        return plan is not None and plan[1] * 5 >= 4 * self.cu_count and self.block_over_library(plan, M, N, K, -0.6e-6 * M * N)
 
     def use_block_gated(self, M, I, K):
         """Whether the tiled product forms silu(gate) * up of more than 64 rows, one kernel where the library's product and the SiLU-mul are two
@@ -1371,7 +1371,7 @@ class HipOps:
         plan = self.block_plan(M, 2 * I, K, True)
         if plan is None or (K > 1024 and plan[1] * 5 < 3 * self.cu_count):
             return False
-        return self.block_over_library(plan, M, 2 * I, K, share=1.0, behind=8.0 + 6e-6 / 8 * M * I)
+        return self.block_over_library(plan, M, 2 * I, K, 8.0 + 6e-6 / 8 * M * I)
 
     def use_block_residual(self, M, N, K):
         """The pieces of K that the tiled product takes for the residual stream (1: a bfloat16 result; else 2, 4 or 8, which the norm's kernel has
@@ -1661,13 +1661,13 @@ class HipOps:
             self._check(self.lib.ra_gemm_sweep_act_bf16(_ptr(x), _ptr(w), _ptr(out), M, N, K, 1 if gated else 0, self.cu_count, act, limit, slope,
                                                         _ptr(bias), self._stream()), "gemm_sweep_act")
             return out
-        # The row kernel's time is in the bargain, 3 us and 4 bytes an element at 6 TB/s. Microseconds of the tiles / of the library's product and squared
+        # The row kernel's time is in the bargain, 3 us and 4 bytes an element at 6 TB/s (0.4 of its 0.67 us a million lost to slower stores). Microseconds of the tiles / of the library's product and squared
         # ReLU, 12,288 x 4,096 at 300, 1,500, 2,304 and 3,072 rows 49 / 58, 147 / 164, 204 / 191, 251 / 264; 4,096 x 12,288 at 512 and 1,024 89 / 85, 114 / 121; 8,192 x
         # 2,048 at 256 and 2,048 19 / 29, 63 / 65: of 144 measured (with biases too) none that is taken is more than 3 % slower, by the number of tiles alone seven.
         if M > 64 and not self.own_gemm and (x.data_ptr() | w.data_ptr() | (bias.data_ptr() if bias is not None else 0)) % 16 == 0:
             plan = self.block_plan(M, w.shape[0], K, gated)
             if plan is not None and (self.use_block_gated(M, N, K) if gated else plan[1] * 5 >= 4 * self.cu_count and
-                                     self.block_over_library(plan, M, N, K, behind=3.0 + 4e-6 / 6 * M * N)):
+                                     self.block_over_library(plan, M, N, K, 3.0 + (4 / 6 - 0.4) * 1e-6 * M * N)):
                 return self._block_product(x, w, gated, plan[0], x.dtype, act, limit, slope, bias)
         return None
 

@@ -106,13 +106,14 @@ def test_which_products_go_by_the_tiles():
     ops = kernel_set("cpu")
     ops.cu_count, ops.own_gemm = 256, False
     # (what was measured on either side stands at the rule)
-    for M, N, K, want in [(64, 8192, 2048, False), (65, 8192, 2048, False), (256, 8192, 2048, True), (256, 6144, 4096, False), (300, 6144, 4096, True),
-                          (536, 6144, 2560, True), (1280, 6144, 2560, True), (536, 6144, 4096, True), (1999, 6144, 4096, False), (2048, 6144, 4096, False),
+    for M, N, K, want in [(64, 8192, 2048, False), (256, 8192, 2048, True), (256, 6144, 4096, False), (300, 6144, 4096, True),
+                          (536, 6144, 2560, True), (1280, 6144, 2560, False), (536, 6144, 4096, True), (1999, 6144, 4096, False), (2048, 6144, 4096, False),
                           (2804, 6144, 4096, True), (384, 4096, 4096, False), (448, 4096, 4096, True), (800, 4096, 4096, True), (1100, 4096, 4096, True),
-                          (1280, 8192, 2048, False), (1999, 8192, 2048, False), (3072, 8192, 2048, False), (1280, 12288, 2048, False),
+                          (1280, 8192, 2048, False), (1999, 8192, 2048, False), (3072, 8192, 2048, False), (1280, 12288, 2048, False), (2804, 12288, 2048, False),
                           (1280, 12288, 4096, False), (2048, 12288, 4096, False), (3072, 12288, 4096, False), (1280, 24576, 1024, False),
-                          (2804, 8256, 2048, True), (256, 10304, 4096, True), (1999, 10304, 4096, True), (1999, 10240, 4096, False),
-                          (1536, 2048, 12288, False), (1536, 2048, 8184, False), (536, 6144, 2568, False), (536, 6140, 2560, False), (536, 32, 4096, False)]:
+                          (2804, 8256, 2048, True), (1024, 8256, 256, True), (2048, 8256, 128, True), (2048, 8192, 128, False), (4096, 16384, 64, False),
+                          (256, 10304, 4096, True), (1999, 10304, 4096, True), (1999, 10240, 4096, False), (1536, 2048, 12288, False), (1536, 2048, 8184, False),
+                          (536, 6144, 2568, False), (536, 6140, 2560, False), (536, 32, 4096, False)]:
         assert ops.use_block(M, N, K) == want, (M, N, K)
     for M, I, K, want in [(64, 12288, 4096, False), (65, 1536, 512, True), (300, 12288, 4096, True), (1024, 12288, 4096, True), (1400, 12288, 4096, True),
                           (2048, 12288, 4096, False), (4096, 12288, 4096, False), (2804, 12288, 4096, True), (536, 9728, 2560, True), (2804, 9728, 2560, True),
