@@ -1329,20 +1329,20 @@ class HipOps:
 
     def block_over_library(self, plan, M, N, K, behind):
         """Whether a plan of the tiled product is taken in place of the library's product, by what both are reckoned with; `behind`: microseconds that the
-        library's way takes beside. A round of the library's of which at most a tenth is there counts for more (it is 0.65 of a full one: 264
+        library's way takes beside. A round of the library's of which at most a fifth is there counts for more from K of 4,096 on (it is 0.65 to 0.8 of a full one: 264
         tiles, the 2,804 rows above, 135 by the tiles here). With K of 8,192 and more and few tiles the library cuts K, which this product does
         not: from 0.2 tiles of 256 x 256 a CU on (1,536 rows of 2,048 x 12,288 98 us, the library 87)."""
         tiles = -(-M // 256) * -(-N // 256)
         begun = tiles % self.cu_count
         if K >= 8192 and tiles * 5 < self.cu_count:
             return False
-        more = 1.15 if tiles > self.cu_count and 0 < begun * 10 <= self.cu_count and K >= 2048 else 1.0
+        more = 1.15 if tiles > self.cu_count and 0 < begun * 5 <= self.cu_count and K >= 4096 else 1.0
         return plan[2] < more * self.library_us(M, N, K) + behind
 
     def use_block(self, M, N, K):
         """Whether the tiled product forms a bfloat16 result of more than 64 rows: where it has 0.8 tiles a CU (the library cuts K where its tiles are
         fewer) and is the faster one by the reckoning, its results stored at 0.6 us a million more than the library's. Over those 5,493 products this takes
-        2.2 % less time than the library alone (geometric mean); 215 are more than 3 % slower by it and 20 more than 10 (by the number of rows, columns
+        2.3 % less time than the library alone (geometric mean); 221 are more than 3 % slower by it and 18 more than 10 (by the number of rows, columns
         and elements alone 817 and 319). Measured on MI355X, microseconds by the tiles / by the library, W from memory, those it takes: 6,144 x 2,560 at 536
         rows 26 / 30; 6,144 x 4,096 at 536 and 2,804 35 / 39, 135 / 212; 4,096 x 4,096 at 800 and 1,100 32 / 38, 42 / 48; 8,192 x 2,048 at 256 19 / 25; 8,256 x
         2,048 at 2,804 93 / 100, x 256 at 1,024 14 / 20, x 128 at 2,048 22 / 31; 10,304 x 4,096 at 256 and 1,999 38 / 50, 156 / 197. Those it leaves: 8,192 x
@@ -1362,7 +1362,7 @@ class HipOps:
         194 / 185, 265 / 278, 505 / 514 (another day 449 / 504); 9,728 x 2,560 at 300, 536 and 2,804 49 / 53, 60 / 65, 265 / 278; 3,072 x 4,096 at 2,804 136 / 224; 8,192 x 2,048 at 300 and 2,804 32 / 36,
         181 / 198; 3,072 x 4,096 at 536 35 / 44; 1,024 x 4,096 at 1,000 29 / 31; 256 x 512 and 256 x 1,024 at 300 7.0 / 9.2, 9.1 / 11. Those it leaves: 104 x
         4,096 at 300 20 / 14; 512 x 12,288 at 300 82 / 42; 1,024 x 4,096 at 300 28 / 24; 768 x 8,192 at 300 50 / 29; 3,072 x 12,288 at 2,048 260 / 240. Of 2,719
-        products measured 96 are more than 3 % slower by it and two more than 10, and 11 % of the time is saved (geometric mean).
+        products measured 98 are more than 3 % slower by it and two more than 10, and 11 % of the time is saved (geometric mean).
         2,048 rows of 12,288 x 4,096, where the library's tiles of 256 x 256 come to whole rounds, are at par alone (313 / 312; 4,096 669 / 602), and in
         a model, whose products the card's power bounds, the library is ahead: whole prompts, the two in turn, 14 times each, 36 layers at 2,048 rows 27.05 to
         27.24 ms / 26.53 to 26.82, 12 layers at 4,096 18.03 to 18.24 / 17.74 to 17.97, at 2,048 9.26 to 9.34 / 9.12 to 9.37."""
